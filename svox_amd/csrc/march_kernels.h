@@ -760,6 +760,8 @@ struct ReplaySpace {
     // > 0: the looks in a row after which a waiting wavefront of render_forward_split_kernel gives up, in place of
     // kSpinLimit (set by a debug flag, so that a test can see what a give-up leaves behind)
     int32_t spin_limit;
+    // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
+    unsigned int* give_ups;
 };
 
 // whether the workspace carries the stamp this launch expects
@@ -1664,9 +1666,6 @@ __device__ __forceinline__ void box_write(int32_t* at, int32_t value) {
     __hip_atomic_store(at, value, kBoxStoreOrder, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Wavefronts of render_forward_split_kernel that gave up waiting since the library was loaded (svox_give_up_count).
-__device__ unsigned int split_give_ups = 0;
-
 // (The density phase stays also where the marks of a launch say that every leaf they let through is shaded,
 // render_forward_kernel's kAllShaded: here the walk is the critical path, and the density read of a leaf brings the
 // last line of its record into L2 ahead of the coefficient reads.)
@@ -1756,7 +1755,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             const bool go = live && written - (taken & ~kEndedBit) < kRing;
             if (!__any(go)) {   // every ring is full: the shading is behind
                 if (++spins > spin_limit) {
-                    if (lane == 0) atomicAdd(&split_give_ups, 1u);
+                    if (lane == 0) atomicAdd(ws.give_ups, 1u);
                     break;
                 }
                 __builtin_amdgcn_s_sleep(1);
@@ -1819,7 +1818,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                 if constexpr (kNoted) {
                     if (active) notes.give_up(r.dscale);
                 }
-                if (lane == 0) atomicAdd(&split_give_ups, 1u);
+                if (lane == 0) atomicAdd(ws.give_ups, 1u);
                 break;
             }
             __builtin_amdgcn_s_sleep(1);

@@ -1,0 +1,129 @@
+// march_launch.h -- the launches of the wavefront-per-tile march kernels, one class per policy and ray source.
+//
+// The kernels of march_kernels.h are templates over the record's format and basis size.  Every policy is compiled in
+// a translation unit of its own (march_policy.hip, once per format and basis size: build.py), so that a build takes
+// as long as its slowest policy and not as long as their sum; svox_hip.hip picks the policy at run time
+// (SVOX_DISPATCH_OCTREE) and calls these functions.
+#pragma once
+
+#include "march_kernels.h"
+
+namespace svox {
+
+template <class P, class Source>
+struct MarchLaunch {
+    static void forward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                        const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool split, bool accum, bool refill,
+                        bool all_shaded);
+    static void noting(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                       const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out, bool split,
+                       bool refill);
+    static void backward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                         const SvoxRenderOptions& opt, const float* grad_out, float* grad_data, const ReplaySpace& ws,
+                         bool refill, bool second_only);
+    static void replay_backward(dim3 blocks, hipStream_t stream, const Source& src, const SvoxRenderOptions& opt,
+                                const float* grad_out, float* grad_data, const ReplaySpace& ws, int ray_shift,
+                                int march1_known, const Lobes& lobes);
+    static void se_grad(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                        const SvoxRenderOptions& opt, const float* color_ref, float* color_out, float* grad, float* hess,
+                        const unsigned long long* only, bool refill);
+    static void replay_se_grad(dim3 blocks, hipStream_t stream, const Source& src, const SvoxRenderOptions& opt,
+                               const float* color_ref, float* color_out, float* grad, float* hess, const ReplaySpace& ws,
+                               int ray_shift, const Lobes& lobes);
+};
+
+#ifdef SVOX_INSTANTIATE_POLICY
+template <class P, class Source>
+void MarchLaunch<P, Source>::forward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                                     const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool split, bool accum,
+                                     bool refill, bool all_shaded) {
+    const float* const no_grad = nullptr;
+#define SVOX_FORWARD(ACCUM, REFILL, ALL)                                                                              \
+    hipLaunchKernelGGL((render_forward_kernel<P, Source, ACCUM, REFILL, false, false, ALL>), blocks,                  \
+                       dim3(kMarchThreads), 0, stream, tr, src, opt, out, ws, no_grad)
+    if (split)
+        hipLaunchKernelGGL((render_forward_split_kernel<P, Source, false>), blocks, dim3(kSplitThreads), 0, stream, tr, src,
+                           opt, out, ws, no_grad);
+    else if (accum)
+        SVOX_FORWARD(true, true, false);   // (accumulation is an analysis pass: one variant is enough)
+    else if (refill && all_shaded)
+        SVOX_FORWARD(false, true, true);
+    else if (refill)
+        SVOX_FORWARD(false, true, false);
+    else if (all_shaded)
+        SVOX_FORWARD(false, false, true);
+    else
+        SVOX_FORWARD(false, false, false);
+#undef SVOX_FORWARD
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                                    const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out,
+                                    bool split, bool refill) {
+#define SVOX_NOTING(THREADS, ...) \
+    hipLaunchKernelGGL((__VA_ARGS__), blocks, dim3(THREADS), 0, stream, tr, src, opt, out, ws, grad_out)
+    if (split && grad_out)
+        SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, true>);
+    else if (split)
+        SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, false>);
+    else if (refill && grad_out)
+        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
+    else if (refill)
+        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, false>);
+    else if (grad_out)
+        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, true>);
+    else
+        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, false>);
+#undef SVOX_NOTING
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::backward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                                      const SvoxRenderOptions& opt, const float* grad_out, float* grad_data,
+                                      const ReplaySpace& ws, bool refill, bool second_only) {
+#define SVOX_BACKWARD(REFILL, MODE)                                                                                   \
+    hipLaunchKernelGGL((render_backward_kernel<P, Source, REFILL, MODE>), blocks, dim3(kMarchThreads), 0, stream, tr, \
+                       src, opt, grad_out, grad_data, ws)
+    if (refill && second_only)
+        SVOX_BACKWARD(true, kBackwardSecond);
+    else if (refill)
+        SVOX_BACKWARD(true, kBackwardPlain);
+    else if (second_only)
+        SVOX_BACKWARD(false, kBackwardSecond);
+    else
+        SVOX_BACKWARD(false, kBackwardPlain);
+#undef SVOX_BACKWARD
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::replay_backward(dim3 blocks, hipStream_t stream, const Source& src,
+                                             const SvoxRenderOptions& opt, const float* grad_out, float* grad_data,
+                                             const ReplaySpace& ws, int ray_shift, int march1_known, const Lobes& lobes) {
+    hipLaunchKernelGGL((replay_backward_kernel<P, Source>), blocks, dim3(kMarchThreads), 0, stream, src, opt, grad_out,
+                       grad_data, ws, ray_shift, march1_known, lobes);
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::se_grad(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                                     const SvoxRenderOptions& opt, const float* color_ref, float* color_out, float* grad,
+                                     float* hess, const unsigned long long* only, bool refill) {
+    if (refill)
+        hipLaunchKernelGGL((se_grad_kernel<P, Source, true>), blocks, dim3(kMarchThreads), 0, stream, tr, src, opt,
+                           color_ref, color_out, grad, hess, only);
+    else
+        hipLaunchKernelGGL((se_grad_kernel<P, Source, false>), blocks, dim3(kMarchThreads), 0, stream, tr, src, opt,
+                           color_ref, color_out, grad, hess, only);
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::replay_se_grad(dim3 blocks, hipStream_t stream, const Source& src,
+                                            const SvoxRenderOptions& opt, const float* color_ref, float* color_out,
+                                            float* grad, float* hess, const ReplaySpace& ws, int ray_shift,
+                                            const Lobes& lobes) {
+    hipLaunchKernelGGL((replay_se_grad_kernel<P, Source>), blocks, dim3(kMarchThreads), 0, stream, src, opt, color_ref,
+                       color_out, grad, hess, ws, ray_shift, lobes);
+}
+#endif  // SVOX_INSTANTIATE_POLICY
+
+}  // namespace svox

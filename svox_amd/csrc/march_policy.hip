@@ -1,0 +1,13 @@
+// march_policy.hip -- the march kernels of one policy.  build.py compiles this file once per record format and basis
+// size, with SVOX_POLICY_FORMAT (SVOX_FORMAT_RGBA, _SH or _SG) and SVOX_POLICY_BASIS defined.
+#include <hip/hip_runtime.h>
+
+#include "../../include/svox_hip.h"
+
+#define SVOX_INSTANTIATE_POLICY
+#include "march_launch.h"
+
+namespace svox {
+template struct MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, BatchSource<float>>;
+template struct MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, ImageSource<float>>;
+}  // namespace svox

@@ -10,7 +10,7 @@
 #include <cstring>
 
 #include "../../include/svox_hip.h"
-#include "march_kernels.h"
+#include "march_launch.h"
 #include "query_kernels.h"
 
 #include <mutex>
@@ -20,6 +20,9 @@
 // is never passed to a kernel or a runtime call as an address.
 static_assert(SVOX_STATIC_WORKSPACE_BYTES % 256 == 0, "whole 256-byte units");
 static __device__ __align__(256) unsigned char scratch[SVOX_STATIC_WORKSPACE_BYTES];
+// Wavefronts of render_forward_split_kernel that gave up waiting since the library was loaded (svox_give_up_count);
+// the kernels get its address in ReplaySpace::give_ups.
+static __device__ unsigned int split_give_ups = 0;
 
 namespace {
 
@@ -78,6 +81,30 @@ int check_launch(const char* what) {
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return fail(SVOX_ERR_LAUNCH, "svox.%s: %s", what, hipGetErrorString(err));
     return SVOX_OK;
+}
+
+// The device address of a __device__ variable of this library on the current device, looked up once per device (every
+// GPU holds its own copy at its own address); nullptr where there is no usable device.
+constexpr int kStaticDevicesMax = 64;
+struct DeviceAddress {
+    std::mutex guard;
+    void* address[kStaticDevicesMax] = {nullptr};
+    template <typename Symbol>
+    void* get(const Symbol& symbol) {
+        int device = -1;
+        if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kStaticDevicesMax) return nullptr;
+        std::lock_guard<std::mutex> lock(guard);
+        if (!address[device]) {
+            void* ptr = nullptr;
+            if (hipGetSymbolAddress(&ptr, symbol) != hipSuccess) return nullptr;
+            address[device] = ptr;
+        }
+        return address[device];
+    }
+};
+unsigned int* give_up_counter() {
+    static DeviceAddress at;
+    return (unsigned int*)at.get(HIP_SYMBOL(split_give_ups));
 }
 
 int check_tree(const SvoxTreeSpec* t, bool need_data) {
@@ -272,6 +299,7 @@ TreeDev<float> march_tree(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt
 ReplaySpace no_notes() {
     ReplaySpace ws{};
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
+    ws.give_ups = give_up_counter();
     return ws;
 }
 
@@ -432,26 +460,10 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
             // registers (5 instead of 6 wavefronts per SIMD): measured 0.70 -> 0.73 ms on 8 poses of 800x800,
             // although the launch sends 17 % fewer requests to L2.
             const bool all_shaded = !tree->weight_accum && marks_decide(tree, opt, opt->sigma_thresh);
-#define SVOX_LAUNCH_FORWARD(ACCUM, REFILL, ALL)                                                                   \
-    SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((render_forward_kernel<P, Source, ACCUM, REFILL, false, false, ALL>), \
-                                               dim3(blocks), dim3(kMarchThreads), 0, stream, tr, dealt, *opt,      \
-                                               (float*)out, none))
             const bool refill = src.per_wave > kMarchThreads;
-            if (!refill && !tree->weight_accum && use_split_forward(blocks, is_image_source(src), opt, all_shaded)) {
-                SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((render_forward_split_kernel<P, Source, false>),
-                                                           dim3(blocks), dim3(kSplitThreads), 0, stream, tr, dealt,
-                                                           *opt, (float*)out, none));
-                return;
-            }
-            if (tree->weight_accum) {
-                // accumulation is an analysis pass: one variant is enough
-                SVOX_LAUNCH_FORWARD(true, true, false);
-            } else if (refill) {
-                if (all_shaded) { SVOX_LAUNCH_FORWARD(false, true, true); } else { SVOX_LAUNCH_FORWARD(false, true, false); }
-            } else {
-                if (all_shaded) { SVOX_LAUNCH_FORWARD(false, false, true); } else { SVOX_LAUNCH_FORWARD(false, false, false); }
-            }
-#undef SVOX_LAUNCH_FORWARD
+            const bool split = !refill && !tree->weight_accum && use_split_forward(blocks, is_image_source(src), opt, all_shaded);
+            SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::forward(dim3(blocks), stream, tr, dealt, *opt, (float*)out, none,
+                                                                    split, tree->weight_accum != nullptr, refill, all_shaded));
             return;
         }
     }
@@ -488,7 +500,7 @@ constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
 bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, ReplaySpace* ws) {
-    *ws = ReplaySpace{nullptr, 0, 0, nullptr, nullptr, {0, 0, 0, 0, 0, 0}, nullptr, nullptr};
+    *ws = ReplaySpace{};
     const int64_t chunks = workspace && n_slots > 0
                                ? (workspace_bytes - kTailBytes - bitmap_bytes(n_slots)) / kChunkBytes : 0;
     if (n_slots <= 0 || chunks < n_slots || chunks >= 0x7fffffffll || ((uintptr_t)workspace & 15u) != 0) return false;
@@ -512,17 +524,9 @@ void launch_backward(const SvoxTreeSpec* tree, const Source& src, const SvoxRend
             const unsigned blocks = blocks_for(items, src.per_wave);
             const Source dealt = dealt_out(src, blocks);
             const ReplaySpace none{};
-            if (src.per_wave > kMarchThreads) {
-                SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((render_backward_kernel<P, Source, true, kBackwardPlain>),
-                                                           dim3(blocks), dim3(kMarchThreads), 0, stream,
-                                                           march_tree(tree, opt), dealt, *opt, (const float*)grad_out,
-                                                           (float*)grad_data, none));
-            } else {
-                SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((render_backward_kernel<P, Source, false, kBackwardPlain>),
-                                                           dim3(blocks), dim3(kMarchThreads), 0, stream,
-                                                           march_tree(tree, opt), dealt, *opt, (const float*)grad_out,
-                                                           (float*)grad_data, none));
-            }
+            SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::backward(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
+                                                                     (const float*)grad_out, (float*)grad_data, none,
+                                                                     src.per_wave > kMarchThreads, false));
             return;
         }
     }
@@ -561,54 +565,11 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     if (rc) return rc;
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
+    ws.give_ups = give_up_counter();
     const bool refill = src.per_wave > kMarchThreads;
     const bool split = !refill && use_split_forward(blocks, is_image_source(src), opt, false);
-    const dim3 threads(split ? kSplitThreads : kMarchThreads);
-#define SVOX_LAUNCH_NOTING(KERNEL)                                                                                   \
-    SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL(KERNEL, dim3(blocks), threads, 0, stream, march_tree(tree, opt), dealt, \
-                                               *opt, (float*)out, ws, (const float*)grad_out))
-    if (grad_out) {
-        if (split) {
-            SVOX_LAUNCH_NOTING((render_forward_split_kernel<P, Source, true, true>));
-        } else if (refill) {
-            SVOX_LAUNCH_NOTING((render_forward_kernel<P, Source, false, true, true, true>));
-        } else {
-            SVOX_LAUNCH_NOTING((render_forward_kernel<P, Source, false, false, true, true>));
-        }
-    } else {
-        if (split) {
-            SVOX_LAUNCH_NOTING((render_forward_split_kernel<P, Source, true, false>));
-        } else if (refill) {
-            SVOX_LAUNCH_NOTING((render_forward_kernel<P, Source, false, true, true, false>));
-        } else {
-            SVOX_LAUNCH_NOTING((render_forward_kernel<P, Source, false, false, true, false>));
-        }
-    }
-#undef SVOX_LAUNCH_NOTING
-    return SVOX_OK;
-}
-
-// The device address of `scratch` on the current device, looked up once per device (every GPU holds
-// its own copy of the array at its own address).
-constexpr int kStaticDevicesMax = 64;
-int static_workspace(void** out) {
-    static std::mutex guard;
-    static void* address[kStaticDevicesMax] = {nullptr};
-    int device = -1;
-    hipError_t err = hipGetDevice(&device);
-    if (err != hipSuccess || device < 0 || device >= kStaticDevicesMax)
-        return fail(SVOX_ERR_NO_DEVICE, "svox.volume_render_backward_static: no usable current device (%s)",
-                    err != hipSuccess ? hipGetErrorString(err) : "device index out of range");
-    std::lock_guard<std::mutex> lock(guard);
-    if (!address[device]) {
-        void* ptr = nullptr;
-        err = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-        if (err != hipSuccess || !ptr)
-            return fail(SVOX_ERR_LAUNCH, "svox.volume_render_backward_static: hipGetSymbolAddress failed (%s)",
-                        hipGetErrorString(err));
-        address[device] = ptr;
-    }
-    *out = address[device];
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
+                                                           (float*)out, ws, (const float*)grad_out, split, refill));
     return SVOX_OK;
 }
 
@@ -628,17 +589,10 @@ void launch_se_grad(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
         if (D >= 0) {
             const unsigned blocks = blocks_for(items, src.per_wave);
             const Source dealt = only ? src : dealt_out(src, blocks);
-            if (src.per_wave > kMarchThreads) {
-                SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((se_grad_kernel<P, Source, true>), dim3(blocks),
-                                                           dim3(kMarchThreads), 0, stream, march_tree(tree, opt),
-                                                           dealt, *opt, (const float*)color_ref, (float*)color_out,
-                                                           (float*)grad, (float*)hess, only));
-            } else {
-                SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((se_grad_kernel<P, Source, false>), dim3(blocks),
-                                                           dim3(kMarchThreads), 0, stream, march_tree(tree, opt),
-                                                           src, *opt, (const float*)color_ref, (float*)color_out,
-                                                           (float*)grad, (float*)hess, only));
-            }
+            SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::se_grad(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
+                                                                    (const float*)color_ref, (float*)color_out,
+                                                                    (float*)grad, (float*)hess, only,
+                                                                    src.per_wave > kMarchThreads));
             return;
         }
     }
@@ -705,25 +659,18 @@ int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest
     ReplaySpace ws;
     carve_workspace(workspace, workspace_bytes, n_slots, &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
-    SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((replay_backward_kernel<P, Source>), dim3(waves), dim3(kMarchThreads), 0,
-                                               stream, all, *opt, (const float*)grad_output, (float*)grad_data_out, ws,
-                                               ray_shift, march1_known ? 1 : 0, lobes_of(tree, opt)));
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(waves), stream, all, *opt, (const float*)grad_output,
+                                                                    (float*)grad_data_out, ws, ray_shift,
+                                                                    march1_known ? 1 : 0, lobes_of(tree, opt)));
     int rc = check_launch("volume_render_backward_noted");
     if (rc) return rc;
     ReplaySpace only{};
     only.base = ws.base;
     only.only = ws.undone;
     const unsigned blocks = blocks_for(total_items_of(rest), rest.per_wave);
-#define SVOX_LAUNCH_REST(REFILL, MODE)                                                                              \
-    SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((render_backward_kernel<P, Source, REFILL, MODE>), dim3(blocks),      \
-                                               dim3(kMarchThreads), 0, stream, march_tree(tree, opt), rest, *opt,    \
-                                               (const float*)grad_output, (float*)grad_data_out, only))
-    if (rest.per_wave > kMarchThreads) {
-        if (march1_known) { SVOX_LAUNCH_REST(true, kBackwardSecond); } else { SVOX_LAUNCH_REST(true, kBackwardPlain); }
-    } else {
-        if (march1_known) { SVOX_LAUNCH_REST(false, kBackwardSecond); } else { SVOX_LAUNCH_REST(false, kBackwardPlain); }
-    }
-#undef SVOX_LAUNCH_REST
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::backward(dim3(blocks), stream, march_tree(tree, opt), rest, *opt,
+                                                             (const float*)grad_output, (float*)grad_data_out, only,
+                                                             rest.per_wave > kMarchThreads, march1_known));
     return check_launch("volume_render_backward_noted");
 }
 
@@ -776,10 +723,9 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
     carve_workspace(workspace, workspace_bytes, n_slots, &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     const int ray_shift = replay_ray_shift(is_image_source(all), n_slots);
-    SVOX_DISPATCH_OCTREE(D, hipLaunchKernelGGL((replay_se_grad_kernel<P, Source>), dim3(blocks_for(n_slots, 1 << ray_shift)),
-                                               dim3(kMarchThreads), 0, stream, all, *opt, (const float*)color_ref,
-                                               (float*)color_out, (float*)grad, (float*)hess, ws, ray_shift,
-                                               lobes_of(tree, opt)));
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_se_grad(dim3(blocks_for(n_slots, 1 << ray_shift)), stream, all, *opt,
+                                                                   (const float*)color_ref, (float*)color_out, (float*)grad,
+                                                                   (float*)hess, ws, ray_shift, lobes_of(tree, opt)));
     rc = check_launch("se_grad");
     if (rc) return rc;
     launch_se_grad<Source, float>(tree, rest, opt, 3, color_ref, color_out, grad, hess, stream, ws.undone);
@@ -1095,9 +1041,9 @@ int svox_volume_render_backward_static(const SvoxTreeSpec* tree, const SvoxRaysS
                     "workspace serves per call; split the batch (accumulate = 1 from the second part on) or "
                     "call svox_volume_render_backward_ws with a workspace of your own",
                     (long long)rays->n_rays, (int)SVOX_STATIC_RAYS_MAX);
-    void* ws = nullptr;
-    rc = static_workspace(&ws);
-    if (rc) return rc;
+    static DeviceAddress workspace_at;
+    void* const ws = workspace_at.get(HIP_SYMBOL(scratch));
+    if (!ws) return fail(SVOX_ERR_NO_DEVICE, "svox.volume_render_backward_static: no usable current device");
     return svox_volume_render_backward_ws(tree, rays, opt, grad_output, grad_data_out, accumulate, ws,
                                           (int64_t)SVOX_STATIC_WORKSPACE_BYTES, stream);
 }
