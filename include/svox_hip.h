@@ -265,6 +265,23 @@ int svox_volume_render_images_backward_noted(const SvoxTreeSpec* tree, const Svo
                                              const SvoxRenderOptions* opt, const void* grad_output,
                                              void* grad_data_out, int32_t accumulate, void* workspace,
                                              int64_t workspace_bytes, void* stream);
+/* The two backward calls from notes with more to say (no reference counterpart; extras may be NULL).
+ * report: NULL, or 8 bytes of host memory the device can write (hipHostMalloc).  The call's kernels leave there how
+ * full the workspace ran, as svox_notes_pool_info describes it -- the stocks asked for in the upper 32 bits, the stocks
+ * there are in the lower --, which the caller may look at at any time without waiting for the device. */
+typedef struct SvoxNotesExtras {
+    int64_t* report;
+} SvoxNotesExtras;
+int svox_volume_render_backward_noted_with(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays,
+                                           const SvoxRenderOptions* opt, const void* grad_output,
+                                           void* grad_data_out, int32_t accumulate, void* workspace,
+                                           int64_t workspace_bytes, const SvoxNotesExtras* extras, void* stream);
+int svox_volume_render_images_backward_noted_with(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam,
+                                                  int32_t n_images, int64_t pose_stride,
+                                                  const SvoxRenderOptions* opt, const void* grad_output,
+                                                  void* grad_data_out, int32_t accumulate, void* workspace,
+                                                  int64_t workspace_bytes, const SvoxNotesExtras* extras,
+                                                  void* stream);
 int64_t svox_volume_render_backward_workspace_bytes(int64_t n_rays, int32_t records_per_ray);
 
 /* No counterpart in the reference.  How full a workspace of notes ran: after a call that takes notes

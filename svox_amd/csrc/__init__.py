@@ -8,6 +8,10 @@ checks its tensors the way the reference's `check()` methods do (svox/csrc/inclu
 allocates the outputs with the reference's shapes / dtypes / devices and calls the matching
 extern "C" entry point of libsvox_hip.so on torch's current stream.
 
+The calls of the hot path -- point queries and their gradient, rendering, gradients, se_grad -- are made in native code
+(host_shim.cpp): a call on a few thousand points or rays lasts as long as the host needs to make it.  The others go
+through ctypes.
+
 There is no CPU implementation here: tensors that are not on a GPU raise, and a missing library
 raises at the first call.
 """
@@ -76,11 +80,21 @@ class RenderOptions:
         self.rgb_padding = 0.0
 
     def _pack(self):
-        return _abi.RenderOptionsC(
-            float(self.step_size), float(self.background_brightness), int(self.format),
-            int(self.basis_dim), int(self.ndc_width), int(self.ndc_height), float(self.ndc_focal),
-            int(self.min_comp), int(self.max_comp), float(self.sigma_thresh),
-            float(self.stop_thresh), int(bool(self.density_softplus)), float(self.rgb_padding))
+        packed = _abi.RenderOptionsC()
+        _shim().fill_options(ctypes.addressof(packed), self)
+        return packed
+
+
+_native = None
+
+
+def _shim():
+    """The native half of this module, bound to the library at the first call."""
+    global _native
+    if _native is None:
+        _abi.load_library()
+        _native = _abi.load_shim()
+    return _native
 
 
 # --------------------------------------------------------------------------------------------
@@ -95,98 +109,15 @@ def _check_input(x, name):
         raise RuntimeError(f"{name} must be contiguous")
 
 
-def _numel(x):
-    return 0 if x is None else x.numel()
-
-
-def _dtype_code(dtype, name):
-    if dtype == torch.float32:
-        return _abi.SVOX_F32
-    if dtype == torch.float64:
-        return _abi.SVOX_F64
-    raise RuntimeError(f"{name} must be a float32 or float64 tensor, got {dtype}")
-
-
 def _same_dtype(x, dtype, name):
     if x.dtype != dtype:
         raise RuntimeError(f"expected scalar type {dtype} for {name} but found {x.dtype}")
 
 
-def _check_tree(tree):
-    """TreeSpec::check, data_spec.hpp:75-88, plus the shape facts the kernels rely on."""
-    _check_input(tree.data, "data")
-    _check_input(tree.child, "child")
-    _check_input(tree.parent_depth, "parent_depth")
-    if _numel(tree.extra_data):
-        _check_input(tree.extra_data, "extra_data")
-    if tree.offset is not None:
-        _check_input(tree.offset, "offset")
-    if tree.scaling is not None:
-        _check_input(tree.scaling, "scaling")
-    if _numel(tree._weight_accum):
-        _check_input(tree._weight_accum, "_weight_accum")
-    if tree.data.dim() != 5 or tree.child.dim() != 4 or tree.parent_depth.dim() != 2:
-        raise RuntimeError("data must be 5-D, child 4-D and parent_depth 2-D")
-    if tree.child.dtype != torch.int32 or tree.parent_depth.dtype != torch.int32:
-        raise RuntimeError("child and parent_depth must be int32 tensors")
-    if tuple(tree.data.shape[:4]) != tuple(tree.child.shape):
-        raise RuntimeError("data and child disagree on (capacity, N, N, N)")
-
-
 def _pack_tree(tree, dtype=None, need_data=True):
-    _check_tree(tree)
-    dt = tree.data.dtype if dtype is None else dtype
-    code = _dtype_code(dt, "data")
-    if need_data:
-        _same_dtype(tree.data, dt, "data")
+    """TreeSpec::check, data_spec.hpp:75-88, and the C struct."""
     spec = _abi.TreeSpecC()
-    spec.data = tree.data.data_ptr()
-    spec.child = tree.child.data_ptr()
-    spec.parent_depth = tree.parent_depth.data_ptr()
-    extra = tree.extra_data if _numel(tree.extra_data) else None
-    if extra is not None:
-        _same_dtype(extra, dt, "extra_data")
-        if extra.dim() != 2:
-            raise RuntimeError("extra_data must be 2-D")
-        spec.extra_data = extra.data_ptr()
-        spec.extra_rows, spec.extra_cols = int(extra.shape[0]), int(extra.shape[1])
-    else:
-        spec.extra_data = None
-        spec.extra_rows = spec.extra_cols = 0
-    for attr in ("offset", "scaling"):
-        t = getattr(tree, attr)
-        if t is not None:
-            _same_dtype(t, dt, attr)
-            if t.numel() != 3:
-                raise RuntimeError(f"{attr} must have 3 elements")
-            setattr(spec, attr, t.data_ptr())
-        else:
-            setattr(spec, attr, None)
-    wa = tree._weight_accum if _numel(tree._weight_accum) else None
-    if wa is not None:
-        _same_dtype(wa, dt, "_weight_accum")
-        if wa.numel() != tree.child.numel():
-            raise RuntimeError("_weight_accum must have one entry per cell of child")
-        spec.weight_accum = wa.data_ptr()
-    else:
-        spec.weight_accum = None
-    spec.weight_accum_max = int(bool(tree._weight_accum_max))
-    marks = getattr(tree, "child_marks", None)
-    if marks is not None:
-        _check_input(marks, "child_marks")
-        if marks.dtype != torch.int32 or marks.shape != tree.child.shape:
-            raise RuntimeError("child_marks must be an int32 tensor shaped like child")
-        spec.child_marks = marks.data_ptr()
-        spec.child_marks_thresh = float(getattr(tree, "child_marks_thresh", 0.0))
-        spec.child_marks_softplus = int(bool(getattr(tree, "child_marks_softplus", False)))
-    else:
-        spec.child_marks = None
-        spec.child_marks_thresh = 0.0
-        spec.child_marks_softplus = 0
-    spec.capacity = int(tree.child.shape[0])
-    spec.N = int(tree.child.shape[1])
-    spec.data_dim = int(tree.data.shape[4])
-    spec.dtype = code
+    _shim().fill_tree(ctypes.addressof(spec), tree, dtype, need_data)
     return spec
 
 
@@ -223,35 +154,12 @@ def out_data_dim(fmt, basis_dim, data_dim):
 # --------------------------------------------------------------------------------------------
 def query_vertical(tree, indices):
     """(values (Q, K) like indices, node_ids (Q,) int64 on child's device); svox_kernel.cu:120-143"""
-    _check_indices(indices)
-    spec = _pack_tree(tree, indices.dtype)
-    if indices.shape[1] != 3:
-        raise RuntimeError("indices must be (Q, 3)")
-    Q, K = indices.shape[0], spec.data_dim
-    values = torch.empty((Q, K), dtype=indices.dtype, device=indices.device)
-    node_ids = torch.empty((Q,), dtype=torch.int64, device=tree.child.device)
-    with torch.cuda.device(indices.device):
-        _call("svox_query_vertical", ctypes.byref(spec), indices.data_ptr(), Q, values.data_ptr(),
-              node_ids.data_ptr(), _stream(indices.device))
-    return values, node_ids
+    return _shim().query_vertical(tree, indices)
 
 
 def query_vertical_backward(tree, indices, grad_output):
     """zeros (M, N, N, N, grad_output.shape[1]) + scatter-add; svox_kernel.cu:160-182"""
-    _check_indices(indices)
-    _check_indices(grad_output, "grad_output")
-    _same_dtype(grad_output, indices.dtype, "grad_output")
-    spec = _pack_tree(tree, indices.dtype, need_data=False)
-    Q, Kg = indices.shape[0], int(grad_output.shape[1])
-    if grad_output.shape[0] != Q:
-        raise RuntimeError("grad_output must have one row per point")
-    N = spec.N
-    grad_data = torch.empty((spec.capacity, N, N, N, Kg), dtype=grad_output.dtype,
-                            device=grad_output.device)
-    with torch.cuda.device(indices.device):
-        _call("svox_query_vertical_backward", ctypes.byref(spec), indices.data_ptr(), Q,
-              grad_output.data_ptr(), Kg, grad_data.data_ptr(), 0, _stream(indices.device))
-    return grad_data
+    return _shim().query_vertical_backward(tree, indices, grad_output)
 
 
 def assign_vertical(tree, indices, values):
@@ -286,31 +194,16 @@ def calc_corners(tree, indexer):
 # --------------------------------------------------------------------------------------------
 def _pack_rays(rays, dtype):
     """RaysSpec::check, data_spec.hpp:56-63"""
-    for name in ("origins", "dirs", "vdirs"):
-        t = getattr(rays, name)
-        _check_input(t, name)
-        if not t.is_floating_point():
-            raise RuntimeError(f"{name} must be a floating point tensor")
-        _same_dtype(t, dtype, name)
-        if t.dim() != 2 or t.shape[1] != 3:
-            raise RuntimeError(f"{name} must be (B, 3)")
-    B = rays.origins.shape[0]
-    if rays.dirs.shape[0] != B or rays.vdirs.shape[0] != B:
-        raise RuntimeError("origins, dirs and vdirs must have the same number of rays")
-    return _abi.RaysSpecC(rays.origins.data_ptr(), rays.dirs.data_ptr(), rays.vdirs.data_ptr(), B)
+    spec = _abi.RaysSpecC()
+    _shim().fill_rays(ctypes.addressof(spec), rays, dtype)
+    return spec
 
 
 def _pack_camera(cam, dtype, batched=False):
     """CameraSpec::check, data_spec.hpp:98-103.  batched: c2w is (n, 3 or 4, 4)."""
-    _check_input(cam.c2w, "c2w")
-    if not cam.c2w.is_floating_point():
-        raise RuntimeError("c2w must be a floating point tensor")
-    want = 3 if batched else 2
-    if cam.c2w.dim() != want or cam.c2w.shape[-1] != 4 or cam.c2w.shape[-2] not in (3, 4):
-        raise RuntimeError("c2w must be (n, 3, 4) or (n, 4, 4)" if batched else "c2w must be (3, 4) or (4, 4)")
-    _same_dtype(cam.c2w, dtype, "c2w")
-    return _abi.CameraSpecC(cam.c2w.data_ptr(), float(cam.fx), float(cam.fy), int(cam.width),
-                            int(cam.height))
+    spec = _abi.CameraSpecC()
+    _shim().fill_camera(ctypes.addressof(spec), cam, dtype, batched)
+    return spec
 
 
 def _render_out_dim(spec, opt):
@@ -321,31 +214,26 @@ def _render_out_dim(spec, opt):
     return od
 
 
+def _n_rays(rays):
+    """Rays of a RaysSpec, as far as it can be told before it is checked."""
+    origins = rays.origins
+    return origins.shape[0] if isinstance(origins, torch.Tensor) and origins.dim() else 0
+
+
+def _n_pixels(cam):
+    c2w = cam.c2w
+    many = isinstance(c2w, torch.Tensor) and c2w.dim() == 3
+    return (c2w.shape[0] if many else 1) * cam.height * cam.width
+
+
 def volume_render(tree, rays, opt):
     """(B, out_dim) like rays.origins; rt_kernel.cu:1019-1036"""
-    spec = _pack_tree(tree, rays.origins.dtype if isinstance(rays.origins, torch.Tensor) else None)
-    rspec = _pack_rays(rays, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    out = torch.empty((rspec.n_rays, od), dtype=rays.origins.dtype, device=rays.origins.device)
-    copt = opt._pack()
-    marks = _attach_marks(spec, tree, opt, rspec.n_rays)  # noqa: F841
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render", ctypes.byref(spec), ctypes.byref(rspec), ctypes.byref(copt),
-              out.data_ptr(), _stream(tree.data.device))
-    return out
+    return _shim().volume_render(tree, rays, opt, _call_marks(tree, opt, _n_rays(rays)))
 
 
 def volume_render_image(tree, cam, opt):
     """(H, W, out_dim) like tree.data; rt_kernel.cu:1038-1057"""
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    out = torch.empty((cspec.height, cspec.width, od), dtype=tree.data.dtype, device=tree.data.device)
-    copt = opt._pack()
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_image", ctypes.byref(spec), ctypes.byref(cspec),
-              ctypes.byref(copt), out.data_ptr(), _stream(tree.data.device))
-    return out
+    return _shim().volume_render_images(tree, cam, opt, False, None)
 
 
 # A render call (forward, noted forward or marching backward) with at least this many rays per cell of
@@ -375,100 +263,43 @@ def _marks_for_this_call(tree, opt, n_rays, every_positive_leaf=False):
     return mark_empty_leaves(tree, thresh, bool(opt.density_softplus)), thresh
 
 
-def _attach_marks(spec, tree, opt, n_rays, every_positive_leaf=False):
-    """Points the packed `spec` to marks made for this call, where they pay; returns the tensor,
-    which the caller keeps until its launch is queued."""
-    made = _marks_for_this_call(tree, opt, n_rays, every_positive_leaf)
-    if made is None:
+def _call_marks(tree, opt, n_rays, every_positive_leaf=False):
+    """(marks, threshold, softplus) made for this call, where they pay, or None."""
+    if n_rays < AUTO_MARK_MIN_RAYS:
         return None
-    marks, thresh = made
-    spec.child_marks = marks.data_ptr()
-    spec.child_marks_thresh = thresh
-    spec.child_marks_softplus = int(bool(opt.density_softplus))
-    return marks
+    made = _marks_for_this_call(tree, opt, n_rays, every_positive_leaf)
+    return None if made is None else (*made, bool(opt.density_softplus))
 
 
 def volume_render_images(tree, cam, opt):
     """(n, H, W, out_dim): n images in one launch; cam.c2w is (n, 3, 4) or (n, 4, 4).
     No counterpart in the reference, whose extension renders one image per call."""
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype, batched=True)
-    n, stride = int(cam.c2w.shape[0]), int(cam.c2w.shape[1]) * 4
-    od = _render_out_dim(spec, opt)
-    out = torch.empty((n, cspec.height, cspec.width, od), dtype=tree.data.dtype, device=tree.data.device)
-    copt = opt._pack()
-    marks = _attach_marks(spec, tree, opt, n * cspec.height * cspec.width)  # noqa: F841 (kept alive for the launch)
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_images", ctypes.byref(spec), ctypes.byref(cspec), n, stride,
-              ctypes.byref(copt), out.data_ptr(), _stream(tree.data.device))
-    return out
+    return _shim().volume_render_images(tree, cam, opt, True, _call_marks(tree, opt, _n_pixels(cam)))
 
 
 def volume_render_images_backward(tree, cam, opt, grad_output, workspace=True):
     """zeros_like(tree.data) + scatter for volume_render_images (workspace: see volume_render_backward)."""
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype, batched=True)
-    n, stride = int(cam.c2w.shape[0]), int(cam.c2w.shape[1]) * 4
-    od = _render_out_dim(spec, opt)
-    _check_grad(grad_output, (n, cspec.height, cspec.width, od), tree.data.dtype)
-    grad = torch.empty_like(tree.data)
-    copt = opt._pack()
-    ws, ws_bytes = _backward_workspace(tree, n * cspec.height * cspec.width) if workspace else (None, 0)
-    marks = _attach_marks(spec, tree, opt, n * cspec.height * cspec.width, True)  # noqa: F841
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_images_backward_ws", ctypes.byref(spec), ctypes.byref(cspec), n, stride,
-              ctypes.byref(copt), grad_output.data_ptr(), grad.data_ptr(), 0,
-              ws.data_ptr() if ws is not None else None, ws_bytes, _stream(tree.data.device))
-    return grad
+    n = _n_pixels(cam)
+    ws = _backward_workspace(tree, n)[0] if workspace else None
+    return _shim().volume_render_images_backward(tree, cam, opt, grad_output, ws, False, 0, 1,
+                                                 _call_marks(tree, opt, n, True))
 
 
 def volume_render_images_noted(tree, cam, opt, records_per_ray=None):
     """(images, notes): volume_render_images that also leaves the notes
     volume_render_images_backward_noted works from (see volume_render_noted).  cam.c2w is
     (n, 3, 4) / (n, 4, 4), or one pose (3, 4) / (4, 4), which gives (H, W, out_dim)."""
-    single = cam.c2w.dim() == 2
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype, batched=not single)
-    n, stride = (1, 12) if single else (int(cam.c2w.shape[0]), int(cam.c2w.shape[1]) * 4)
-    od = _render_out_dim(spec, opt)
-    shape = (cspec.height, cspec.width, od) if single else (n, cspec.height, cspec.width, od)
-    out = torch.empty(shape, dtype=tree.data.dtype, device=tree.data.device)
-    copt = opt._pack()
-    ws, ws_bytes = _notes_workspace(tree, spec, copt, n * cspec.height * cspec.width, records_per_ray)
-    marks = _attach_marks(spec, tree, opt, n * cspec.height * cspec.width, ws is not None)  # noqa: F841
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_images_noted", ctypes.byref(spec), ctypes.byref(cspec), n, stride,
-              ctypes.byref(copt), out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes,
-              _stream(tree.data.device))
-    return out, ws
+    n = _n_pixels(cam)
+    ws = _notes_workspace(tree, opt, n, records_per_ray)
+    return _shim().volume_render_images_noted(tree, cam, opt, ws, _call_marks(tree, opt, n, ws is not None)), ws
 
 
-def volume_render_images_backward_noted(tree, cam, opt, grad_output, notes):
+def volume_render_images_backward_noted(tree, cam, opt, grad_output, notes, report=0):
     """The gradient of volume_render_images_noted's picture(s) from its notes (notes None: by marching)."""
-    single = cam.c2w.dim() == 2
     if notes is None:
-        fn = volume_render_image_backward if single else volume_render_images_backward
+        fn = volume_render_image_backward if cam.c2w.dim() == 2 else volume_render_images_backward
         return fn(tree, cam, opt, grad_output)
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype, batched=not single)
-    n, stride = (1, 12) if single else (int(cam.c2w.shape[0]), int(cam.c2w.shape[1]) * 4)
-    od = _render_out_dim(spec, opt)
-    shape = (cspec.height, cspec.width, od) if single else (n, cspec.height, cspec.width, od)
-    _check_grad(grad_output, shape, tree.data.dtype)
-    grad = torch.empty_like(tree.data)
-    copt = opt._pack()
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_images_backward_noted", ctypes.byref(spec), ctypes.byref(cspec), n, stride,
-              ctypes.byref(copt), grad_output.data_ptr(), grad.data_ptr(), 0, notes.data_ptr(),
-              notes.numel() * notes.element_size(), _stream(tree.data.device))
-    return grad
-
-
-def _check_grad(grad_output, shape, dtype):
-    _check_input(grad_output, "grad_output")
-    _same_dtype(grad_output, dtype, "grad_output")
-    if tuple(grad_output.shape) != tuple(shape):
-        raise RuntimeError(f"grad_output must have shape {tuple(shape)}, got {tuple(grad_output.shape)}")
+    return _shim().volume_render_images_backward(tree, cam, opt, grad_output, notes, True, report, -1, None)
 
 
 # Leaves per ray (on average) the backward's workspace has room for, and the most memory it may take:
@@ -513,13 +344,13 @@ def _backward_workspace(tree, n_rays, records_per_ray=None):
         return None, 0
 
 
-def _notes_workspace(tree, spec, copt, n_rays, records_per_ray=None):
-    """_backward_workspace for the notes of a forward pass: (None, 0) also where the library would take no notes
+def _notes_workspace(tree, opt, n_rays, records_per_ray=None):
+    """_backward_workspace for the notes of a forward pass: None also where the library would take no notes
     for this tree under these options (svox_notes_serve: the one-ray-per-lane kernels, a weight accumulator, a
     negative sigma_thresh) -- the pass then runs as the plain forward pass and its caller keeps nothing."""
-    if _abi.load_library().svox_notes_serve(ctypes.byref(spec), ctypes.byref(copt)) != 1:
-        return None, 0
-    return _backward_workspace(tree, n_rays, records_per_ray)
+    if _shim().notes_serve(tree, opt) != 1:
+        return None
+    return _backward_workspace(tree, n_rays, records_per_ray)[0]
 
 
 def volume_render_backward(tree, rays, opt, grad_output, workspace=True):
@@ -529,19 +360,9 @@ def volume_render_backward(tree, rays, opt, grad_output, workspace=True):
     that a ray whose notes fit is marched once (fp32 octrees; room for BACKWARD_RECORDS_PER_RAY
     leaves per ray on average, at most BACKWARD_WORKSPACE_LIMIT bytes, from torch's allocator).
     The gradient is the same."""
-    spec = _pack_tree(tree)
-    rspec = _pack_rays(rays, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    _check_grad(grad_output, (rspec.n_rays, od), tree.data.dtype)
-    grad = torch.empty_like(tree.data)
-    copt = opt._pack()
-    ws, ws_bytes = _backward_workspace(tree, rspec.n_rays) if workspace else (None, 0)
-    marks = _attach_marks(spec, tree, opt, rspec.n_rays, True)  # noqa: F841
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_backward_ws", ctypes.byref(spec), ctypes.byref(rspec),
-              ctypes.byref(copt), grad_output.data_ptr(), grad.data_ptr(), 0,
-              ws.data_ptr() if ws is not None else None, ws_bytes, _stream(tree.data.device))
-    return grad
+    n = _n_rays(rays)
+    ws = _backward_workspace(tree, n)[0] if workspace else None
+    return _shim().volume_render_backward(tree, rays, opt, grad_output, ws, False, 0, _call_marks(tree, opt, n, True))
 
 
 def volume_render_backward_static(tree, rays, opt, grad_output, grad_data_out, accumulate=False):
@@ -552,7 +373,10 @@ def volume_render_backward_static(tree, rays, opt, grad_output, grad_data_out, a
     spec = _pack_tree(tree)
     rspec = _pack_rays(rays, tree.data.dtype)
     od = _render_out_dim(spec, opt)
-    _check_grad(grad_output, (rspec.n_rays, od), tree.data.dtype)
+    _check_input(grad_output, "grad_output")
+    _same_dtype(grad_output, tree.data.dtype, "grad_output")
+    if tuple(grad_output.shape) != (rspec.n_rays, od):
+        raise RuntimeError(f"grad_output must have shape {(rspec.n_rays, od)}, got {tuple(grad_output.shape)}")
     _check_input(grad_data_out, "grad_data_out")
     _same_dtype(grad_data_out, tree.data.dtype, "grad_data_out")
     if tuple(grad_data_out.shape) != tuple(tree.data.shape):
@@ -586,65 +410,25 @@ def volume_render_noted(tree, rays, opt, records_per_ray=None):
     records_per_ray: room for that many leaves per ray on average (default BACKWARD_RECORDS_PER_RAY).
     No counterpart in the reference: it is what an autograd function keeps between forward and
     backward."""
-    spec = _pack_tree(tree, rays.origins.dtype if isinstance(rays.origins, torch.Tensor) else None)
-    rspec = _pack_rays(rays, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    out = torch.empty((rspec.n_rays, od), dtype=rays.origins.dtype, device=rays.origins.device)
-    copt = opt._pack()
-    ws, ws_bytes = _notes_workspace(tree, spec, copt, rspec.n_rays, records_per_ray)
-    marks = _attach_marks(spec, tree, opt, rspec.n_rays, ws is not None)  # noqa: F841
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_noted", ctypes.byref(spec), ctypes.byref(rspec), ctypes.byref(copt),
-              out.data_ptr(), ws.data_ptr() if ws is not None else None, ws_bytes, _stream(tree.data.device))
-    return out, ws
+    n = _n_rays(rays)
+    ws = _notes_workspace(tree, opt, n, records_per_ray)
+    return _shim().volume_render_noted(tree, rays, opt, ws, _call_marks(tree, opt, n, ws is not None)), ws
 
 
-def volume_render_backward_noted(tree, rays, opt, grad_output, notes):
+def volume_render_backward_noted(tree, rays, opt, grad_output, notes, report=0):
     """volume_render_backward from the notes volume_render_noted left for the same tree, rays and
-    options (notes None: volume_render_backward).  tree.data must not have changed in between."""
+    options (notes None: volume_render_backward).  tree.data must not have changed in between.
+    report: 0, or the address of 8 bytes of pinned host memory that receive how full the notes ran
+    (SvoxNotesExtras.report)."""
     if notes is None:
         return volume_render_backward(tree, rays, opt, grad_output)
-    spec = _pack_tree(tree)
-    rspec = _pack_rays(rays, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    _check_grad(grad_output, (rspec.n_rays, od), tree.data.dtype)
-    grad = torch.empty_like(tree.data)
-    copt = opt._pack()
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_backward_noted", ctypes.byref(spec), ctypes.byref(rspec), ctypes.byref(copt),
-              grad_output.data_ptr(), grad.data_ptr(), 0, notes.data_ptr(), notes.numel() * notes.element_size(),
-              _stream(tree.data.device))
-    return grad
+    return _shim().volume_render_backward(tree, rays, opt, grad_output, notes, True, report, None)
 
 
 def volume_render_image_backward(tree, cam, opt, grad_output, workspace=True):
     """zeros_like(tree.data) + scatter; rt_kernel.cu:1085-1109 (workspace: see volume_render_backward)"""
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype)
-    od = _render_out_dim(spec, opt)
-    _check_grad(grad_output, (cspec.height, cspec.width, od), tree.data.dtype)
-    grad = torch.empty_like(tree.data)
-    copt = opt._pack()
-    ws, ws_bytes = _backward_workspace(tree, cspec.height * cspec.width) if workspace else (None, 0)
-    with torch.cuda.device(tree.data.device):
-        _call("svox_volume_render_images_backward_ws", ctypes.byref(spec), ctypes.byref(cspec), 1, 12,
-              ctypes.byref(copt), grad_output.data_ptr(), grad.data_ptr(), 0,
-              ws.data_ptr() if ws is not None else None, ws_bytes, _stream(tree.data.device))
-    return grad
-
-
-def _check_color(color, shape, dtype):
-    _check_input(color, "color")
-    _same_dtype(color, dtype, "color")
-    if tuple(color.shape) != tuple(shape):
-        raise RuntimeError(f"color must have shape {tuple(shape)}, got {tuple(color.shape)}")
-
-
-def _se_out_dim(spec, opt):
-    od = _render_out_dim(spec, opt)
-    if od > 4:
-        raise RuntimeError("Tree's output dim cannot be > 4 for se_grad")   # rt_kernel.cu:1123-1125
-    return od
+    ws = _backward_workspace(tree, cam.height * cam.width)[0] if workspace else None
+    return _shim().volume_render_images_backward(tree, cam, opt, grad_output, ws, False, 0, 0, None)
 
 
 def se_grad(tree, rays, color, opt, workspace=True):
@@ -652,39 +436,15 @@ def se_grad(tree, rays, color, opt, workspace=True):
     svox.cpp:115, rt_kernel.cu:1111-1139.  Argument order as in the reference: color before opt.
     With `workspace` (default) the rays are marched once and their notes used for the rest
     (svox_se_grad_ws); without, the rays are marched twice."""
-    spec = _pack_tree(tree)
-    rspec = _pack_rays(rays, tree.data.dtype)
-    od = _se_out_dim(spec, opt)
-    _check_color(color, (rspec.n_rays, od), tree.data.dtype)
-    result = torch.empty((rspec.n_rays, od), dtype=tree.data.dtype, device=tree.data.device)
-    grad = torch.empty_like(tree.data)
-    hessdiag = torch.empty_like(tree.data)
-    copt = opt._pack()
-    ws, ws_bytes = _backward_workspace(tree, rspec.n_rays) if workspace else (None, 0)
-    with torch.cuda.device(tree.data.device):
-        _call("svox_se_grad_ws", ctypes.byref(spec), ctypes.byref(rspec), ctypes.byref(copt), color.data_ptr(),
-              result.data_ptr(), grad.data_ptr(), hessdiag.data_ptr(), ws.data_ptr() if ws is not None else None,
-              ws_bytes, _stream(tree.data.device))
-    return result, grad, hessdiag
+    ws = _backward_workspace(tree, _n_rays(rays))[0] if workspace else None
+    return _shim().se_grad(tree, rays, opt, color, False, ws)
 
 
 def se_grad_persp(tree, cam, opt, color, workspace=True):
     """Image version: color and result are (H, W, C); svox.cpp:116, rt_kernel.cu:1141-1173.
     Argument order as in the reference: opt before color.  `workspace` as in se_grad."""
-    spec = _pack_tree(tree)
-    cspec = _pack_camera(cam, tree.data.dtype)
-    od = _se_out_dim(spec, opt)
-    _check_color(color, (cspec.height, cspec.width, od), tree.data.dtype)
-    result = torch.empty((cspec.height, cspec.width, od), dtype=tree.data.dtype, device=tree.data.device)
-    grad = torch.empty_like(tree.data)
-    hessdiag = torch.empty_like(tree.data)
-    copt = opt._pack()
-    ws, ws_bytes = _backward_workspace(tree, cspec.height * cspec.width) if workspace else (None, 0)
-    with torch.cuda.device(tree.data.device):
-        _call("svox_se_grad_image_ws", ctypes.byref(spec), ctypes.byref(cspec), ctypes.byref(copt),
-              color.data_ptr(), result.data_ptr(), grad.data_ptr(), hessdiag.data_ptr(),
-              ws.data_ptr() if ws is not None else None, ws_bytes, _stream(tree.data.device))
-    return result, grad, hessdiag
+    ws = _backward_workspace(tree, cam.height * cam.width)[0] if workspace else None
+    return _shim().se_grad(tree, cam, opt, color, True, ws)
 
 
 def mark_empty_leaves(tree, sigma_thresh=0.0, density_softplus=False):

@@ -100,6 +100,10 @@ class MarchStatsC(ctypes.Structure):
         return {name: int(getattr(self, name)) for name, _ in self._fields_}
 
 
+class NotesExtrasC(ctypes.Structure):
+    _fields_ = [("report", c_void_p)]
+
+
 P = ctypes.POINTER
 
 # name -> (restype, argtypes); the entry points of include/svox_hip.h
@@ -137,6 +141,12 @@ SIGNATURES = {
     "svox_volume_render_backward_noted": (
         ctypes.c_int, [P(TreeSpecC), P(RaysSpecC), P(RenderOptionsC), c_void_p, c_void_p, c_int32, c_void_p, c_int64,
                        c_void_p]),
+    "svox_volume_render_backward_noted_with": (
+        ctypes.c_int, [P(TreeSpecC), P(RaysSpecC), P(RenderOptionsC), c_void_p, c_void_p, c_int32, c_void_p, c_int64,
+                       P(NotesExtrasC), c_void_p]),
+    "svox_volume_render_images_backward_noted_with": (
+        ctypes.c_int, [P(TreeSpecC), P(CameraSpecC), c_int32, c_int64, P(RenderOptionsC), c_void_p, c_void_p, c_int32,
+                       c_void_p, c_int64, P(NotesExtrasC), c_void_p]),
     "svox_volume_render_images_noted": (
         ctypes.c_int, [P(TreeSpecC), P(CameraSpecC), c_int32, c_int64, P(RenderOptionsC), c_void_p, c_void_p, c_int64,
                        c_void_p]),
@@ -203,6 +213,17 @@ def load_library(path=None):
     if path is None:
         _lib = lib
     return lib
+
+
+def load_shim():
+    """The extension module host_shim.cpp is built into, bound to the library.  Raises if it is not built."""
+    try:
+        from . import _host_shim
+    except ImportError as e:
+        raise RuntimeError(f"the host extension of svox_amd.csrc cannot be loaded ({e}): build it "
+                           "(run `python -m svox_amd.csrc.build`)") from e
+    _host_shim.init(LIB_PATH)
+    return _host_shim
 
 
 def library_loaded():

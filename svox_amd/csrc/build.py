@@ -1,14 +1,17 @@
 """Build libsvox_hip.so for gfx950 with hipcc, in-tree (next to the sources): one object for the entry points and one
-per policy of the march kernels, compiled side by side and linked."""
+per policy of the march kernels, compiled side by side and linked; and, beside them, the host extension _host_shim.so
+(host_shim.cpp: plain C++ against torch's headers, no device code)."""
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libsvox_hip.so"
+SHIM_NAME = "_host_shim.so"
 
 # -ffp-contract=off: the kernels spell their fused multiply-adds out; the compiler adds none.
 # -munsafe-fp-atomics: floating-point atomicAdd becomes the hardware global_atomic_add.
@@ -40,12 +43,24 @@ def _run(cmd):
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     log = "\n".join(l for l in proc.stdout.splitlines() if "packed-fp32-ops" not in l)
     if proc.returncode != 0:
-        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + log)
+        raise RuntimeError("build failed: " + " ".join(cmd) + "\n" + log)
     return log
 
 
+def _shim_command(out):
+    import torch
+    root = os.path.dirname(torch.__file__)
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    libs = ["c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python", "dl"]
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+             "-DTORCH_EXTENSION_NAME=" + SHIM_NAME[:-3], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+            + [f for i in includes for f in ("-isystem", i)] + [os.path.join(HERE, "host_shim.cpp"), "-o", out]
+            + ["-L" + os.path.join(root, "lib")] + ["-l" + name for name in libs])
+
+
 def build_library(verbose=True):
-    """Compile the HIP sources into svox_amd/csrc/libsvox_hip.so.  Raises on failure."""
+    """Compile the sources into svox_amd/csrc/libsvox_hip.so and _host_shim.so.  Raises on failure."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     out = library_path()
     with tempfile.TemporaryDirectory(prefix="svox_build_") as scratch:
@@ -57,13 +72,19 @@ def build_library(verbose=True):
         if verbose:
             print(" ".join([hipcc] + HIPCC_FLAGS), "-c: one object per policy of the march kernels", flush=True)
         workers = int(os.environ.get("MAX_JOBS", 0)) or min(8, os.cpu_count() or 1)
+        shim = os.path.join(HERE, SHIM_NAME)
         with ThreadPoolExecutor(max_workers=workers) as pool:
+            host = pool.submit(_run, _shim_command(shim + ".tmp"))
             made = list(pool.map(compile_unit, list(_units())))
+            log = host.result()
+        if verbose and log.strip():
+            print(log)
         for _, log in made:
             if verbose and log.strip():
                 print(log)
         _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out + ".tmp"] + [obj for obj, _ in made])
     os.replace(out + ".tmp", out)
+    os.replace(shim + ".tmp", shim)
     return out
 
 

@@ -760,6 +760,10 @@ struct ReplaySpace {
     // > 0: the looks in a row after which a waiting wavefront of render_forward_split_kernel gives up, in place of
     // kSpinLimit (set by a debug flag, so that a test can see what a give-up leaves behind)
     int32_t spin_limit;
+    // where replay_backward_kernel reports how full the notes ran, for the caller to look at whenever it likes (host
+    // memory the device can write, or nullptr): stocks asked for in the upper half, stocks there are in the lower
+    unsigned long long* report;
+    uint32_t n_stocks;
     // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
     unsigned int* give_ups;
 };
@@ -2078,6 +2082,8 @@ __global__ __launch_bounds__(kMarchThreads) __attribute__((amdgpu_waves_per_eu(3
     const int64_t ray = ((int64_t)blockIdx.x << ray_shift) + lane;
     const bool seated = lane < (1 << ray_shift);
     const bool stamped = stamp_matches(ws);
+    if (ws.report && stamped && blockIdx.x == 0 && lane == 0)
+        __hip_atomic_store(ws.report, *ws.stocks_taken << 32 | ws.n_stocks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const float2* first = ws.base + ray * kChunkFloat2;
     int count = 0;
     int32_t first_link = 0;

@@ -507,6 +507,7 @@ bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, 
     ws->base = (float2*)workspace;
     ws->first_shared = n_slots;
     ws->n_chunks = chunks;
+    ws->n_stocks = (uint32_t)((chunks - n_slots + kChunkStock - 1) / kChunkStock);
     ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
     ws->stamp_at = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStampOffset);
     ws->stocks_taken = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStockCounterOffset);
@@ -652,13 +653,15 @@ int replay_ray_shift(bool image, int64_t n_rays) {
 template <class Source>
 int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest, const SvoxRenderOptions* opt,
                                const void* grad_output, void* grad_data_out, void* workspace, int64_t workspace_bytes,
-                               int64_t n_slots, const NoteStamp& stamp, hipStream_t stream, bool march1_known = false) {
+                               int64_t n_slots, const NoteStamp& stamp, hipStream_t stream, bool march1_known = false,
+                               int64_t* report = nullptr) {
     const int D = fast_basis(tree, opt);
     const int ray_shift = replay_ray_shift(is_image_source(all), n_slots);
     const unsigned waves = blocks_for(n_slots, 1 << ray_shift);
     ReplaySpace ws;
     carve_workspace(workspace, workspace_bytes, n_slots, &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
+    ws.report = (unsigned long long*)report;
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(waves), stream, all, *opt, (const float*)grad_output,
                                                                     (float*)grad_data_out, ws, ray_shift,
                                                                     march1_known ? 1 : 0, lobes_of(tree, opt)));
@@ -862,6 +865,14 @@ int svox_volume_render_noted(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays,
 int svox_volume_render_backward_noted(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays,
                                       const SvoxRenderOptions* opt, const void* grad_output, void* grad_data_out,
                                       int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
+    return svox_volume_render_backward_noted_with(tree, rays, opt, grad_output, grad_data_out, accumulate, workspace,
+                                                  workspace_bytes, nullptr, stream);
+}
+
+int svox_volume_render_backward_noted_with(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays,
+                                           const SvoxRenderOptions* opt, const void* grad_output, void* grad_data_out,
+                                           int32_t accumulate, void* workspace, int64_t workspace_bytes,
+                                           const SvoxNotesExtras* extras, void* stream) {
     int od;
     int rc = check_render(tree, opt, &od);
     if (rc) return rc;
@@ -880,7 +891,8 @@ int svox_volume_render_backward_noted(const SvoxTreeSpec* tree, const SvoxRaysSp
     if (!grad_output) return fail(SVOX_ERR_NULL_POINTER, "grad_output is NULL");
     const BatchSource<float> all = batch_source<float>(rays, true);
     return backward_from_notes(tree, all, all, opt, grad_output, grad_data_out, workspace, workspace_bytes,
-                               rays->n_rays, stamp_of(tree, rays, opt), (hipStream_t)stream);
+                               rays->n_rays, stamp_of(tree, rays, opt), (hipStream_t)stream, false,
+                               extras ? extras->report : nullptr);
 }
 
 int svox_volume_render_images_noted(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam, int32_t n_images,
@@ -908,6 +920,15 @@ int svox_volume_render_images_backward_noted(const SvoxTreeSpec* tree, const Svo
                                              int64_t pose_stride, const SvoxRenderOptions* opt,
                                              const void* grad_output, void* grad_data_out, int32_t accumulate,
                                              void* workspace, int64_t workspace_bytes, void* stream) {
+    return svox_volume_render_images_backward_noted_with(tree, cam, n_images, pose_stride, opt, grad_output, grad_data_out,
+                                                         accumulate, workspace, workspace_bytes, nullptr, stream);
+}
+
+int svox_volume_render_images_backward_noted_with(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam, int32_t n_images,
+                                                  int64_t pose_stride, const SvoxRenderOptions* opt,
+                                                  const void* grad_output, void* grad_data_out, int32_t accumulate,
+                                                  void* workspace, int64_t workspace_bytes, const SvoxNotesExtras* extras,
+                                                  void* stream) {
     int od;
     int rc = check_render(tree, opt, &od);
     if (rc) return rc;
@@ -927,7 +948,8 @@ int svox_volume_render_images_backward_noted(const SvoxTreeSpec* tree, const Svo
     if (!grad_output) return fail(SVOX_ERR_NULL_POINTER, "grad_output is NULL");
     const ImageSource<float> all = image_source<float>(cam, n_images, pose_stride, opt);
     return backward_from_notes(tree, all, all, opt, grad_output, grad_data_out, workspace, workspace_bytes, n_slots,
-                               stamp_of_image(tree, cam, n_images, opt), (hipStream_t)stream);
+                               stamp_of_image(tree, cam, n_images, opt), (hipStream_t)stream, false,
+                               extras ? extras->report : nullptr);
 }
 
 int svox_volume_render(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const SvoxRenderOptions* opt, void* out,
@@ -986,7 +1008,7 @@ int svox_notes_pool_info(int64_t n_rays, int64_t workspace_bytes, int64_t* count
     if (!carve_workspace(base, workspace_bytes, n_rays, &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "svox_notes_pool_info: the workspace does not hold a chunk per ray");
     *counter_offset = (int64_t)((char*)ws.stocks_taken - base);
-    *pool_stocks = (ws.n_chunks - ws.first_shared + kChunkStock - 1) / kChunkStock;
+    *pool_stocks = ws.n_stocks;
     return SVOX_OK;
 }
 

@@ -51,20 +51,22 @@ class NotesBudget:
     passes after it, up to MAX_FACTOR times the start (and to the memory limits of
     csrc._backward_workspace); passes that use less than a quarter of their room halve it again.
 
-    Nothing here waits for the GPU: the counter a pass leaves is copied to pinned memory behind the
-    pass, and looked at by a later pass only once the copy has arrived.  While the stream is being
-    captured into a graph (torch.cuda.graph) nothing is observed: a replay cannot change the size of
-    the buffers it was captured with, so the room stays what it was when the capture began."""
+    Nothing here waits for the GPU: the backward pass that uses the notes leaves in pinned memory how full
+    they ran (csrc.volume_render_backward_noted, `report`), and a later forward pass looks there.  While the stream is
+    being captured into a graph (torch.cuda.graph) nothing is observed: a replay cannot change the size of the
+    buffers it was captured with, so the room stays what it was when the capture began."""
 
     MAX_FACTOR = 16
+    _free = []                    # landing places of budgets that are gone (a place is used again, never given back:
+    #                               a kernel still under way may yet write to it -- then the next owner sees a stray figure)
 
     def __init__(self):
         self.factor = 1
-        self._pending = None      # (pinned int64[1], event, pool stocks) of the last pass looked after
-        self._landing = None      # the pinned buffer, allocated on first use
+        self._pending = None      # the landing place (a pinned tensor seen through numpy) while a report is awaited
+        self._landing = None      # (array, its address), taken at the first use
 
     def __getstate__(self):
-        # (a copy or a pickle of the renderer takes the figure along, not the buffer and the event)
+        # (a copy or a pickle of the renderer takes the figure along, not the landing place)
         return {"factor": self.factor}
 
     def __setstate__(self, state):
@@ -72,18 +74,20 @@ class NotesBudget:
         self._pending = None
         self._landing = None
 
+    def __del__(self):
+        if getattr(self, "_landing", None) is not None:
+            NotesBudget._free.append(self._landing)
+
     def records_per_ray(self):
         self._settle()
         return int(_C.BACKWARD_RECORDS_PER_RAY) * self.factor
 
     def _settle(self):
-        if self._pending is None or torch.cuda.is_current_stream_capturing():
+        if self._pending is None or self._pending[0] < 0 or torch.cuda.is_current_stream_capturing():
             return
-        landing, event, pool = self._pending
-        if not event.query():
-            return
+        said = int(self._pending[0])
         self._pending = None
-        self.adjust(int(landing[0]), pool)
+        self.adjust(said >> 32, said & 0xffffffff)
 
     def adjust(self, asked, pool):
         """One observation: `asked` stocks of chunks were asked for, the workspace had `pool`."""
@@ -92,17 +96,25 @@ class NotesBudget:
         elif asked * 4 < pool and self.factor > 1:
             self.factor //= 2
 
-    def observe(self, notes, n_rays):
-        """Called right after the launch of a noted forward pass (on the current stream)."""
-        if notes is None or self._pending is not None or torch.cuda.is_current_stream_capturing():
-            return
-        counter, pool = _C.notes_pool_use(notes, n_rays)
+    def report(self):
+        """Where a backward pass that starts now is to report: an address, or 0 (a report is awaited already, or the
+        pass is being captured)."""
+        if torch.cuda.is_current_stream_capturing():
+            return 0
+        if self._pending is not None:
+            # (a pass whose notes turned out not to be its own leaves no report: ask again after a while)
+            self._waited += 1
+            return self._landing[1] if self._waited > 64 else 0
         if self._landing is None:
-            self._landing = torch.empty(1, dtype=torch.int64, pin_memory=True)
-        self._landing.copy_(counter, non_blocking=True)
-        event = torch.cuda.Event()
-        event.record()
-        self._pending = (self._landing, event, pool)
+            if NotesBudget._free:
+                self._landing = NotesBudget._free.pop()
+            else:
+                pinned = torch.empty(1, dtype=torch.int64, pin_memory=True)
+                self._landing = (pinned.numpy(), pinned.data_ptr(), pinned)
+        self._waited = 0
+        self._pending = self._landing[0]
+        self._pending[0] = -1
+        return self._landing[1]
 
 
 class _VolumeRenderFunction(torch.autograd.Function):
@@ -116,13 +128,11 @@ class _VolumeRenderFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, data, tree, rays, opt, keep_notes=False, budget=None):
-        ctx.tree, ctx.rays, ctx.opt = tree, rays, opt
+        ctx.tree, ctx.rays, ctx.opt, ctx.budget = tree, rays, opt, budget
         ctx.notes = None
         ctx.versions = _versions(tree, rays)
         if keep_notes:
             out, ctx.notes = _C.volume_render_noted(tree, rays, opt, budget.records_per_ray() if budget else None)
-            if budget:
-                budget.observe(ctx.notes, int(rays.origins.shape[0]))
             return out
         return _C.volume_render(tree, rays, opt)
 
@@ -136,7 +146,8 @@ class _VolumeRenderFunction(torch.autograd.Function):
             # the empty leaves it ran with describe the old values; march through the tree as it is
             notes, ctx.tree.child_marks = None, None
         if notes is not None:
-            grad = _C.volume_render_backward_noted(ctx.tree, ctx.rays, ctx.opt, grad_out.contiguous(), notes)
+            grad = _C.volume_render_backward_noted(ctx.tree, ctx.rays, ctx.opt, grad_out.contiguous(), notes,
+                                                   ctx.budget.report() if ctx.budget else 0)
         else:
             grad = _C.volume_render_backward(ctx.tree, ctx.rays, ctx.opt, grad_out.contiguous())
         return grad, None, None, None, None, None
@@ -161,15 +172,12 @@ class _VolumeRenderImageFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, data, tree, cam, opt, keep_notes=False, budget=None):
-        ctx.tree, ctx.cam, ctx.opt = tree, cam, opt
+        ctx.tree, ctx.cam, ctx.opt, ctx.budget = tree, cam, opt, budget
         ctx.notes = None
         ctx.versions = _image_versions(tree, cam)
         if keep_notes:
             out, ctx.notes = _C.volume_render_images_noted(tree, cam, opt,
                                                            budget.records_per_ray() if budget else None)
-            if budget:
-                n_images = 1 if cam.c2w.dim() == 2 else int(cam.c2w.shape[0])
-                budget.observe(ctx.notes, n_images * cam.height * cam.width)
             return out
         return _C.volume_render_image(tree, cam, opt) if cam.c2w.dim() == 2 else _C.volume_render_images(tree, cam, opt)
 
@@ -180,7 +188,8 @@ class _VolumeRenderImageFunction(torch.autograd.Function):
         notes, ctx.notes = ctx.notes, None
         if ctx.versions != _image_versions(ctx.tree, ctx.cam):
             notes, ctx.tree.child_marks = None, None     # as in _VolumeRenderFunction.backward
-        grad = _C.volume_render_images_backward_noted(ctx.tree, ctx.cam, ctx.opt, grad_out.contiguous(), notes)
+        report = ctx.budget.report() if ctx.budget and notes is not None else 0
+        grad = _C.volume_render_images_backward_noted(ctx.tree, ctx.cam, ctx.opt, grad_out.contiguous(), notes, report)
         return grad, None, None, None, None, None
 
 
@@ -347,8 +356,8 @@ class VolumeRenderer(nn.Module):
         else:
             opts.ndc_width = -1
         opts.sigma_thresh = opts.stop_thresh = 1e-2 if fast else 0.0
-        if hasattr(self, "sigma_thresh"):
-            opts.sigma_thresh = self.sigma_thresh
-        if hasattr(self, "stop_thresh"):
-            opts.stop_thresh = self.stop_thresh
+        # (asked of the class and the instance's own attributes first: nn.Module takes microseconds to say no)
+        for name in ("sigma_thresh", "stop_thresh"):
+            if name in self.__dict__ or hasattr(type(self), name) or name in self._buffers or name in self._parameters:
+                setattr(opts, name, getattr(self, name))
         return opts
