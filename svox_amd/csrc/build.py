@@ -36,6 +36,7 @@ def _units():
     for fmt, basis in POLICIES:
         yield (f"march_{fmt.lower()}{basis}", "march_policy.hip",
                [f"-DSVOX_POLICY_FORMAT=SVOX_FORMAT_{fmt}", f"-DSVOX_POLICY_BASIS={basis}"])
+    yield "march_double", "march_double.hip", []
     yield "svox_hip", "svox_hip.hip", []
 
 
