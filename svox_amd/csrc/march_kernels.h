@@ -11,6 +11,7 @@
 #pragma once
 
 #include <cstddef>
+#include <type_traits>
 
 #include "basis.h"
 #include "tree_walk.h"
@@ -890,6 +891,21 @@ struct NoteTaker {
         first[kHeadFloat2 + 1] = make_float2(dscale, broken ? 2.0f : 0.0f);
         first[kHeadFloat2 + 2] = make_float2(march1_sum, 0.0f);
     }
+    // The end of a ray of a pass that takes the notes for replay_se_grad_kernel: its pixel, whose colour and light in
+    // front of the background are acc and light, as se_grad_kernel's first march leaves it (rt_kernel.cu:560-563,
+    // 635-637, 711-713), and in the head, in place of flag and sum, the residual against the reference colour.
+    __device__ __forceinline__ void finish_residual(bool broken, float dscale, const float* acc, float light, float bg,
+                                                    const float* __restrict__ color_ref, float* __restrict__ pixel) {
+        float resid[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            resid[c] = acc[c] + fma_(light, bg, -color_ref[c]);
+            pixel[c] = resid[c] + color_ref[c];
+        }
+        ((float*)(first + kHeadFloat2))[1] = __int_as_float(lost || broken ? -1 : count);
+        first[kHeadFloat2 + 1] = make_float2(dscale, resid[0]);
+        first[kHeadFloat2 + 2] = make_float2(resid[1], resid[2]);
+    }
 };
 
 // What a noting pass that has the gradient of the picture at hand accumulates per ray beside its notes:
@@ -947,7 +963,9 @@ struct March1Sum {
 // sigma > 0 of the whole ray, so a ray is walked to its end also after its picture stopped early, and
 // the colours of the leaves at or below sigma_thresh are evaluated too.  With out == nullptr only the
 // notes are taken (the backward pass without a forward pass before it); kGrad: that backward pass's
-// grad_out is given, and the sum of its first march is formed on the way (March1Sum).
+// grad_out is given, and the sum of its first march is formed on the way (March1Sum).  A pass that takes notes for
+// replay_se_grad_kernel (not kGrad, stop_thresh 0) is given the reference colours in grad_out's place
+// (NoteTaker::finish_residual).
 // kAllShaded: tr.child is a marked copy of the child table made with this launch's sigma_thresh (and softplus
 // setting): a leaf that is not marked has sigma > sigma_thresh, so the round has no density phase -- every
 // unmarked leaf goes on the shade list and its density arrives with its coefficients (one round trip to memory
@@ -1121,12 +1139,16 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
                     active = false;
             }
             if (active && (broken || !(r.t < r.tmax))) {
-                if (!painted) {
-                    out[slot * 3] = fma_(light, bg, acc[0]);
-                    out[slot * 3 + 1] = fma_(light, bg, acc[1]);
-                    out[slot * 3 + 2] = fma_(light, bg, acc[2]);
+                if (kNoted && !kGrad && grad_out) {
+                    notes.finish_residual(broken, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
+                } else {
+                    if (!painted) {
+                        out[slot * 3] = fma_(light, bg, acc[0]);
+                        out[slot * 3 + 1] = fma_(light, bg, acc[1]);
+                        out[slot * 3 + 2] = fma_(light, bg, acc[2]);
+                    }
+                    if constexpr (kNoted) notes.finish(broken, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
                 }
-                if constexpr (kNoted) notes.finish(broken, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
                 active = false;
             }
         }
@@ -1431,10 +1453,21 @@ __device__ __forceinline__ void add_records_by_leaf(int n, int lane, const int32
 // density terms and colour factors (20 bytes a record) fill ShadeShared::leaf and ::who exactly; the
 // owners follow the GroupScratch in ShadeShared::colour.
 constexpr int kEmitCap = kMarchThreads;
+// (kByRecord: the replay kernel's list, in ReplayShared.)
+constexpr int kReplayRows = 32;   // rays of a batch at most (more would cost wavefronts per CU in LDS)
+template <int D>
+struct ReplayShared {
+    int32_t leaf[kEmitCap];
+    float factor[kEmitCap * 4];
+    uint8_t owner[kEmitCap];
+    uint8_t start[kMarchThreads];    // ReplayRays::take
+    GroupScratch group;
+    float basis[kReplayRows * D];
+};
 template <class P, int D, bool kByRecord = false>
 struct RecordList {
     static constexpr int K = P::kRecord;
-    ShadeShared<D, true>& sh;
+    std::conditional_t<kByRecord, ReplayShared<D>, ShadeShared<D, true>>& sh;
     float* grad_data;
     int lane;
     MergeState& merge;
@@ -1442,8 +1475,18 @@ struct RecordList {
 
     __device__ __forceinline__ int32_t* leaves() const { return sh.leaf; }
     // per record four factors: the three colour factors tmp2[c], then the density term
-    __device__ __forceinline__ float* factors() const { return (float*)(sh.leaf + kEmitCap); }
-    __device__ __forceinline__ uint8_t* owners() const { return (uint8_t*)sh.colour + sizeof(GroupScratch); }
+    __device__ __forceinline__ float* factors() const {
+        if constexpr (kByRecord)
+            return sh.factor;
+        else
+            return (float*)(sh.leaf + kEmitCap);
+    }
+    __device__ __forceinline__ uint8_t* owners() const {
+        if constexpr (kByRecord)
+            return sh.owner;
+        else
+            return (uint8_t*)sh.colour + sizeof(GroupScratch);
+    }
 
     // element e of record rec: basis[i] * tmp2[c] for a colour coefficient, g_sigma for the density
     __device__ __forceinline__ float element(int rec, int e) const {
@@ -1456,7 +1499,12 @@ struct RecordList {
     }
 
     // The colours of the round are in registers by the time records are added: their LDS is free.
-    __device__ __forceinline__ GroupScratch& scratch() const { return *(GroupScratch*)sh.colour; }
+    __device__ __forceinline__ GroupScratch& scratch() const {
+        if constexpr (kByRecord)
+            return sh.group;
+        else
+            return *(GroupScratch*)sh.colour;
+    }
 
     // add_records_by_leaf for records longer than half a wavefront (one record at a time, lane e on
     // element e).  What the lanes need to find a record's values -- its place in the list, its leaf,
@@ -1800,12 +1848,16 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         const int32_t avail = (w & ~(kEndedBit | kBrokenBit)) - taken;
         if (active && (w & kEndedBit) && avail == 0) {
             // the ray left the tree: the background shows through what is left of the light
-            if (!painted) {
-                out[slot * 3] = fma_(light, bg, acc[0]);
-                out[slot * 3 + 1] = fma_(light, bg, acc[1]);
-                out[slot * 3 + 2] = fma_(light, bg, acc[2]);
+            if (kNoted && !kGrad && grad_out) {
+                notes.finish_residual((w & kBrokenBit) != 0, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
+            } else {
+                if (!painted) {
+                    out[slot * 3] = fma_(light, bg, acc[0]);
+                    out[slot * 3 + 1] = fma_(light, bg, acc[1]);
+                    out[slot * 3 + 2] = fma_(light, bg, acc[2]);
+                }
+                if constexpr (kNoted) notes.finish((w & kBrokenBit) != 0, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
             }
-            if constexpr (kNoted) notes.finish((w & kBrokenBit) != 0, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
             active = false;
         }
         if (!__any(active)) break;
@@ -2056,157 +2108,350 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
     }
 }
 
-// The backward pass from the notes a noting forward kernel left (NoteTaker): one lane per ray, no
-// tree walk.  The notes of a ray (leaf, step length, sigma, the three sigmoids of every leaf with
-// sigma > 0) are read twice, five at a time: first for the sum the reference's first march forms
-// (rt_kernel.cu:358-419), then for the gradient records of its second march (:421-475), which the
-// wavefront adds together as render_backward_kernel does.  A ray whose notes are incomplete, or every
-// ray if the workspace carries another stamp, is left to a launch of render_backward_kernel with the
-// bitmap this kernel writes (one word per wavefront).
-constexpr int kReplayGroup = 5;
-static_assert(kChunkRecords % kReplayGroup == 0, "a group of notes never straddles two chunks");
+// ---- notes read back ---------------------------------------------------------------------------
+// The replay kernels give every NOTE a lane.  A block of four wavefronts owns 2^ray_shift rays (16 to 64) and lists
+// those that have notes; then its wavefronts take from the list, each time as many rays as fit with all their notes
+// into 64 lanes, lane l the l-th note: exponentials, colours and factors of 64 leaves at a time.  What has to be formed
+// one leaf after the other -- the transmittance in front of a leaf, the colour that lies behind it -- is passed from
+// lane to lane (each_in_turn).  A ray with more than 64 notes is taken alone, 64 notes at a time, once for its sum and
+// once for its records.
+// (One lane per ray, as the march has it, is the wrong shape here: where one ray in five meets the scene, and those
+// differ in length, 60 to 95 % of the lanes idle, and every ray's notes are read twice, first for the sum of the first
+// march.  replay_backward_kernel from that to this: 4 096 rays of a 16^3 RGBA tree 22.6 -> 9.1 us, 50 001 rays of a
+// 256^3 SH9 shell with softplus 244 -> 82 us, 1 Mi rays of a 512^3 SH16 shell 457 -> 378 us, an 800x800 picture of
+// it 414 -> 296 us; replay_se_grad_kernel, 200 003 rays, 256^3 SH9: 199 -> 111 us.  What is left of the large cases is the
+// rate of the atomic additions, about 16 requests of 64 bytes a nanosecond: without them 159 and 151 us.)
+// A ray whose notes are incomplete, or every ray if the workspace carries another stamp, is marked in the bitmap for a
+// launch of the marching kernel.
+constexpr int kReplayMaxShift = 6;
+constexpr int kReplayWaves = 4;
+constexpr int kReplayThreads = kReplayWaves * kMarchThreads;
 
+// one ray of the list; link: its second chunk, or, if `known`, where ReplayRays::chunks has its chunks from the second on
+struct ReplayRay {
+    int32_t ray;
+    uint32_t known : 1;
+    int32_t count : 31;
+    int32_t link;
+    float dscale;
+};
+// one lane's note
+struct ReplayNote {
+    bool valid;
+    int owner;      // row of the ray in LDS
+    int32_t ray;
+    int p, count;   // place among the notes of the ray that are in this batch, and their number
+    int last;       // lane of the last of them
+    int32_t leaf;
+    float dt, raw, s[3], dscale;
+};
+struct ReplayRays {
+    // The chunks of a ray's notes are a chain, and to follow it is one trip to memory after the other.  The rays of the
+    // list follow theirs all at once, before the first note is read, as long as there is room to keep what they find.
+    static constexpr int kChunks = 512;
+    ReplayRay list[1 << kReplayMaxShift];
+    int32_t chunks[kChunks];
+    int n, cursor;   // of the list: rays, and rays taken
+    int n_chunks;
+
+    // Lists the rays of block `block` of `blocks` that have notes and writes its part of the bitmap of undone rays.
+    // The rays are dealt out in pieces of 16 neighbours: neighbouring pixels share leaves, whose records are added
+    // together.  They are also all long or all short together, so the pieces of a block come from all over the launch:
+    // piece number b of the k-th `blocks` pieces goes to block b - k * 0.618 blocks (without the turn a block would get
+    // pieces below one another wherever the width of a picture divides `blocks`).
+    __device__ __forceinline__ void gather(const ReplaySpace& ws, bool stamped, int64_t n_slots, int block, int blocks,
+                                           int ray_shift) {
+        static_assert(1 << kReplayMaxShift <= kMarchThreads, "one wavefront looks the rays up");
+        const int lane = threadIdx.x;
+        if (lane < kMarchThreads) {
+            if (lane == 0) cursor = n_chunks = 0;
+            const unsigned k = (unsigned)lane >> 4, turn = (unsigned)((float)blocks * 0.618f);
+            const int64_t ray = (((int64_t)k * blocks + ((unsigned)block + k * turn) % (unsigned)blocks) << 4) + (lane & 15);
+            const bool seated = lane < (1 << ray_shift) && ray < n_slots;
+            int32_t count = 0, link = 0;
+            float dscale = 0.0f;
+            if (seated) {
+                const float2* first = ws.base + ray * kChunkFloat2;
+                const float2 head = first[kHeadFloat2], tail = first[kHeadFloat2 + 1];
+                link = __float_as_int(head.x);
+                count = stamped ? __float_as_int(head.y) : -1;
+                dscale = tail.x;
+            }
+            const unsigned long long undone = __ballot(count < 0), m = __ballot(count > 0);
+            if ((lane & 15) == 0 && seated) ((uint16_t*)ws.undone)[ray >> 4] = (uint16_t)(undone >> lane);
+            if (lane == 0) n = __popcll(m);
+            wave_lds_sync();
+            if (count > 0) {
+                const int more = (count - 1) / kChunkRecords;
+                const int to = more > 0 && more <= kChunks ? atomicAdd(&n_chunks, more) : 0;
+                const bool known = more > 0 && more <= kChunks && to + more <= kChunks;
+                list[rank_in(m)] = ReplayRay{(int32_t)ray, known ? 1u : 0u, count, known ? to : link, dscale};
+                if (known) {
+                    int32_t index = link;
+                    for (int at = 0; at < more; ++at) {
+                        if (at > 0) index = __float_as_int(ws.base[(int64_t)index * kChunkFloat2 + kHeadFloat2].x);
+                        chunks[to + at] = index;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // reads note i of ray r; chunk, index: number and place of a chunk at or before the note's (0 and the first chunk
+    // if nothing is known), moved on to the note's
+    __device__ __forceinline__ void read(const ReplaySpace& ws, const ReplayRay& r, int i, int& chunk, int32_t& index,
+                                         ReplayNote& g) const {
+        const int want = i / kChunkRecords;
+        const bool known = r.known != 0;
+        if (g.valid && want > 0) {
+            if (known) index = chunks[r.link + want - 1];
+            if (known) chunk = want;
+        }
+        while (__any(g.valid && chunk < want)) {
+            if (g.valid && chunk < want) {
+                index = chunk == 0 ? r.link : __float_as_int(ws.base[(int64_t)index * kChunkFloat2 + kHeadFloat2].x);
+                chunk += 1;
+            }
+        }
+        if (g.valid) {
+            const float2* e = ws.base + (int64_t)index * kChunkFloat2 + (i - want * kChunkRecords) * 3;
+            const float2 a = e[0], b = e[1], c = e[2];
+            g.leaf = __float_as_int(a.x);
+            g.dt = a.y;
+            g.raw = b.x;
+            g.s[0] = b.y;
+            g.s[1] = c.x;
+            g.s[2] = c.y;
+        }
+    }
+
+    // Takes the next rays of the list whose notes fit into the wavefront: `at` receives the first of them (n: the list
+    // is used up), n_notes the number of their notes, g each lane's note.  Returns how many rays these are; 0: one ray
+    // that has more than 64 notes.
+    __device__ __forceinline__ int take(const ReplaySpace& ws, uint8_t* start, int lane, int& at, int& n_notes,
+                                        ReplayNote& g) {
+        int rays, sum, count;
+        bool fits;
+        at = __builtin_amdgcn_readfirstlane(__atomic_load_n(&cursor, __ATOMIC_RELAXED));
+        while (true) {
+            if (at >= n) return 0;
+            count = at + lane < n ? list[at + lane].count : 0;
+            sum = count <= kMarchThreads ? count : kMarchThreads + 1;
+#pragma unroll
+            for (int off = 1; off < kMarchThreads; off <<= 1) {
+                const int other = __shfl_up(sum, off);
+                if (lane >= off) sum += other;
+            }
+            fits = at + lane < n && sum <= kMarchThreads && lane < kReplayRows;
+            rays = __popcll(__ballot(fits));
+            int seen = at;
+            if (lane == 0) seen = atomicCAS(&cursor, at, at + (rays > 0 ? rays : 1));
+            seen = __builtin_amdgcn_readfirstlane(seen);
+            if (seen == at) break;
+            at = seen;   // (another wavefront was faster)
+        }
+        if (rays == 0) return 0;
+        n_notes = __builtin_amdgcn_readlane(sum, rays - 1);
+        start[lane] = 0;
+        wave_lds_sync();
+        if (fits) start[sum - count] = 1;
+        wave_lds_sync();
+        const unsigned long long starts = __ballot(start[lane] != 0);
+        const unsigned long long upto = starts & (~0ull >> (63 - lane));
+        g.valid = lane < n_notes;
+        g.owner = __popcll(upto) - 1;
+        const int first = 63 - __builtin_clzll(upto);
+        g.p = lane - first;
+        const ReplayRay r = list[at + g.owner];
+        g.ray = r.ray;
+        g.count = r.count;
+        g.last = first + r.count - 1;
+        g.dscale = r.dscale;
+        int chunk = 0;
+        int32_t index = r.ray;
+        read(ws, r, g.p, chunk, index, g);
+        return rays;
+    }
+
+    // notes [64 * segment, 64 * segment + 64) of entry `at`; chunk, index: where the segment before it left off
+    __device__ __forceinline__ void take_segment(const ReplaySpace& ws, int at, int segment, int lane, int& chunk,
+                                                 int32_t& index, ReplayNote& g) {
+        const ReplayRay r = list[at];
+        if (segment == 0) {
+            chunk = 0;
+            index = r.ray;
+        }
+        const int i = segment * kMarchThreads + lane;
+        g.valid = i < r.count;
+        g.owner = 0;
+        g.ray = r.ray;
+        g.p = lane;
+        g.count = r.count - segment * kMarchThreads < kMarchThreads ? r.count - segment * kMarchThreads : kMarchThreads;
+        g.last = g.count - 1;
+        g.dscale = r.dscale;
+        read(ws, r, i, chunk, index, g);
+        chunk = __builtin_amdgcn_readlane(chunk, __builtin_amdgcn_readfirstlane(g.last));
+        index = __builtin_amdgcn_readlane(index, __builtin_amdgcn_readfirstlane(g.last));
+    }
+};
+
+// The march's running values over the lanes of every ray: each lane applies its leaf to the value of the lane before it
+// (the first lane of a ray to `seed`), over and over; after k turns the first k lanes of every ray hold their final
+// values.  In this order, and not as prefix sums of fewer turns, because what lies behind a leaf is a difference of
+// sums: the rounding of the reference's order is part of small gradients.
+// A turn is two or three instructions for all rays of the batch.
+template <class Step>
+__device__ __forceinline__ void each_in_turn(const ReplayNote& g, Step&& step) {
+    for (int turn = 0; __any(g.valid && g.p >= turn); turn += 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) step();
+    }
+}
+__device__ __forceinline__ float lane_before(float v) {
+    constexpr int kWaveShiftRight1 = 0x138;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kWaveShiftRight1, 0xf, 0xf, false));
+}
+// transmittance in front of the lane's leaf (first leaf of a ray: seed)
+__device__ __forceinline__ float light_before(const ReplayNote& g, float att, float seed) {
+    float before = seed, after = 0.0f;
+    each_in_turn(g, [&]() {
+        const float neighbour = lane_before(after);   // (read by every lane, whatever it does with it)
+        before = g.p == 0 ? seed : neighbour;
+        after = before * att;
+    });
+    return before;
+}
+// running sums of weight * value[i], the lane's own included, into sum
+template <int N>
+__device__ __forceinline__ void running_sums(const ReplayNote& g, float weight, const float (&value)[N],
+                                             const float (&seed)[N], float (&sum)[N]) {
+    float run[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) run[i] = 0.0f;
+    each_in_turn(g, [&]() {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float neighbour = lane_before(run[i]);
+            run[i] = fma_(weight, value[i], g.p == 0 ? seed[i] : neighbour);
+        }
+    });
+#pragma unroll
+    for (int i = 0; i < N; ++i) sum[i] = run[i];
+}
+
+// The backward pass from the notes a noting forward kernel left (NoteTaker), trace_ray_backward's second march
+// (rt_kernel.cu:358-475: the sum of the first march, then the records of the second).
 template <class P, class Source>
-__global__ __launch_bounds__(kMarchThreads) __attribute__((amdgpu_waves_per_eu(3))) void replay_backward_kernel(Source src, SvoxRenderOptions opt,
-                                                                        const float* __restrict__ grad_out,
-                                                                        float* __restrict__ grad_data,
-                                                                        ReplaySpace ws, int ray_shift,
-                                                                        int march1_known, Lobes lobes) {
+__global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source src, SvoxRenderOptions opt,
+                                                                         const float* __restrict__ grad_out,
+                                                                         float* __restrict__ grad_data, ReplaySpace ws,
+                                                                         int ray_shift, Lobes lobes) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
-    __shared__ ShadeShared<D, true> sh;
-    const int lane = threadIdx.x;
-    // A wavefront takes 2^ray_shift consecutive rays (64 or 16), one per lane from lane 0.  Adding a
-    // step's records is work of the whole wavefront, one record after the other; where the rays of a
-    // wavefront are neighbours (the pixels of an image) they are all long or all short together, and
-    // fewer of them per wavefront spread a long run of pixels over several wavefronts.
-    const int64_t ray = ((int64_t)blockIdx.x << ray_shift) + lane;
-    const bool seated = lane < (1 << ray_shift);
+    __shared__ ReplayShared<D> shared[kReplayWaves];
+    __shared__ ReplayRays rays;
+    const int lane = threadIdx.x & (kMarchThreads - 1);
+    ReplayShared<D>& sh = shared[threadIdx.x / kMarchThreads];
     const bool stamped = stamp_matches(ws);
-    if (ws.report && stamped && blockIdx.x == 0 && lane == 0)
+    if (ws.report && stamped && blockIdx.x == 0 && threadIdx.x == 0)
         __hip_atomic_store(ws.report, *ws.stocks_taken << 32 | ws.n_stocks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    const float2* first = ws.base + ray * kChunkFloat2;
-    int count = 0;
-    int32_t first_link = 0;
-    float dscale = 0.0f;
-    if (seated && ray < src.n_slots()) {
-        const float2 head = first[kHeadFloat2], tail = first[kHeadFloat2 + 1];
-        first_link = __float_as_int(head.x);
-        count = stamped ? __float_as_int(head.y) : -1;
-        dscale = tail.x;
-    }
-    // (the wavefront's part of the bitmap: a word or a quarter of one)
-    const unsigned long long undone = __ballot(count < 0);
-    if (lane == 0) {
-        if (ray_shift == 6)
-            ws.undone[blockIdx.x] = undone;
-        else
-            ((uint16_t*)ws.undone)[blockIdx.x] = (uint16_t)undone;
-    }
-    const bool work = count > 0;
-    if (!__any(work)) return;
+    rays.gather(ws, stamped, src.n_slots(), (int)blockIdx.x, (int)gridDim.x, ray_shift);
 
     const float bg = opt.background_brightness;
     const float pad = opt.rgb_padding;
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
-    float go[3] = {0.f, 0.f, 0.f};
-    if (work) {
-        if constexpr (P::kFormat != SVOX_FORMAT_RGBA) {
-            float vdir[3];
-            src.view_dir(ray, vdir);
-            float basis[D];
-            policy_basis<P>(lobes, opt, vdir, basis);
-#pragma unroll
-            for (int i = 0; i < D; ++i) sh.basis[lane * D + i] = basis[i];
-        }
-        go[0] = grad_out[ray * 3];
-        go[1] = grad_out[ray * 3 + 1];
-        go[2] = grad_out[ray * 3 + 2];
-    }
-    wave_lds_sync();   // the basis rows are read by other lanes when the records are added
-
-    float light = 1.0f, accum = 0.0f;
-    // march1_known: the pass that took the notes had grad_out and left the sum of the first march in
-    // the head of the ray's notes (March1Sum: the same expressions in the same order as pass 0 below)
-    if (march1_known && work) accum = first[kHeadFloat2 + 2].x;
-    MergeState merge{2};   // (a wavefront of 64 unrelated rays flushes about twice: it never looks)
+    MergeState merge;
     RecordList<P, D, true> records{sh, grad_data, lane, merge};
-    struct Group {
-        float2 note[kReplayGroup][3];
-    };
-#pragma unroll 1
-    for (int pass = march1_known ? 1 : 0; pass < 2; ++pass) {
-        const float2* chunk = first;
-        int32_t link = first_link;
-        int pos = 0;
-        // asks for the group of notes that starts at note `base` (the loads are waited for where the
-        // group is worked on: meanwhile the group before it is)
-        auto fetch = [&](Group& g, int base) {
-            if (work && base < count) {
-                if (pos == kChunkRecords) {
-                    chunk = ws.base + (int64_t)link * kChunkFloat2;
-                    link = __float_as_int(chunk[kHeadFloat2].x);
-                    pos = 0;
-                }
+    // the basis rows of the rays of a batch (entry at + lane by lane)
+    auto set_rows = [&](int at, int n_rays) {
+        if constexpr (P::kFormat != SVOX_FORMAT_RGBA) {
+            if (lane < n_rays) {
+                float vdir[3];
+                src.view_dir(rays.list[at + lane].ray, vdir);
+                float basis[D];
+                policy_basis<P>(lobes, opt, vdir, basis);
 #pragma unroll
-                for (int k = 0; k < kReplayGroup; ++k) {
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) g.note[k][j] = chunk[(pos + k) * 3 + j];
-                }
-                pos += kReplayGroup;
+                for (int i = 0; i < D; ++i) sh.basis[lane * D + i] = basis[i];
             }
-        };
-        auto work_on = [&](const Group& g, int base) {
-#pragma unroll
-            for (int k = 0; k < kReplayGroup; ++k) {
-                const bool have = work && base + k < count;
-                const int32_t leaf = __float_as_int(g.note[k][0].x);
-                const float dt = g.note[k][0].y, raw = g.note[k][1].x;   // (the stored density)
-                const float s[3] = {g.note[k][1].y, g.note[k][2].x, g.note[k][2].y};
-                float tmp2[3] = {0.f, 0.f, 0.f};
-                float g_sigma = 0.0f;
-                if (have) {
-                    const float sigma = opt.density_softplus ? softplus_m1(raw) : raw;
-                    const float att = expf_fixed(-dt * sigma * dscale);
-                    const float weight = light * (1.0f - att);
-                    float total_color = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) total_color = fma_(fma_(s[c], d_rgb_pad, -pad), go[c], total_color);
-                    light *= att;
-                    if (pass == 0) {
-                        accum = fma_(weight, total_color, accum);
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            if constexpr (P::kFormat == SVOX_FORMAT_RGBA) {
-                                tmp2[c] = weight * s[c] * (1.0f - s[c]) * go[c] * d_rgb_pad;
-                            } else {
-                                tmp2[c] = (float)((double)(weight * s[c]) * (1.0 - (double)s[c]) * (double)go[c] *
-                                                  (double)d_rgb_pad);
-                            }
-                        }
-                        accum = fma_(-weight, total_color, accum);
-                        g_sigma = dt * dscale * fma_(total_color, light, -accum);
-                        if (opt.density_softplus) g_sigma *= sigmoid_(raw - 1.0f);
-                    }
-                }
-                if (pass == 1) records.append(have, leaf, tmp2, g_sigma);
-            }
-        };
-        Group a, b;
-        fetch(a, 0);
-        for (int base = 0; __any(work && base < count); base += 2 * kReplayGroup) {
-            fetch(b, base + kReplayGroup);
-            work_on(a, base);
-            fetch(a, base + 2 * kReplayGroup);
-            work_on(b, base + kReplayGroup);
         }
-        if (pass == 0) {
-            const float total_grad = (go[0] + go[1]) + go[2];
-            accum = fma_(light * bg, total_grad, accum);
-            light = 1.0f;
+    };
+    float go[3];
+    float att, total_color[1];   // of the lane's leaf
+    auto look = [&](const ReplayNote& g) {
+        go[0] = go[1] = go[2] = 0.0f;
+        att = 1.0f;
+        total_color[0] = 0.0f;
+        if (g.valid) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) go[c] = grad_out[(int64_t)g.ray * 3 + c];
+            const float sigma = opt.density_softplus ? softplus_m1(g.raw) : g.raw;
+            att = expf_fixed(-g.dt * sigma * g.dscale);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) total_color[0] = fma_(fma_(g.s[c], d_rgb_pad, -pad), go[c], total_color[0]);
+        }
+    };
+    // the records of a batch; behind: what lies behind the lane's leaf
+    auto add = [&](const ReplayNote& g, int n_notes, float light, float behind) {
+        if (g.valid) {
+            const float weight = light * (1.0f - att);
+            sh.leaf[lane] = g.leaf;
+            records.owners()[lane] = (uint8_t)g.owner;
+            float* const f = records.factors() + lane * 4;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                if constexpr (P::kFormat == SVOX_FORMAT_RGBA) {
+                    f[c] = weight * g.s[c] * (1.0f - g.s[c]) * go[c] * d_rgb_pad;
+                } else {
+                    f[c] = (float)((double)(weight * g.s[c]) * (1.0 - (double)g.s[c]) * (double)go[c] * (double)d_rgb_pad);
+                }
+            }
+            float g_sigma = g.dt * g.dscale * fma_(total_color[0], light * att, -behind);
+            if (opt.density_softplus) g_sigma *= sigmoid_(g.raw - 1.0f);   // rt_kernel.cu:471-474
+            f[3] = g_sigma;
+        }
+        records.n = n_notes;
+        records.flush();
+    };
+    while (true) {
+        ReplayNote g;
+        int at, n_notes = 0;
+        const int taken = rays.take(ws, sh.start, lane, at, n_notes, g);
+        if (at >= rays.n) break;
+        if (taken > 0) {
+            set_rows(at, taken);
+            look(g);
+            const float light = light_before(g, att, 1.0f);
+            const float weight = light * (1.0f - att);
+            float run[1] = {0.0f};
+            running_sums(g, weight, total_color, run, run);
+            const int last = g.valid ? g.last : lane;
+            run[0] = fma_(__shfl(light * att, last) * bg, (go[0] + go[1]) + go[2], __shfl(run[0], last));
+            running_sums(g, -weight, total_color, run, run);
+            add(g, n_notes, light, run[0]);
+            continue;
+        }
+        set_rows(at, 1);
+        const int segments = (rays.list[at].count + kMarchThreads - 1) / kMarchThreads;
+        float run[1] = {0.0f};
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+            float through = 1.0f;   // transmittance in front of the segment
+            int chunk = 0;
+            int32_t index = 0;
+            for (int k = 0; k < segments; ++k) {
+                rays.take_segment(ws, at, k, lane, chunk, index, g);
+                look(g);
+                const float light = light_before(g, att, through);
+                const float weight = light * (1.0f - att);
+                float behind[1];
+                running_sums(g, pass == 0 ? weight : -weight, total_color, run, behind);
+                run[0] = __shfl(behind[0], g.last);
+                through = __shfl(light * att, g.last);
+                if (pass == 1) add(g, g.count, light, behind[0]);
+            }
+            if (pass == 0) run[0] = fma_(through * bg, __shfl((go[0] + go[1]) + go[2], 0), run[0]);
         }
     }
-    records.flush();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2608,91 +2853,37 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
     }
 }
 
-// se_grad from the notes a noting forward kernel left (NoteTaker; taken with both thresholds at
-// zero): one lane per ray, no tree walk.  The first pass over a ray's notes forms the residual and the
-// rendered colour as march 1 of se_grad_kernel does, the second pass the gradient and Hessian records
-// of its march 2, term by term the same values; the wavefront adds the records of its rays together,
-// each lane serving one element of one record (RecordList::flush_by_record's scheme, with two output
-// arrays).  Rays that miss the tree keep the background colour the noting launch wrote; a ray whose
-// notes are incomplete, or every ray if the workspace carries another stamp, is marked in the bitmap
-// for a launch of se_grad_kernel.
-constexpr int kSeRecordCap = 48;
-static_assert(kSeRecordCap <= kMarchThreads, "group_by_leaf holds one record per lane");
-
+// se_grad from the notes a noting forward kernel left (NoteTaker; taken with both thresholds at zero, the colours
+// written and the residuals left in the heads by finish_residual): the records of march 2 of se_grad_kernel, term by
+// term the same values, a note to a lane (ReplayRays).  A ray whose notes are incomplete, or every ray if the workspace
+// carries another stamp, is marked in the bitmap for a launch of se_grad_kernel.
+template <int D>
+struct ReplaySeShared : ReplayShared<D> {
+    float hess_sigma[kEmitCap];             // the density term of the Hessian (factor[3]: that of the gradient)
+    float resid[kReplayRows * 3];
+};
 template <class P, class Source>
-__global__ __launch_bounds__(kMarchThreads) void replay_se_grad_kernel(Source src, SvoxRenderOptions opt,
-                                                                       const float* __restrict__ color_ref,
-                                                                       float* __restrict__ color_out,
-                                                                       float* __restrict__ grad_data,
-                                                                       float* __restrict__ hess_data,
-                                                                       ReplaySpace ws, int ray_shift, Lobes lobes) {
+__global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source src, SvoxRenderOptions opt,
+                                                                        float* __restrict__ grad_data,
+                                                                        float* __restrict__ hess_data, ReplaySpace ws,
+                                                                        int ray_shift, Lobes lobes) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
     constexpr bool kRgba = P::kFormat == SVOX_FORMAT_RGBA;
-    __shared__ float basis_rows[kMarchThreads * D];
-    __shared__ float resid_rows[kMarchThreads * 3];
-    __shared__ int32_t l_leaf[kSeRecordCap];
-    // per record four gradient factors (the three colour factors, then the density term) and the
-    // density term of the Hessian
-    __shared__ float l_factor[kSeRecordCap * 4], l_hs[kSeRecordCap];
-    __shared__ uint8_t l_owner[kSeRecordCap];
-    __shared__ GroupScratch group;
-    const int lane = threadIdx.x;
-    // 2^ray_shift consecutive rays per wavefront (64, or 16 for the pixels of images), as in
-    // replay_backward_kernel
-    const int64_t ray = ((int64_t)blockIdx.x << ray_shift) + lane;
-    const bool seated = lane < (1 << ray_shift);
-    const bool stamped = stamp_matches(ws);
-    const float2* first = ws.base + ray * kChunkFloat2;
-    int count = 0;
-    int32_t first_link = 0;
-    float dscale = 0.0f;
-    bool missed = true;
-    if (seated && ray < src.n_slots()) {
-        const float2 head = first[kHeadFloat2], tail = first[kHeadFloat2 + 1];
-        first_link = __float_as_int(head.x);
-        count = stamped ? __float_as_int(head.y) : -1;
-        dscale = tail.x;
-        missed = tail.y != 0.0f;
-    }
-    const unsigned long long undone = __ballot(count < 0);
-    if (lane == 0) {
-        if (ray_shift == 6)
-            ws.undone[blockIdx.x] = undone;
-        else
-            ((uint16_t*)ws.undone)[blockIdx.x] = (uint16_t)undone;
-    }
-    const bool hit = count >= 0 && !missed;   // the rays this launch answers
-    const bool work = hit && count > 0;
-    if (!__any(hit)) return;
+    __shared__ ReplaySeShared<D> shared[kReplayWaves];
+    __shared__ ReplayRays rays;
+    const int lane = threadIdx.x & (kMarchThreads - 1);
+    ReplaySeShared<D>& sh = shared[threadIdx.x / kMarchThreads];
+    rays.gather(ws, stamp_matches(ws), src.n_slots(), (int)blockIdx.x, (int)gridDim.x, ray_shift);
 
     const float bg = opt.background_brightness;
     const float pad = opt.rgb_padding;
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
-    float ref[3] = {0.f, 0.f, 0.f};
-    if (hit) {
-        ref[0] = color_ref[ray * 3];
-        ref[1] = color_ref[ray * 3 + 1];
-        ref[2] = color_ref[ray * 3 + 2];
-    }
-    if (work) {
-        if constexpr (!kRgba) {
-            float vdir[3];
-            src.view_dir(ray, vdir);
-            float basis[D];
-            policy_basis<P>(lobes, opt, vdir, basis);
-#pragma unroll
-            for (int i = 0; i < D; ++i) basis_rows[lane * D + i] = basis[i];
-        }
-    }
-
-    int n = 0;   // records in the list (wavefront-uniform)
-    MergeState merge{2};
-    auto flush = [&]() {
-        if (n == 0) return;
+    MergeState merge;
+    auto flush = [&](int n) {
         wave_lds_sync();
         // where enough records share a leaf, the records of a leaf are brought together first
-        const bool grouped = group_by_leaf(group, merge, l_leaf, n, lane);
+        const bool grouped = group_by_leaf(sh.group, merge, sh.leaf, n, lane);
         auto emit = [&](int32_t leaf, int e, const float* sum) {
             const int64_t at = (int64_t)leaf * K + e;
             atomicAdd(grad_data + at, sum[0]);
@@ -2704,9 +2895,9 @@ __global__ __launch_bounds__(kMarchThreads) void replay_se_grad_kernel(Source sr
             // record have their addresses from scalars and those of four records are in flight together
             // (RecordList::add_held).
             const bool mine = lane < n;
-            const int my_rec = mine ? (grouped ? group.order[lane] : lane) : 0;
-            const int my_leaf = l_leaf[my_rec];
-            const int my_owner = l_owner[my_rec];
+            const int my_rec = mine ? (grouped ? sh.group.order[lane] : lane) : 0;
+            const int my_leaf = sh.leaf[my_rec];
+            const int my_owner = sh.owner[my_rec];
             constexpr int kBlock = 4;
             // (a loop every lane runs, so that every lane holds its record when readlane looks: see add_held)
             for (int e0 = 0; e0 < K; e0 += kMarchThreads) {
@@ -2727,10 +2918,10 @@ __global__ __launch_bounds__(kMarchThreads) void replay_se_grad_kernel(Source sr
                         const int rec = __builtin_amdgcn_readlane(my_rec, a);
                         const int owner = __builtin_amdgcn_readlane(my_owner, a);
                         leaf[u] = __builtin_amdgcn_readlane(my_leaf, a);
-                        f[u] = l_factor[rec * 4 + c];
-                        b[u] = kRgba ? 1.0f : basis_rows[owner * D + i];
-                        rs[u] = resid_rows[owner * 3 + cc];
-                        hs[u] = l_hs[rec];
+                        f[u] = sh.factor[rec * 4 + c];
+                        b[u] = kRgba ? 1.0f : sh.basis[owner * D + i];
+                        rs[u] = sh.resid[owner * 3 + cc];
+                        hs[u] = sh.hess_sigma[rec];
                     }
 #pragma unroll
                     for (int u = 0; u < kBlock; ++u) {
@@ -2750,151 +2941,131 @@ __global__ __launch_bounds__(kMarchThreads) void replay_se_grad_kernel(Source sr
             }
         } else {
             add_records_by_leaf<K, 2>(
-                n, lane, grouped ? group.leaf : l_leaf,
+                n, lane, grouped ? sh.group.leaf : sh.leaf,
                 // element e of a record: colour coefficient (c, i) or, last, the density
                 [&](int at, int e, float* t) {
-                    const int rec = grouped ? group.order[at] : at;
+                    const int rec = grouped ? sh.group.order[at] : at;
                     const int c = kRgba ? e : e / D;
                     if (c < 3) {
-                        const int owner = l_owner[rec];
-                        const float v = l_factor[rec * 4 + c];
-                        const float gw = kRgba ? v : basis_rows[owner * D + (e - c * D)] * v;
-                        t[0] = gw * resid_rows[owner * 3 + c];
+                        const int owner = sh.owner[rec];
+                        const float v = sh.factor[rec * 4 + c];
+                        const float gw = kRgba ? v : sh.basis[owner * D + (e - c * D)] * v;
+                        t[0] = gw * sh.resid[owner * 3 + c];
                         t[1] = gw * gw;
                     } else {
-                        t[0] = l_factor[rec * 4 + 3];
-                        t[1] = l_hs[rec];
+                        t[0] = sh.factor[rec * 4 + 3];
+                        t[1] = sh.hess_sigma[rec];
                     }
                 },
                 emit);
         }
         wave_lds_sync();
-        n = 0;
     };
-    // the record of every lane with `emit` set joins the list (in lane order)
-    auto append = [&](bool emit, int32_t leaf, const float* gci, float g_sigma, float h_sigma) {
-        unsigned long long todo = __ballot(emit);
-        while (todo) {
-            if (n == kSeRecordCap) flush();
-            const bool pending = (todo >> lane) & 1ull;
-            const int at = n + rank_in(todo);
-            const bool take = pending && at < kSeRecordCap;
-            if (take) {
-                l_leaf[at] = leaf;
-                l_owner[at] = (uint8_t)lane;
-                l_hs[at] = h_sigma;
-                l_factor[at * 4] = gci[0];
-                l_factor[at * 4 + 1] = gci[1];
-                l_factor[at * 4 + 2] = gci[2];
-                l_factor[at * 4 + 3] = g_sigma;
+    // what the march of a ray starts from, entry at + lane by lane
+    auto set_rows = [&](int at, int n_rays) {
+        if (lane < n_rays) {
+            const int64_t ray = rays.list[at + lane].ray;
+            const float2* head = ws.base + ray * kChunkFloat2 + kHeadFloat2;
+            const float2 r = head[2];
+            sh.resid[lane * 3] = head[1].y;
+            sh.resid[lane * 3 + 1] = r.x;
+            sh.resid[lane * 3 + 2] = r.y;
+            if constexpr (!kRgba) {
+                float vdir[3];
+                src.view_dir(ray, vdir);
+                float basis[D];
+                policy_basis<P>(lobes, opt, vdir, basis);
+#pragma unroll
+                for (int i = 0; i < D; ++i) sh.basis[lane * D + i] = basis[i];
             }
-            const unsigned long long taken = __ballot(take);
-            n += __popcll(taken);
-            todo &= ~taken;
         }
+        wave_lds_sync();
     };
-
-    float resid[3] = {0.f, 0.f, 0.f};    // pass 0: colour so far; afterwards the residual
-    float caccum[3] = {0.f, 0.f, 0.f};   // rendered colour not yet passed (second spelling)
-    float light = 1.0f, light1 = 1.0f;
-    struct Group {
-        float2 note[kReplayGroup][3];
+    float att, col[3];   // of the lane's leaf
+    auto look = [&](const ReplayNote& g) {
+        const float sigma = opt.density_softplus ? softplus_m1(g.raw) : g.raw;
+        att = g.valid ? expf_fixed(-g.dt * sigma * g.dscale) : 1.0f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) col[c] = g.valid ? fma_(g.s[c], d_rgb_pad, -pad) : 0.0f;
     };
+    // the records of a batch; behind: the colour that lies behind the lane's leaf
+    auto add = [&](const ReplayNote& g, int n_notes, float light, const float* behind) {
+        if (g.valid) {
+            const float weight = light * (1.0f - att), after = light * att;
+            const float sg = opt.density_softplus ? sigmoid_(g.raw - 1.0f) : 1.0f;
+            const float d_sg = sg * (1.0f - sg);
+            float g_sigma = 0.0f, h_sigma = 0.0f;
+            sh.leaf[lane] = g.leaf;
+            sh.owner[lane] = (uint8_t)g.owner;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                if constexpr (kRgba) {
+                    sh.factor[lane * 4 + c] = weight * g.s[c] * (1.0f - g.s[c]) * d_rgb_pad;
+                } else {
+                    sh.factor[lane * 4 + c] =
+                        (float)((double)(weight * g.s[c]) * (1.0 - (double)g.s[c]) * (double)d_rgb_pad);
+                }
+                const float gs = g.dt * g.dscale * fma_(col[c], after, -behind[c]);
+                const float resid = sh.resid[g.owner * 3 + c];
+                if (opt.density_softplus) {
+                    g_sigma += gs * resid * sg;
+                    h_sigma += fma_(gs * gs * sg, sg, gs * d_sg);
+                } else {
+                    g_sigma += gs * resid;
+                    h_sigma += gs * gs;
+                }
+            }
+            sh.factor[lane * 4 + 3] = g_sigma;
+            sh.hess_sigma[lane] = h_sigma;
+        }
+        flush(n_notes);
+    };
+    while (true) {
+        ReplayNote g;
+        int at, n_notes = 0;
+        const int taken = rays.take(ws, sh.start, lane, at, n_notes, g);
+        if (at >= rays.n) break;
+        if (taken > 0) {
+            set_rows(at, taken);
+            look(g);
+            const float light = light_before(g, att, 1.0f);
+            const float weight = light * (1.0f - att);
+            const int last = g.valid ? g.last : lane;
+            const float through = __shfl(light * att, last);
+            float run[3] = {0.0f, 0.0f, 0.0f};
+            running_sums(g, weight, col, run, run);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) run[c] = fma_(through, bg, __shfl(run[c], last));
+            running_sums(g, -weight, col, run, run);
+            add(g, n_notes, light, run);
+            continue;
+        }
+        set_rows(at, 1);
+        const int segments = (rays.list[at].count + kMarchThreads - 1) / kMarchThreads;
+        float run[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-    for (int pass = 0; pass < 2; ++pass) {
-        const float2* chunk = first;
-        int32_t link = first_link;
-        int pos = 0;
-        auto fetch = [&](Group& g, int base) {
-            if (work && base < count) {
-                if (pos == kChunkRecords) {
-                    chunk = ws.base + (int64_t)link * kChunkFloat2;
-                    link = __float_as_int(chunk[kHeadFloat2].x);
-                    pos = 0;
-                }
+        for (int pass = 0; pass < 2; ++pass) {
+            float through = 1.0f;   // transmittance in front of the segment
+            int chunk = 0;
+            int32_t index = 0;
+            for (int k = 0; k < segments; ++k) {
+                rays.take_segment(ws, at, k, lane, chunk, index, g);
+                look(g);
+                const float light = light_before(g, att, through);
+                const float weight = light * (1.0f - att);
+                float behind[3];
+                running_sums(g, pass == 0 ? weight : -weight, col, run, behind);
 #pragma unroll
-                for (int k = 0; k < kReplayGroup; ++k) {
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) g.note[k][j] = chunk[(pos + k) * 3 + j];
-                }
-                pos += kReplayGroup;
+                for (int c = 0; c < 3; ++c) run[c] = __shfl(behind[c], g.last);
+                through = __shfl(light * att, g.last);
+                if (pass == 1) add(g, g.count, light, behind);
             }
-        };
-        auto work_on = [&](const Group& g, int base) {
+            if (pass == 0) {
 #pragma unroll
-            for (int k = 0; k < kReplayGroup; ++k) {
-                const bool have = work && base + k < count;
-                const int32_t leaf = __float_as_int(g.note[k][0].x);
-                const float dt = g.note[k][0].y, raw = g.note[k][1].x;   // (the stored density)
-                const float s[3] = {g.note[k][1].y, g.note[k][2].x, g.note[k][2].y};
-                float gci[3] = {0.f, 0.f, 0.f};
-                float g_sigma = 0.0f, h_sigma = 0.0f;
-                if (have) {
-                    const float sigma = opt.density_softplus ? softplus_m1(raw) : raw;
-                    const float att = expf_fixed(-dt * sigma * dscale);
-                    const float weight = light * (1.0f - att);
-                    float col[3];
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) col[c] = fma_(s[c], d_rgb_pad, -pad);
-                    light *= att;
-                    if (pass == 0) {
-                        const float att1 = expf_fixed(-dt * dscale * sigma);
-                        const float weight1 = light1 * (1.0f - att1);
-                        light1 *= att1;
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            resid[c] = fma_(weight1, col[c], resid[c]);
-                            caccum[c] = fma_(weight, col[c], caccum[c]);
-                        }
-                    } else {
-                        const float sg = opt.density_softplus ? sigmoid_(raw - 1.0f) : 1.0f;
-                        const float d_sg = sg * (1.0f - sg);
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            if constexpr (kRgba) {
-                                gci[c] = weight * s[c] * (1.0f - s[c]) * d_rgb_pad;
-                            } else {
-                                gci[c] = (float)((double)(weight * s[c]) * (1.0 - (double)s[c]) * (double)d_rgb_pad);
-                            }
-                            caccum[c] = fma_(-weight, col[c], caccum[c]);
-                            const float gs = dt * dscale * fma_(col[c], light, -caccum[c]);
-                            if (opt.density_softplus) {
-                                g_sigma += gs * resid[c] * sg;
-                                h_sigma += fma_(gs * gs * sg, sg, gs * d_sg);
-                            } else {
-                                g_sigma += gs * resid[c];
-                                h_sigma += gs * gs;
-                            }
-                        }
-                    }
-                }
-                if (pass == 1) append(have, leaf, gci, g_sigma, h_sigma);
+                for (int c = 0; c < 3; ++c) run[c] = fma_(through, bg, run[c]);
             }
-        };
-        Group a, b;
-        fetch(a, 0);
-        for (int base = 0; __any(work && base < count); base += 2 * kReplayGroup) {
-            fetch(b, base + kReplayGroup);
-            work_on(a, base);
-            fetch(a, base + 2 * kReplayGroup);
-            work_on(b, base + kReplayGroup);
-        }
-        if (pass == 0) {
-            // the end of march 1 (rt_kernel.cu:560-563, the background of :635-637, and :711-713)
-            if (hit) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    resid[c] += fma_(light1, bg, -ref[c]);
-                    caccum[c] = fma_(light, bg, caccum[c]);
-                    color_out[ray * 3 + c] = resid[c] + ref[c];
-                    resid_rows[lane * 3 + c] = resid[c];
-                }
-            }
-            light = 1.0f;
-            wave_lds_sync();   // basis and residual rows are read by other lanes when the records are added
         }
     }
-    flush();
 }
 
 // ------------------------------------------------------------------------------------------------

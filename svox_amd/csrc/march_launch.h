@@ -16,20 +16,19 @@ struct MarchLaunch {
                         const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool split, bool accum, bool refill,
                         bool all_shaded);
     static void noting(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
-                       const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out, bool split,
-                       bool refill);
+                       const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out,
+                       const float* color_ref, bool split, bool refill);
     static void backward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                          const SvoxRenderOptions& opt, const float* grad_out, float* grad_data, const ReplaySpace& ws,
                          bool refill, bool second_only);
     static void replay_backward(dim3 blocks, hipStream_t stream, const Source& src, const SvoxRenderOptions& opt,
                                 const float* grad_out, float* grad_data, const ReplaySpace& ws, int ray_shift,
-                                int march1_known, const Lobes& lobes);
+                                const Lobes& lobes);
     static void se_grad(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                         const SvoxRenderOptions& opt, const float* color_ref, float* color_out, float* grad, float* hess,
                         const unsigned long long* only, bool refill);
     static void replay_se_grad(dim3 blocks, hipStream_t stream, const Source& src, const SvoxRenderOptions& opt,
-                               const float* color_ref, float* color_out, float* grad, float* hess, const ReplaySpace& ws,
-                               int ray_shift, const Lobes& lobes);
+                               float* grad, float* hess, const ReplaySpace& ws, int ray_shift, const Lobes& lobes);
 };
 
 #ifdef SVOX_INSTANTIATE_POLICY
@@ -60,9 +59,10 @@ void MarchLaunch<P, Source>::forward(dim3 blocks, hipStream_t stream, const Tree
 template <class P, class Source>
 void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                                     const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out,
-                                    bool split, bool refill) {
-#define SVOX_NOTING(THREADS, ...) \
-    hipLaunchKernelGGL((__VA_ARGS__), blocks, dim3(THREADS), 0, stream, tr, src, opt, out, ws, grad_out)
+                                    const float* color_ref, bool split, bool refill) {
+    // (the colours take the gradient's place in the variants without it)
+#define SVOX_NOTING(THREADS, ...)                                                                                        \
+    hipLaunchKernelGGL((__VA_ARGS__), blocks, dim3(THREADS), 0, stream, tr, src, opt, out, ws, grad_out ? grad_out : color_ref)
     if (split && grad_out)
         SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, true>);
     else if (split)
@@ -99,9 +99,9 @@ void MarchLaunch<P, Source>::backward(dim3 blocks, hipStream_t stream, const Tre
 template <class P, class Source>
 void MarchLaunch<P, Source>::replay_backward(dim3 blocks, hipStream_t stream, const Source& src,
                                              const SvoxRenderOptions& opt, const float* grad_out, float* grad_data,
-                                             const ReplaySpace& ws, int ray_shift, int march1_known, const Lobes& lobes) {
-    hipLaunchKernelGGL((replay_backward_kernel<P, Source>), blocks, dim3(kMarchThreads), 0, stream, src, opt, grad_out,
-                       grad_data, ws, ray_shift, march1_known, lobes);
+                                             const ReplaySpace& ws, int ray_shift, const Lobes& lobes) {
+    hipLaunchKernelGGL((replay_backward_kernel<P, Source>), blocks, dim3(kReplayThreads), 0, stream, src, opt, grad_out,
+                       grad_data, ws, ray_shift, lobes);
 }
 
 template <class P, class Source>
@@ -118,11 +118,10 @@ void MarchLaunch<P, Source>::se_grad(dim3 blocks, hipStream_t stream, const Tree
 
 template <class P, class Source>
 void MarchLaunch<P, Source>::replay_se_grad(dim3 blocks, hipStream_t stream, const Source& src,
-                                            const SvoxRenderOptions& opt, const float* color_ref, float* color_out,
-                                            float* grad, float* hess, const ReplaySpace& ws, int ray_shift,
-                                            const Lobes& lobes) {
-    hipLaunchKernelGGL((replay_se_grad_kernel<P, Source>), blocks, dim3(kMarchThreads), 0, stream, src, opt, color_ref,
-                       color_out, grad, hess, ws, ray_shift, lobes);
+                                            const SvoxRenderOptions& opt, float* grad, float* hess,
+                                            const ReplaySpace& ws, int ray_shift, const Lobes& lobes) {
+    hipLaunchKernelGGL((replay_se_grad_kernel<P, Source>), blocks, dim3(kReplayThreads), 0, stream, src, opt, grad, hess,
+                       ws, ray_shift, lobes);
 }
 #endif  // SVOX_INSTANTIATE_POLICY
 

@@ -45,7 +45,7 @@ thread_local int g_debug_flags = 0;
 //   SVOX_IMAGE_RUN     16x16 blocks of one image in a row before the next image's, in multi-image launches
 //   SVOX_SPLIT_FORWARD 0 / 1: forward launches never / always on two wavefronts per tile
 //   SVOX_SPLIT_BLOCKS  largest forward launch (in tiles) that takes two wavefronts per tile
-//   SVOX_REPLAY_SHIFT  4 or 6: log2 of the rays a wavefront of the replay kernels takes
+//   SVOX_REPLAY_SHIFT  4, 5 or 6: log2 of the rays a block of the replay kernels takes
 struct Tuning {
     int per_wave = 0, refill = 0, xcd_group = 0, tile_order = -1, image_run = -1, split_forward = -1, replay_shift = -1;
     long split_blocks = -1;
@@ -590,7 +590,7 @@ ImageSource<T> noting_shape(const ImageSource<T>& s) { return s; }
 template <class Source>
 int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, void* out,
                  void* workspace, int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp,
-                 hipStream_t stream, const void* grad_out = nullptr) {
+                 hipStream_t stream, const void* grad_out = nullptr, const void* color_ref = nullptr) {
     const int D = fast_basis(tree, opt);
     const unsigned blocks = blocks_for(total_items_of(src), src.per_wave);
     const Source dealt = dealt_out(src, blocks);
@@ -605,7 +605,8 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     const bool refill = src.per_wave > kMarchThreads;
     const bool split = !refill && use_split_forward(blocks, is_image_source(src), opt, false);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
-                                                           (float*)out, ws, (const float*)grad_out, split, refill));
+                                                           (float*)out, ws, (const float*)grad_out,
+                                                           (const float*)color_ref, split, refill));
     return SVOX_OK;
 }
 
@@ -672,13 +673,16 @@ NoteStamp stamp_of_image(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam, in
     return stamp_of(tree, &as_rays, opt);
 }
 
-// log2 of the rays a wavefront of the replay kernels takes: 16 rays for the pixels of images (neighbours,
-// long together) and for batches that do not fill the GPU with 64 (up to 64 Ki rays: 4 096 rays of a 16^3
-// tree 246 -> 196 us, 64 Ki rays 350 -> 333 us), 64 for larger ray batches (1 Mi rays: 0.68 against 0.83 ms
-// with 16).
-int replay_ray_shift(bool image, int64_t n_rays) {
-    const int forced_shift = tuning().replay_shift;
-    return forced_shift == 4 || forced_shift == 6 ? forced_shift : (image || n_rays <= 65536 ? 4 : 6);
+// log2 of the rays a block of the replay kernels takes: as many as leave 1024 blocks (four wavefronts for every SIMD),
+// between 16 and 64.  Fewer cost the blocks' own time (start, heads of the notes), more leave the last blocks running
+// alone: 50 001 rays 99 / 91 / 96 us with 16 / 32 / 64, an 800x800 picture 337 / 300 / 310 / 333 us with
+// 32 / 64 / 128 / 256, 1 Mi rays 376 / 376 / 381 / 398 us.
+int replay_shift(int64_t n_rays) {
+    const int forced = tuning().replay_shift;
+    if (forced >= 4 && forced <= kReplayMaxShift) return forced;
+    int shift = 4;
+    while (shift < kReplayMaxShift && n_rays >= ((int64_t)1024 << (shift + 1))) ++shift;
+    return shift;
 }
 
 // The backward pass of `all` from the notes in the workspace: the rays with complete notes by
@@ -691,15 +695,15 @@ int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest
                                int64_t n_slots, const NoteStamp& stamp, hipStream_t stream, bool march1_known = false,
                                int64_t* report = nullptr) {
     const int D = fast_basis(tree, opt);
-    const int ray_shift = replay_ray_shift(is_image_source(all), n_slots);
-    const unsigned waves = blocks_for(n_slots, 1 << ray_shift);
+    const int ray_shift = replay_shift(n_slots);
+    const unsigned replay_blocks = blocks_for(n_slots, 1 << ray_shift);
     ReplaySpace ws;
     carve_workspace(workspace, workspace_bytes, n_slots, &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.report = (unsigned long long*)report;
-    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(waves), stream, all, *opt, (const float*)grad_output,
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(replay_blocks), stream, all, *opt, (const float*)grad_output,
                                                                     (float*)grad_data_out, ws, ray_shift,
-                                                                    march1_known ? 1 : 0, lobes_of(tree, opt)));
+                                                                    lobes_of(tree, opt)));
     int rc = check_launch("volume_render_backward_noted");
     if (rc) return rc;
     ReplaySpace only{};
@@ -753,17 +757,18 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
                        const void* color_ref, void* color_out, void* grad, void* hess, void* workspace,
                        int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp, hipStream_t stream) {
     const int D = fast_basis(tree, opt);
-    int rc = launch_noted(tree, noting_shape(all), opt, color_out, workspace, workspace_bytes, n_slots, stamp, stream);
+    int rc = launch_noted(tree, noting_shape(all), opt, color_out, workspace, workspace_bytes, n_slots, stamp, stream, nullptr,
+                          color_ref);
     if (rc) return rc;
     rc = check_launch("se_grad");
     if (rc) return rc;
     ReplaySpace ws;
     carve_workspace(workspace, workspace_bytes, n_slots, &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
-    const int ray_shift = replay_ray_shift(is_image_source(all), n_slots);
+    const int ray_shift = replay_shift(n_slots);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_se_grad(dim3(blocks_for(n_slots, 1 << ray_shift)), stream, all, *opt,
-                                                                   (const float*)color_ref, (float*)color_out, (float*)grad,
-                                                                   (float*)hess, ws, ray_shift, lobes_of(tree, opt)));
+                                                                   (float*)grad, (float*)hess, ws, ray_shift,
+                                                                   lobes_of(tree, opt)));
     rc = check_launch("se_grad");
     if (rc) return rc;
     launch_se_grad<Source, float>(tree, rest, opt, 3, color_ref, color_out, grad, hess, stream, ws.undone);
