@@ -18,6 +18,7 @@
 namespace svox {
 
 constexpr int kGroupLanes = 4;
+constexpr int kGroupSeekBudget = 2;   // child reads in a turn of the walk
 constexpr int kGroupRays = kMarchThreads / kGroupLanes;
 
 // value of lane k of the caller's group of four (every lane of the group takes part)
@@ -34,7 +35,7 @@ __device__ __forceinline__ double from_group(double v) {
 
 // The march of one ray.  Lane c of the group keeps axis c of the ray (lane 3 axis 0 again) and the group puts the three
 // together where all are needed: double-precision arithmetic is what a turn consists of.  A turn makes at most
-// kSeekBudget child reads; a longer descent goes on in the next turn, so that the other rays of the wavefront do not
+// kGroupSeekBudget child reads; a longer descent goes on in the next turn, so that the other rays of the wavefront do not
 // wait for it.
 struct GroupWalk {
     double o, d, inv, up;      // this lane's axis; up = max(inv, 0), see leaf_exit
@@ -80,7 +81,7 @@ struct GroupWalk {
         bool open = true, deep = false;
         int32_t cell = 0;
 #pragma unroll
-        for (int it = 0; it < kSeekBudget; ++it) {
+        for (int it = 0; it < kGroupSeekBudget; ++it) {
             if (open) {
                 path[(min(level, kPathLevels + 1) - 1) * kMarchThreads] = node;
                 cell = (node << 3) | cell_at(nx, ny, nz, level);

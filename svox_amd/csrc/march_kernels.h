@@ -27,6 +27,9 @@ constexpr int kMarchThreads = 64;  // one wavefront per block: finished tiles fr
 // nothing here has to wait for.)
 __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// __any without the detour through vector registers that the library's takes
+__device__ __forceinline__ bool any_lane(bool b) { return __builtin_amdgcn_ballot_w64(b) != 0ull; }
+
 // ------------------------------------------------------------------------------------------------
 // ray sources
 // ------------------------------------------------------------------------------------------------
@@ -314,11 +317,11 @@ __device__ __forceinline__ void advance(RayState<T>& r, T delta_t) {
 }
 
 struct Visit {
-    int64_t leaf;  // cell index node*N^3 + cell; -1 ends the ray (malformed tree); -2 descent pending
+    int64_t leaf;  // cell index node*N^3 + cell; -1 ends the ray (malformed tree)
     int levels;
 };
 
-// Child entries one lane reads per turn of the octree walk (OctreeCursor::seek_flat).  A lane that needs
+// Child entries one lane reads per turn of the octree walk (OctreeCursor::turn).  A lane that needs
 // more (its ray crossed the boundary of a large cell and has to descend many levels) goes on in its
 // next turn, so that the other lanes of the wavefront do not wait for it: measured, the lanes need
 // 2.0 entries per leaf on average, but the slowest lane of a wavefront 4.8.  (Budgets of 1 and 3, and
@@ -341,49 +344,143 @@ __device__ __forceinline__ Visit step_generic(const TreeDev<T>& tr, const RaySta
     return v;
 }
 
-// One turn of the octree walk for the whole wavefront, written flat: the lanes with `go` take one
-// sample (slot_leaf, slot_dt) and advance, or keep a descent pending (slot_leaf -1); the others run
-// the same instructions without effect.  `broken`: the tree is malformed, the ray ends here.
+// The walk of one lane's ray through the tree, sample after sample.  A sample's integer coordinates (24 bits an axis)
+// say which cell it lies in at every level, and those it shares with the sample before say how far up the next search
+// has to start: the node ids of the previous path are kept in LDS, one column per lane (`path`, laid out
+// [kPathLevels + 1][64]: path[64 * l], l < kPathLevels, is the node whose child row is indexed at level l + 1, path[0]
+// the root, node 0; the last row is a dump for the levels below, which no search resumes from).
+//
+// The march waits for this chain -- position, coordinates, path, child reads, step -- once per leaf, and where no other
+// wavefront fills the gaps its instructions count as much as its reads.  So the ray's origin and direction are kept
+// times 2^24 (exact: the coordinates need no further product), the sample is looked up in the path as soon as it is
+// known (aim) rather than when its turn comes, and there is no state but (level, node): an interrupted descent is one
+// that has not found its leaf yet.  (Before, as selects over pending
+// and finished searches, a turn was 145 vector instructions instead of 110.  Forward kernels: 800x800 picture of a
+// 512^3 SH16 shell 369 -> 343 us, 8 such pictures 688 -> 660 us, an NDC picture 616 -> 583 us; noting: 50 001 rays
+// 266 -> 240 us, 1 Mi rays 710 -> 661 us.  Keeping whole child rows of the last four levels in LDS as well, so that a
+// step costs one read instead of two, made the two-wavefront kernel 3 to 8 % faster where it runs alone on a CU, and
+// everything else up to 45 % slower.)
+struct OctreeCursor {
+    int32_t* rows;         // the lane's column of the path, counted from level 1: rows[64 * level]
+    float p[3];            // the sample, clamped, times 2^24
+    uint32_t ix, iy, iz;   // its integer coordinates
+    int level;             // where the search for its leaf stands: the child row to look into at this level ...
+    int32_t node;          // ... is that of this node
+    int levels;            // of the previous leaf (1: none, or one the path says nothing of)
+
+    // `lane_path`: this lane's column
+    __device__ __forceinline__ void reset(int32_t* lane_path) {
+        rows = lane_path - kMarchThreads;
+        lane_path[0] = 0;
+        p[0] = p[1] = p[2] = 0.0f;
+        ix = iy = iz = 0;
+        level = levels = 1;
+        node = 0;
+    }
+    // the first sample of a ray fresh from setup_ray
+    __device__ __forceinline__ void begin(RayState<float>& r) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            r.o[i] *= 16777216.0f;
+            r.d[i] *= 16777216.0f;
+        }
+        levels = 1;
+        aim(r);
+    }
+    // the sample at r.t
+    __device__ __forceinline__ void aim(const RayState<float>& r) {
+        // (clamp01, times 2^24)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            p[i] = max_(0.0f, min_(__uint_as_float(0x3F7FFFEFu) * 16777216.0f, fma_(r.t, r.d[i], r.o[i])));
+        const uint32_t nx = (uint32_t)p[0], ny = (uint32_t)p[1], nz = (uint32_t)p[2];
+        const uint32_t diff = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
+        // the first level the two samples differ at (a huge number: none)
+        const uint32_t first_diff = (diff ? (uint32_t)__builtin_clz(diff) : 0xffffffffu) - (31 - kCoordBits);
+        level = (int)min(min(first_diff, (uint32_t)levels), (uint32_t)kPathLevels);
+        node = rows[level * kMarchThreads];
+        ix = nx;
+        iy = ny;
+        iz = nz;
+    }
+    // One turn of the lanes with `go`: up to kSeekBudget child reads, and if the leaf is found its index (with
+    // kEmptyLeafBit if it is marked empty) in slot_leaf, the step of the sample in slot_dt, and the ray moved on; else
+    // slot_leaf is -1.  Returns whether the lane's sample lies deeper than the coordinates resolve.
+    // Node ids read from the table are clamped into [0, last_node]: a malformed tree yields a wrong leaf, never an
+    // access outside the table.  The table is smaller than 4 GiB (checked on the host): a 32-bit byte offset from the
+    // uniform base lets the load use the scalar-base form.
+    __device__ __forceinline__ bool turn(RayState<float>& r, bool go, const int32_t* __restrict__ child, int32_t last_node,
+                                         float step_size, int32_t& slot_leaf, float& slot_dt) {
+        slot_leaf = -1;
+        slot_dt = 0.0f;
+        int32_t cell = 0, skip = 1;   // (a lane that does not search keeps its 1)
+#pragma unroll
+        for (int it = 0; it < kSeekBudget; ++it) {
+            if (go && skip > 0 && level <= kCoordBits) {
+                rows[min(level, kPathLevels + 1) * kMarchThreads] = node;
+                cell = (node << 3) | cell_at(ix, iy, iz, level);
+                skip = *(const int32_t*)((const char*)child + ((uint32_t)cell << 2));
+                // (of a lane that has found its leaf the node is of no more use)
+                node = (int32_t)min((uint32_t)(node + skip), (uint32_t)last_node);
+                level += skip > 0 ? 1 : 0;
+            }
+        }
+        const bool deep = go && level > kCoordBits;
+        if (skip <= 0) {
+            // 2^(levels - 24) and 2^-levels: dividing by the power of two is the multiplication by its reciprocal
+            const uint32_t level_bits = (uint32_t)level << 23;
+            const float to_leaf = __uint_as_float(level_bits + ((uint32_t)(127 - kCoordBits) << 23));
+            const float inv_cube = __uint_as_float((127u << 23) - level_bits);
+            // leaf-local position frac(pos * 2^levels): s - floor(s), exact for the non-negative s of a clamped
+            // coordinate, in one instruction
+            float local[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) local[j] = __builtin_amdgcn_fractf(p[j] * to_leaf);
+            slot_leaf = skip < 0 ? cell | kEmptyLeafBit : cell;
+            slot_dt = leaf_exit(local, r.inv) * inv_cube + step_size;
+            const float t_next = r.t + slot_dt;
+            r.t = t_next > r.t ? t_next : r.tmax;   // (advance())
+            levels = level;
+            aim(r);
+        }
+        return deep;
+    }
+};
+
+// One turn of the walk for the whole wavefront: the lanes with `go` take one sample (slot_leaf, slot_dt) and advance,
+// or keep a descent open (slot_leaf -1).  `broken`: the tree is malformed, the ray ends here.
 __device__ __forceinline__ void walk_turn_flat(const TreeDev<float>& tr, RayState<float>& r, OctreeCursor& cur,
                                                float step_size, bool go, bool& broken, int32_t& slot_leaf,
                                                float& slot_dt) {
-    float pc[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) pc[j] = clamp01(fma_(r.t, r.d[j], r.o[j]));
     // (trees with another branching factor have no exact integer formulation: every lane takes the reference's
     // floating-point walk below, from the root for every sample, and shares everything else with the octrees)
     const bool octree = tr.N == 2;
-    int32_t leaf = go ? -1 : OctreeCursor::kIdle;
-    if (octree)
-        leaf = cur.seek_flat<kSeekBudget>(go, tr.child, (int32_t)(tr.capacity - 1), cell_coord(pc[0]), cell_coord(pc[1]),
-                                          cell_coord(pc[2]));
-    // 2^levels and 2^-levels: dividing by the power of two is the multiplication by its reciprocal
-    const float cube = __uint_as_float((uint32_t)(127 + cur.levels) << 23);
-    float inv_cube = __uint_as_float((uint32_t)(127 - cur.levels) << 23);
-    float cells_per_axis = 1.0f;   // N^levels where it is no power of two
-    float local[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) local[j] = leaf_local(pc[j], cube);
-    const bool deep = leaf == -1;
-    if (__any(deep)) {
+    bool deep = go;
+    slot_leaf = -1;
+    slot_dt = 0.0f;
+    if (octree) deep = cur.turn(r, go, tr.child, (int32_t)(tr.capacity - 1), step_size, slot_leaf, slot_dt);
+    if (__builtin_expect(any_lane(deep), 0)) {
         if (deep) {
             // more levels than the integer coordinates hold, another branching factor, or a broken tree
+            float local[3], cells_per_axis;
             int levels_f;
 #pragma unroll
-            for (int j = 0; j < 3; ++j) local[j] = pc[j];
-            leaf = (int32_t)descend_generic<float>(tr.child, tr.capacity, tr.N, local, &cells_per_axis, &levels_f, true);
-            inv_cube = 1.0f / cells_per_axis;
-            broken = broken || leaf < 0;
+            for (int j = 0; j < 3; ++j) local[j] = cur.p[j] * (1.0f / 16777216.0f);
+            slot_leaf = (int32_t)descend_generic<float>(tr.child, tr.capacity, tr.N, local, &cells_per_axis, &levels_f, true);
+            cur.levels = 1;
+            if (slot_leaf >= 0) {
+                // (rt_kernel.cu:274 divides by the cell count; for a power of two the product with the reciprocal is
+                // the same number)
+                const float segment = leaf_exit(local, r.inv);
+                slot_dt = (octree ? segment * (1.0f / cells_per_axis) : segment / cells_per_axis) + step_size;
+                const float t_next = r.t + slot_dt;
+                r.t = t_next > r.t ? t_next : r.tmax;
+                cur.aim(r);
+            } else {
+                broken = true;
+            }
         }
     }
-    const float segment = leaf_exit(local, r.inv);
-    // (rt_kernel.cu:274 divides by the cell count; for a power of two the product with the reciprocal is the same number)
-    const float delta_t = (octree ? segment * inv_cube : segment / cells_per_axis) + step_size;
-    const bool ok = leaf >= 0;
-    slot_leaf = ok ? leaf : -1;
-    slot_dt = ok ? delta_t : 0.0f;
-    const float t_next = r.t + delta_t;
-    r.t = ok ? (t_next > r.t ? t_next : r.tmax) : r.t;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -670,7 +767,7 @@ __device__ __forceinline__ void walk_turns(const TreeDev<float>& tr, RayState<fl
         const bool go = active && !broken && r.t < r.tmax;
         q_leaf[q] = -1;
         q_dt[q] = 0.0f;
-        if (__any(go)) walk_turn_flat(tr, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
+        if (any_lane(go)) walk_turn_flat(tr, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
     }
 }
 
@@ -1008,7 +1105,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     March1Sum sum1;
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
     OctreeCursor cur;
-    cur.reset(path + lane, kMarchThreads);
+    cur.reset(path + lane);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
     auto start = [&](int64_t item) {
@@ -1028,7 +1125,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
             }
             acc[0] = acc[1] = acc[2] = 0.0f;
             light = 1.0f;
-            cur.restart();
+            cur.begin(r);
             active = true;
             if constexpr (kNoted) {
                 painted = out == nullptr;   // no picture asked for: nothing to compose
@@ -1054,7 +1151,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
             if (state == kRoundRefilled) continue;
             if (state == kRoundDone) break;
         } else {
-            if (!__any(active)) break;
+            if (!any_lane(active)) break;
         }
 
         // ---- walk
@@ -1217,7 +1314,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_generic_kernel(
     T accum = T(0);
     {
         T light = T(1);
-        while (__any(alive && r.t < r.tmax)) {
+        while (any_lane(alive && r.t < r.tmax)) {
             bool emit = false;
             if (alive && r.t < r.tmax) {
                 T delta_t;
@@ -1777,7 +1874,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             }
         }
     }
-    if (!__any(active)) return;   // (both wavefronts see the same rays: both leave or both stay)
+    if (!any_lane(active)) return;   // (both wavefronts see the same rays: both leave or both stay)
     if (walks)
         box.written[lane] = 0;
     else
@@ -1787,33 +1884,36 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     if (walks) {
         // ---- the walk: one leaf per live lane and turn, into the ring
         OctreeCursor cur;
-        cur.reset(path + lane, kMarchThreads);
-        int32_t written = 0;
+        cur.reset(path + lane);
+        if (active) cur.begin(r);
+        int32_t written = 0, taken = 0;
         bool live = active, broken = false;
         int spins = 0;
-        // the walk is the longest chain of a tile: it goes first where wavefronts share a SIMD
-        // (measured: -10 % on a dense image, nothing elsewhere)
-        __builtin_amdgcn_s_setprio(3);
-        while (true) {
-            // (reading the shading's count only every few turns was measured slower: rays that have
-            // stopped are then walked further)
-            const int32_t taken = box_read(&box.taken[lane]);
-            live = live && !(taken & kEndedBit);
-            if (live && (broken || !(r.t < r.tmax))) {   // the walk of this ray is over: say so once
+        // the walk of a ray is over: say so once
+        auto end_walk = [&]() {
+            if (live && (broken || !(r.t < r.tmax))) {
                 box_write(&box.written[lane], written | kEndedBit | (broken ? kBrokenBit : 0));
                 live = false;
             }
-            if (!__any(live)) break;
-            const bool go = live && written - (taken & ~kEndedBit) < kRing;
-            if (!__any(go)) {   // every ring is full: the shading is behind
+        };
+        // the walk is the longest chain of a tile: it goes first where wavefronts share a SIMD
+        // (measured: -10 % on a dense image, nothing elsewhere)
+        __builtin_amdgcn_s_setprio(3);
+        end_walk();
+        while (any_lane(live)) {
+            const bool go = live && written - taken < kRing;
+            if (!any_lane(go)) {   // every ring is full: the shading is behind (and the turn below does nothing)
                 if (++spins > spin_limit) {
                     if (lane == 0) atomicAdd(ws.give_ups, 1u);
                     break;
                 }
                 __builtin_amdgcn_s_sleep(1);
-                continue;
+            } else {
+                spins = 0;
             }
-            spins = 0;
+            // asked for here, looked at after the turn: not waited for.  (Reading the shading's count only every few
+            // turns was measured slower: rays that have stopped are then walked further.)
+            const int32_t taken_next = __hip_atomic_load(&box.taken[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             int32_t leaf;
             float dt;
             walk_turn_flat(tr, r, cur, step, go, broken, leaf, dt);
@@ -1823,9 +1923,14 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                 box.leaf[at] = leaf;
                 box.dt[at] = dt;
                 written += 1;
+                // (release: the leaf is in the ring before the count says so)
+                box_write(&box.written[lane], written);
             }
-            // (release: the leaf is in the ring before the count says so)
-            if (put) box_write(&box.written[lane], written);
+            // (acquire: what the shading had taken is no longer needed before it is overwritten)
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            live = live && !(taken_next & kEndedBit);
+            taken = taken_next & ~kEndedBit;
+            end_walk();
         }
         return;
     }
@@ -1860,11 +1965,11 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             }
             active = false;
         }
-        if (!__any(active)) break;
+        if (!any_lane(active)) break;
         const int n_take = active ? (avail < kQueue ? avail : kQueue) : 0;
         // (waiting for fuller hands -- two or four leaves per lane, a few looks of patience -- and a ring
         // of 16 were measured: no gain, the larger ring costs LDS)
-        if (!__any(n_take > 0)) {   // the walk has found nothing new yet
+        if (!any_lane(n_take > 0)) {   // the walk has found nothing new yet
             if (++spins > spin_limit) {
                 // Cannot happen while the walk runs.  If it ever does, nothing plausible is left behind: the pixel
                 // is NaN, the ray's notes say "march me" (the backward pass then does, twice), and the library's
@@ -1979,7 +2084,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
     int phase = kMarch1;
     MergeState merge;
     OctreeCursor cur;
-    cur.reset(path + lane, kMarchThreads);
+    cur.reset(path + lane);
 
     // takes ray `item` into this lane if it hits the tree
     auto start = [&](int64_t item) {
@@ -2011,7 +2116,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
             light = 1.0f;
             accum = march1_sum;
             tmin = r.t;
-            cur.restart();
+            cur.begin(r);
             phase = kMode == kBackwardSecond && !first_march_too ? kMarch2 : kMarch1;
             active = true;
         }
@@ -2027,7 +2132,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
             if (state == kRoundRefilled) continue;
             if (state == kRoundDone) break;
         } else {
-            if (!__any(active)) break;
+            if (!any_lane(active)) break;
         }
 
         // ---- walk
@@ -2101,6 +2206,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
                 light = 1.0f;
                 phase = kMarch2;
                 r.t = tmin;
+                cur.aim(r);
             } else {
                 active = false;
             }
@@ -2208,7 +2314,7 @@ struct ReplayRays {
             if (known) index = chunks[r.link + want - 1];
             if (known) chunk = want;
         }
-        while (__any(g.valid && chunk < want)) {
+        while (any_lane(g.valid && chunk < want)) {
             if (g.valid && chunk < want) {
                 index = chunk == 0 ? r.link : __float_as_int(ws.base[(int64_t)index * kChunkFloat2 + kHeadFloat2].x);
                 chunk += 1;
@@ -2303,7 +2409,7 @@ struct ReplayRays {
 // A turn is two or three instructions for all rays of the batch.
 template <class Step>
 __device__ __forceinline__ void each_in_turn(const ReplayNote& g, Step&& step) {
-    for (int turn = 0; __any(g.valid && g.p >= turn); turn += 4) {
+    for (int turn = 0; any_lane(g.valid && g.p >= turn); turn += 4) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) step();
     }
@@ -2547,7 +2653,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_generic_kernel(TreeDev<
         T light = T(1);
         if (alive) r.t = tmin;
         bool marching = alive;   // (a broken tree ends this march, not the ray: the reference breaks out of the loop)
-        while (__any(marching && r.t < r.tmax)) {
+        while (any_lane(marching && r.t < r.tmax)) {
             bool emit = false;
             if (marching && r.t < r.tmax) {
                 T delta_t;
@@ -2679,7 +2785,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
     int64_t slot = -1;
     bool active = false, second = false;
     OctreeCursor cur;
-    cur.reset(path + lane, kMarchThreads);
+    cur.reset(path + lane);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
     // (with a bitmap `only` the launch does the rays whose bit is set and no others; a batch launch
@@ -2705,7 +2811,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
             }
             light = light1 = 1.0f;
             tmin = r.t;
-            cur.restart();
+            cur.begin(r);
             second = false;
             active = true;
         } else {
@@ -2725,7 +2831,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
             if (state == kRoundRefilled) continue;
             if (state == kRoundDone) break;
         } else {
-            if (!__any(active)) break;
+            if (!any_lane(active)) break;
         }
 
         // ---- walk
@@ -2843,6 +2949,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
                 }
                 light = 1.0f;
                 r.t = tmin;
+                cur.aim(r);
                 second = true;
             } else {
 #pragma unroll

@@ -443,9 +443,10 @@ unsigned blocks_for(int64_t items, int per_block) { return (unsigned)((items + p
 // leaf's density with its coefficients, the two-wavefront kernel gains nothing from them) the balance tips earlier,
 // launches alone: radius 4, 4 poses 0.48 / 0.47, 8 poses 0.69 / 0.72, 16 poses 1.13 / 1.30; radius 2.5, 8 poses
 // 1.22 / 1.33.  The launcher cannot know how many rays hit, so the rule goes by tiles: images of up to 65 536 tiles
-// (six 800x800 poses) -- 49 152 with deciding marks, 16 384 under NDC, where every ray passes through the tree --,
-// ray batches of up to 128 Ki rays (dense 128^3 tree: 1 pose 0.54 / 0.37, 4 poses 0.84 / 0.75; 4 NDC poses of 47 628
-// tiles 3.54 / 3.67; 256 Ki unrelated rays 0.29 / 0.39).
+// (six 800x800 poses) -- 49 152 with deciding marks, 6 144 under NDC, where every ray passes through the tree (us, one /
+// two, SH16 trees of 128^3 and 512^3: 3 024 tiles 117 / 115 and 310 / 279, 6 745 tiles 155 / 190 and 423 / 420, 11 970
+// tiles 201 / 243 and 482 / 506) --, ray batches of up to 128 Ki rays (dense 128^3 tree: 1 pose 0.54 / 0.37, 4 poses
+// 0.84 / 0.75; 256 Ki unrelated rays 0.29 / 0.39).
 bool use_split_forward(unsigned blocks, bool image, const SvoxRenderOptions* opt, bool decided) {
     const int forced = tuning().split_forward;
     const long limit = tuning().split_blocks;
@@ -453,7 +454,7 @@ bool use_split_forward(unsigned blocks, bool image, const SvoxRenderOptions* opt
     if (forced >= 0) return forced > 0;
     if (limit >= 0) return (long)blocks <= limit;
     if (!image) return blocks <= 2048u;
-    if (opt->ndc_width > 0) return blocks <= 16384u;
+    if (opt->ndc_width > 0) return blocks <= 6144u;
     return blocks <= (decided ? 49152u : 65536u);
 }
 template <typename T>

@@ -6,7 +6,7 @@
 //   descend_generic<T>   the reference's floating-point walk (multiply by N, floor, subtract) for
 //                        any branching factor and scalar type.
 //
-//   OctreeCursor         N == 2, fp32.  Multiplying by 2, taking the floor and subtracting it are
+//   OctreeCursor         (march_kernels.h) N == 2, fp32.  Multiplying by 2, taking the floor and subtracting it are
 //                        exact in binary floating point, so the cell chosen at level l is bit
 //                        (24 - l) of trunc(p * 2^24) and the leaf-local position at depth L is
 //                        frac(p * 2^L).  The walk therefore runs on integers, and because a ray's
@@ -184,98 +184,5 @@ __device__ __forceinline__ void descend_octree_multi(const int32_t* __restrict__
         }
     }
 }
-
-// leaf-local position frac(pc * 2^levels): s - floor(s), exact for the non-negative s of a clamped coordinate, in
-// one instruction
-__device__ __forceinline__ float leaf_local(float pc, float cube_sz) {
-    return __builtin_amdgcn_fractf(pc * cube_sz);
-}
-
-// Per-lane cursor that remembers the previous descent.  `path` points at this lane's column of an
-// LDS array laid out [kPathLevels + 1][block threads]: path[l * stride], l < kPathLevels, is the node
-// whose child row is indexed at level l + 1 (path[0] is the root, node 0); the last row is a dump
-// for the levels below kPathLevels, which a restart never resumes from.
-struct OctreeCursor {
-    int32_t* path;
-    int stride;
-    uint32_t ix, iy, iz;  // coordinates of the previous query
-    int levels;           // levels of the previous leaf, 0 = no previous query
-    int32_t leaf;         // its cell index
-    int pend_level;       // > 0: a descent was interrupted before reading the child row at this level
-    int32_t pend_node;    //      of this node
-
-    static constexpr int32_t kPending = -2;
-
-    __device__ __forceinline__ void reset(int32_t* lane_path, int lane_stride) {
-        path = lane_path;
-        stride = lane_stride;
-        levels = 0;
-        leaf = -1;
-        pend_level = 0;
-        pend_node = 0;
-        ix = iy = iz = 0;
-    }
-
-    // forget the previous query (a new ray)
-    __device__ __forceinline__ void restart() {
-        levels = 0;
-        pend_level = 0;
-    }
-
-    static constexpr int32_t kIdle = -3;
-
-    // Finds the leaf of the point with integer coordinates (nx, ny, nz), reading at most kBudget
-    // child entries.  Returns the leaf cell index; kPending if the budget ran out (call again with
-    // the same point to go on); -1 if the tree has more levels than the coordinates hold (`levels`
-    // becomes 0).  The budget bounds how long the lanes of a wavefront wait for the one lane that
-    // has to descend many levels: that lane continues in its next turn instead.
-    // Node ids read from the table are clamped into [0, capacity): a malformed tree yields a wrong
-    // leaf, never an access outside the table.  The table is smaller than 4 GiB (checked on the
-    // host): a 32-bit byte offset from the uniform base lets the load use the scalar-base form.
-    //
-    // The bookkeeping is written as selects: every lane runs every instruction (in a wavefront that
-    // costs nothing more than running it for one lane) and only the table reads sit under a
-    // condition.  `go`: this lane searches; a lane that does not keeps its state and returns kIdle.
-    template <int kBudget>
-    __device__ __forceinline__ int32_t seek_flat(bool go, const int32_t* __restrict__ child, int32_t last_node,
-                                                 uint32_t nx, uint32_t ny, uint32_t nz) {
-        const bool pending = pend_level > 0;
-        const bool have = levels > 0;
-        const uint32_t diff = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
-        const int first_diff = diff ? (kCoordBits - 31 + __builtin_clz(diff)) : kCoordBits + 1;
-        const bool same = !pending && have && first_diff > levels;   // still inside the previous leaf
-        const int from = first_diff < kPathLevels ? first_diff : kPathLevels;
-        const int32_t remembered = path[(from - 1) * stride];   // a row of the array for every lane
-        int level = pending ? pend_level : (have ? from : 1);
-        int32_t node = pending ? pend_node : (have ? remembered : 0);
-        const bool moved = go && !pending;
-        ix = moved ? nx : ix;
-        iy = moved ? ny : iy;
-        iz = moved ? nz : iz;
-        const bool search = go && !same;
-        bool want = search;
-        int32_t cell = 0, skip = 0;
-#pragma unroll
-        for (int it = 0; it < kBudget; ++it) {
-            if (want) {
-                path[((level <= kPathLevels ? level : kPathLevels + 1) - 1) * stride] = node;
-                cell = (node << 3) | cell_at(nx, ny, nz, level);
-                skip = *(const int32_t*)((const char*)child + ((uint32_t)cell << 2));
-            }
-            want = want && skip > 0 && level != kCoordBits;
-            node = want ? (int32_t)min((uint32_t)(node + skip), (uint32_t)last_node) : node;
-            level = want ? level + 1 : level;
-        }
-        // want: the budget ran out; skip == 0: found; else more levels than the coordinates hold
-        const bool empty = skip < 0;   // a leaf marked empty
-        const bool found = search && skip <= 0;
-        const bool open = search && skip > 0;
-        pend_level = go ? (want ? level : 0) : pend_level;
-        pend_node = want ? node : pend_node;
-        levels = found ? level : (open ? 0 : levels);
-        leaf = found ? (empty ? cell | kEmptyLeafBit : cell) : (open ? -1 : leaf);
-        return !go ? kIdle : (want ? kPending : leaf);
-    }
-};
 
 }  // namespace svox
