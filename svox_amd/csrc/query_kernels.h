@@ -8,8 +8,8 @@
 //      wavefront is one contiguous run of 64*K scalars, so consecutive lanes touch consecutive
 //      addresses on that side and K-long runs on the tree side, instead of one lane copying K
 //      scalars in a serial loop.
-// Blocks are persistent (grid-stride over tiles of 512 points, two per lane) so the LDS copy of the
-// child rows is filled once per block.
+// Blocks are persistent (grid-stride over tiles of 256 points) so the LDS copy of the child rows is
+// filled once per block.
 #pragma once
 
 #include "tree_walk.h"
@@ -22,45 +22,71 @@ constexpr int kWave = 64;
 enum QueryMode { kQueryGather = 0, kQueryScatterAdd = 1, kQueryAssign = 2 };
 typedef unsigned int Piece16 __attribute__((ext_vector_type(4)));   // 16 bytes as the non-temporal builtins take them
 
-constexpr int kQueryPts = 2;   // points a lane walks in lockstep (their child reads overlap)
-
-// Leaves of a lane's kQueryPts points: leaf[u] = packed leaf id or -1.
+// Leaf of a point (packed leaf id or -1).  lds_child: the child rows of the nodes below lds_nodes.
 template <typename T, bool kOctree>
-__device__ __forceinline__ void query_leaves(const TreeDev<T>& tr, const int32_t* lds_child, int32_t lds_nodes,
-                                             const T* offset, const T* scaling, const T* __restrict__ points,
-                                             const int64_t* q, int64_t n_points, int64_t* leaf) {
-    T xyz[kQueryPts][3];
-    bool valid[kQueryPts];
+__device__ __forceinline__ int64_t query_leaf(const TreeDev<T>& tr, const int32_t* lds_child, int32_t lds_nodes,
+                                              const T* offset, const T* scaling, const T* __restrict__ points, int64_t q,
+                                              bool valid) {
+    T xyz[3];
 #pragma unroll
-    for (int u = 0; u < kQueryPts; ++u) {
-        valid[u] = q[u] < n_points;
-        leaf[u] = -1;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) xyz[u][k] = valid[u] ? points[q[u] * 3 + k] : T(0);
-        transform_coord(xyz[u], offset, scaling);
-    }
+    for (int k = 0; k < 3; ++k) xyz[k] = valid ? points[q * 3 + k] : T(0);
+    transform_coord(xyz, offset, scaling);
+    int64_t leaf = -1;
     if constexpr (kOctree) {
-        uint32_t ix[kQueryPts], iy[kQueryPts], iz[kQueryPts];
-        int32_t cell[kQueryPts];
-#pragma unroll
-        for (int u = 0; u < kQueryPts; ++u) {
-            ix[u] = cell_coord(clamp01(xyz[u][0]));
-            iy[u] = cell_coord(clamp01(xyz[u][1]));
-            iz[u] = cell_coord(clamp01(xyz[u][2]));
-        }
-        descend_octree_multi<kQueryPts>(tr.child, lds_child, lds_nodes, tr.capacity, ix, iy, iz, valid, cell);
-#pragma unroll
-        for (int u = 0; u < kQueryPts; ++u) {
-            leaf[u] = cell[u];
-            valid[u] = valid[u] && cell[u] < 0;   // deeper than the integer coordinates resolve:
-        }                                         // repeat those with the floating-point walk
+        if (valid)
+            leaf = descend_octree(tr.child, lds_child, lds_nodes, tr.capacity, cell_coord(clamp01(xyz[0])),
+                                  cell_coord(clamp01(xyz[1])), cell_coord(clamp01(xyz[2])));
     }
+    if (valid && leaf < 0) {   // deeper than the integer coordinates resolve: once more with the floating-point walk
+        T cube;
+        int levels;
+        leaf = descend_generic<T>(tr.child, tr.capacity, tr.N, xyz, &cube, &levels);
+    }
+    return leaf;
+}
+
+// The rows of one run, scalar by scalar: flat index f = p * Kx + e of the run's contiguous side (`lin`) to lane f mod 64,
+// row_leaf(p) the leaf of row p (called by every lane).  kBatch scalars per lane are read before the first is written:
+// the compiler must assume that the two sides overlap, so it would wait for every read before the write behind it
+// (1 000 points, 49 scalars: 32.4 -> 6.7 us, with query_few_kernel's smaller wavefronts).
+template <typename T, int MODE, class RowLeaf>
+__device__ __forceinline__ void move_rows(int lane, int n_rows, int32_t Kx, int64_t row, RowLeaf&& row_leaf, T* data, T* lin,
+                                          T* target) {
+    constexpr int kBatch = 4;
+    const int total = n_rows * Kx;
+    const int step_e = kWave % Kx, step_p = kWave / Kx;
+    int p = lane / Kx, e = lane % Kx;
+    for (int f0 = 0; f0 < total; f0 += kWave * kBatch) {
+        T buf[kBatch];
+        int64_t at[kBatch];   // on the tree's side; -1: no leaf (malformed tree) or past the end
 #pragma unroll
-    for (int u = 0; u < kQueryPts; ++u) {
-        if (valid[u]) {
-            T cube;
-            int levels;
-            leaf[u] = descend_generic<T>(tr.child, tr.capacity, tr.N, xyz[u], &cube, &levels);
+        for (int b = 0; b < kBatch; ++b) {
+            const int f = f0 + b * kWave + lane;
+            const int64_t leaf = row_leaf(f < total ? p : 0);
+            at[b] = f < total && leaf >= 0 ? leaf * row + e : -1;
+            buf[b] = T(0);
+            if (MODE == kQueryGather) {
+                if (at[b] >= 0) buf[b] = data[at[b]];
+            } else {
+                if (at[b] >= 0) buf[b] = __builtin_nontemporal_load(&lin[f]);
+            }
+            e += step_e;
+            p += step_p;
+            if (e >= Kx) {
+                e -= Kx;
+                p += 1;
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const int f = f0 + b * kWave + lane;
+            if (MODE == kQueryGather) {
+                if (f < total) __builtin_nontemporal_store(buf[b], &lin[f]);
+            } else if (MODE == kQueryScatterAdd) {
+                if (at[b] >= 0) atomicAdd(target + at[b], buf[b]);
+            } else {
+                if (at[b] >= 0) data[at[b]] = buf[b];
+            }
         }
     }
 }
@@ -81,100 +107,90 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(TreeDev<T> tr, con
     T offset[3], scaling[3];
     load_transform(tr, offset, scaling);
     const int lane = threadIdx.x & (kWave - 1);
-    constexpr int kTile = kQueryThreads * kQueryPts;   // points per block and iteration
-    const int64_t n_tiles = (n_points + kTile - 1) / kTile;
+    const int64_t n_tiles = (n_points + kQueryThreads - 1) / kQueryThreads;
     const int64_t row = (MODE == kQueryAssign) ? (int64_t)tr.K : (int64_t)Kx;
     // records and output rows start on 16-byte boundaries: move 16-byte pieces
     const bool vec16 = (Kx * (int)sizeof(T)) % 16 == 0 && (((uintptr_t)tr.data | (uintptr_t)values) & 15u) == 0;
 
     for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        // a wavefront owns kQueryPts runs of 64 consecutive points; lane l walks point l of each run
-        const int64_t wave_first = tile * kTile + (int64_t)(threadIdx.x / kWave) * (kWave * kQueryPts);
-        int64_t q[kQueryPts], leaves[kQueryPts];
+        // a wavefront owns 64 consecutive points; lane l walks point l
+        const int64_t wave_base = tile * kQueryThreads + (int64_t)(threadIdx.x / kWave) * kWave;
+        const int64_t q = wave_base + lane;
+        const int64_t leaf = query_leaf<T, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, q < n_points);
+        if (MODE == kQueryGather && ids && q < n_points) ids[q] = leaf;
+        // phase 2: the 64 rows of the run, flat index f = p * Kx + e
+        const int64_t remaining = n_points - wave_base;
+        const int n_rows = remaining < kWave ? (int)(remaining > 0 ? remaining : 0) : kWave;
+        T* lin = values + wave_base * Kx;
+        const int leaf_lo = (int)(leaf & 0xffffffff), leaf_hi = (int)(leaf >> 32);
+        if (MODE == kQueryGather && vec16) {
+            // 16-byte pieces: a record is `pieces` of them, and kBatch loads per lane are in flight
+            // before the first store (the compiler must assume that the output aliases the tree)
+            constexpr int kPer = 16 / (int)sizeof(T);
+            constexpr int kBatch = 4;
+            const int pieces = Kx / kPer;
+            const int total = n_rows * pieces;
+            const int step_e = kWave % pieces, step_p = kWave / pieces;
+            int p = lane / pieces, e = lane % pieces;
+            uint4* lin16 = (uint4*)lin;
+            for (int f0 = 0; f0 < total; f0 += kWave * kBatch) {
+                uint4 buf[kBatch];
 #pragma unroll
-        for (int u = 0; u < kQueryPts; ++u) q[u] = wave_first + u * kWave + lane;
-        query_leaves<T, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, n_points, leaves);
-        if (MODE == kQueryGather && ids) {
-#pragma unroll
-            for (int u = 0; u < kQueryPts; ++u)
-                if (q[u] < n_points) ids[q[u]] = leaves[u];
-        }
-        // phase 2, run by run: the 64 rows of a run, flat index f = p * Kx + e
-#pragma unroll
-        for (int u = 0; u < kQueryPts; ++u) {
-            const int64_t wave_base = wave_first + u * kWave;
-            const int64_t leaf = leaves[u];
-            const int64_t remaining = n_points - wave_base;
-            const int n_rows = remaining < kWave ? (int)(remaining > 0 ? remaining : 0) : kWave;
-            T* lin = values + wave_base * Kx;
-            const int leaf_lo = (int)(leaf & 0xffffffff), leaf_hi = (int)(leaf >> 32);
-            if (MODE == kQueryGather && vec16) {
-                // 16-byte pieces: a record is `pieces` of them, and kBatch loads per lane are in flight
-                // before the first store (the compiler must assume that the output aliases the tree)
-                constexpr int kPer = 16 / (int)sizeof(T);
-                constexpr int kBatch = 4;
-                const int pieces = Kx / kPer;
-                const int total = n_rows * pieces;
-                const int step_e = kWave % pieces, step_p = kWave / pieces;
-                int p = lane / pieces, e = lane % pieces;
-                uint4* lin16 = (uint4*)lin;
-                for (int f0 = 0; f0 < total; f0 += kWave * kBatch) {
-                    uint4 buf[kBatch];
-#pragma unroll
-                    for (int b = 0; b < kBatch; ++b) {
-                        const int f = f0 + b * kWave + lane;
-                        // every lane takes part in the shuffle; rows past the end read lane 0's leaf
-                        const int src_lane = f < total ? p : 0;
-                        const int lo = __shfl(leaf_lo, src_lane);
-                        const int hi = __shfl(leaf_hi, src_lane);
-                        const int64_t lf = ((int64_t)hi << 32) | (uint32_t)lo;
-                        buf[b] = make_uint4(0u, 0u, 0u, 0u);
-                        if (f < total && lf >= 0) buf[b] = ((const uint4*)(tr.data + lf * row))[e];
-                        e += step_e;
-                        p += step_p;
-                        if (e >= pieces) {
-                            e -= pieces;
-                            p += 1;
-                        }
-                    }
-#pragma unroll
-                    for (int b = 0; b < kBatch; ++b) {
-                        const int f = f0 + b * kWave + lane;
-                        // (stored past the caches' keep-list: the output is written once, and the tree it is gathered
-                        // from should stay in the last-level cache: 4 Mi points of a 268 MB tree 0.346 -> 0.332 ms)
-                        if (f < total) __builtin_nontemporal_store((Piece16){buf[b].x, buf[b].y, buf[b].z, buf[b].w}, (Piece16*)lin16 + f);
+                for (int b = 0; b < kBatch; ++b) {
+                    const int f = f0 + b * kWave + lane;
+                    // every lane takes part in the shuffle; rows past the end read lane 0's leaf
+                    const int src_lane = f < total ? p : 0;
+                    const int lo = __shfl(leaf_lo, src_lane);
+                    const int hi = __shfl(leaf_hi, src_lane);
+                    const int64_t lf = ((int64_t)hi << 32) | (uint32_t)lo;
+                    buf[b] = make_uint4(0u, 0u, 0u, 0u);
+                    if (f < total && lf >= 0) buf[b] = ((const uint4*)(tr.data + lf * row))[e];
+                    e += step_e;
+                    p += step_p;
+                    if (e >= pieces) {
+                        e -= pieces;
+                        p += 1;
                     }
                 }
-                continue;
-            }
-            const int total = n_rows * Kx;
-            const int step_e = kWave % Kx, step_p = kWave / Kx;
-            int p = lane / Kx, e = lane % Kx;
-            for (int f = lane; __any(f < total); f += kWave) {
-                const int src_lane = f < total ? p : 0;
-                const int lo = __shfl(leaf_lo, src_lane);
-                const int hi = __shfl(leaf_hi, src_lane);
-                const int64_t lf = ((int64_t)hi << 32) | (uint32_t)lo;
-                if (f < total && lf >= 0) {
-                    if (MODE == kQueryGather) {
-                        __builtin_nontemporal_store(tr.data[lf * row + e], &lin[f]);
-                    } else if (MODE == kQueryScatterAdd) {
-                        atomicAdd(target + lf * row + e, __builtin_nontemporal_load(&lin[f]));
-                    } else {
-                        tr.data[lf * row + e] = lin[f];
-                    }
-                } else if (MODE == kQueryGather && f < total) {
-                    lin[f] = T(0);   // malformed tree: no leaf
-                }
-                e += step_e;
-                p += step_p;
-                if (e >= Kx) {
-                    e -= Kx;
-                    p += 1;
+#pragma unroll
+                for (int b = 0; b < kBatch; ++b) {
+                    const int f = f0 + b * kWave + lane;
+                    // (stored past the caches' keep-list: the output is written once, and the tree it is gathered
+                    // from should stay in the last-level cache: 4 Mi points of a 268 MB tree 0.346 -> 0.332 ms)
+                    if (f < total) __builtin_nontemporal_store((Piece16){buf[b].x, buf[b].y, buf[b].z, buf[b].w}, (Piece16*)lin16 + f);
                 }
             }
+        } else {
+            move_rows<T, MODE>(lane, n_rows, Kx, row, [&](int p) {
+                const int lo = __shfl(leaf_lo, p), hi = __shfl(leaf_hi, p);
+                return ((int64_t)hi << 32) | (uint32_t)lo;
+            }, tr.data, lin, target);
         }
     }
+}
+
+// Few points: 16 to a wavefront, four lanes walking each, nothing staged in LDS -- a call this small is one chain of
+// dependent reads, and the shorter its pieces the sooner it is over.  (Before, as two runs of 64 points per wavefront:
+// 1 000 points of a 32^3 SH4 tree 13.7 -> 4.7 us.)
+constexpr int kFewPoints = 16;
+template <typename T, int MODE, bool kOctree>
+__global__ __launch_bounds__(kWave) void query_few_kernel(TreeDev<T> tr, const T* __restrict__ points, int64_t n_points,
+                                                          T* values, T* target, int64_t* __restrict__ ids, int32_t Kx) {
+    const int lane = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * kFewPoints, q = base + lane / (kWave / kFewPoints);
+    const bool valid = q < n_points;
+    T offset[3], scaling[3];
+    load_transform(tr, offset, scaling);
+    const int64_t leaf = query_leaf<T, kOctree>(tr, nullptr, 0, offset, scaling, points, q, valid);
+    if (MODE == kQueryGather && ids && valid && lane % (kWave / kFewPoints) == 0) ids[q] = leaf;
+    const int64_t remaining = n_points - base;
+    const int n_rows = remaining < kFewPoints ? (int)remaining : kFewPoints;
+    const int leaf_lo = (int)(leaf & 0xffffffff), leaf_hi = (int)(leaf >> 32);
+    move_rows<T, MODE>(lane, n_rows, Kx, MODE == kQueryAssign ? (int64_t)tr.K : (int64_t)Kx, [&](int p) {
+        const int from = p * (kWave / kFewPoints);
+        const int lo = __shfl(leaf_lo, from), hi = __shfl(leaf_hi, from);
+        return ((int64_t)hi << 32) | (uint32_t)lo;
+    }, tr.data, values + base * Kx, target);
 }
 
 // calc_corner_kernel, svox_kernel.cu:91-115: climb parent links from the leaf's node to the

@@ -171,6 +171,12 @@ int zero_fill(void* ptr, int64_t bytes, hipStream_t stream) {
 // ---------------------------------------------------------------------------------------------
 // queries
 // ---------------------------------------------------------------------------------------------
+// Calls of up to kFewPointsMax points take query_few_kernel: its wavefronts have 16 points instead of 64, so that small
+// calls spread further and end sooner, but each walks from the root through memory and moves scalars.  Gather, us, 64 /
+// 16 points: 262 144 points, SH9 25.7 / 25.2, SH4 11.7 / 11.5, SH16 36.9 / 30.2; 524 288 points 44.7 / 44.6, 16.3 / 19.3,
+// 52.7 / 54.8.  (Larger wavefronts of 128 points, two to a lane, for the rest: SH16, 1 Mi points 92 / 92, 262 144 points
+// 37 / 47.)
+constexpr int64_t kFewPointsMax = 262144;
 constexpr int kLdsNodesMax = 584;  // child rows kept in LDS per block: 584 * 32 B = 18.25 KiB
 
 template <typename T, int MODE>
@@ -178,8 +184,17 @@ int launch_query(const SvoxTreeSpec* tree, const void* points, int64_t n, void* 
                  int64_t* ids, int32_t Kx, hipStream_t stream, const char* what) {
     if (n == 0) return SVOX_OK;
     const TreeDev<T> tr = make_tree<T>(tree);
-    const int64_t per_tile = (int64_t)kQueryThreads * kQueryPts;
-    const int64_t tiles = (n + per_tile - 1) / per_tile;
+    if (n <= kFewPointsMax) {
+        const dim3 blocks((unsigned)((n + kFewPoints - 1) / kFewPoints));
+        if (sizeof(T) == 4 && octree_fast_ok(tree))
+            hipLaunchKernelGGL((query_few_kernel<T, MODE, sizeof(T) == 4>), blocks, dim3(kWave), 0, stream, tr, (const T*)points, n,
+                               (T*)values, (T*)target, ids, Kx);
+        else
+            hipLaunchKernelGGL((query_few_kernel<T, MODE, false>), blocks, dim3(kWave), 0, stream, tr, (const T*)points, n,
+                               (T*)values, (T*)target, ids, Kx);
+        return check_launch(what);
+    }
+    const int64_t tiles = (n + kQueryThreads - 1) / kQueryThreads;
     const int64_t blocks = tiles < 256 * 8 ? tiles : 256 * 8;
     if constexpr (sizeof(T) == 4) {
         if (octree_fast_ok(tree)) {

@@ -122,67 +122,25 @@ __device__ __forceinline__ int32_t child_entry(const int32_t* __restrict__ child
 }
 
 // Octree walk over integer coordinates with no path memory (point queries).
-// `lds_child` holds the child rows of nodes [0, lds_nodes); deeper nodes are read from memory.
-// Returns the leaf cell index node*8 + cell (or -1) and the number of levels visited.
-__device__ __forceinline__ int32_t descend_octree(const int32_t* __restrict__ child,
-                                                  const int32_t* lds_child, int32_t lds_nodes,
-                                                  int64_t capacity, uint32_t ix, uint32_t iy,
-                                                  uint32_t iz, int* levels) {
-    int32_t node = 0;
-    for (int level = 1; level <= kCoordBits; ++level) {
+// `lds_child` holds the child rows of nodes [0, lds_nodes); deeper nodes are read from memory (lds_nodes 0: all of them).
+// Returns the leaf cell index node*8 + cell, or -1.
+__device__ __forceinline__ int32_t descend_octree(const int32_t* __restrict__ child, const int32_t* lds_child,
+                                                  int32_t lds_nodes, int64_t capacity, uint32_t ix, uint32_t iy,
+                                                  uint32_t iz) {
+    int32_t node = 0, leaf = -1;
+    bool live = true;
+    for (int level = 1; level <= kCoordBits && live; ++level) {
         const int32_t cell = node * 8 + cell_at(ix, iy, iz, level);
-        const int32_t skip = child_entry(child, lds_child, lds_nodes, node, cell);
+        const int32_t skip = lds_child ? child_entry(child, lds_child, lds_nodes, node, cell) : child[cell];
         if (skip == 0) {
-            *levels = level;
-            return cell;
-        }
-        node += skip;
-        if (node < 0 || node >= capacity) return -1;
-    }
-    return -1;  // deeper than the integer coordinates resolve; the host routes such trees elsewhere
-}
-
-// The same walk for kPts points of one lane in lockstep: the child reads of the points are
-// independent, so they are in flight together and the lane waits once per level instead of once
-// per level and point.  leaf[u] = cell index or -1.
-template <int kPts>
-__device__ __forceinline__ void descend_octree_multi(const int32_t* __restrict__ child, const int32_t* lds_child,
-                                                     int32_t lds_nodes, int64_t capacity, const uint32_t* ix,
-                                                     const uint32_t* iy, const uint32_t* iz, const bool* valid,
-                                                     int32_t* leaf) {
-    int32_t node[kPts];
-    bool live[kPts];
-    bool any_live = false;
-#pragma unroll
-    for (int u = 0; u < kPts; ++u) {
-        node[u] = 0;
-        leaf[u] = -1;
-        live[u] = valid[u];
-        any_live |= live[u];
-    }
-    for (int level = 1; level <= kCoordBits && any_live; ++level) {
-        int32_t cell[kPts], skip[kPts];
-#pragma unroll
-        for (int u = 0; u < kPts; ++u) {
-            cell[u] = node[u] * 8 + cell_at(ix[u], iy[u], iz[u], level);
-            skip[u] = 0;
-            if (live[u]) skip[u] = child_entry(child, lds_child, lds_nodes, node[u], cell[u]);
-        }
-        any_live = false;
-#pragma unroll
-        for (int u = 0; u < kPts; ++u) {
-            if (live[u]) {
-                if (skip[u] == 0) {
-                    leaf[u] = cell[u];
-                    live[u] = false;
-                } else {
-                    node[u] += skip[u];
-                    if (node[u] < 0 || node[u] >= capacity) live[u] = false;
-                }
-            }
-            any_live |= live[u];
+            leaf = cell;
+            live = false;
+        } else {
+            node += skip;
+            if (node < 0 || node >= capacity) live = false;
         }
     }
+    return leaf;  // (-1 also where the tree is deeper than the integer coordinates resolve)
 }
 
 }  // namespace svox
