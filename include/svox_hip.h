@@ -154,6 +154,14 @@ int svox_query_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n
 int svox_query_vertical_backward(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                                  const void* grad_output, int32_t grad_dim, void* grad_data_out,
                                  int32_t accumulate, void* stream);
+/* The same with a workspace (no reference counterpart): where the points are many beside the tree, and unless
+ * `accumulate` is nonzero, they are brought together by leaf in it and every row of the gradient is written once, instead
+ * of being cleared and added to.  _workspace_bytes: how large it has to be for these calls (8-byte aligned); 0 where the
+ * call would make no use of one.  A smaller workspace, or NULL, is the plain call. */
+int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
+                                    const void* grad_output, int32_t grad_dim, void* grad_data_out,
+                                    int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t svox_query_vertical_backward_workspace_bytes(const SvoxTreeSpec* tree, int64_t n_points, int32_t grad_dim);
 
 /* assign_vertical(TreeSpec&, indices, values); svox_kernel.cu:145-158.  values (n_points, value_dim),
  * value_dim <= data_dim.  Two points in one leaf race; the last writer wins, as in the reference. */

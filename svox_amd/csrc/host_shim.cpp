@@ -24,7 +24,8 @@ namespace {
 
 // ---- the library
 #define SVOX_CALLS(X)                                                                                                   \
-    X(svox_last_error) X(svox_status_string) X(svox_out_data_dim) X(svox_query_vertical) X(svox_query_vertical_backward) \
+    X(svox_last_error) X(svox_status_string) X(svox_out_data_dim) X(svox_query_vertical) \
+    X(svox_query_vertical_backward_ws) X(svox_query_vertical_backward_workspace_bytes)                                  \
     X(svox_assign_vertical) X(svox_calc_corners) X(svox_volume_render) X(svox_volume_render_images)                     \
     X(svox_volume_render_noted) X(svox_volume_render_images_noted) X(svox_volume_render_backward_ws)                    \
     X(svox_volume_render_images_backward_ws) X(svox_volume_render_backward_noted_with)                                  \
@@ -349,8 +350,11 @@ Tensor query_vertical_backward(py::handle tree, const py::object& points, const 
     if (g.size(0) != p.size(0)) fail("grad_output must have one row per point");
     Tensor grad = like(g, {t.spec.capacity, t.spec.N, t.spec.N, t.spec.N, g.size(1)});
     const On on(p);
-    status(lib.svox_query_vertical_backward(&t.spec, p.data_ptr(), p.size(0), g.data_ptr(), (int32_t)g.size(1),
-                                            grad.data_ptr(), 0, on.stream),
+    const int64_t bytes = lib.svox_query_vertical_backward_workspace_bytes(&t.spec, p.size(0), (int32_t)g.size(1));
+    Tensor space;
+    if (bytes > 0) space = at::empty({bytes}, p.options().dtype(at::kByte));
+    status(lib.svox_query_vertical_backward_ws(&t.spec, p.data_ptr(), p.size(0), g.data_ptr(), (int32_t)g.size(1),
+                                               grad.data_ptr(), 0, bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
            "query_vertical_backward");
     return grad;
 }

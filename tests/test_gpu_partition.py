@@ -1,0 +1,35 @@
+"""The gradient of point queries collected row by row (partition_kernels.h), against an exact sum on the CPU.
+
+Bar: 1e-5 of the largest element.
+"""
+import pytest
+import torch
+
+import svox_amd as svox
+from svox_amd import csrc as C
+from svox_amd.csrc import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,levels,dim,n,spread", [
+    (2, 5, 28, 700001, 1.0),         # rows of 16 bytes' multiples
+    (2, 4, 49, 300007, 1.0),         # ... and not; many points to a row
+    (2, 5, 13, 1200000, 0.05),       # most rows empty, the others full: several rounds to a tile
+    (2, 0, 49, 300000, 1.0),         # one node
+    (2, 3, 76, 400000, 1e-6),        # all points in one leaf
+    (3, 3, 49, 500000, 1.0),         # 27 cells to a node, a number of rows that no tile divides
+])
+def test_gradient_by_rows(gpu, N, levels, dim, n, spread):
+    import ctypes
+    tree = svox.N3Tree(N=N, data_dim=dim, init_refine=levels, data_format="RGBA").to(gpu)
+    gen = torch.Generator().manual_seed(n)
+    points = ((torch.rand(n, 3, generator=gen) - 0.5) * spread + 0.51).to(gpu)
+    grad = torch.randn(n, dim, generator=gen).to(gpu)
+    spec = C._pack_tree(tree._spec(world=False))
+    assert _abi.load_library().svox_query_vertical_backward_workspace_bytes(ctypes.byref(spec), n, dim) > 0
+    got = C.query_vertical_backward(tree._spec(world=False), points, grad)
+    _, ids = C.query_vertical(tree._spec(world=False), points)
+    want = torch.zeros(tree.data.numel() // dim, dim, dtype=torch.float64)
+    want.index_add_(0, ids.cpu(), grad.double().cpu())
+    assert (got.view(-1, dim).cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
