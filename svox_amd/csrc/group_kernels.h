@@ -38,38 +38,39 @@ __device__ __forceinline__ double from_group(double v) {
 // kGroupSeekBudget child reads; a longer descent goes on in the next turn, so that the other rays of the wavefront do not
 // wait for it.
 struct GroupWalk {
-    double o, d, inv, up;      // this lane's axis; up = max(inv, 0), see leaf_exit
+    double o, d, inv, up;      // this lane's axis, o and d times 2^24; up = max(inv, 0), see leaf_exit
     double t, tmax, dscale;
-    double p;                  // the sample's clamped coordinate on this lane's axis
-    int32_t* path;             // this lane's column of the previous descent's path, stride kMarchThreads
+    double p;                  // the sample's clamped coordinate on this lane's axis, times 2^24
+    int32_t* rows;             // this lane's column of the path, counted from level 1 (OctreeCursor)
     uint32_t nx, ny, nz;       // integer cell coordinates of the sample
-    int levels;                // of the previous leaf; 0: none
+    int levels;                // of the previous leaf (1: none)
     int level;                 // where the search for the sample's leaf stands
     int32_t node;
 
     __device__ __forceinline__ void begin(const RayState<double>& r, int axis, int32_t* lane_path) {
-        o = axis == 1 ? r.o[1] : axis == 2 ? r.o[2] : r.o[0];
-        d = axis == 1 ? r.d[1] : axis == 2 ? r.d[2] : r.d[0];
+        o = (axis == 1 ? r.o[1] : axis == 2 ? r.o[2] : r.o[0]) * 16777216.0;
+        d = (axis == 1 ? r.d[1] : axis == 2 ? r.d[2] : r.d[0]) * 16777216.0;
         inv = axis == 1 ? r.inv[1] : axis == 2 ? r.inv[2] : r.inv[0];
         up = max_(inv, 0.0);
         t = r.t;
         tmax = r.tmax;
         dscale = r.dscale;
-        path = lane_path;
+        rows = lane_path - kMarchThreads;
+        rows[kMarchThreads] = 0;
         nx = ny = nz = 0;
-        levels = 0;
+        levels = 1;
     }
     __device__ __forceinline__ bool ended() const { return !(t < tmax); }
 
     // the sample at t: its position, and the deepest node of the previous path it still lies in
     __device__ __forceinline__ void aim() {
-        p = clamp01(fma_(t, d, o));
-        const int n = (int)(uint32_t)(p * 16777216.0);
+        p = max_(0.0, min_((1.0 - 1e-6) * 16777216.0, fma_(t, d, o)));   // (clamp01, times 2^24)
+        const int n = (int)(uint32_t)p;
         const uint32_t mx = (uint32_t)from_group<0>(n), my = (uint32_t)from_group<1>(n), mz = (uint32_t)from_group<2>(n);
         const uint32_t diff = (nx ^ mx) | (ny ^ my) | (nz ^ mz);
-        const int first_diff = diff ? kCoordBits - 31 + __builtin_clz(diff) : kCoordBits + 1;
-        level = min(min(first_diff, levels > 0 ? levels : 1), kPathLevels);
-        node = level > 1 ? path[(level - 1) * kMarchThreads] : 0;
+        const uint32_t first_diff = (diff ? (uint32_t)__builtin_clz(diff) : 0xffffffffu) - (31 - kCoordBits);
+        level = (int)min(min(first_diff, (uint32_t)levels), (uint32_t)kPathLevels);
+        node = rows[level * kMarchThreads];
         nx = mx;
         ny = my;
         nz = mz;
@@ -78,39 +79,34 @@ struct GroupWalk {
     // One turn of the search.  True: the leaf is found (its cell index, -1 in a malformed tree), delta_t is the step of
     // the sample and the ray stands at the next one (aim() is still to be called).  rt_kernel.cu:262-275, 315.
     __device__ __forceinline__ bool turn(const TreeDev<double>& tr, double step_size, int64_t& leaf, double& delta_t) {
-        bool open = true, deep = false;
-        int32_t cell = 0;
+        int32_t cell = 0, skip = 1;
 #pragma unroll
         for (int it = 0; it < kGroupSeekBudget; ++it) {
-            if (open) {
-                path[(min(level, kPathLevels + 1) - 1) * kMarchThreads] = node;
+            if (skip > 0 && level <= kCoordBits) {
+                rows[min(level, kPathLevels + 1) * kMarchThreads] = node;
                 cell = (node << 3) | cell_at(nx, ny, nz, level);
-                const int32_t skip = tr.child[cell];
-                if (skip == 0) {
-                    open = false;
-                } else if (level == kCoordBits || (uint32_t)(node + skip) >= (uint32_t)tr.capacity) {
-                    open = false;
-                    deep = true;
-                } else {
-                    node += skip;
-                    level += 1;
-                }
+                skip = tr.child[cell];
+                // (negative: no entry of a well-formed tree; the walk from the root says what comes of it)
+                const bool down = skip != 0;
+                node += skip;
+                level = down ? ((uint32_t)node >= (uint32_t)tr.capacity ? kCoordBits + 1 : level + 1) : level;
+                skip = down ? 1 : 0;
             }
         }
-        if (open) return false;
+        if (skip > 0 && level <= kCoordBits) return false;
         double segment;
         leaf = cell;
-        if (!deep) {
+        if (skip == 0) {
             levels = level;
-            const double x = p * __longlong_as_double((long long)(1023 + level) << 52);
             // (dda_unit for a point inside the cube: the entry distance is 0, see leaf_exit)
-            const double e = -(x - floor_(x)) * inv + up;
+            const double e = -__builtin_amdgcn_fract(p * __longlong_as_double((long long)(1023 - kCoordBits + level) << 52)) * inv + up;
             const double hi = min_(min_(min_((double)1e9f, from_group<0>(e)), from_group<1>(e)), from_group<2>(e));
             segment = hi * __longlong_as_double((long long)(1023 - level) << 52);
         } else {
             // more levels than the integer coordinates hold, or a malformed tree
-            levels = 0;
-            double local[3] = {from_group<0>(p), from_group<1>(p), from_group<2>(p)};
+            levels = 1;
+            const double q = p * (1.0 / 16777216.0);
+            double local[3] = {from_group<0>(q), from_group<1>(q), from_group<2>(q)};
             const double all_inv[3] = {from_group<0>(inv), from_group<1>(inv), from_group<2>(inv)};
             double cells_per_axis, s0, s1;
             int levels_f;
