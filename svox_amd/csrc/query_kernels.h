@@ -249,12 +249,14 @@ __global__ __launch_bounds__(256) void mark_leaves_kernel(const T* __restrict__ 
     marks[i] = m;
 }
 
-// Zero-fill used in place of a memset so that a caller may capture the call in a graph.
+// Zero-fill used in place of a memset so that a caller may capture the call in a graph.  16 bytes a thread and no loop: the
+// blocks finish in the order they start, so what is written at any time lies close together (1.21 GB: 178 us, 6.8 TB/s;
+// 8192 blocks that stride through all of it 210 to 272 us, 16 pieces a thread 215 us, non-temporal stores 199 us and more;
+// 268 MB: 34 us instead of 37).
 __global__ __launch_bounds__(256) void zero_kernel(uint4* __restrict__ p16, int64_t n16,
                                                    uint32_t* __restrict__ tail, int n_tail) {
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n16; i += stride) p16[i] = z;
+    const int64_t i = blockIdx.x * 256ll + threadIdx.x;
+    if (i < n16) p16[i] = make_uint4(0u, 0u, 0u, 0u);
     if (blockIdx.x == 0 && (int)threadIdx.x < n_tail) tail[threadIdx.x] = 0u;
 }
 

@@ -161,7 +161,6 @@ int zero_fill(void* ptr, int64_t bytes, hipStream_t stream) {
     const int64_t n16 = bytes / 16;
     const int n_tail = (int)((bytes - n16 * 16) / 4);
     int64_t blocks = (n16 + 255) / 256;
-    if (blocks > 256 * 32) blocks = 256 * 32;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(zero_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (uint4*)ptr, n16,
                        (uint32_t*)((char*)ptr + n16 * 16), n_tail);
