@@ -168,6 +168,11 @@ int64_t svox_query_vertical_backward_workspace_bytes(const SvoxTreeSpec* tree, i
 int svox_assign_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                          const void* values, int32_t value_dim, void* stream);
 
+/* The same where the leaves of the points are known: node_ids (n_points) as svox_query_vertical left them, or NULL.  The tree is
+ * not walked then; a point whose id is no cell of the tree adds nothing. */
+int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
+                                     const void* grad_output, int32_t grad_dim, void* grad_data_out,
+                                     int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
 /* calc_corners(TreeSpec&, indexer) -> (n,3); svox_kernel.cu:184-203.  indexer (n_leaves,4) int64
  * rows [node, x, y, z]; corners_out (n_leaves,3) scalar of tree->dtype. */
 int svox_calc_corners(const SvoxTreeSpec* tree, const int64_t* indexer, int64_t n_leaves,

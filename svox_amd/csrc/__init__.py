@@ -157,9 +157,9 @@ def query_vertical(tree, indices):
     return _shim().query_vertical(tree, indices)
 
 
-def query_vertical_backward(tree, indices, grad_output):
+def query_vertical_backward(tree, indices, grad_output, node_ids=None):
     """zeros (M, N, N, N, grad_output.shape[1]) + scatter-add; svox_kernel.cu:160-182"""
-    return _shim().query_vertical_backward(tree, indices, grad_output)
+    return _shim().query_vertical_backward(tree, indices, grad_output, node_ids)
 
 
 def assign_vertical(tree, indices, values):

@@ -25,7 +25,7 @@ namespace {
 // ---- the library
 #define SVOX_CALLS(X)                                                                                                   \
     X(svox_last_error) X(svox_status_string) X(svox_out_data_dim) X(svox_query_vertical) \
-    X(svox_query_vertical_backward_ws) X(svox_query_vertical_backward_workspace_bytes)                                  \
+    X(svox_query_vertical_backward_ids) X(svox_query_vertical_backward_workspace_bytes)                                  \
     X(svox_assign_vertical) X(svox_calc_corners) X(svox_volume_render) X(svox_volume_render_images)                     \
     X(svox_volume_render_noted) X(svox_volume_render_images_noted) X(svox_volume_render_backward_ws)                    \
     X(svox_volume_render_images_backward_ws) X(svox_volume_render_backward_noted_with)                                  \
@@ -337,7 +337,8 @@ py::tuple query_vertical(py::handle tree, const py::object& points) {
     return py::make_tuple(values, ids);
 }
 
-Tensor query_vertical_backward(py::handle tree, const py::object& points, const py::object& grad_output) {
+// node_ids: the leaves of the points as query_vertical left them, or None
+Tensor query_vertical_backward(py::handle tree, const py::object& points, const py::object& grad_output, const py::object& node_ids) {
     const Tensor &p = tensor(points, "indices"), &g = tensor(grad_output, "grad_output");
     check_input(p, "indices");
     if (p.dim() != 2) fail("indices must be 2-D");
@@ -353,8 +354,14 @@ Tensor query_vertical_backward(py::handle tree, const py::object& points, const 
     const int64_t bytes = lib.svox_query_vertical_backward_workspace_bytes(&t.spec, p.size(0), (int32_t)g.size(1));
     Tensor space;
     if (bytes > 0) space = at::empty({bytes}, p.options().dtype(at::kByte));
-    status(lib.svox_query_vertical_backward_ws(&t.spec, p.data_ptr(), p.size(0), g.data_ptr(), (int32_t)g.size(1),
-                                               grad.data_ptr(), 0, bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
+    const int64_t* ids = nullptr;
+    if (!node_ids.is_none()) {
+        const Tensor& i = tensor(node_ids, "node_ids");
+        check_shaped(i, "node_ids", at::kLong, {p.size(0)});
+        ids = (const int64_t*)i.data_ptr();
+    }
+    status(lib.svox_query_vertical_backward_ids(&t.spec, p.data_ptr(), ids, p.size(0), g.data_ptr(), (int32_t)g.size(1),
+                                                grad.data_ptr(), 0, bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
            "query_vertical_backward");
     return grad;
 }

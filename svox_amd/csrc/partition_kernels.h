@@ -3,7 +3,8 @@
 // Adding a point's gradient row to its leaf with atomics (query_kernel) costs the memory system a request per 64 bytes,
 // about 16 a nanosecond, after the gradient has been cleared.  Where the points are many beside the tree, it is cheaper to
 // bring the points of neighbouring leaves together and write every row of the gradient once:
-//   count    every block of points counts how many fall into each bin of rows (a bin: a few thousand rows);
+//   count    every block of points counts how many fall into each bin of rows (a bin: a few thousand rows), from the leaves
+//            the query found where the caller kept them (28 -> 9 us for the points below);
 //   offsets  prefix sums of the counts over the blocks, bin by bin;
 //   place    (row, point) pairs, bin after bin;
 //   collect  a block per tile of rows (up to 256) picks its pairs out of the bin, puts them in order and
@@ -26,6 +27,7 @@ struct Partition {
     int32_t n_blocks, n_bins;
     int32_t bin_shift;      // rows of a bin, log2
     int32_t tile_shift;     // rows of a tile, log2
+    const int64_t* ids;     // [n_points]: leaves of the points, where the caller knows them, or null
     int32_t* leaf;          // [n_points]
     int32_t* counts;        // [n_bins][n_blocks]
     int32_t* totals;        // [n_bins]
@@ -49,7 +51,7 @@ static __global__ __launch_bounds__(kPointThreads) void partition_count_kernel(T
     for (int i = threadIdx.x; i < part.per_block; i += kPointThreads) {
         const int64_t q = first + i;
         if (q >= part.n_points) break;
-        const int64_t leaf = query_leaf<float, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, true);
+        const int64_t leaf = part.ids ? part.ids[q] : query_leaf<float, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, true);
         // (no leaf: a malformed tree; and what is no row of this tree is left out)
         const bool ok = leaf >= 0 && leaf < part.n_rows;
         part.leaf[q] = ok ? (int32_t)leaf : -1;

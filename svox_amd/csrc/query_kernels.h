@@ -92,9 +92,17 @@ __device__ __forceinline__ void move_rows(int lane, int n_rows, int32_t Kx, int6
 }
 
 // MODE gather:      values[q][0..Kx) = data[leaf_q][0..Kx), ids[q] = leaf_q        (Kx = K)
-// MODE scatter-add: target[leaf_q][0..Kx) += values[q][0..Kx)   (target row stride Kx)
+// MODE scatter-add: target[leaf_q][0..Kx) += values[q][0..Kx)   (target row stride Kx); with ids given, leaf_q = ids[q], and the
+//                   points are not looked up
 // MODE assign:      data[leaf_q][0..Kx) = values[q][0..Kx)      (tree row stride K)
 template <typename T, int MODE, bool kOctree>
+// The leaf the scatter was told of, -1 if it is none of the tree's.
+template <typename T>
+__device__ __forceinline__ int64_t known_leaf(const TreeDev<T>& tr, const int64_t* __restrict__ ids, int64_t q, bool valid) {
+    const int64_t leaf = valid ? ids[q] : -1;
+    return leaf < tr.capacity * tr.N * tr.N * tr.N ? leaf : -1;
+}
+
 __global__ __launch_bounds__(kQueryThreads) void query_kernel(TreeDev<T> tr, const T* __restrict__ points,
                                                               int64_t n_points, T* values, T* target,
                                                               int64_t* __restrict__ ids, int32_t Kx,
@@ -116,7 +124,8 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(TreeDev<T> tr, con
         // a wavefront owns 64 consecutive points; lane l walks point l
         const int64_t wave_base = tile * kQueryThreads + (int64_t)(threadIdx.x / kWave) * kWave;
         const int64_t q = wave_base + lane;
-        const int64_t leaf = query_leaf<T, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, q < n_points);
+        const int64_t leaf = MODE == kQueryScatterAdd && ids ? known_leaf(tr, ids, q, q < n_points)
+                                                             : query_leaf<T, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, q < n_points);
         if (MODE == kQueryGather && ids && q < n_points) ids[q] = leaf;
         // phase 2: the 64 rows of the run, flat index f = p * Kx + e
         const int64_t remaining = n_points - wave_base;
@@ -181,7 +190,8 @@ __global__ __launch_bounds__(kWave) void query_few_kernel(TreeDev<T> tr, const T
     const bool valid = q < n_points;
     T offset[3], scaling[3];
     load_transform(tr, offset, scaling);
-    const int64_t leaf = query_leaf<T, kOctree>(tr, nullptr, 0, offset, scaling, points, q, valid);
+    const int64_t leaf = MODE == kQueryScatterAdd && ids ? known_leaf(tr, ids, q, valid)
+                                                         : query_leaf<T, kOctree>(tr, nullptr, 0, offset, scaling, points, q, valid);
     if (MODE == kQueryGather && ids && valid && lane % (kWave / kFewPoints) == 0) ids[q] = leaf;
     const int64_t remaining = n_points - base;
     const int n_rows = remaining < kFewPoints ? (int)remaining : kFewPoints;

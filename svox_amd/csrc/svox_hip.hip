@@ -239,8 +239,9 @@ int64_t plan_partition(const SvoxTreeSpec* tree, int64_t n, int32_t K, Partition
     part->n_blocks = (int32_t)((n + part->per_block - 1) / part->per_block);
     return n * 12 + ((int64_t)part->n_bins * part->n_blocks + 2 * part->n_bins + 16) * 4;
 }
-int launch_partition(const SvoxTreeSpec* tree, Partition part, const float* points, const float* values, int32_t K, float* grad,
-                     void* workspace, hipStream_t stream) {
+int launch_partition(const SvoxTreeSpec* tree, Partition part, const float* points, const int64_t* ids, const float* values, int32_t K,
+                     float* grad, void* workspace, hipStream_t stream) {
+    part.ids = ids;
     part.pairs = (uint2*)workspace;
     part.leaf = (int32_t*)(part.pairs + part.n_points);
     part.counts = part.leaf + part.n_points;
@@ -248,7 +249,7 @@ int launch_partition(const SvoxTreeSpec* tree, Partition part, const float* poin
     part.starts = part.totals + part.n_bins;
     const TreeDev<float> tr = make_tree<float>(tree);
     const dim3 threads(kPartThreads);
-    const int32_t lds_nodes = tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
+    const int32_t lds_nodes = ids ? 0 : tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
     if (octree_fast_ok(tree))
         hipLaunchKernelGGL((partition_count_kernel<true>), dim3(part.n_blocks), dim3(kPointThreads), (size_t)lds_nodes * 32, stream, tr, points,
                            part, lds_nodes);
@@ -919,7 +920,7 @@ int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indice
         Partition part;
         const int64_t need = plan_partition(tree, n_points, grad_dim, &part);
         if (need > 0 && need <= workspace_bytes)
-            return launch_partition(tree, part, (const float*)indices, (const float*)grad_output, grad_dim,
+            return launch_partition(tree, part, (const float*)indices, node_ids, (const float*)grad_output, grad_dim,
                                     (float*)grad_data_out, workspace, (hipStream_t)stream);
     }
     const int64_t esz = tree->dtype == SVOX_F32 ? 4 : 8;
@@ -932,14 +933,21 @@ int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indice
     if (!indices || !grad_output) return fail(SVOX_ERR_NULL_POINTER, "indices / grad_output is NULL");
     if (tree->dtype == SVOX_F32)
         return launch_query<float, kQueryScatterAdd>(tree, indices, n_points, (void*)grad_output, grad_data_out,
-                                                     nullptr, grad_dim, (hipStream_t)stream,
+                                                     (int64_t*)node_ids, grad_dim, (hipStream_t)stream,
                                                      "query_vertical_backward");
     return launch_query<double, kQueryScatterAdd>(tree, indices, n_points, (void*)grad_output, grad_data_out,
-                                                  nullptr, grad_dim, (hipStream_t)stream,
+                                                  (int64_t*)node_ids, grad_dim, (hipStream_t)stream,
                                                   "query_vertical_backward");
 }
 
 int svox_assign_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points, const void* values,
+    return svox_query_vertical_backward_ids(tree, indices, nullptr, n_points, grad_output, grad_dim, grad_data_out, accumulate,
+                                            workspace, workspace_bytes, stream);
+}
+
+int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
+                                     const void* grad_output, int32_t grad_dim, void* grad_data_out, int32_t accumulate,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
                          int32_t value_dim, void* stream) {
     int rc = check_tree(tree, true);
     if (rc) return rc;

@@ -30,6 +30,39 @@ def test_gradient_by_rows(gpu, N, levels, dim, n, spread):
     assert _abi.load_library().svox_query_vertical_backward_workspace_bytes(ctypes.byref(spec), n, dim) > 0
     got = C.query_vertical_backward(tree._spec(world=False), points, grad)
     _, ids = C.query_vertical(tree._spec(world=False), points)
+    again = C.query_vertical_backward(tree._spec(world=False), points, grad, ids)   # (the leaves known: nothing is looked up)
     want = torch.zeros(tree.data.numel() // dim, dim, dtype=torch.float64)
     want.index_add_(0, ids.cpu(), grad.double().cpu())
-    assert (got.view(-1, dim).cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
+    for g in (got, again):
+        assert (g.view(-1, dim).cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("n,dtype,N", [(65536, torch.float32, 2), (70001, torch.float64, 2), (300001, torch.float32, 3)])
+def test_gradient_at_known_leaves(gpu, n, dtype, N):
+    """Atomics at leaves the query kept: both launch shapes, both scalar types; ids that are no cell add nothing; and what
+    makes the leaves void (the tree or the ids written to before the backward pass)."""
+    tree = svox.N3Tree(N=N, data_dim=4, init_refine=3, data_format="RGBA", dtype=dtype).to(gpu)
+    gen = torch.Generator().manual_seed(n)
+    points = torch.rand(n, 3, generator=gen, dtype=dtype).to(gpu)
+    grad = torch.randn(n, 4, generator=gen, dtype=dtype).to(gpu)
+    spec = tree._spec()
+    _, ids = C.query_vertical(spec, points)
+
+    def sums(ids):
+        want = torch.zeros(tree.data.numel() // 4, 4, dtype=torch.float64)
+        ok = (ids >= 0) & (ids < want.shape[0])
+        return want.index_add_(0, ids[ok].cpu(), grad[ok].double().cpu())
+    odd = ids.clone()
+    odd[::7], odd[3::7] = -1, tree.child.numel()
+    for known in (ids, odd):
+        got = C.query_vertical_backward(spec, points, grad, known).view(-1, 4).cpu().double()
+        want = sums(known)
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()
+    for void in (False, True):
+        tree.data.grad = None
+        values, node_ids = tree(points, want_node_ids=True)
+        if void:
+            node_ids.zero_()
+        values.backward(grad)
+        want = sums(ids)
+        assert (tree.data.grad.view(-1, 4).cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
