@@ -147,6 +147,13 @@ int svox_give_up_count(int64_t* count_out);
 int svox_query_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                         void* values_out, int64_t* node_ids_out, void* stream);
 
+/* The same with a workspace (no reference counterpart): where the points are many beside the tree, the call first makes a copy
+ * of the child table in it that saves every point the last step of its search.  _workspace_bytes: how large it has to be for
+ * these calls (4-byte aligned); 0 where the call would make no use of one.  A smaller workspace, or NULL, is the plain call. */
+int svox_query_vertical_ws(const SvoxTreeSpec* tree, const void* indices, int64_t n_points, void* values_out,
+                           int64_t* node_ids_out, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t svox_query_vertical_workspace_bytes(const SvoxTreeSpec* tree, int64_t n_points);
+
 /* query_vertical_backward(TreeSpec&, indices, grad_output) -> grad_data; svox_kernel.cu:160-182.
  * grad_output (n_points, grad_dim); grad_data_out (capacity, N, N, N, grad_dim).  The reference
  * returns a fresh zero-filled tensor; here the library zero-fills grad_data_out first unless
@@ -161,6 +168,11 @@ int svox_query_vertical_backward(const SvoxTreeSpec* tree, const void* indices, 
 int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                                     const void* grad_output, int32_t grad_dim, void* grad_data_out,
                                     int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same where the leaves of the points are known: node_ids (n_points) as svox_query_vertical left them, or NULL.  The tree is
+ * not walked then; a point whose id is no cell of the tree adds nothing. */
+int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
+                                     const void* grad_output, int32_t grad_dim, void* grad_data_out,
+                                     int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t svox_query_vertical_backward_workspace_bytes(const SvoxTreeSpec* tree, int64_t n_points, int32_t grad_dim);
 
 /* assign_vertical(TreeSpec&, indices, values); svox_kernel.cu:145-158.  values (n_points, value_dim),
@@ -168,11 +180,6 @@ int64_t svox_query_vertical_backward_workspace_bytes(const SvoxTreeSpec* tree, i
 int svox_assign_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                          const void* values, int32_t value_dim, void* stream);
 
-/* The same where the leaves of the points are known: node_ids (n_points) as svox_query_vertical left them, or NULL.  The tree is
- * not walked then; a point whose id is no cell of the tree adds nothing. */
-int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
-                                     const void* grad_output, int32_t grad_dim, void* grad_data_out,
-                                     int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
 /* calc_corners(TreeSpec&, indexer) -> (n,3); svox_kernel.cu:184-203.  indexer (n_leaves,4) int64
  * rows [node, x, y, z]; corners_out (n_leaves,3) scalar of tree->dtype. */
 int svox_calc_corners(const SvoxTreeSpec* tree, const int64_t* indexer, int64_t n_leaves,

@@ -114,15 +114,18 @@ SIGNATURES = {
     "svox_set_debug_flags": (None, [ctypes.c_int]),
     "svox_out_data_dim": (ctypes.c_int, [c_int32, c_int32, c_int32]),
     "svox_query_vertical": (ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+    "svox_query_vertical_ws": (
+        ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "svox_query_vertical_workspace_bytes": (c_int64, [P(TreeSpecC), c_int64]),
     "svox_query_vertical_backward": (
         ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_void_p]),
     "svox_query_vertical_backward_ws": (
         ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
+    "svox_query_vertical_backward_ids": (
+        ctypes.c_int, [P(TreeSpecC), c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
     "svox_query_vertical_backward_workspace_bytes": (c_int64, [P(TreeSpecC), c_int64, c_int32]),
     "svox_assign_vertical": (ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_int32, c_void_p]),
     "svox_calc_corners": (ctypes.c_int, [P(TreeSpecC), c_void_p, c_int64, c_void_p, c_void_p]),
-    "svox_query_vertical_backward_ids": (
-        ctypes.c_int, [P(TreeSpecC), c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
     "svox_volume_render": (ctypes.c_int, [P(TreeSpecC), P(RaysSpecC), P(RenderOptionsC), c_void_p, c_void_p]),
     "svox_volume_render_image": (
         ctypes.c_int, [P(TreeSpecC), P(CameraSpecC), P(RenderOptionsC), c_void_p, c_void_p]),

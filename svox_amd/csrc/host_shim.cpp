@@ -24,7 +24,8 @@ namespace {
 
 // ---- the library
 #define SVOX_CALLS(X)                                                                                                   \
-    X(svox_last_error) X(svox_status_string) X(svox_out_data_dim) X(svox_query_vertical) \
+    X(svox_last_error) X(svox_status_string) X(svox_out_data_dim) X(svox_query_vertical_ws) \
+    X(svox_query_vertical_workspace_bytes)                                                            \
     X(svox_query_vertical_backward_ids) X(svox_query_vertical_backward_workspace_bytes)                                  \
     X(svox_assign_vertical) X(svox_calc_corners) X(svox_volume_render) X(svox_volume_render_images)                     \
     X(svox_volume_render_noted) X(svox_volume_render_images_noted) X(svox_volume_render_backward_ws)                    \
@@ -332,7 +333,11 @@ py::tuple query_vertical(py::handle tree, const py::object& points) {
     Tensor values = like(p, {p.size(0), t.spec.data_dim});
     Tensor ids = at::empty({p.size(0)}, t.child.options().dtype(at::kLong));
     const On on(p);
-    status(lib.svox_query_vertical(&t.spec, p.data_ptr(), p.size(0), values.data_ptr(), (int64_t*)ids.data_ptr(), on.stream),
+    const int64_t bytes = lib.svox_query_vertical_workspace_bytes(&t.spec, p.size(0));
+    Tensor space;
+    if (bytes > 0) space = at::empty({bytes}, t.child.options().dtype(at::kByte));
+    status(lib.svox_query_vertical_ws(&t.spec, p.data_ptr(), p.size(0), values.data_ptr(), (int64_t*)ids.data_ptr(),
+                                      bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
            "query_vertical");
     return py::make_tuple(values, ids);
 }
@@ -349,17 +354,17 @@ Tensor query_vertical_backward(py::handle tree, const py::object& points, const 
     same_dtype(g, p.scalar_type(), "grad_output");
     const Tree t = pack_tree(tree, p.scalar_type(), false);
     if (g.size(0) != p.size(0)) fail("grad_output must have one row per point");
-    Tensor grad = like(g, {t.spec.capacity, t.spec.N, t.spec.N, t.spec.N, g.size(1)});
-    const On on(p);
-    const int64_t bytes = lib.svox_query_vertical_backward_workspace_bytes(&t.spec, p.size(0), (int32_t)g.size(1));
-    Tensor space;
-    if (bytes > 0) space = at::empty({bytes}, p.options().dtype(at::kByte));
     const int64_t* ids = nullptr;
     if (!node_ids.is_none()) {
         const Tensor& i = tensor(node_ids, "node_ids");
         check_shaped(i, "node_ids", at::kLong, {p.size(0)});
         ids = (const int64_t*)i.data_ptr();
     }
+    Tensor grad = like(g, {t.spec.capacity, t.spec.N, t.spec.N, t.spec.N, g.size(1)});
+    const On on(p);
+    const int64_t bytes = lib.svox_query_vertical_backward_workspace_bytes(&t.spec, p.size(0), (int32_t)g.size(1));
+    Tensor space;
+    if (bytes > 0) space = at::empty({bytes}, p.options().dtype(at::kByte));
     status(lib.svox_query_vertical_backward_ids(&t.spec, p.data_ptr(), ids, p.size(0), g.data_ptr(), (int32_t)g.size(1),
                                                 grad.data_ptr(), 0, bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
            "query_vertical_backward");

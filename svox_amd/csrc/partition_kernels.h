@@ -51,7 +51,7 @@ static __global__ __launch_bounds__(kPointThreads) void partition_count_kernel(T
     for (int i = threadIdx.x; i < part.per_block; i += kPointThreads) {
         const int64_t q = first + i;
         if (q >= part.n_points) break;
-        const int64_t leaf = part.ids ? part.ids[q] : query_leaf<float, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, true);
+        const int64_t leaf = part.ids ? part.ids[q] : query_leaf<float, kOctree>(tr, tr.child, lds_child, lds_nodes, offset, scaling, points, q, true);
         // (no leaf: a malformed tree; and what is no row of this tree is left out)
         const bool ok = leaf >= 0 && leaf < part.n_rows;
         part.leaf[q] = ok ? (int32_t)leaf : -1;

@@ -22,9 +22,10 @@ constexpr int kWave = 64;
 enum QueryMode { kQueryGather = 0, kQueryScatterAdd = 1, kQueryAssign = 2 };
 typedef unsigned int Piece16 __attribute__((ext_vector_type(4)));   // 16 bytes as the non-temporal builtins take them
 
-// Leaf of a point (packed leaf id or -1).  lds_child: the child rows of the nodes below lds_nodes.
+// Leaf of a point (packed leaf id or -1).  lds_child: the child rows of the nodes below lds_nodes; walk: the child table or its
+// copy with kLastNodeBit (octrees).
 template <typename T, bool kOctree>
-__device__ __forceinline__ int64_t query_leaf(const TreeDev<T>& tr, const int32_t* lds_child, int32_t lds_nodes,
+__device__ __forceinline__ int64_t query_leaf(const TreeDev<T>& tr, const int32_t* __restrict__ walk, const int32_t* lds_child, int32_t lds_nodes,
                                               const T* offset, const T* scaling, const T* __restrict__ points, int64_t q,
                                               bool valid) {
     T xyz[3];
@@ -34,7 +35,7 @@ __device__ __forceinline__ int64_t query_leaf(const TreeDev<T>& tr, const int32_
     int64_t leaf = -1;
     if constexpr (kOctree) {
         if (valid)
-            leaf = descend_octree(tr.child, lds_child, lds_nodes, tr.capacity, cell_coord(clamp01(xyz[0])),
+            leaf = descend_octree(walk, lds_child, lds_nodes, tr.capacity, cell_coord(clamp01(xyz[0])),
                                   cell_coord(clamp01(xyz[1])), cell_coord(clamp01(xyz[2])));
     }
     if (valid && leaf < 0) {   // deeper than the integer coordinates resolve: once more with the floating-point walk
@@ -95,7 +96,6 @@ __device__ __forceinline__ void move_rows(int lane, int n_rows, int32_t Kx, int6
 // MODE scatter-add: target[leaf_q][0..Kx) += values[q][0..Kx)   (target row stride Kx); with ids given, leaf_q = ids[q], and the
 //                   points are not looked up
 // MODE assign:      data[leaf_q][0..Kx) = values[q][0..Kx)      (tree row stride K)
-template <typename T, int MODE, bool kOctree>
 // The leaf the scatter was told of, -1 if it is none of the tree's.
 template <typename T>
 __device__ __forceinline__ int64_t known_leaf(const TreeDev<T>& tr, const int64_t* __restrict__ ids, int64_t q, bool valid) {
@@ -103,13 +103,14 @@ __device__ __forceinline__ int64_t known_leaf(const TreeDev<T>& tr, const int64_
     return leaf < tr.capacity * tr.N * tr.N * tr.N ? leaf : -1;
 }
 
+template <typename T, int MODE, bool kOctree>
 __global__ __launch_bounds__(kQueryThreads) void query_kernel(TreeDev<T> tr, const T* __restrict__ points,
                                                               int64_t n_points, T* values, T* target,
                                                               int64_t* __restrict__ ids, int32_t Kx,
-                                                              int32_t lds_nodes) {
+                                                              const int32_t* __restrict__ walk, int32_t lds_nodes) {
     extern __shared__ int32_t lds_child[];
     if constexpr (kOctree) {
-        for (int i = threadIdx.x; i < lds_nodes * 8; i += kQueryThreads) lds_child[i] = tr.child[i];
+        for (int i = threadIdx.x; i < lds_nodes * 8; i += kQueryThreads) lds_child[i] = walk[i];
         __syncthreads();
     }
     T offset[3], scaling[3];
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kQueryThreads) void query_kernel(TreeDev<T> tr, con
         const int64_t wave_base = tile * kQueryThreads + (int64_t)(threadIdx.x / kWave) * kWave;
         const int64_t q = wave_base + lane;
         const int64_t leaf = MODE == kQueryScatterAdd && ids ? known_leaf(tr, ids, q, q < n_points)
-                                                             : query_leaf<T, kOctree>(tr, lds_child, lds_nodes, offset, scaling, points, q, q < n_points);
+                                                             : query_leaf<T, kOctree>(tr, walk, lds_child, lds_nodes, offset, scaling, points, q, q < n_points);
         if (MODE == kQueryGather && ids && q < n_points) ids[q] = leaf;
         // phase 2: the 64 rows of the run, flat index f = p * Kx + e
         const int64_t remaining = n_points - wave_base;
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(kWave) void query_few_kernel(TreeDev<T> tr, const T
     T offset[3], scaling[3];
     load_transform(tr, offset, scaling);
     const int64_t leaf = MODE == kQueryScatterAdd && ids ? known_leaf(tr, ids, q, valid)
-                                                         : query_leaf<T, kOctree>(tr, nullptr, 0, offset, scaling, points, q, valid);
+                                                         : query_leaf<T, kOctree>(tr, tr.child, nullptr, 0, offset, scaling, points, q, valid);
     if (MODE == kQueryGather && ids && valid && lane % (kWave / kFewPoints) == 0) ids[q] = leaf;
     const int64_t remaining = n_points - base;
     const int n_rows = remaining < kFewPoints ? (int)remaining : kFewPoints;
@@ -201,6 +202,22 @@ __global__ __launch_bounds__(kWave) void query_few_kernel(TreeDev<T> tr, const T
         const int lo = __shfl(leaf_lo, from), hi = __shfl(leaf_hi, from);
         return ((int64_t)hi << 32) | (uint32_t)lo;
     }, tr.data, values + base * Kx, target);
+}
+
+// The octree's child table with kLastNodeBit (tree_walk.h).  One thread per cell.
+static __global__ __launch_bounds__(256) void last_nodes_kernel(const int32_t* __restrict__ child, int32_t capacity,
+                                                                int32_t* __restrict__ walk) {
+    const int64_t i = blockIdx.x * 256ll + threadIdx.x;
+    if (i >= capacity * 8ll) return;
+    int32_t c = child[i];
+    const int64_t node = (i >> 3) + c;
+    if (c >= kLastNodeBit) {
+        c = kLastNodeBit - 1;   // (a malformed tree's: still past the end)
+    } else if (c > 0 && node < capacity) {
+        const int4 lo = ((const int4*)child)[node * 2], hi = ((const int4*)child)[node * 2 + 1];
+        if ((lo.x | lo.y | lo.z | lo.w | hi.x | hi.y | hi.z | hi.w) == 0) c |= kLastNodeBit;
+    }
+    walk[i] = c;
 }
 
 // calc_corner_kernel, svox_kernel.cu:91-115: climb parent links from the leaf's node to the

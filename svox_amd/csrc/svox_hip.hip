@@ -176,11 +176,20 @@ int zero_fill(void* ptr, int64_t bytes, hipStream_t stream) {
 // 52.7 / 54.8.  (Larger wavefronts of 128 points, two to a lane, for the rest: SH16, 1 Mi points 92 / 92, 262 144 points
 // 37 / 47.)
 constexpr int64_t kFewPointsMax = 262144;
+// Whether a query of n points is worth a copy of the child table in which the nodes of leaves only are marked
+// (last_nodes_kernel).  It takes 5 us and 14 ps a node, and what it saves -- a request for a line of the table, which the
+// memory system serves 55 of a nanosecond once the table is larger than an L2 cache -- goes to the points that end in such a
+// node: all of a dense tree's, few of those thrown at random on a sparse one, which the line lies between.  (us, plain / with
+// the copy, its making included; 4 Mi points: 128^3 RGBA 173 / 111 and SH9 285 / 257, 64^3 RGBA 81 / 63, 256^3 shell SH9
+// 122 / 121, 512^3 shell SH4 105 / 119, 32^3 SH4 83 / 82; 1 000 003 points: 128^3 SH9 75 / 66, 256^3 shell SH9 36 / 40.)
+bool walk_copy_pays(const SvoxTreeSpec* tree, int64_t n) {
+    return octree_fast_ok(tree) && tree->dtype == SVOX_F32 && tree->capacity >= 30000 && n >= 12 * tree->capacity;
+}
 constexpr int kLdsNodesMax = 584;  // child rows kept in LDS per block: 584 * 32 B = 18.25 KiB
 
 template <typename T, int MODE>
 int launch_query(const SvoxTreeSpec* tree, const void* points, int64_t n, void* values, void* target,
-                 int64_t* ids, int32_t Kx, hipStream_t stream, const char* what) {
+                 int64_t* ids, int32_t Kx, hipStream_t stream, const char* what, int32_t* walk_space = nullptr) {
     if (n == 0) return SVOX_OK;
     const TreeDev<T> tr = make_tree<T>(tree);
     if (n <= kFewPointsMax) {
@@ -197,15 +206,23 @@ int launch_query(const SvoxTreeSpec* tree, const void* points, int64_t n, void* 
     const int64_t blocks = tiles < 256 * 8 ? tiles : 256 * 8;
     if constexpr (sizeof(T) == 4) {
         if (octree_fast_ok(tree)) {
-            const int32_t lds_nodes = tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
+            // (a scatter with the leaves at hand walks nothing)
+            const bool walks = MODE != kQueryScatterAdd || !ids;
+            const int32_t lds_nodes = !walks ? 0 : tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
+            const int32_t* walk = tr.child;
+            if (walk_space) {
+                hipLaunchKernelGGL(last_nodes_kernel, dim3((unsigned)((tree->capacity * 8 + 255) / 256)), dim3(256), 0, stream, tr.child,
+                                   (int32_t)tree->capacity, walk_space);
+                walk = walk_space;
+            }
             hipLaunchKernelGGL((query_kernel<T, MODE, true>), dim3((unsigned)blocks), dim3(kQueryThreads),
                                (size_t)lds_nodes * 32, stream, tr, (const T*)points, n, (T*)values,
-                               (T*)target, ids, Kx, lds_nodes);
+                               (T*)target, ids, Kx, walk, lds_nodes);
             return check_launch(what);
         }
     }
     hipLaunchKernelGGL((query_kernel<T, MODE, false>), dim3((unsigned)blocks), dim3(kQueryThreads), 0, stream,
-                       tr, (const T*)points, n, (T*)values, (T*)target, ids, Kx, 0);
+                       tr, (const T*)points, n, (T*)values, (T*)target, ids, Kx, tr.child, 0);
     return check_launch(what);
 }
 
@@ -883,14 +900,27 @@ int svox_out_data_dim(int32_t format, int32_t basis_dim, int32_t data_dim) {
 
 int svox_query_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points, void* values_out,
                         int64_t* node_ids_out, void* stream) {
+    return svox_query_vertical_ws(tree, indices, n_points, values_out, node_ids_out, nullptr, 0, stream);
+}
+
+int64_t svox_query_vertical_workspace_bytes(const SvoxTreeSpec* tree, int64_t n_points) {
+    if (check_tree(tree, false) || n_points <= 0 || !walk_copy_pays(tree, n_points)) return 0;
+    return tree->capacity * 32;
+}
+
+int svox_query_vertical_ws(const SvoxTreeSpec* tree, const void* indices, int64_t n_points, void* values_out,
+                           int64_t* node_ids_out, void* workspace, int64_t workspace_bytes, void* stream) {
     int rc = check_tree(tree, true);
     if (rc) return rc;
     if (n_points < 0) return fail(SVOX_ERR_BAD_SHAPE, "negative point count");
     if (n_points == 0) return SVOX_OK;
     if (!indices || !values_out || !node_ids_out) return fail(SVOX_ERR_NULL_POINTER, "indices / values_out / node_ids_out is NULL");
+    const bool copy = workspace && ((uintptr_t)workspace & 3u) == 0 && ((uintptr_t)tree->child & 15u) == 0 &&
+                      workspace_bytes >= tree->capacity * 32 && walk_copy_pays(tree, n_points);
     if (tree->dtype == SVOX_F32)
         return launch_query<float, kQueryGather>(tree, indices, n_points, values_out, nullptr, node_ids_out,
-                                                 tree->data_dim, (hipStream_t)stream, "query_vertical");
+                                                 tree->data_dim, (hipStream_t)stream, "query_vertical",
+                                                 copy ? (int32_t*)workspace : nullptr);
     return launch_query<double, kQueryGather>(tree, indices, n_points, values_out, nullptr, node_ids_out,
                                               tree->data_dim, (hipStream_t)stream, "query_vertical");
 }
@@ -911,6 +941,13 @@ int64_t svox_query_vertical_backward_workspace_bytes(const SvoxTreeSpec* tree, i
 int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indices, int64_t n_points,
                                     const void* grad_output, int32_t grad_dim, void* grad_data_out, int32_t accumulate,
                                     void* workspace, int64_t workspace_bytes, void* stream) {
+    return svox_query_vertical_backward_ids(tree, indices, nullptr, n_points, grad_output, grad_dim, grad_data_out, accumulate,
+                                            workspace, workspace_bytes, stream);
+}
+
+int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
+                                     const void* grad_output, int32_t grad_dim, void* grad_data_out, int32_t accumulate,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
     int rc = check_tree(tree, false);
     if (rc) return rc;
     if (n_points < 0 || grad_dim < 1) return fail(SVOX_ERR_BAD_SHAPE, "negative point count or grad_dim < 1");
@@ -941,13 +978,6 @@ int svox_query_vertical_backward_ws(const SvoxTreeSpec* tree, const void* indice
 }
 
 int svox_assign_vertical(const SvoxTreeSpec* tree, const void* indices, int64_t n_points, const void* values,
-    return svox_query_vertical_backward_ids(tree, indices, nullptr, n_points, grad_output, grad_dim, grad_data_out, accumulate,
-                                            workspace, workspace_bytes, stream);
-}
-
-int svox_query_vertical_backward_ids(const SvoxTreeSpec* tree, const void* indices, const int64_t* node_ids, int64_t n_points,
-                                     const void* grad_output, int32_t grad_dim, void* grad_data_out, int32_t accumulate,
-                                     void* workspace, int64_t workspace_bytes, void* stream) {
                          int32_t value_dim, void* stream) {
     int rc = check_tree(tree, true);
     if (rc) return rc;

@@ -47,6 +47,10 @@ struct TreeDev {
 // and sets this bit in the leaf id it returns for such a leaf (octree leaf ids stay below 2^30).
 constexpr int32_t kEmptyLeafBit = 1 << 30;
 
+// The point queries may be given a copy of an octree's child table in which an entry whose node has leaves only carries this
+// bit: the row of such a node, where most searches end, need not be read.  (Entries of a well-formed table stay below 2^28.)
+constexpr int32_t kLastNodeBit = 1 << 30;
+
 template <typename T>
 __device__ __forceinline__ void load_transform(const TreeDev<T>& tr, T* offset, T* scaling) {
 #pragma unroll
@@ -136,8 +140,14 @@ __device__ __forceinline__ int32_t descend_octree(const int32_t* __restrict__ ch
             leaf = cell;
             live = false;
         } else {
-            node += skip;
-            if (node < 0 || node >= capacity) live = false;
+            const bool last = skip >= kLastNodeBit;
+            node += last ? skip - kLastNodeBit : skip;
+            if (node < 0 || node >= capacity) {
+                live = false;
+            } else if (last) {
+                if (level < kCoordBits) leaf = node * 8 + cell_at(ix, iy, iz, level + 1);
+                live = false;
+            }
         }
     }
     return leaf;  // (-1 also where the tree is deeper than the integer coordinates resolve)

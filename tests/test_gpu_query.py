@@ -1,5 +1,7 @@
 """GPU parity of the point-query operators against the CPU oracle (bit-exact bar for ids, values,
 corners; 1e-4 relative for the atomically summed query gradient)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -7,6 +9,7 @@ import torch
 import svox_amd as svox
 from svox_amd import csrc as C
 from svox_amd import synth
+from svox_amd.csrc import _abi
 from util import on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -177,3 +180,30 @@ def test_from_grid_and_merge_on_the_gpu(gpu, oracle_mod):
     ref = oracle_mod.volume_render(ot, rays.origins, rays.dirs, rays.viewdirs, opt)
     out = C.volume_render(tree._spec(), rays_spec(rays, gpu), opt)
     assert np.array_equal(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("chain", [0, 9, 21])
+def test_query_of_many_points_beside_the_table(gpu, chain):
+    """A query with so many points that it copies the child table first (svox_query_vertical_ws) finds the leaves that small
+    calls find: in nodes of leaves only, in nodes of both kinds, and at the end of a chain of nodes longer than the integer
+    coordinates hold."""
+    tree = svox.N3Tree(N=2, data_format="RGBA", init_refine=5, depth_limit=40, device=gpu)
+    tree.data.data.copy_(torch.arange(tree.data.numel(), device=gpu, dtype=torch.float32).view_as(tree.data))
+    at = torch.tensor([[0.7301, 0.2107, 0.5519]])
+    for _ in range(chain):
+        tree[at.to(gpu)].refine()
+    tree.shrink_to_fit()
+    n = 12 * tree.child.shape[0] + 77
+    gen = torch.Generator().manual_seed(chain)
+    points = torch.rand(n, 3, generator=gen)
+    scale = 2.0 ** -torch.randint(1, 27, (n // 3, 1), generator=gen).float()
+    points[: n // 3] = (at + (torch.rand(n // 3, 3, generator=gen) * 2 - 1) * scale)
+    points[-1] = 1.0
+    points = points.to(gpu)
+    spec = tree._spec(world=False)
+    assert _abi.load_library().svox_query_vertical_workspace_bytes(ctypes.byref(C._pack_tree(spec)), n) > 0
+    values, ids = C.query_vertical(spec, points)
+    step = 200000
+    for i in range(0, n, step):
+        few_values, few_ids = C.query_vertical(spec, points[i:i + step].contiguous())
+        assert torch.equal(ids[i:i + step], few_ids) and torch.equal(values[i:i + step], few_values)
