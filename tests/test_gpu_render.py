@@ -1320,3 +1320,25 @@ def test_a_training_step_replays_from_a_hip_graph(gpu):
         err, ok = grad_close(tree.data.detach().cpu().numpy(), eager_data[i].cpu().numpy(), rel=1e-5)
         assert ok, (i, err)
         assert float((torch.rand(1000, device=gpu) * 2).sum()) > 0          # eager work between the replays
+
+
+@pytest.mark.parametrize("n", [2816 * 64, 2816 * 64 + 1, 3200 * 64, 3200 * 64 + 1])
+def test_ray_batches_where_the_launch_changes(gpu, n):
+    """The largest batches on two wavefronts per tile and the smallest on one, plain and with notes: the same pictures and
+    gradients as with either kernel forced (the forced kernels are held to the oracle above)."""
+    tree = on_gpu(synth.shell_tree(depth=5, n_spheres=4, data_format="SH4", seed=3), gpu)
+    rays = synth.sphere_rays(n, seed=n)
+    rs, opt = rays_spec(rays, gpu), options(tree)
+    grad = torch.randn(n, 3, generator=torch.Generator().manual_seed(1)).to(gpu)
+    got = []
+    for flags in (0, 4, 8):
+        C.set_debug_flags(flags)
+        try:
+            out = C.volume_render(tree._spec(), rs, opt)
+            noted, notes = C.volume_render_noted(tree._spec(), rs, opt)
+        finally:
+            C.set_debug_flags(0)
+        got.append((out, noted, C.volume_render_backward_noted(tree._spec(), rs, opt, grad, notes)))
+    for out, noted, data_grad in got[1:]:
+        assert torch.equal(out, got[0][0]) and torch.equal(noted, got[0][1]) and torch.equal(noted, out)
+        assert (data_grad - got[0][2]).abs().max() <= 1e-4 * data_grad.abs().max()
