@@ -226,20 +226,31 @@ int launch_query(const SvoxTreeSpec* tree, const void* points, int64_t n, void* 
     return check_launch(what);
 }
 
+// log2 of the rows of a bin, from that of a tile on: 2 048 bins at most while that leaves them small (2 048 rows: 8 tiles, each of
+// which looks through the bin's pairs), because every block of points writes a count for every bin; more in larger trees.
+int bin_shift_of(int64_t n_rows, int shift) {
+    auto bins = [&] { return ((n_rows - 1) >> shift) + 1; };
+    while (bins() > kPartBins || (bins() > 2048 && shift < 11)) ++shift;
+    return shift;
+}
+
 // How the gradient of n points is collected row by row (partition_kernels.h): fills `part` and returns the bytes of
-// workspace it needs, or returns 0 where the points are added with atomics, whichever is estimated to take less.  With
-// atomics: the gradient cleared at 6.8 bytes a picosecond, then 16.5 requests a nanosecond, a request for every 64 bytes a
-// row touches.  By rows: four launches, 45 ps a point to count and place it, and rows and points' rows at 4.4 bytes a
-// picosecond.  (us, atomics / rows; 1 000 003 points: 128^3 SH9 197 / 149, 64^3 SH16 254 / 125, 32^3 SH4 106 / 72, 128^3
-// RGBA 74 / 85; 262 144 points: 32^3 SH4 33 / 46, 64^3 SH16 80 / 61; 131 072 points of the latter 47 / 58.)
+// workspace it needs, or returns 0 where the points are added with atomics, whichever is estimated to take less where the
+// points are spread evenly over the rows.  With atomics: the gradient cleared at 6.8 bytes a picosecond, then 16.5 requests a
+// nanosecond, a request for every 64 bytes a row touches.  By rows: the launches, 45 ps a point to count and place it, rows and
+// points' rows at 4.4 bytes a picosecond, and the pairs of a bin once for each of its tiles at 8.
+// Where the points crowd, atomics on one address wait for one another and rows gain by more; the cost of the runs can eat that up
+// again where a run has one or two points to a row (the slab and the blob below).
+// (us, atomics / rows, leaves known.  Even: 1 000 003 points, 128^3 SH9 178 / 131, 64^3 SH16 253 / 101, 32^3 SH4 106 / 61, 128^3
+// RGBA 62 / 76; 4 Mi points, 128^3 SH9 612 / 319, RGBA 216 / 198; 262 144 points, 32^3 SH4 34 / 40, 64^3 SH16 78 / 60; 131 072 of
+// the latter 47 / 52; 16 Mi points, 256^3 SH1 869 / 1120.  All of space, in shells: 1 Mi points, 64^3 SH16 559 / 152, 256^3 SH9
+// 465 / 131, 512^3 SH16 887 / 554; 262 144 points, 64^3 SH16 148 / 86; 16 Mi points, 48 M rows of SH25 8030 / 6740.  1 Mi points of
+// the 128^3 SH9 tree: in 1 % of the volume 200 / 173, in 0.1 % 291 / 148, in a slab of 2 % 190 / 194, around the middle with a
+// deviation of 0.12 184 / 188, in one leaf 23 300 / 160; around the middle of the 64^3 SH16 tree 272 / 181, in 1 % of it 318 / 134.)
 int64_t plan_partition(const SvoxTreeSpec* tree, int64_t n, int32_t K, Partition* part) {
     const double rows = (double)tree->capacity * tree->N * tree->N * tree->N;
-    if (tree->dtype != SVOX_F32 || (g_debug_flags & 1) || rows > 1.5e9 || n > (1 << 30)) return 0;
-    const double row_bytes = 4.0 * K;
-    const int align = K % 16 == 0 ? 64 : K % 8 == 0 ? 32 : K % 4 == 0 ? 16 : K % 2 == 0 ? 8 : 4;   // where rows may start
-    const double atomics_us = rows * row_bytes / 6.8e6 + (double)n * (row_bytes + 64.0 - align) / 64.0 / 16500.0;
-    const double rows_us = 30.0 + (double)n * 45e-6 + (rows * row_bytes + (double)n * (row_bytes + 32.0)) / 4.4e6;
-    if (atomics_us <= rows_us) return 0;
+    const double most_rows = (double)((int64_t)kPartBins << kMaxBinShift);
+    if (tree->dtype != SVOX_F32 || (g_debug_flags & 1) || rows > most_rows || n > (1 << 30) || K > (1 << 20)) return 0;
     *part = Partition{};
     part->n_points = n;
     part->n_rows = (int64_t)rows;
@@ -247,38 +258,60 @@ int64_t plan_partition(const SvoxTreeSpec* tree, int64_t n, int32_t K, Partition
     int tile = 8;
     while (tile > 2 && (double)n * (1 << tile) > 512.0 * rows) --tile;
     part->tile_shift = tile;
-    part->bin_shift = tile;
-    while (((part->n_rows - 1) >> part->bin_shift) >= kPartBins) ++part->bin_shift;
+    part->bin_shift = bin_shift_of(part->n_rows, tile);
     part->n_bins = (int32_t)(((part->n_rows - 1) >> part->bin_shift) + 1);
+    const double row_bytes = 4.0 * K;
+    const int align = K % 16 == 0 ? 64 : K % 8 == 0 ? 32 : K % 4 == 0 ? 16 : K % 2 == 0 ? 8 : 4;   // where rows may start
+    const double atomics_us = rows * row_bytes / 6.8e6 + (double)n * (row_bytes + 64.0 - align) / 64.0 / 16500.0;
+    const double looks = (double)n * 8.0 * (1 << (part->bin_shift - tile));   // bytes
+    const double rows_us = 30.0 + (double)n * 45e-6 + (rows * row_bytes + (double)n * (row_bytes + 32.0)) / 4.4e6 + looks / 8e6;
+    if (atomics_us <= rows_us) return 0;
     int64_t per = (n + kPartBlocks - 1) / kPartBlocks;
     if (per < 2048) per = 2048;
     part->per_block = (int32_t)((per + kPointThreads - 1) / kPointThreads * kPointThreads);
     part->n_blocks = (int32_t)((n + part->per_block - 1) / part->per_block);
-    return n * 12 + ((int64_t)part->n_bins * part->n_blocks + 2 * part->n_bins + 16) * 4;
+    // Crowded: beyond twice the even share, and 1 024 pairs, which a tile sorts at once.  (us, twice and 1 024 / three times and 1 024 /
+    // four times and 2 048; 1 Mi points: deviation of 0.12 in the 64^3 SH16 tree 189 / 255 / 262, 64^3 SH16 shell 157 / 207 / 215, slab
+    // 200 / 190 / 190; 262 144 points in the shell 87 / 87 / 166; even points, half of the capacity unused, 216 / 192 / 192, atomics 253.)
+    // Runs: two for every CU, 512 to 4 096 pairs.  (262 144 points in the shell: the crowded kernel 96 us at 4 096, 23 at 512.)
+    // And not beyond 2 048 pairs a tile, however few the rows are.  (40 000 points in one node of 300 numbers: 2 280 us as two tiles,
+    // 195 with atomics.)
+    const int64_t even = (n + part->n_bins - 1) / part->n_bins, most = 2048ll << (part->bin_shift - tile);
+    part->crowded = (int32_t)(even * 2 < 1024 ? 1024 : even * 2 < most ? even * 2 : most);
+    part->run_pairs = n < 512 * 512 ? 512 : n > 512 * kRunPairs ? kRunPairs : (int32_t)(n / 512);
+    part->max_runs = (int32_t)(n / part->run_pairs + n / part->crowded + 1);
+    return n * 12 + part->max_runs * 8ll + ((int64_t)part->n_bins * part->n_blocks + 2 * part->n_bins + 16) * 4;
 }
 int launch_partition(const SvoxTreeSpec* tree, Partition part, const float* points, const int64_t* ids, const float* values, int32_t K,
                      float* grad, void* workspace, hipStream_t stream) {
     part.ids = ids;
     part.pairs = (uint2*)workspace;
-    part.leaf = (int32_t*)(part.pairs + part.n_points);
+    part.runs = (int2*)(part.pairs + part.n_points);
+    part.leaf = (int32_t*)(part.runs + part.max_runs);
     part.counts = part.leaf + part.n_points;
     part.totals = part.counts + (int64_t)part.n_bins * part.n_blocks;
     part.starts = part.totals + part.n_bins;
+    part.n_runs = part.starts + part.n_bins + 1;
     const TreeDev<float> tr = make_tree<float>(tree);
     const dim3 threads(kPartThreads);
-    const int32_t lds_nodes = ids ? 0 : tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
-    if (octree_fast_ok(tree))
-        hipLaunchKernelGGL((partition_count_kernel<true>), dim3(part.n_blocks), dim3(kPointThreads), (size_t)lds_nodes * 32, stream, tr, points,
-                           part, lds_nodes);
-    else
-        hipLaunchKernelGGL((partition_count_kernel<false>), dim3(part.n_blocks), dim3(kPointThreads), 0, stream, tr, points, part, 0);
-    hipLaunchKernelGGL(partition_offsets_kernel, dim3(part.n_bins), threads, 0, stream, part);
-    hipLaunchKernelGGL(partition_place_kernel, dim3(part.n_blocks), dim3(kPointThreads), 0, stream, part);
+    const size_t bin_words = (size_t)part.n_bins * 4;
+    if (octree_fast_ok(tree)) {
+        const int32_t lds_nodes = ids ? 0 : tree->capacity < kLdsNodesMax ? (int32_t)tree->capacity : kLdsNodesMax;
+        hipLaunchKernelGGL((partition_count_kernel<true>), dim3(part.n_blocks), dim3(kPointThreads), (size_t)lds_nodes * 32 + bin_words,
+                           stream, tr, points, part, lds_nodes);
+    } else {
+        hipLaunchKernelGGL((partition_count_kernel<false>), dim3(part.n_blocks), dim3(kPointThreads), bin_words, stream, tr, points, part, 0);
+    }
+    hipLaunchKernelGGL(partition_offsets_kernel, dim3(part.n_bins), threads, 0, stream, part, K, grad);
+    hipLaunchKernelGGL(partition_place_kernel, dim3(part.n_blocks), dim3(kPointThreads), bin_words, stream, part);
     const unsigned tiles = (unsigned)(((part.n_rows - 1) >> part.tile_shift) + 1);
     if (K % 4 == 0 && (((uintptr_t)values | (uintptr_t)grad) & 15u) == 0)
         hipLaunchKernelGGL((partition_collect_kernel<true>), dim3(tiles), threads, 0, stream, part, values, K, grad);
     else
         hipLaunchKernelGGL((partition_collect_kernel<false>), dim3(tiles), threads, 0, stream, part, values, K, grad);
+    const unsigned run_blocks = (unsigned)(part.max_runs < 512 ? part.max_runs : 512);
+    hipLaunchKernelGGL(partition_crowded_kernel, dim3(run_blocks), dim3(kPointThreads), ((size_t)4 << part.bin_shift) + 4, stream, part,
+                       values, K, grad);
     return check_launch("query_vertical_backward");
 }
 

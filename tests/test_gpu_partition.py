@@ -7,6 +7,7 @@ import torch
 
 import svox_amd as svox
 from svox_amd import csrc as C
+from svox_amd import synth
 from svox_amd.csrc import _abi
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,59 @@ def test_gradient_at_known_leaves(gpu, n, dtype, N):
         values.backward(grad)
         want = sums(ids)
         assert (tree.data.grad.view(-1, 4).cpu().double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+def _crowd(gen, n, kind):
+    if kind == "space":
+        return torch.rand(n, 3, generator=gen)
+    if kind == "leaf":
+        return torch.rand(n, 3, generator=gen) * 1e-6 + 0.51
+    return (torch.randn(n, 3, generator=gen) * 0.1 + 0.5).clamp(0, 1)      # "blob"
+
+
+@pytest.mark.parametrize("tree,dim,n,kind,shifted", [
+    (("shell", 6), 49, 262145, "space", False),    # runs of 512 pairs, rows that no 16-byte piece divides
+    (("shell", 8), 28, 800001, "space", False),    # ... of 1 562, 16-byte pieces
+    (("shell", 8), 28, 800001, "space", True),     # the same from an address that 16 bytes do not divide
+    (("shell", 9), 28, 2200001, "space", False),   # more than 2 048 bins, runs of 4 096
+    (("dense", 6), 49, 1000003, "blob", False),    # crowded bins beside others with several rounds to a tile
+    (("dense", 6), 28, 1000003, "leaf", False),    # one row has all the pairs of every run
+    (("dense", 1), 300, 40000, "blob", False),     # two tiles for everything
+])
+def test_gradient_by_rows_where_points_crowd(gpu, tree, dim, n, kind, shifted):
+    """Values where many points share few rows: crowded bins, their runs and the long rows of tiles, against a sum in double
+    precision; and the time, which must not be far from that of atomics (the workspace withheld) wherever the points fall."""
+    import ctypes
+    gen = torch.Generator().manual_seed(n)
+    if tree[0] == "shell":
+        tree = synth.shell_tree(depth=tree[1], n_spheres=24, data_format="RGBA", seed=0, device=gpu)
+    else:
+        tree = svox.N3Tree(data_format="RGBA", init_refine=tree[1] - 1, device=gpu)
+    points = _crowd(gen, n, kind).to(gpu)
+    grad = torch.randn(n * dim + 1, generator=gen).to(gpu)[int(shifted):][:n * dim].view(n, dim)
+    spec = tree._spec(world=False)
+    packed = C._pack_tree(spec)
+    lib = _abi.load_library()
+    need = lib.svox_query_vertical_backward_workspace_bytes(ctypes.byref(packed), n, dim)
+    assert need > 0
+    _, ids = C.query_vertical(spec, points)
+    want = torch.zeros(tree.child.numel(), dim, dtype=torch.float64, device=gpu).index_add_(0, ids, grad.double())
+    # (a sum of m terms of about 1 in single precision, in runs, is off by less than sqrt(m) 2^-24 times the largest partial sum)
+    for known in (None, ids):
+        got = C.query_vertical_backward(spec, points, grad, known).view(-1, dim)
+        assert (got.double() - want).abs().max() <= 1e-5 * want.abs().max()
+    out = torch.empty(tree.child.numel(), dim, device=gpu)
+    space = torch.empty(need, dtype=torch.uint8, device=gpu)
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    times = {}
+    for way, at, size in [("rows", space.data_ptr(), need), ("atomics", None, 0)] * 8:
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        assert lib.svox_query_vertical_backward_ids(ctypes.byref(packed), points.data_ptr(), ids.data_ptr(), n, grad.data_ptr(), dim,
+                                                    out.data_ptr(), 0, at, size, stream) == 0
+        end.record()
+        end.synchronize()
+        times.setdefault(way, []).append(begin.elapsed_time(end) * 1e3)
+    rows, atomics = (sorted(times[w])[4] for w in ("rows", "atomics"))
+    print(f"[rows] {kind} {n}: by rows {rows:.0f} us, with atomics {atomics:.0f} us", flush=True)
+    assert rows <= 1.5 * atomics + 30.0
