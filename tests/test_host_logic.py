@@ -418,3 +418,37 @@ def test_the_public_names_of_the_reference_are_all_there():
     tree /= 2.0
     assert torch.all(tree[:].values == 1.5)            # (the leaves; cells of inner nodes are no part of tree[:])
     assert torch.equal((tree[0] / 3.0), tree[0].values / 3.0)
+
+
+def test_spec_finds_tensors_that_are_not_plain_parameters_and_buffers():
+    """What reads the tensors past nn.Module's lookup still finds them where a caller has put them elsewhere."""
+    def spec_of(tree):
+        s = tree._spec()
+        assert s.child is tree.child and s.parent_depth is tree.parent_depth and s.scaling is tree.invradius
+        assert s.offset is tree.offset and s.extra_data is tree.extra_data
+        return s
+
+    tree = svox.N3Tree(extra_data=torch.zeros(2, 4))
+    assert spec_of(tree).data is tree.data and tree.extra_data is not None
+
+    class Halved(torch.nn.Module):
+        def forward(self, x):
+            return 0.5 * x
+
+    torch.nn.utils.parametrize.register_parametrization(tree, "data", Halved())
+    tree.parametrizations.data.original.data.fill_(4.0)
+    assert torch.equal(spec_of(tree).data, torch.full(tree.data.shape, 2.0))
+
+    tree = svox.N3Tree()                       # what replicas are made of: a plain attribute, no parameter
+    values = tree.data.data.clone()
+    del tree.data
+    tree.data = values
+    assert spec_of(tree).data is values
+
+    tree = svox.N3Tree(extra_data=torch.zeros(2, 4))
+    for name in ("offset", "invradius", "extra_data"):
+        value = torch.nn.Parameter(getattr(tree, name).clone())
+        delattr(tree, name)
+        setattr(tree, name, value)
+    assert spec_of(tree).offset is tree._parameters["offset"]
+    assert tree._spec(world=False).offset is None
