@@ -452,3 +452,44 @@ def test_spec_finds_tensors_that_are_not_plain_parameters_and_buffers():
         setattr(tree, name, value)
     assert spec_of(tree).offset is tree._parameters["offset"]
     assert tree._spec(world=False).offset is None
+
+
+def _query_on_the_cpu(monkeypatch):
+    """N3Tree.forward with the operators replaced: every point lies in leaf 0.  Returns what the gradient was called with."""
+    calls = []
+
+    def backward(spec, indices, grad_values, node_ids=None):
+        calls.append(node_ids)
+        grad = torch.zeros_like(spec.data)
+        grad[0, 0, 0, 0] = grad_values.sum(dim=0)
+        return grad
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    monkeypatch.setattr(C, "query_vertical", lambda spec, indices: (spec.data.detach()[0, 0, 0, 0].expand(indices.shape[0], -1).clone(),
+                                                                   torch.zeros(indices.shape[0], dtype=torch.int64)))
+    monkeypatch.setattr(C, "query_vertical_backward", backward)
+    return calls
+
+
+def test_a_query_never_drops_a_tangent(monkeypatch):
+    """Forward-mode derivatives of a query are refused, with and without grad mode, whichever argument carries them."""
+    from torch.autograd import forward_ad
+    from torch.func import functional_call, jvp
+    _query_on_the_cpu(monkeypatch)
+    tree = svox.N3Tree()
+    points = torch.rand(5, 3)
+    for mode in (torch.enable_grad, torch.no_grad):
+        with mode(), forward_ad.dual_level():
+            dual = forward_ad.make_dual(tree.data.detach().clone(), torch.ones_like(tree.data))
+            with pytest.raises(NotImplementedError):
+                functional_call(tree, {"data": dual}, (points,))
+            with pytest.raises(NotImplementedError):
+                tree(forward_ad.make_dual(points, torch.ones_like(points)))
+            assert tree(points).shape == (5, 4)      # (nothing dual here)
+        with mode(), pytest.raises(RuntimeError):
+            jvp(lambda data: functional_call(tree, {"data": data}, (points,)), (tree.data.detach(),), (torch.ones_like(tree.data),))
+        with mode(), pytest.raises(RuntimeError):
+            torch.func.vmap(lambda p: tree(p))(points[None].expand(2, 5, 3))
+    with torch.no_grad():
+        assert not tree(points).requires_grad
+    assert tree(points).requires_grad
