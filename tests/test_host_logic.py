@@ -493,3 +493,22 @@ def test_a_query_never_drops_a_tangent(monkeypatch):
     with torch.no_grad():
         assert not tree(points).requires_grad
     assert tree(points).requires_grad
+
+
+def test_leaves_kept_for_the_gradient_go_with_the_backward_pass(monkeypatch):
+    """The leaves a large query keeps are used by its backward pass and freed by it, although the graph is still referenced."""
+    import weakref
+
+    from svox_amd import tree as tree_module
+    calls = _query_on_the_cpu(monkeypatch)
+    monkeypatch.setattr(tree_module, "KEEP_IDS_FROM", 4)
+    tree = svox.N3Tree()
+    values, ids = tree(torch.rand(5, 3), want_node_ids=True)
+    kept = weakref.ref(values.grad_fn.node_ids)
+    del ids
+    values.backward(torch.ones_like(values), retain_graph=True)
+    assert calls[0] is not None and calls[0].shape == (5,)
+    del calls[0]
+    assert kept() is None
+    values.backward(torch.ones_like(values))       # (the points are looked up)
+    assert calls == [None] and float(tree.data.grad[0, 0, 0, 0, 0]) == 10.0
