@@ -52,6 +52,10 @@ void init(const std::string& path) {
 void status(int rc, const char* name) {
     if (rc != SVOX_OK) fail(std::string("svox.") + name + ": " + lib.svox_last_error() + " (" + lib.svox_status_string(rc) + ")");
 }
+// What allocates and launches runs without the interpreter's lock: a launch may wait for room in its queue, an allocation for
+// memory, and other Python threads go on meanwhile.  No Python object is touched while one of these lives; those that a function
+// holds are declared before it and so released after it.
+using Unlocked = py::gil_scoped_release;
 
 // ---- attributes of the spec objects
 struct Name {
@@ -330,15 +334,19 @@ py::tuple query_vertical(py::handle tree, const py::object& points) {
     check_floating(p, "indices");
     const Tree t = pack_tree(tree, p.scalar_type(), true);
     if (p.size(1) != 3) fail("indices must be (Q, 3)");
-    Tensor values = like(p, {p.size(0), t.spec.data_dim});
-    Tensor ids = at::empty({p.size(0)}, t.child.options().dtype(at::kLong));
-    const On on(p);
-    const int64_t bytes = lib.svox_query_vertical_workspace_bytes(&t.spec, p.size(0));
-    Tensor space;
-    if (bytes > 0) space = at::empty({bytes}, t.child.options().dtype(at::kByte));
-    status(lib.svox_query_vertical_ws(&t.spec, p.data_ptr(), p.size(0), values.data_ptr(), (int64_t*)ids.data_ptr(),
-                                      bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
-           "query_vertical");
+    Tensor values, ids;
+    {
+        const Unlocked unlocked;
+        values = like(p, {p.size(0), t.spec.data_dim});
+        ids = at::empty({p.size(0)}, t.child.options().dtype(at::kLong));
+        const On on(p);
+        const int64_t bytes = lib.svox_query_vertical_workspace_bytes(&t.spec, p.size(0));
+        Tensor space;
+        if (bytes > 0) space = at::empty({bytes}, t.child.options().dtype(at::kByte));
+        status(lib.svox_query_vertical_ws(&t.spec, p.data_ptr(), p.size(0), values.data_ptr(), (int64_t*)ids.data_ptr(),
+                                          bytes > 0 ? space.data_ptr() : nullptr, bytes, on.stream),
+               "query_vertical");
+    }
     return py::make_tuple(values, ids);
 }
 
@@ -360,6 +368,7 @@ Tensor query_vertical_backward(py::handle tree, const py::object& points, const 
         check_shaped(i, "node_ids", at::kLong, {p.size(0)});
         ids = (const int64_t*)i.data_ptr();
     }
+    const Unlocked unlocked;
     Tensor grad = like(g, {t.spec.capacity, t.spec.N, t.spec.N, t.spec.N, g.size(1)});
     const On on(p);
     const int64_t bytes = lib.svox_query_vertical_backward_workspace_bytes(&t.spec, p.size(0), (int32_t)g.size(1));
@@ -379,8 +388,9 @@ Tensor volume_render(py::handle tree, py::handle rays, py::handle opt, const py:
                        true);
     const Rays r = pack_rays(rays, t.data.scalar_type());
     const SvoxRenderOptions c = pack_options(opt);
-    Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     attach_marks(t, marks);
+    const Unlocked unlocked;
+    Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
     status(lib.svox_volume_render(&t.spec, &r.spec, &c, out.data_ptr(), on.stream), "volume_render");
     return out;
@@ -390,8 +400,9 @@ Tensor volume_render_images(py::handle tree, py::handle cam, py::handle opt, boo
     Tree t = pack_tree(tree, at::ScalarType::Undefined, true);
     const Camera k = pack_camera(cam, t.data.scalar_type(), batched ? 1 : 0);
     const SvoxRenderOptions c = pack_options(opt);
-    Tensor out = like(t.data, k.shape(out_dim(t, c)));
     attach_marks(t, marks);
+    const Unlocked unlocked;
+    Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
     status(lib.svox_volume_render_images(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), on.stream), "volume_render_images");
     return out;
@@ -405,9 +416,10 @@ Tensor volume_render_noted(py::handle tree, py::handle rays, py::handle opt, con
                        true);
     const Rays r = pack_rays(rays, t.data.scalar_type());
     const SvoxRenderOptions c = pack_options(opt);
-    Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     attach_marks(t, marks);
     const Space ws(workspace);
+    const Unlocked unlocked;
+    Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
     status(lib.svox_volume_render_noted(&t.spec, &r.spec, &c, out.data_ptr(), ws.at, ws.bytes, on.stream), "volume_render_noted");
     return out;
@@ -418,9 +430,10 @@ Tensor volume_render_images_noted(py::handle tree, py::handle cam, py::handle op
     Tree t = pack_tree(tree, at::ScalarType::Undefined, true);
     const Camera k = pack_camera(cam, t.data.scalar_type(), -1);
     const SvoxRenderOptions c = pack_options(opt);
-    Tensor out = like(t.data, k.shape(out_dim(t, c)));
     attach_marks(t, marks);
     const Space ws(workspace);
+    const Unlocked unlocked;
+    Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
     status(lib.svox_volume_render_images_noted(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), ws.at, ws.bytes, on.stream),
            "volume_render_images_noted");
@@ -435,9 +448,10 @@ Tensor volume_render_backward(py::handle tree, py::handle rays, py::handle opt, 
     const SvoxRenderOptions c = pack_options(opt);
     const Tensor& g = tensor(grad_output, "grad_output");
     check_shaped(g, "grad_output", t.data.scalar_type(), {r.spec.n_rays, out_dim(t, c)});
-    Tensor grad = like_data(t);
     attach_marks(t, marks);
     const Space ws(workspace);
+    const Unlocked unlocked;
+    Tensor grad = like_data(t);
     const On on(t.data);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
@@ -460,9 +474,10 @@ Tensor volume_render_images_backward(py::handle tree, py::handle cam, py::handle
     const SvoxRenderOptions c = pack_options(opt);
     const Tensor& g = tensor(grad_output, "grad_output");
     check_shaped(g, "grad_output", t.data.scalar_type(), k.shape(out_dim(t, c)));
-    Tensor grad = like_data(t);
     attach_marks(t, marks);
     const Space ws(workspace);
+    const Unlocked unlocked;
+    Tensor grad = like_data(t);
     const On on(t.data);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
@@ -493,17 +508,23 @@ py::tuple se_grad(py::handle tree, py::handle rays_or_cam, py::handle opt, const
     const std::vector<int64_t> shape = image ? k.shape(od) : std::vector<int64_t>{r.spec.n_rays, od};
     const Tensor& ref = tensor(color, "color");
     check_shaped(ref, "color", t.data.scalar_type(), shape);
-    Tensor result = like(t.data, shape), grad = like_data(t), hess = like_data(t);
     const Space ws(workspace);
-    const On on(t.data);
-    if (image)
-        status(lib.svox_se_grad_image_ws(&t.spec, &k.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(),
-                                         hess.data_ptr(), ws.at, ws.bytes, on.stream),
-               "se_grad_persp");
-    else
-        status(lib.svox_se_grad_ws(&t.spec, &r.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(), hess.data_ptr(),
-                                   ws.at, ws.bytes, on.stream),
-               "se_grad");
+    Tensor result, grad, hess;
+    {
+        const Unlocked unlocked;
+        result = like(t.data, shape);
+        grad = like_data(t);
+        hess = like_data(t);
+        const On on(t.data);
+        if (image)
+            status(lib.svox_se_grad_image_ws(&t.spec, &k.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(),
+                                             hess.data_ptr(), ws.at, ws.bytes, on.stream),
+                   "se_grad_persp");
+        else
+            status(lib.svox_se_grad_ws(&t.spec, &r.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(), hess.data_ptr(),
+                                       ws.at, ws.bytes, on.stream),
+                   "se_grad");
+    }
     return py::make_tuple(result, grad, hess);
 }
 
