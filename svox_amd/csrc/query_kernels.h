@@ -36,7 +36,7 @@ __device__ __forceinline__ int64_t query_leaf(const TreeDev<T>& tr, const int32_
     if constexpr (kOctree) {
         if (valid)
             leaf = descend_octree(walk, lds_child, lds_nodes, tr.capacity, cell_coord(clamp01(xyz[0])),
-                                  cell_coord(clamp01(xyz[1])), cell_coord(clamp01(xyz[2])));
+                                  cell_coord(clamp01(xyz[1])), cell_coord(clamp01(xyz[2])), walk != tr.child);
     }
     if (valid && leaf < 0) {   // deeper than the integer coordinates resolve: once more with the floating-point walk
         T cube;

@@ -127,10 +127,11 @@ __device__ __forceinline__ int32_t child_entry(const int32_t* __restrict__ child
 
 // Octree walk over integer coordinates with no path memory (point queries).
 // `lds_child` holds the child rows of nodes [0, lds_nodes); deeper nodes are read from memory (lds_nodes 0: all of them).
+// `marked`: `child` is the copy with kLastNodeBit; in the table itself an entry that large leads past the end (malformed tree).
 // Returns the leaf cell index node*8 + cell, or -1.
 __device__ __forceinline__ int32_t descend_octree(const int32_t* __restrict__ child, const int32_t* lds_child,
                                                   int32_t lds_nodes, int64_t capacity, uint32_t ix, uint32_t iy,
-                                                  uint32_t iz) {
+                                                  uint32_t iz, bool marked) {
     int32_t node = 0, leaf = -1;
     bool live = true;
     for (int level = 1; level <= kCoordBits && live; ++level) {
@@ -140,8 +141,8 @@ __device__ __forceinline__ int32_t descend_octree(const int32_t* __restrict__ ch
             leaf = cell;
             live = false;
         } else {
-            const bool last = skip >= kLastNodeBit;
-            node += last ? skip - kLastNodeBit : skip;
+            const bool last = marked && skip >= kLastNodeBit;
+            node = (int32_t)((uint32_t)node + (uint32_t)(last ? skip - kLastNodeBit : skip));
             if (node < 0 || node >= capacity) {
                 live = false;
             } else if (last) {

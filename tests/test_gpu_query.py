@@ -207,3 +207,27 @@ def test_query_of_many_points_beside_the_table(gpu, chain):
     for i in range(0, n, step):
         few_values, few_ids = C.query_vertical(spec, points[i:i + step].contiguous())
         assert torch.equal(ids[i:i + step], few_ids) and torch.equal(values[i:i + step], few_values)
+
+
+@pytest.mark.parametrize("n", [1000, 300000, 500000])      # few points, many, and many beside the table
+def test_child_entries_that_lead_past_the_end(gpu, n):
+    """A malformed table: entries beyond every node, up to the largest ones, end the search with leaf -1 and value 0, and the
+    gradient of such a point goes nowhere; all other points are found as before."""
+    tree = svox.N3Tree(data_format="SH1", init_refine=5, device=gpu)
+    tree.data.data.normal_(generator=torch.Generator(device=gpu).manual_seed(n))
+    points = torch.rand(n, 3, generator=torch.Generator().manual_seed(n)).to(gpu)
+    with torch.no_grad():
+        values, ids = tree(points, want_node_ids=True)
+        flat = tree.child.view(-1)
+        bad = torch.zeros(n, dtype=torch.bool, device=gpu)
+        for cell, entry in ((1, (1 << 30) + 2), (2, (1 << 31) - 1), (3, -3), (4, tree.capacity)):      # of the root: a corner each
+            flat[cell] = entry
+            corner = torch.tensor([cell >> 2 & 1, cell >> 1 & 1, cell & 1], device=gpu)
+            bad |= ((points * 2).long() == corner).all(dim=1)
+        got, got_ids = tree(points, want_node_ids=True)
+    assert bad.any() and torch.equal(got_ids, torch.where(bad, torch.full_like(ids, -1), ids))
+    assert torch.equal(got, torch.where(bad[:, None], torch.zeros_like(values), values))
+    grad = torch.randn(n, 4, generator=torch.Generator().manual_seed(n + 1)).to(gpu)
+    want = torch.zeros(flat.numel(), 4, dtype=torch.float64, device=gpu).index_add_(0, ids[~bad], grad[~bad].double())
+    out = C.query_vertical_backward(tree._spec(), points, grad).view(-1, 4)
+    assert (out.double() - want).abs().max() <= 1e-5 * want.abs().max()
