@@ -158,12 +158,15 @@ int zero_fill(void* ptr, int64_t bytes, hipStream_t stream) {
     if (bytes <= 0) return SVOX_OK;
     if (((uintptr_t)ptr & 15u) != 0 || (bytes & 3) != 0)
         return fail(SVOX_ERR_BAD_SHAPE, "gradient buffer must be 16-byte aligned and a multiple of 4 bytes");
-    const int64_t n16 = bytes / 16;
-    const int n_tail = (int)((bytes - n16 * 16) / 4);
-    int64_t blocks = (n16 + 255) / 256;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(zero_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (uint4*)ptr, n16,
-                       (uint32_t*)((char*)ptr + n16 * 16), n_tail);
+    // (a launch has fewer than 2^32 threads, and each of these clears 16 bytes)
+    constexpr int64_t kMost = (int64_t)0xffffff * 256;
+    int64_t left = bytes / 16;
+    uint4* at = (uint4*)ptr;
+    for (; left > kMost; left -= kMost, at += kMost)
+        hipLaunchKernelGGL(zero_kernel, dim3((unsigned)(kMost / 256)), dim3(256), 0, stream, at, kMost, (uint32_t*)nullptr, 0);
+    const int64_t blocks = left < 1 ? 1 : (left + 255) / 256;
+    hipLaunchKernelGGL(zero_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, at, left, (uint32_t*)(at + left),
+                       (int)(bytes % 16 / 4));
     return check_launch("zero_fill");
 }
 

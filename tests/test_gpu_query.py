@@ -231,3 +231,23 @@ def test_child_entries_that_lead_past_the_end(gpu, n):
     want = torch.zeros(flat.numel(), 4, dtype=torch.float64, device=gpu).index_add_(0, ids[~bad], grad[~bad].double())
     out = C.query_vertical_backward(tree._spec(), points, grad).view(-1, 4)
     assert (out.double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("extra", [0, 4099])
+def test_a_gradient_beyond_64_gib_is_cleared(gpu, extra):
+    """One launch clears less than 64 GiB (fewer than 2^32 threads of 16 bytes): a gradient that large and one beyond it."""
+    tree = svox.N3Tree(init_reserve=2, device=gpu)
+    dim = (1 << 30) + extra                     # 16 cells of 4 GiB and more
+    if torch.cuda.mem_get_info(gpu)[0] < 16 * 4 * dim + (8 << 30):
+        pytest.skip("not enough free device memory")
+    out = torch.empty(16 * dim + 4, device=gpu)
+    out.fill_(7.0)
+    spec = C._pack_tree(tree._spec())
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    rc = _abi.load_library().svox_query_vertical_backward(ctypes.byref(spec), None, 0, None, dim, out.data_ptr(), 0, stream)
+    assert rc == 0, _abi.load_library().svox_last_error()
+    assert torch.equal(out[16 * dim:], torch.full_like(out[16 * dim:], 7.0))
+    step = 1 << 30
+    for i in range(0, 16 * dim, step):
+        part = out[i:min(i + step, 16 * dim)]
+        assert float(part.min()) == 0.0 and float(part.max()) == 0.0
