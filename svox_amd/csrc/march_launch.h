@@ -12,6 +12,9 @@ namespace svox {
 
 template <class P, class Source>
 struct MarchLaunch {
+    // How many tiles of a forward launch (noting: one that takes notes; graded: with the gradient at hand) the GPU holds at once
+    // with two wavefronts to a tile.
+    static unsigned split_tiles_at_once(bool noting, bool graded);
     static void forward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                         const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool split, bool accum, bool refill,
                         bool all_shaded);
@@ -32,6 +35,31 @@ struct MarchLaunch {
 };
 
 #ifdef SVOX_INSTANTIATE_POLICY
+// What the runtime tells of the kernel's registers -- 12 tiles to a CU up to 80 of them, 10 up to 96, 8 up to 128 -- but not more
+// than 12, which is all the LDS holds (12.25 KiB a tile and more).
+template <class P, class Source>
+unsigned MarchLaunch<P, Source>::split_tiles_at_once(bool noting, bool graded) {
+    auto tiles = [](auto* kernel) {
+        constexpr unsigned kCus = 256, kMost = 12;
+        int blocks = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, kSplitThreads, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            blocks = 8;
+        }
+        return kCus * ((unsigned)blocks < kMost ? (unsigned)blocks : kMost);
+    };
+    if (noting && graded) {
+        static const unsigned n = tiles(render_forward_split_kernel<P, Source, true, true>);
+        return n;
+    }
+    if (noting) {
+        static const unsigned n = tiles(render_forward_split_kernel<P, Source, true, false>);
+        return n;
+    }
+    static const unsigned n = tiles(render_forward_split_kernel<P, Source, false>);
+    return n;
+}
+
 template <class P, class Source>
 void MarchLaunch<P, Source>::forward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                                      const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool split, bool accum,

@@ -568,28 +568,35 @@ unsigned blocks_for(int64_t items, int per_block) { return (unsigned)((items + p
 // 1.22 / 1.33.  The launcher cannot know how many rays hit, so the rule goes by tiles: images of up to 65 536 tiles
 // (six 800x800 poses) -- 49 152 with deciding marks, 6 144 under NDC, where every ray passes through the tree (us, one /
 // two, SH16 trees of 128^3 and 512^3: 3 024 tiles 117 / 115 and 310 / 279, 6 745 tiles 155 / 190 and 423 / 420, 11 970
-// tiles 201 / 243 and 482 / 506) --, ray batches of up to 2 816 (180 224 rays), 2 048 on complete octrees of 64^3 leaves and more:
-// there no ray is short, a leaf to every layer of the grid, and the second wavefront has paid for itself sooner; on sparse trees
-// lengths differ and a launch waits for its longest ray up to where its blocks, 10 to 12 to a CU, no longer run at once.  us, one /
-// two wavefronts, forward, training step, squared error; unrelated rays:
-//   150 001 rays: 256^3 SH9 shell 300 / 264, 553 / 477, 690 / 622; 512^3 SH16 shell 365 / 310, 850 / 765, 1069 / 972; dense 64^3 SH4
-//   367 / 319, 1234 / 1191, 1794 / 1740, SH16 491 / 531, 2064 / 2087, 3284 / 3296; 128^3 SH9 1036 / 1062, 3076 / 3175, 4522 / 4633;
-//   180 001 rays: the shells 304 / 270, 565 / 486, 634 / 561; 367 / 314, 865 / 794, 1092 / 1014; dense 64^3 SH4 387 / 346, 1364 / 1343,
-//   2052 / 2019, SH16 555 / 615, 2432 / 2557, 3828 / 3951; 128^3 SH9 1215 / 1316, 3546 / 3686, 5242 / 5389; 32^3 SH4 167 / 151, 739 / 721;
-//   196 001 rays: the shells 300 / 266, 565 / 497, 629 / 557; 386 / 325, 884 / 906, 1113 / 1126; dense 64^3 SH4 398 / 369, 1471 / 1476;
-//   131 001 rays: dense 64^3 SH16 443 / 412, 1841 / 1971, 2866 / 2852; 128^3 SH9 895 / 866, 2888 / 2897, 4046 / 4069.
+// tiles 201 / 243 and 482 / 506) --, ray batches as
+// long as all their blocks run at once (`at_once`; 3 072 tiles with up to 80 registers, fewer with more of them), beyond which the
+// longest chain waits for a place: us, one / two wavefronts, unrelated rays that all hit, forward, training step, squared error:
+//   SH9, at once 3 072 / 3 072: 256^3 shell, 196 001 rays 481 / 438, 1150 / 1074, 1543 / 1469; 200 003 rays 486 / 543, 1171 / 1194,
+//   1563 / 1579; SH4 in a 512^3 shell 621 / 556, 1185 / 1086, 1494 / 1390 and 581 / 680, 1146 / 1208, 1466 / 1525;
+//   SH16, 3 072 / 2 560: 256^3 shell, 160 001 rays 473 / 417, 1282 / 1195, 1818 / 1731; 170 001 rays 490 / 429, 1313 / 1378, 1904 / 1957;
+//   SH25, 2 560 / 2 048: 256^3 shell, 130 001 rays 500 / 422, 1473 / 1366, 2174 / 2066; 150 001 rays 505 / 460, 1582 / 1628, 2381 / 2416;
+//   170 001 rays 540 / 637, 1689 / 1752, 2591 / 2624;
+//   the gradient by itself (2 560 to SH9, 2 048 beyond): SH9, 163 001 rays 1060 / 957, 170 001 rays 1081 / 1109.
+// (Where most rays miss, as in pictures of a shell, noting passes gain a little beyond: SH9, 200 003 rays 572 / 533, 230 401 598 / 597;
+// SH16 loses there too.)  On complete octrees of 64^3 leaves and more not beyond 2 048: no ray is short there, a leaf to every layer
+// of the grid, and the second wavefront has paid for itself sooner:
+//   131 001 rays: 64^3 SH16 443 / 412, 1841 / 1971, 2866 / 2852; 128^3 SH9 895 / 866, 2888 / 2897, 4046 / 4069;
+//   150 001 rays: 64^3 SH4 367 / 319, 1234 / 1191, 1794 / 1740, SH16 491 / 531, 2064 / 2087, 3284 / 3296; 128^3 SH9 1036 / 1062, 3076 /
+//   3175, 4522 / 4633; 180 001 rays: 64^3 SH4 387 / 346, 1364 / 1343, 2052 / 2019, SH16 555 / 615, 2432 / 2557, 3828 / 3951; 128^3 SH9
+//   1215 / 1316, 3546 / 3686, 5242 / 5389; 32^3 SH4 167 / 151, 739 / 721.
 bool is_complete_octree(const SvoxTreeSpec* tree) {
     int64_t nodes = 1;
     while (nodes < tree->capacity) nodes = nodes * 8 + 1;
     return tree->N == 2 && nodes == tree->capacity;
 }
-bool use_split_forward(const SvoxTreeSpec* tree, unsigned blocks, bool image, const SvoxRenderOptions* opt, bool decided) {
+bool use_split_forward(const SvoxTreeSpec* tree, unsigned blocks, bool image, const SvoxRenderOptions* opt, bool decided,
+                       unsigned at_once) {
     const int forced = tuning().split_forward;
     const long limit = tuning().split_blocks;
     if (g_debug_flags & 12) return (g_debug_flags & 8) != 0;
     if (forced >= 0) return forced > 0;
     if (limit >= 0) return (long)blocks <= limit;
-    if (!image) return blocks <= (tree->capacity >= 37449 && is_complete_octree(tree) ? 2048u : 2816u);
+    if (!image) return blocks <= at_once && (blocks <= 2048u || tree->capacity < 37449 || !is_complete_octree(tree));
     if (opt->ndc_width > 0) return blocks <= 6144u;
     return blocks <= (decided ? 49152u : 65536u);
 }
@@ -618,7 +625,10 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
             // although the launch sends 17 % fewer requests to L2.
             const bool all_shaded = !tree->weight_accum && marks_decide(tree, opt, opt->sigma_thresh);
             const bool refill = src.per_wave > kMarchThreads;
-            const bool split = !refill && !tree->weight_accum && use_split_forward(tree, blocks, is_image_source(src), opt, all_shaded);
+            unsigned at_once = 0;
+            SVOX_DISPATCH_OCTREE(D, at_once = MarchLaunch<P, Source>::split_tiles_at_once(false, false));
+            const bool split = !refill && !tree->weight_accum &&
+                               use_split_forward(tree, blocks, is_image_source(src), opt, all_shaded, at_once);
             SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::forward(dim3(blocks), stream, tr, dealt, *opt, (float*)out, none,
                                                                     split, tree->weight_accum != nullptr, refill, all_shaded));
             return;
@@ -740,7 +750,9 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
     ws.give_ups = give_up_counter();
     const bool refill = src.per_wave > kMarchThreads;
-    const bool split = !refill && use_split_forward(tree, blocks, is_image_source(src), opt, false);
+    unsigned at_once = 0;
+    SVOX_DISPATCH_OCTREE(D, at_once = MarchLaunch<P, Source>::split_tiles_at_once(true, grad_out != nullptr));
+    const bool split = !refill && use_split_forward(tree, blocks, is_image_source(src), opt, false, at_once);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
                                                            (float*)out, ws, (const float*)grad_out,
                                                            (const float*)color_ref, split, refill));

@@ -1344,25 +1344,30 @@ def test_ray_batches_where_the_launch_changes(gpu, n):
         assert (data_grad - got[0][2]).abs().max() <= 1e-4 * data_grad.abs().max()
 
 
-@pytest.mark.parametrize("kind,depth,tiles,two", [
-    ("dense", 6, 2048, True), ("dense", 6, 2049, False),       # a complete octree of 64^3 leaves: every ray is long
-    ("dense", 5, 2816, True), ("dense", 5, 2817, False),
-    ("shell", 6, 2816, True), ("shell", 6, 2817, False),
-    ("shell", 6, 3126, False),
+@pytest.mark.parametrize("kind,depth,fmt,most", [
+    ("dense", 6, "RGBA", (2048, 2048, 2048)),       # a complete octree of 64^3 leaves: every ray is long
+    ("dense", 5, "RGBA", (3072, 3072, 2560)),
+    ("shell", 6, "SH9", (3072, 3072, 2560)),
+    ("shell", 6, "SH16", (3072, 2560, 2048)),
+    ("shell", 6, "SH25", (2560, 2048, 2048)),
 ])
-def test_which_ray_batches_run_on_two_wavefronts_per_tile(gpu, kind, depth, tiles, two):
-    """The size from which on a ray batch runs on one wavefront per tile, for passes with and without notes.  Waits that
-    give up at the first look (debug flag 16) tell which kernel ran: only the two-wavefront one has any."""
-    tree = (synth.dense_tree(depth - 1, "RGBA", seed=1) if kind == "dense" else
-            synth.shell_tree(depth=depth, n_spheres=5, data_format="RGBA", seed=3))
+def test_which_ray_batches_run_on_two_wavefronts_per_tile(gpu, kind, depth, fmt, most):
+    """The size from which on a ray batch runs on one wavefront per tile: forward passes, those that take notes and the
+    gradient by itself.  Waits that give up at the first look (debug flag 16) tell which kernel ran: only the two-wavefront
+    one has any."""
+    tree = (synth.dense_tree(depth - 1, fmt, seed=1) if kind == "dense" else
+            synth.shell_tree(depth=depth, n_spheres=5, data_format=fmt, seed=3))
     dev = on_gpu(tree, gpu)
-    rays = rays_spec(synth.sphere_rays(64 * tiles, seed=6), gpu)
     opt = options(tree, step_size=1e-3)
-    for call in (C.volume_render, C.volume_render_noted):
-        before = C.give_up_count()
-        C.set_debug_flags(16)
-        try:
-            call(dev._spec(), rays, opt)
-        finally:
-            C.set_debug_flags(0)
-        assert (C.give_up_count() > before) == two, call.__name__
+    calls = (C.volume_render, C.volume_render_noted,
+             lambda spec, rays, opt: C.volume_render_backward(spec, rays, opt, torch.ones(rays.origins.shape[0], 3, device=gpu)))
+    for call, limit in zip(calls, most):
+        for tiles in (limit, limit + 1):
+            rays = rays_spec(synth.sphere_rays(64 * tiles, seed=6), gpu)
+            before = C.give_up_count()
+            C.set_debug_flags(16)
+            try:
+                call(dev._spec(), rays, opt)
+            finally:
+                C.set_debug_flags(0)
+            assert (C.give_up_count() > before) == (tiles == limit), tiles
