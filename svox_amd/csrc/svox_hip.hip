@@ -179,14 +179,28 @@ int zero_fill(void* ptr, int64_t bytes, hipStream_t stream) {
 // 52.7 / 54.8.  (Larger wavefronts of 128 points, two to a lane, for the rest: SH16, 1 Mi points 92 / 92, 262 144 points
 // 37 / 47.)
 constexpr int64_t kFewPointsMax = 262144;
+// Whether a tree's nodes number as many as a complete octree's, or up to an eighth more: a grid that is as fine everywhere, perhaps
+// refined here and there.  (A tree of another shape with such a number only takes a rule that is not made for it.)
+bool like_complete_octree(const SvoxTreeSpec* tree) {
+    int64_t nodes = 1;
+    while (nodes * 8 + 1 <= tree->capacity) nodes = nodes * 8 + 1;
+    return tree->N == 2 && tree->capacity - nodes <= nodes / 8;
+}
 // Whether a query of n points is worth a copy of the child table in which the nodes of leaves only are marked
 // (last_nodes_kernel).  It takes 5 us and 14 ps a node, and what it saves -- a request for a line of the table, which the
 // memory system serves 55 of a nanosecond once the table is larger than an L2 cache -- goes to the points that end in such a
-// node: all of a dense tree's, few of those thrown at random on a sparse one, which the line lies between.  (us, plain / with
-// the copy, its making included; 4 Mi points: 128^3 RGBA 173 / 111 and SH9 285 / 257, 64^3 RGBA 81 / 63, 256^3 shell SH9
-// 122 / 121, 512^3 shell SH4 105 / 119, 32^3 SH4 83 / 82; 1 000 003 points: 128^3 SH9 75 / 66, 256^3 shell SH9 36 / 40.)
+// node: all of a grid's, few of those thrown at random on a sparse tree.  So for a grid by that cost, with 17 ps saved a point and
+// a quarter in hand (a table that L2 holds: from 12 points a node on, even at 27); for others from 24 points a node on, where it is
+// even, and not where L2 holds the table.
+// (us, plain / with the copy, its making included.  Grids: 128^3 SH9, 600 000 points 52 / 48, 1 000 003 78 / 69, 4 M 274 / 249; RGBA
+// 36 / 33, 52 / 43, 167 / 109; 64^3 SH4, 450 000 points 26 / 28, 1.0 M 44 / 43, 4 M 131 / 120, SH16 45 / 48, 83 / 85, 285 / 274; 256^3
+// SH1, 2 M points 134 / 133, 4 M 257 / 214; 32^3 SH4, 4 M 77 / 77.  Shells, 13 / 24 / 48 points a node: 256^3 RGBA 40 / 43, 62 / 64,
+// 114 / 113, SH9 79 / 81, 136 / 134, 417 / 415; 512^3 SH4 338 / 349, 622 / 623, 1238 / 1224; 128^3 RGBA 18 / 21, 24 / 31, 35 / 37.)
 bool walk_copy_pays(const SvoxTreeSpec* tree, int64_t n) {
-    return octree_fast_ok(tree) && tree->dtype == SVOX_F32 && tree->capacity >= 30000 && n >= 12 * tree->capacity;
+    if (!octree_fast_ok(tree) || tree->capacity < 30000 || n <= kFewPointsMax) return false;
+    const bool beyond_l2 = tree->capacity >= 131072;   // (32 bytes a node, 4 MB)
+    if (!like_complete_octree(tree)) return beyond_l2 && n >= 24 * tree->capacity;
+    return beyond_l2 ? (double)n * 17.0 >= 1.25 * (5e6 + 14.0 * (double)tree->capacity) : n >= 12 * tree->capacity;
 }
 constexpr int kLdsNodesMax = 584;  // child rows kept in LDS per block: 584 * 32 B = 18.25 KiB
 
@@ -578,17 +592,12 @@ unsigned blocks_for(int64_t items, int per_block) { return (unsigned)((items + p
 //   170 001 rays 540 / 637, 1689 / 1752, 2591 / 2624;
 //   the gradient by itself (2 560 to SH9, 2 048 beyond): SH9, 163 001 rays 1060 / 957, 170 001 rays 1081 / 1109.
 // (Where most rays miss, as in pictures of a shell, noting passes gain a little beyond: SH9, 200 003 rays 572 / 533, 230 401 598 / 597;
-// SH16 loses there too.)  On complete octrees of 64^3 leaves and more not beyond 2 048: no ray is short there, a leaf to every layer
+// SH16 loses there too.)  On grids of 64^3 leaves and more not beyond 2 048: no ray is short there, a leaf to every layer
 // of the grid, and the second wavefront has paid for itself sooner:
 //   131 001 rays: 64^3 SH16 443 / 412, 1841 / 1971, 2866 / 2852; 128^3 SH9 895 / 866, 2888 / 2897, 4046 / 4069;
 //   150 001 rays: 64^3 SH4 367 / 319, 1234 / 1191, 1794 / 1740, SH16 491 / 531, 2064 / 2087, 3284 / 3296; 128^3 SH9 1036 / 1062, 3076 /
 //   3175, 4522 / 4633; 180 001 rays: 64^3 SH4 387 / 346, 1364 / 1343, 2052 / 2019, SH16 555 / 615, 2432 / 2557, 3828 / 3951; 128^3 SH9
 //   1215 / 1316, 3546 / 3686, 5242 / 5389; 32^3 SH4 167 / 151, 739 / 721.
-bool is_complete_octree(const SvoxTreeSpec* tree) {
-    int64_t nodes = 1;
-    while (nodes < tree->capacity) nodes = nodes * 8 + 1;
-    return tree->N == 2 && nodes == tree->capacity;
-}
 bool use_split_forward(const SvoxTreeSpec* tree, unsigned blocks, bool image, const SvoxRenderOptions* opt, bool decided,
                        unsigned at_once) {
     const int forced = tuning().split_forward;
@@ -596,7 +605,7 @@ bool use_split_forward(const SvoxTreeSpec* tree, unsigned blocks, bool image, co
     if (g_debug_flags & 12) return (g_debug_flags & 8) != 0;
     if (forced >= 0) return forced > 0;
     if (limit >= 0) return (long)blocks <= limit;
-    if (!image) return blocks <= at_once && (blocks <= 2048u || tree->capacity < 37449 || !is_complete_octree(tree));
+    if (!image) return blocks <= at_once && (blocks <= 2048u || tree->capacity < 37449 || !like_complete_octree(tree));
     if (opt->ndc_width > 0) return blocks <= 6144u;
     return blocks <= (decided ? 49152u : 65536u);
 }

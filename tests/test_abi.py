@@ -82,3 +82,31 @@ def test_oracle_library_builds_and_exports_its_checker_symbols():
     for name in ("oracle_query_vertical", "oracle_volume_render", "oracle_volume_render_backward",
                  "oracle_volume_render_image", "oracle_calc_corners", "oracle_expf"):
         assert hasattr(lib, name)
+
+
+def test_which_queries_copy_the_child_table():
+    """Points from which on a query asks for room for its copy of the child table, by the number of nodes and points alone."""
+    lib = _abi.load_library()
+    spec = _abi.TreeSpecC()
+    spec.data = spec.child = spec.parent_depth = 16
+    spec.N, spec.data_dim, spec.dtype = 2, 4, 0
+
+    def first(nodes, low=1, high=1 << 30):
+        spec.capacity = nodes
+        while low < high:
+            middle = (low + high) // 2
+            if lib.svox_query_vertical_workspace_bytes(ctypes.byref(spec), middle) > 0:
+                high = middle
+            else:
+                low = middle + 1
+        assert lib.svox_query_vertical_workspace_bytes(ctypes.byref(spec), low - 1) == 0
+        return low
+
+    grid64, grid128, grid256 = 37449, 299593, 2396745
+    assert first(grid64) == first(grid64 + 21) - 12 * 21 == 12 * grid64
+    assert 500000 < first(grid128) < 800000 and first(grid128 + grid128 // 8) < 800000
+    assert 2000000 < first(grid256) < 3500000
+    for nodes in (192314, 774208, grid128 + grid128 // 8 + 1):       # sparse trees, by their number of nodes
+        assert first(nodes) == 24 * nodes
+    for nodes in (4681, 47433, grid64 + grid64 // 8 + 1):            # ... whose tables L2 holds, and small grids
+        assert first(nodes) == 1 << 30
