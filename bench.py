@@ -652,7 +652,8 @@ def main():
         log(f"[bench] query {query}")
 
     # ---------------------------------------------------------------- what the generic kernels do
-    # (fp64 data, spherical-Gaussian lobes, density_softplus: one ray per lane, the reference's loop)
+    # (fp64 pictures and what is forced onto them: one ray per lane, the reference's loop; beside them spherical-Gaussian
+    # lobes, density_softplus and N = 3, which the wavefront kernels serve)
     generic = None
     if not args.no_generic:
         def ev_time(fn, n=3):

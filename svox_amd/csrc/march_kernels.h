@@ -5,9 +5,11 @@
 // The tree kernels exist in two flavours that compute the same numbers:
 //   GenericPolicy<T>   any branching factor, scalar type, data format, component range, softplus;
 //                      the reference's floating-point walk from the root for every sample.
-//   OctreePolicy<FMT,D> fp32 octree with the default options (SH with D in {1,4,9,16,25}, or RGBA
-//                      with 3 colours): integer-coordinate walk restarted from the previous path
-//                      (OctreeCursor), record length and basis size known at compile time.
+//   OctreePolicy<FMT,D> fp32 trees of three colours (RGBA, or SH and lobes with D in {1,4,9,16,25}):
+//                      record length and basis size known at compile time, a wavefront to 64 rays that
+//                      share their work; octrees walk on integer coordinates, restarted from the
+//                      previous path (OctreeCursor), other branching factors as above.
+// (Small batches through fp64 octrees have kernels of their own: group_kernels.h.)
 #pragma once
 
 #include <cstddef>

@@ -597,7 +597,8 @@ unsigned blocks_for(int64_t items, int per_block) { return (unsigned)((items + p
 //   131 001 rays: 64^3 SH16 443 / 412, 1841 / 1971, 2866 / 2852; 128^3 SH9 895 / 866, 2888 / 2897, 4046 / 4069;
 //   150 001 rays: 64^3 SH4 367 / 319, 1234 / 1191, 1794 / 1740, SH16 491 / 531, 2064 / 2087, 3284 / 3296; 128^3 SH9 1036 / 1062, 3076 /
 //   3175, 4522 / 4633; 180 001 rays: 64^3 SH4 387 / 346, 1364 / 1343, 2052 / 2019, SH16 555 / 615, 2432 / 2557, 3828 / 3951; 128^3 SH9
-//   1215 / 1316, 3546 / 3686, 5242 / 5389; 32^3 SH4 167 / 151, 739 / 721.
+//   1215 / 1316, 3546 / 3686, 5242 / 5389; 32^3 SH4 167 / 151, 739 / 721.  (N = 3, 81^3 SH9, walks longer: 736 / 665, 2517 / 2470,
+//   3597 / 3617.)
 bool use_split_forward(const SvoxTreeSpec* tree, unsigned blocks, bool image, const SvoxRenderOptions* opt, bool decided,
                        unsigned at_once) {
     const int forced = tuning().split_forward;
