@@ -2229,6 +2229,17 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
 // one leaf after the other -- the transmittance in front of a leaf, the colour that lies behind it -- is passed from
 // lane to lane (each_in_turn).  A ray with more than 64 notes is taken alone, 64 notes at a time, once for its sum and
 // once for its records.
+// Neighbours that share leaves are taken first, and in slices: 64 / 2^k notes of each of up to 16 rays, so that
+// records of one leaf stand in the same batch and leave the wavefront as one (a ray passes a leaf once: rays taken
+// alone, or packed end to end, have next to none to add together).  It pays where the atomic additions bound the
+// kernel, and costs two passes over the notes instead of one, so it goes by what neighbours have in common: half of
+// the rays of a piece of 16 begin in the leaf of the one to their left.  Steps of training (forward and backward pass,
+// us), 800x800 pictures unless stated, with the rays packed or alone -> with slices: dense 128^3 SH9, from 1.2 of its
+// edges away 9 090 -> 5 680, from 2 5 030 -> 4 050, from 4 1 480 -> 1 475; 64^3 RGBA from 1.2 2 480 -> 1 465; 64^3
+// SH16 from 2 3 800 -> 1 830; N = 3, 81^3 SH9 from 2 3 360 -> 2 035; a 256^3 SH9 shell from 1.5 1 690 -> 1 470, from 4
+// 685 -> 655, 50 001 rays of it 650 -> 638; 65 536 scattered rays of 64^3 RGBA with softplus 725 -> 722; 262 144 of
+// 128^3 SH9 5 190 -> 5 140.  (The line at a third: the same; at three quarters the pictures from 2 away are lost to
+// it.)
 // (One lane per ray, as the march has it, is the wrong shape here: where one ray in five meets the scene, and those
 // differ in length, 60 to 95 % of the lanes idle, and every ray's notes are read twice, first for the sum of the first
 // march.  replay_backward_kernel from that to this: 4 096 rays of a 16^3 RGBA tree 22.6 -> 9.1 us, 50 001 rays of a
@@ -2259,13 +2270,27 @@ struct ReplayNote {
     int32_t leaf;
     float dt, raw, s[3], dscale;
 };
+// What a wavefront keeps of a ray from one slice of its notes to the next, in LDS, by the ray's row: the transmittance
+// in front of the slice, N running sums, and where the notes go on.
+template <int N>
+struct ReplayCarry {
+    static constexpr int kRows = 16;
+    float through[kRows], run[N][kRows];
+    int32_t chunk[kRows], index[kRows];
+    __device__ __forceinline__ void begin(int row, int32_t ray) {
+        through[row] = 1.0f;
+        chunk[row] = 0;
+        index[row] = ray;
+    }
+};
 struct ReplayRays {
     // The chunks of a ray's notes are a chain, and to follow it is one trip to memory after the other.  The rays of the
     // list follow theirs all at once, before the first note is read, as long as there is room to keep what they find.
     static constexpr int kChunks = 512;
     ReplayRay list[1 << kReplayMaxShift];
     int32_t chunks[kChunks];
-    int n, cursor;   // of the list: rays, and rays taken
+    int n, cursor;                 // of the list: rays, and rays taken
+    int n_shared, shared_cursor;   // ... of those that come first, which share leaves with their neighbours
     int n_chunks;
 
     // Lists the rays of block `block` of `blocks` that have notes and writes its part of the bitmap of undone rays.
@@ -2278,11 +2303,11 @@ struct ReplayRays {
         static_assert(1 << kReplayMaxShift <= kMarchThreads, "one wavefront looks the rays up");
         const int lane = threadIdx.x;
         if (lane < kMarchThreads) {
-            if (lane == 0) cursor = n_chunks = 0;
+            if (lane == 0) shared_cursor = n_chunks = 0;
             const unsigned k = (unsigned)lane >> 4, turn = (unsigned)((float)blocks * 0.618f);
             const int64_t ray = (((int64_t)k * blocks + ((unsigned)block + k * turn) % (unsigned)blocks) << 4) + (lane & 15);
             const bool seated = lane < (1 << ray_shift) && ray < n_slots;
-            int32_t count = 0, link = 0;
+            int32_t count = 0, link = 0, leaf = -1;
             float dscale = 0.0f;
             if (seated) {
                 const float2* first = ws.base + ray * kChunkFloat2;
@@ -2290,16 +2315,19 @@ struct ReplayRays {
                 link = __float_as_int(head.x);
                 count = stamped ? __float_as_int(head.y) : -1;
                 dscale = tail.x;
+                if (count > 0) leaf = __float_as_int(first[0].x);
             }
             const unsigned long long undone = __ballot(count < 0), m = __ballot(count > 0);
             if ((lane & 15) == 0 && seated) ((uint16_t*)ws.undone)[ray >> 4] = (uint16_t)(undone >> lane);
             if (lane == 0) n = __popcll(m);
             wave_lds_sync();
+            bool known = false;
+            int place = 0;
             if (count > 0) {
                 const int more = (count - 1) / kChunkRecords;
                 const int to = more > 0 && more <= kChunks ? atomicAdd(&n_chunks, more) : 0;
-                const bool known = more > 0 && more <= kChunks && to + more <= kChunks;
-                list[rank_in(m)] = ReplayRay{(int32_t)ray, known ? 1u : 0u, count, known ? to : link, dscale};
+                known = more > 0 && more <= kChunks && to + more <= kChunks;
+                place = to;
                 if (known) {
                     int32_t index = link;
                     for (int at = 0; at < more; ++at) {
@@ -2307,6 +2335,19 @@ struct ReplayRays {
                         chunks[to + at] = index;
                     }
                 }
+            }
+            // Neighbours share leaves if half of them begin in the leaf of the one to their left (16 of them are two
+            // rows of 8 pixels).
+            const int32_t left = __shfl_up(leaf, 1);
+            const unsigned long long alike = __ballot(leaf >= 0 && leaf == left && (lane & 7) != 0);
+            const unsigned like_left = (unsigned)(alike >> (lane & 48)) & 0xffffu;
+            const unsigned with_notes = (unsigned)(m >> (lane & 48)) & 0xffffu;
+            const unsigned long long shared = __ballot(count > 0 && 2 * __popc(like_left) >= __popc(with_notes));
+            if (lane == 0) cursor = n_shared = __popcll(shared);
+            if (count > 0) {
+                const bool first = (shared >> lane & 1ull) != 0;
+                list[first ? rank_in(shared) : __popcll(shared) + rank_in(m & ~shared)] =
+                    ReplayRay{(int32_t)ray, known ? 1u : 0u, count, known ? place : link, dscale};
             }
         }
         __syncthreads();
@@ -2341,10 +2382,8 @@ struct ReplayRays {
     }
 
     // Takes the next rays of the list whose notes fit into the wavefront: `at` receives the first of them (n: the list
-    // is used up), n_notes the number of their notes, g each lane's note.  Returns how many rays these are; 0: one ray
-    // that has more than 64 notes.
-    __device__ __forceinline__ int take(const ReplaySpace& ws, uint8_t* start, int lane, int& at, int& n_notes,
-                                        ReplayNote& g) {
+    // is used up), g each lane's note.  Returns how many rays these are; 0: one ray that has more than 64 notes.
+    __device__ __forceinline__ int take(const ReplaySpace& ws, uint8_t* start, int lane, int& at, ReplayNote& g) {
         int rays, sum, count;
         bool fits;
         at = __builtin_amdgcn_readfirstlane(__atomic_load_n(&cursor, __ATOMIC_RELAXED));
@@ -2366,7 +2405,7 @@ struct ReplayRays {
             at = seen;   // (another wavefront was faster)
         }
         if (rays == 0) return 0;
-        n_notes = __builtin_amdgcn_readlane(sum, rays - 1);
+        const int n_notes = __builtin_amdgcn_readlane(sum, rays - 1);
         start[lane] = 0;
         wave_lds_sync();
         if (fits) start[sum - count] = 1;
@@ -2386,6 +2425,51 @@ struct ReplayRays {
         int32_t index = r.ray;
         read(ws, r, g.p, chunk, index, g);
         return rays;
+    }
+
+    // Takes the next neighbours that share leaves, 16 at most and not more than a wavefront's part of all: `at` receives
+    // the first of them.  Returns how many; 0: all are taken.
+    __device__ __forceinline__ int take_shared(int lane, int& at) {
+        at = __builtin_amdgcn_readfirstlane(__atomic_load_n(&shared_cursor, __ATOMIC_RELAXED));
+        while (at < n_shared) {
+            const int piece = list[at + lane < n_shared ? at + lane : n_shared - 1].ray >> 4;
+            const bool with_first = piece == __builtin_amdgcn_readfirstlane(piece) && at + lane < n_shared;
+            const bool its_part = lane * kReplayWaves < n_shared && lane < ReplayCarry<1>::kRows;
+            const int rays = __builtin_ctzll(~__ballot(with_first && its_part));
+            int seen = at;
+            if (lane == 0) seen = atomicCAS(&shared_cursor, at, at + rays);
+            seen = __builtin_amdgcn_readfirstlane(seen);
+            if (seen == at) return rays;
+            at = seen;   // (another wavefront was faster)
+        }
+        return 0;
+    }
+
+    // Slice number k of the `taken` rays from entry `at` on: as many notes of each, one after the other, as there are
+    // lanes for (a power of two).  Returns whether any ray has notes in it.
+    template <int N>
+    __device__ __forceinline__ bool take_slice(const ReplaySpace& ws, int at, int taken, int k, int lane,
+                                               ReplayCarry<N>& carry, ReplayNote& g) {
+        const int shift = taken > 1 ? 6 - (32 - __builtin_clz((unsigned)taken - 1u)) : 6, wide = 1 << shift;
+        const bool seated = lane >> shift < taken;
+        g.owner = seated ? lane >> shift : 0;
+        const ReplayRay r = list[at + g.owner];
+        const int left = seated ? r.count - (k << shift) : 0;
+        g.ray = r.ray;
+        g.p = lane & (wide - 1);
+        g.count = left < wide ? left : wide;
+        g.valid = g.p < g.count;
+        g.last = lane - g.p + g.count - 1;
+        g.dscale = r.dscale;
+        if (!any_lane(g.valid)) return false;
+        int chunk = carry.chunk[g.owner];
+        int32_t index = carry.index[g.owner];
+        read(ws, r, (k << shift) + g.p, chunk, index, g);
+        if (g.valid && lane == g.last) {
+            carry.chunk[g.owner] = chunk;
+            carry.index[g.owner] = index;
+        }
+        return true;
     }
 
     // notes [64 * segment, 64 * segment + 64) of entry `at`; chunk, index: where the segment before it left off
@@ -2454,18 +2538,28 @@ __device__ __forceinline__ void running_sums(const ReplayNote& g, float weight, 
     for (int i = 0; i < N; ++i) sum[i] = run[i];
 }
 
+// Wavefronts per SIMD that the replay kernels' registers are cut to.  The loop over slices would else take one step
+// more of them than the loops beside it do without it: replay_backward_kernel, SH9 rays, 79 without that loop, 78
+// uncut, 74 cut; none spills.
+template <class P, class Source>
+constexpr int replay_waves(bool squared_error) {
+    if (P::kFormat == SVOX_FORMAT_SG || P::kBasis > 16) return 3;
+    if (std::is_same_v<Source, ImageSource<float>>) return 5;
+    return squared_error && P::kBasis > 9 ? 5 : 6;
+}
 // The backward pass from the notes a noting forward kernel left (NoteTaker), trace_ray_backward's second march
 // (rt_kernel.cu:358-475: the sum of the first march, then the records of the second).
 template <class P, class Source>
-__global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source src, SvoxRenderOptions opt,
-                                                                         const float* __restrict__ grad_out,
-                                                                         float* __restrict__ grad_data, ReplaySpace ws,
-                                                                         int ray_shift, Lobes lobes) {
+__global__ __launch_bounds__(kReplayThreads, (replay_waves<P, Source>(false))) void replay_backward_kernel(
+    Source src, SvoxRenderOptions opt, const float* __restrict__ grad_out, float* __restrict__ grad_data, ReplaySpace ws,
+    int ray_shift, Lobes lobes) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     __shared__ ReplayShared<D> shared[kReplayWaves];
+    __shared__ ReplayCarry<1> carries[kReplayWaves];
     __shared__ ReplayRays rays;
     const int lane = threadIdx.x & (kMarchThreads - 1);
     ReplayShared<D>& sh = shared[threadIdx.x / kMarchThreads];
+    ReplayCarry<1>& carry = carries[threadIdx.x / kMarchThreads];
     const bool stamped = stamp_matches(ws);
     if (ws.report && stamped && blockIdx.x == 0 && threadIdx.x == 0)
         __hip_atomic_store(ws.report, *ws.stocks_taken << 32 | ws.n_stocks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2505,12 +2599,14 @@ __global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source 
         }
     };
     // the records of a batch; behind: what lies behind the lane's leaf
-    auto add = [&](const ReplayNote& g, int n_notes, float light, float behind) {
+    auto add = [&](const ReplayNote& g, float light, float behind) {
+        const unsigned long long m = __ballot(g.valid);
+        const int place = rank_in(m);
         if (g.valid) {
             const float weight = light * (1.0f - att);
-            sh.leaf[lane] = g.leaf;
-            records.owners()[lane] = (uint8_t)g.owner;
-            float* const f = records.factors() + lane * 4;
+            sh.leaf[place] = g.leaf;
+            records.owners()[place] = (uint8_t)g.owner;
+            float* const f = records.factors() + place * 4;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 if constexpr (P::kFormat == SVOX_FORMAT_RGBA) {
@@ -2523,13 +2619,47 @@ __global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source 
             if (opt.density_softplus) g_sigma *= sigmoid_(g.raw - 1.0f);   // rt_kernel.cu:471-474
             f[3] = g_sigma;
         }
-        records.n = n_notes;
+        records.n = __popcll(m);
         records.flush();
     };
+    // neighbours that share leaves: slice by slice, once for the sum of the first march, once for the records
+    int at, n_rays;
+    while ((n_rays = rays.take_shared(lane, at)) > 0) {
+        ReplayNote g;
+        set_rows(at, n_rays);
+        if (lane < n_rays) {
+            carry.run[0][lane] = 0.0f;
+            carry.begin(lane, rays.list[at + lane].ray);
+        }
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+            wave_lds_sync();
+#pragma unroll 1
+            for (int k = 0; rays.take_slice(ws, at, n_rays, k, lane, carry, g); ++k) {
+                look(g);
+                const float light = light_before(g, att, carry.through[g.owner]);
+                const float weight = light * (1.0f - att);
+                float run[1] = {carry.run[0][g.owner]};
+                running_sums(g, pass == 0 ? weight : -weight, total_color, run, run);
+                if (g.valid && lane == g.last) {
+                    carry.through[g.owner] = light * att;
+                    carry.run[0][g.owner] = run[0];
+                }
+                if (pass == 1) add(g, light, run[0]);
+                wave_lds_sync();
+            }
+            if (pass == 0 && lane < n_rays) {
+                // the background behind the last leaf
+                const int32_t ray = rays.list[at + lane].ray;
+                const float* const grad = grad_out + (int64_t)ray * 3;
+                carry.run[0][lane] = fma_(carry.through[lane] * bg, (grad[0] + grad[1]) + grad[2], carry.run[0][lane]);
+                carry.begin(lane, ray);
+            }
+        }
+    }
     while (true) {
         ReplayNote g;
-        int at, n_notes = 0;
-        const int taken = rays.take(ws, sh.start, lane, at, n_notes, g);
+        const int taken = rays.take(ws, sh.start, lane, at, g);
         if (at >= rays.n) break;
         if (taken > 0) {
             set_rows(at, taken);
@@ -2541,7 +2671,7 @@ __global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source 
             const int last = g.valid ? g.last : lane;
             run[0] = fma_(__shfl(light * att, last) * bg, (go[0] + go[1]) + go[2], __shfl(run[0], last));
             running_sums(g, -weight, total_color, run, run);
-            add(g, n_notes, light, run[0]);
+            add(g, light, run[0]);
             continue;
         }
         set_rows(at, 1);
@@ -2561,7 +2691,7 @@ __global__ __launch_bounds__(kReplayThreads) void replay_backward_kernel(Source 
                 running_sums(g, pass == 0 ? weight : -weight, total_color, run, behind);
                 run[0] = __shfl(behind[0], g.last);
                 through = __shfl(light * att, g.last);
-                if (pass == 1) add(g, g.count, light, behind[0]);
+                if (pass == 1) add(g, light, behind[0]);
             }
             if (pass == 0) run[0] = fma_(through * bg, __shfl((go[0] + go[1]) + go[2], 0), run[0]);
         }
@@ -2978,17 +3108,18 @@ struct ReplaySeShared : ReplayShared<D> {
     float resid[kReplayRows * 3];
 };
 template <class P, class Source>
-__global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source src, SvoxRenderOptions opt,
-                                                                        float* __restrict__ grad_data,
-                                                                        float* __restrict__ hess_data, ReplaySpace ws,
-                                                                        int ray_shift, Lobes lobes) {
+__global__ __launch_bounds__(kReplayThreads, (replay_waves<P, Source>(true))) void replay_se_grad_kernel(
+    Source src, SvoxRenderOptions opt, float* __restrict__ grad_data, float* __restrict__ hess_data, ReplaySpace ws,
+    int ray_shift, Lobes lobes) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
     constexpr bool kRgba = P::kFormat == SVOX_FORMAT_RGBA;
     __shared__ ReplaySeShared<D> shared[kReplayWaves];
+    __shared__ ReplayCarry<3> carries[kReplayWaves];
     __shared__ ReplayRays rays;
     const int lane = threadIdx.x & (kMarchThreads - 1);
     ReplaySeShared<D>& sh = shared[threadIdx.x / kMarchThreads];
+    ReplayCarry<3>& carry = carries[threadIdx.x / kMarchThreads];
     rays.gather(ws, stamp_matches(ws), src.n_slots(), (int)blockIdx.x, (int)gridDim.x, ray_shift);
 
     const float bg = opt.background_brightness;
@@ -3104,20 +3235,22 @@ __global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source s
         for (int c = 0; c < 3; ++c) col[c] = g.valid ? fma_(g.s[c], d_rgb_pad, -pad) : 0.0f;
     };
     // the records of a batch; behind: the colour that lies behind the lane's leaf
-    auto add = [&](const ReplayNote& g, int n_notes, float light, const float* behind) {
+    auto add = [&](const ReplayNote& g, float light, const float* behind) {
+        const unsigned long long m = __ballot(g.valid);
+        const int place = rank_in(m);
         if (g.valid) {
             const float weight = light * (1.0f - att), after = light * att;
             const float sg = opt.density_softplus ? sigmoid_(g.raw - 1.0f) : 1.0f;
             const float d_sg = sg * (1.0f - sg);
             float g_sigma = 0.0f, h_sigma = 0.0f;
-            sh.leaf[lane] = g.leaf;
-            sh.owner[lane] = (uint8_t)g.owner;
+            sh.leaf[place] = g.leaf;
+            sh.owner[place] = (uint8_t)g.owner;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 if constexpr (kRgba) {
-                    sh.factor[lane * 4 + c] = weight * g.s[c] * (1.0f - g.s[c]) * d_rgb_pad;
+                    sh.factor[place * 4 + c] = weight * g.s[c] * (1.0f - g.s[c]) * d_rgb_pad;
                 } else {
-                    sh.factor[lane * 4 + c] =
+                    sh.factor[place * 4 + c] =
                         (float)((double)(weight * g.s[c]) * (1.0 - (double)g.s[c]) * (double)d_rgb_pad);
                 }
                 const float gs = g.dt * g.dscale * fma_(col[c], after, -behind[c]);
@@ -3130,15 +3263,52 @@ __global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source s
                     h_sigma += gs * gs;
                 }
             }
-            sh.factor[lane * 4 + 3] = g_sigma;
-            sh.hess_sigma[lane] = h_sigma;
+            sh.factor[place * 4 + 3] = g_sigma;
+            sh.hess_sigma[place] = h_sigma;
         }
-        flush(n_notes);
+        flush(__popcll(m));
     };
+    // neighbours that share leaves: slice by slice, once for the ray's colour, once for the records
+    int at, n_rays;
+    while ((n_rays = rays.take_shared(lane, at)) > 0) {
+        ReplayNote g;
+        set_rows(at, n_rays);
+        if (lane < n_rays) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) carry.run[c][lane] = 0.0f;
+            carry.begin(lane, rays.list[at + lane].ray);
+        }
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+            wave_lds_sync();
+#pragma unroll 1
+            for (int k = 0; rays.take_slice(ws, at, n_rays, k, lane, carry, g); ++k) {
+                look(g);
+                const float light = light_before(g, att, carry.through[g.owner]);
+                const float weight = light * (1.0f - att);
+                float run[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) run[c] = carry.run[c][g.owner];
+                running_sums(g, pass == 0 ? weight : -weight, col, run, run);
+                if (g.valid && lane == g.last) {
+                    carry.through[g.owner] = light * att;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) carry.run[c][g.owner] = run[c];
+                }
+                if (pass == 1) add(g, light, run);
+                wave_lds_sync();
+            }
+            if (pass == 0 && lane < n_rays) {
+                // the background behind the last leaf
+#pragma unroll
+                for (int c = 0; c < 3; ++c) carry.run[c][lane] = fma_(carry.through[lane], bg, carry.run[c][lane]);
+                carry.begin(lane, rays.list[at + lane].ray);
+            }
+        }
+    }
     while (true) {
         ReplayNote g;
-        int at, n_notes = 0;
-        const int taken = rays.take(ws, sh.start, lane, at, n_notes, g);
+        const int taken = rays.take(ws, sh.start, lane, at, g);
         if (at >= rays.n) break;
         if (taken > 0) {
             set_rows(at, taken);
@@ -3152,7 +3322,7 @@ __global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source s
 #pragma unroll
             for (int c = 0; c < 3; ++c) run[c] = fma_(through, bg, __shfl(run[c], last));
             running_sums(g, -weight, col, run, run);
-            add(g, n_notes, light, run);
+            add(g, light, run);
             continue;
         }
         set_rows(at, 1);
@@ -3173,7 +3343,7 @@ __global__ __launch_bounds__(kReplayThreads) void replay_se_grad_kernel(Source s
 #pragma unroll
                 for (int c = 0; c < 3; ++c) run[c] = __shfl(behind[c], g.last);
                 through = __shfl(light * att, g.last);
-                if (pass == 1) add(g, g.count, light, behind);
+                if (pass == 1) add(g, light, behind);
             }
             if (pass == 0) {
 #pragma unroll

@@ -47,3 +47,84 @@ def test_notes_of_every_number(gpu, oracle_mod, levels, keep, n, fmt):
     for a, b in zip(replayed[1:], marched[1:]):
         err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy())
         assert ok, err
+
+
+@pytest.mark.parametrize("levels,n,softplus", [(1, 160, False), (5, 1600, False), (5, 40007, True), (4, 40000, False), (5, 70001, False)])
+@pytest.mark.parametrize("fmt", ["RGBA", "SH9"])
+def test_notes_of_neighbours_that_share_leaves(gpu, oracle_mod, levels, n, softplus, fmt):
+    """Pieces of 16 rays of which 1, 2, 3 ... 16 meet the scene, next to one another or (every fourth piece) from all
+    over; their notes are read in slices of 64, 32, 16, 8 or 4 of each, up to 150 of them.
+
+    With softplus the generic kernels are the only reference: every leaf counts there, a leaf's density gradient is a
+    difference of nearly equal sums, and the last bit of an exponential, which the device and the oracle round
+    differently, is 1.9e-4 of the smallest of them, in the marching kernels' gradient bit for bit as in this one."""
+    tree = svox.N3Tree(N=2, data_format=fmt, init_refine=levels)
+    gen = torch.Generator().manual_seed(levels)
+    tree.data.data.normal_(generator=gen)
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.5 * (torch.rand(tree.child.shape, generator=gen) < 0.8)
+    rays = synth.sphere_rays(n, seed=n)
+    at = torch.arange(n)
+    piece, place = at // 16, at % 16
+    near = piece % 4 != 3
+    first = piece * 16
+    dirs, origins = rays.dirs.clone(), rays.origins.clone()
+    jitter = (torch.rand(n, 3, generator=gen) - 0.5) * 2e-3
+    dirs[near] = torch.nn.functional.normalize(rays.dirs[first][near] + jitter[near], dim=-1)
+    origins[near] = rays.origins[first][near]
+    away = near & (place >= piece % 16 + 1)
+    dirs[away] = -dirs[away]
+    rays = svox.Rays(origins, dirs, dirs)
+    opt = options(tree, step_size=1e-3, density_softplus=softplus)
+    dev, rs = on_gpu(tree, gpu), rays_spec(rays, gpu)
+    go = torch.randn(n, 3, generator=gen) * 1e-2
+    out, notes = C.volume_render_noted(dev._spec(), rs, opt, records_per_ray=256)
+    assert notes is not None
+    got = C.volume_render_backward_noted(dev._spec(), rs, opt, go.to(gpu), notes)
+    if n <= 2000:
+        ot = oracle_mod.Tree.from_n3tree(tree)
+        want = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go)
+    else:
+        C.set_debug_flags(1)
+        try:
+            want = C.volume_render_backward(dev._spec(), rs, opt, go.to(gpu)).cpu().numpy()
+        finally:
+            C.set_debug_flags(0)
+    err, ok = grad_close(got.cpu().numpy(), want)
+    assert ok, err
+    target = torch.rand(n, 3, generator=gen).to(gpu)
+    replayed, marched = C.se_grad(dev._spec(), rs, target, opt), C.se_grad(dev._spec(), rs, target, opt, workspace=False)
+    assert torch.equal(replayed[0], marched[0])
+    for a, b in zip(replayed[1:], marched[1:]):
+        err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy())
+        assert ok, err
+
+
+def test_notes_of_a_picture_taken_close_up(gpu):
+    """Where neighbours share leaves their records are added together before they go to memory: the gradient of a
+    picture taken from close to the tree is faster from notes than from a march of its own.  (A ray alone in its
+    wavefront, whose records go out one by one, takes 5 780 us here, a march 4 360, rays with their neighbours 2 510.)"""
+    tree = synth.dense_tree(6, data_format="SH16", seed=7, zero_fraction=0.5)
+    dev = on_gpu(tree, gpu)
+    opt = options(tree, step_size=1e-3)
+    cam = C.CameraSpec()
+    cam.c2w = synth.orbit_poses(1, seed=1, radius=1.2)[0][None].to(gpu)
+    cam.width = cam.height = 800
+    cam.fx = cam.fy = 1111.111
+    go = torch.randn(1, 800, 800, 3, generator=torch.Generator().manual_seed(1)).to(gpu) * 1e-2
+    spec = dev._spec()
+    notes = C.volume_render_images_noted(spec, cam, opt, records_per_ray=256)[1]
+    assert notes is not None
+    times = {}
+    for way in ["notes", "march"] * 6:
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        if way == "notes":
+            C.volume_render_images_backward_noted(spec, cam, opt, go, notes)
+        else:
+            C.volume_render_images_backward(spec, cam, opt, go, workspace=False)
+        end.record()
+        end.synchronize()
+        times.setdefault(way, []).append(begin.elapsed_time(end) * 1e3)
+    noted, marched = (sorted(times[w])[3] for w in ("notes", "march"))
+    print(f"[notes] close up: from notes {noted:.0f} us, from a march {marched:.0f} us", flush=True)
+    assert noted <= 0.9 * marched
