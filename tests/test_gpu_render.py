@@ -823,10 +823,13 @@ def test_writes_past_the_version_counters_between_forward_and_backward(gpu, orac
 
     def oracle_grads():
         ot = oracle_mod.Tree.from_n3tree(tree)      # the tree as it is now
-        a = oracle_mod.volume_render_backward(ot, rays.origins.cpu(), rays.dirs.cpu(), rays.viewdirs.cpu(), opt, go.cpu())
+        a = oracle_mod.volume_render_backward(ot, rays.origins.cpu(), rays.dirs.cpu(), rays.viewdirs.cpu(), opt, go.cpu(),
+                                              want_slack=True)
         b = oracle_mod.volume_render_image_backward(ot, c2w.cpu(), 50.0, 50.0, 64, 48, opt, gi.cpu())
         return a, b
 
+    # (the batch's order slack is taken off: once view_write has made the large leaves around the shell dense, hundreds of
+    # rays add into each of them, and the bare difference is 2e-5 to 1.1e-4 with the order the GPU happens to take)
     def check(write):
         tree.data.grad = None
         out = r(rays, fast=True)
@@ -834,9 +837,9 @@ def test_writes_past_the_version_counters_between_forward_and_backward(gpu, orac
         versions = (tree.data._version, tree.child._version)
         write()
         assert (tree.data._version, tree.child._version) == versions    # torch has not seen the write
-        want_batch, want_image = oracle_grads()
+        (want_batch, slack), want_image = oracle_grads()
         out.backward(go)
-        err, ok = grad_close(tree.data.grad.cpu().numpy(), want_batch)
+        err, ok = grad_close(tree.data.grad.cpu().numpy(), want_batch, slack=slack)
         assert ok, err
         tree.data.grad = None
         img.backward(gi)

@@ -55,6 +55,8 @@ def test_notes_of_neighbours_that_share_leaves(gpu, oracle_mod, levels, n, softp
     """Pieces of 16 rays of which 1, 2, 3 ... 16 meet the scene, next to one another or (every fourth piece) from all
     over; their notes are read in slices of 64, 32, 16, 8 or 4 of each, up to 150 of them.
 
+    The order slack of the oracle is taken off: up to 70 001 rays add into the leaves of a 32^3 or 64^3 grid in the order the
+    GPU happens to take them, and the bare difference of two such sums is 4e-5 to 9.8e-5 from run to run.
     With softplus the generic kernels are the only reference: every leaf counts there, a leaf's density gradient is a
     difference of nearly equal sums, and the last bit of an exponential, which the device and the oracle round
     differently, is 1.9e-4 of the smallest of them, in the marching kernels' gradient bit for bit as in this one."""
@@ -80,22 +82,25 @@ def test_notes_of_neighbours_that_share_leaves(gpu, oracle_mod, levels, n, softp
     out, notes = C.volume_render_noted(dev._spec(), rs, opt, records_per_ray=256)
     assert notes is not None
     got = C.volume_render_backward_noted(dev._spec(), rs, opt, go.to(gpu), notes)
-    if n <= 2000:
-        ot = oracle_mod.Tree.from_n3tree(tree)
-        want = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go)
-    else:
+    target = torch.rand(n, 3, generator=gen)
+    replayed = C.se_grad(dev._spec(), rs, target.to(gpu), opt)
+    marched = C.se_grad(dev._spec(), rs, target.to(gpu), opt, workspace=False)
+    assert torch.equal(replayed[0], marched[0])
+    if softplus:
         C.set_debug_flags(1)
         try:
             want = C.volume_render_backward(dev._spec(), rs, opt, go.to(gpu)).cpu().numpy()
         finally:
             C.set_debug_flags(0)
-    err, ok = grad_close(got.cpu().numpy(), want)
-    assert ok, err
-    target = torch.rand(n, 3, generator=gen).to(gpu)
-    replayed, marched = C.se_grad(dev._spec(), rs, target, opt), C.se_grad(dev._spec(), rs, target, opt, workspace=False)
-    assert torch.equal(replayed[0], marched[0])
-    for a, b in zip(replayed[1:], marched[1:]):
-        err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy())
+        checks = [(got, want, None)] + [(a, b.cpu().numpy(), None) for a, b in zip(replayed[1:], marched[1:])]
+    else:
+        ot = oracle_mod.Tree.from_n3tree(tree)
+        ray_args = (ot, rays.origins, rays.dirs, rays.viewdirs)
+        want, slack = oracle_mod.volume_render_backward(*ray_args, opt, go, n_threads=8, want_slack=True)
+        _, g, h, g_slack, h_slack = oracle_mod.se_grad(*ray_args, target, opt, n_threads=8, want_slack=True)
+        checks = [(got, want, slack), (replayed[1], g, g_slack), (replayed[2], h, h_slack)]
+    for a, b, slack in checks:
+        err, ok = grad_close(a.cpu().numpy(), b, slack=slack)
         assert ok, err
 
 
