@@ -1007,6 +1007,14 @@ struct NoteTaker {
     }
 };
 
+// A noting pass follows a ray beyond the early stop of its picture, but not beyond the leaf behind which the transmittance of what
+// it shades is less than the smallest normal float, 2^-126: every weight further on is less than that, and with it every term of
+// the picture, of the sum of the first march and of a gradient.  (What the reference adds to the density gradients of such leaves
+// is the rounding that is left of `accum`, where the exact term is below 2^-126.)  The chain of a batch's longest rays is what such
+// a pass waits for, and those that graze a surface are long because of what they pass through: 50 001 rays of a 256^3 SH9 shell with
+// softplus, march 240 -> 80 us, training step 391 -> 203 us.  Scenes without such densities: within 0.2 %.
+constexpr float kOpaqueLight = 1.17549435e-38f;
+
 // What a noting pass that has the gradient of the picture at hand accumulates per ray beside its notes:
 // the sum the backward pass forms in its first march (rt_kernel.cu:358-419; the same expressions, in
 // the same order, as march 1 of render_backward_kernel), so that a ray whose notes do not fit needs
@@ -1201,11 +1209,13 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
             }
 #pragma unroll
             for (int q = 0; q < kQueue; ++q) {
-                const bool take = active && !painted && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
+                // (the light of a ray whose picture is finished goes on: kOpaqueLight)
+                const bool shade = active && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
+                const bool take = shade && !painted;
                 const float weight = light * (1.0f - q_att[q]);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) acc[c] = take ? fma_(weight, q_rgb[q][c], acc[c]) : acc[c];
-                light = take ? light * q_att[q] : light;
+                light = shade ? light * q_att[q] : light;
                 if constexpr (kAccum) {
                     if (take) {
                         if (tr.weight_accum_max)
@@ -1237,7 +1247,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
                 else
                     active = false;
             }
-            if (active && (broken || !(r.t < r.tmax))) {
+            if (active && (broken || !(r.t < r.tmax) || (kNoted && light < kOpaqueLight))) {
                 if (kNoted && !kGrad && grad_out) {
                     notes.finish_residual(broken, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
                 } else {
@@ -1943,6 +1953,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     // kNoted: the picture of a ray may be finished (early stop) while its notes go on; without `out`
     // there is no picture to compose
     bool painted = kNoted && out == nullptr;
+    bool opaque = false;   // kNoted: nothing behind the leaves seen so far counts any more
     NoteTaker notes;
     March1Sum sum1;
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
@@ -1954,7 +1965,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) place[q] = ring_read(&box.place[((taken + q) & (kRing - 1)) * kMarchThreads + lane]);
         int n_take = 0;
-        bool run = active;
+        bool run = active && !opaque;
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) {
             const uint32_t code = (uint32_t)place[q];
@@ -1962,17 +1973,19 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             n_take += run ? 1 : 0;
         }
         const uint32_t next = (uint32_t)place[0];
-        if (active && (next & kOverBit) && (next & kRoundBit) == ring_round(taken)) {
+        const bool over = (next & kOverBit) && (next & kRoundBit) == ring_round(taken);
+        if (active && (over || (kNoted && opaque))) {
             // the ray left the tree: the background shows through what is left of the light
+            const bool broken = over && (next & 1u) != 0;
             if (kNoted && !kGrad && grad_out) {
-                notes.finish_residual((next & 1u) != 0, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
+                notes.finish_residual(broken, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
             } else {
                 if (!painted) {
                     out[slot * 3] = fma_(light, bg, acc[0]);
                     out[slot * 3 + 1] = fma_(light, bg, acc[1]);
                     out[slot * 3 + 2] = fma_(light, bg, acc[2]);
                 }
-                if constexpr (kNoted) notes.finish((next & 1u) != 0, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
+                if constexpr (kNoted) notes.finish(broken, r.dscale, kGrad ? sum1.end(bg) : 0.0f);
             }
             active = false;
         }
@@ -2027,11 +2040,13 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             }
 #pragma unroll
             for (int q = 0; q < kQueue; ++q) {
-                const bool take = active && !painted && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
+                // (the light of a ray whose picture is finished goes on: kOpaqueLight)
+                const bool shade = active && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
+                const bool take = shade && !painted;
                 const float weight = light * (1.0f - q_att[q]);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) acc[c] = take ? fma_(weight, q_rgb[q][c], acc[c]) : acc[c];
-                light = take ? light * q_att[q] : light;
+                light = shade ? light * q_att[q] : light;
                 stopped = stopped || (take && light <= stop_thresh);
                 if constexpr (kNoted) {
                     const bool note = active && q_leaf[q] >= 0 && q_sigma[q] > 0.0f;
@@ -2053,6 +2068,12 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                 painted = true;   // the picture is done; the notes go on to the end of the ray
             } else {
                 active = false;
+                taken_write(&box.taken[lane], taken | kEndedBit);
+            }
+        }
+        if constexpr (kNoted) {
+            if (active && !opaque && light < kOpaqueLight) {
+                opaque = true;
                 taken_write(&box.taken[lane], taken | kEndedBit);
             }
         }

@@ -133,3 +133,48 @@ def test_notes_of_a_picture_taken_close_up(gpu):
     noted, marched = (sorted(times[w])[3] for w in ("notes", "march"))
     print(f"[notes] close up: from notes {noted:.0f} us, from a march {marched:.0f} us", flush=True)
     assert noted <= 0.9 * marched
+
+
+@pytest.mark.parametrize("fmt,softplus,density", [("SH4", False, 2000.0), ("RGBA", False, 1e4), ("SH9", False, 1e36), ("SH1", True, 300.0)])
+@pytest.mark.parametrize("flags", [0, 2, 4, 8])
+def test_noted_rays_end_where_nothing_shines_through(gpu, oracle_mod, fmt, softplus, density, flags):
+    """Leaves so dense that a ray's transmittance falls below the smallest float inside the tree: its notes end there, picture and
+    gradients stay those of the whole ray.  Where the picture shades none of them, none are left out."""
+    n = 700
+    tree = svox.N3Tree(N=2, data_format=fmt, init_refine=4)
+    gen = torch.Generator().manual_seed(11)
+    tree.data.data.normal_(generator=gen)
+    dense = torch.rand(tree.child.shape, generator=gen)
+    tree.data.data[..., -1] = torch.where(dense < 0.5, density * dense, -3.0 * dense)
+    rays = synth.sphere_rays(n, seed=12)
+    dev, rs = on_gpu(tree, gpu), rays_spec(rays, gpu)
+    spec, ot = dev._spec(), oracle_mod.Tree.from_n3tree(tree)
+    go, target = torch.randn(n, 3, generator=gen) * 1e-2, torch.full((n, 3), 0.5, device=gpu)
+    for thresh in (0.0, float("inf")):
+        opt = options(tree, step_size=1e-3, density_softplus=softplus, sigma_thresh=thresh, stop_thresh=0.0)
+        positive = C.volume_render_stats(spec, rs, opt)["samples_bwd_pos"]
+        C.set_debug_flags(flags)
+        try:
+            out, notes = C.volume_render_noted(spec, rs, opt, records_per_ray=256)
+            got = C.volume_render_backward_noted(spec, rs, opt, go.to(gpu), notes)
+            alone = C.volume_render_backward(spec, rs, opt, go.to(gpu))
+            colours = C.se_grad(spec, rs, target, opt)[0]
+        finally:
+            C.set_debug_flags(0)
+        noted = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91]      # (how many notes a ray has: beside the link of its first chunk)
+        assert bool((noted >= 0).all())
+        assert int(noted.sum()) == positive if thresh > 0 else int(noted.sum()) < 0.9 * positive
+        # (with softplus the last bit of its exponential differs between device and oracle: the marching kernels are the reference)
+        C.set_debug_flags(1 if softplus else 0)
+        try:
+            march, march_se = C.volume_render(spec, rs, opt), C.se_grad(spec, rs, target, opt, workspace=False)[0]
+            march_grad = C.volume_render_backward(spec, rs, opt, go.to(gpu), workspace=False).cpu().numpy()
+        finally:
+            C.set_debug_flags(0)
+        if not softplus:
+            assert (out.cpu().numpy() == oracle_mod.volume_render(ot, rays.origins, rays.dirs, rays.viewdirs, opt)).all()
+            march_grad = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go)
+        assert torch.equal(out, march) and torch.equal(colours, march_se)
+        for what, grad in (("from notes", got), ("alone", alone)):
+            err, ok = grad_close(grad.cpu().numpy(), march_grad, what=what)
+            assert ok, (thresh, what, err)
