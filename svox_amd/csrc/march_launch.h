@@ -6,6 +6,7 @@
 // (SVOX_DISPATCH_OCTREE) and calls these functions.
 #pragma once
 
+#include "cut_kernel.h"
 #include "march_kernels.h"
 
 namespace svox {
@@ -21,6 +22,9 @@ struct MarchLaunch {
     static void noting(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                        const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, const float* grad_out,
                        const float* color_ref, bool split, bool refill);
+    // either of them with every ray cut into pieces (cut_kernel.h), per_wave rays to a wavefront, 2^most_cut pieces at most
+    static void cut(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src, const SvoxRenderOptions& opt,
+                    float* out, const ReplaySpace& ws, bool noted, const float* grad_out, const float* color_ref, int per_wave, int most_cut);
     static void backward(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                          const SvoxRenderOptions& opt, const float* grad_out, float* grad_data, const ReplaySpace& ws,
                          bool refill, bool second_only);
@@ -104,6 +108,22 @@ void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeD
     else
         SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, false>);
 #undef SVOX_NOTING
+}
+
+template <class P, class Source>
+void MarchLaunch<P, Source>::cut(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
+                                 const SvoxRenderOptions& opt, float* out, const ReplaySpace& ws, bool noted,
+                                 const float* grad_out, const float* color_ref, int per_wave, int most_cut) {
+#define SVOX_CUT(...)                                                                                                \
+    hipLaunchKernelGGL((render_forward_cut_kernel<P, Source, __VA_ARGS__>), blocks, dim3(kMarchThreads), 0, stream, tr, src, opt, out, \
+                       ws, grad_out ? grad_out : color_ref, per_wave, most_cut)
+    if (noted && grad_out)
+        SVOX_CUT(true, true);
+    else if (noted)
+        SVOX_CUT(true, false);
+    else
+        SVOX_CUT(false, false);
+#undef SVOX_CUT
 }
 
 template <class P, class Source>

@@ -32,7 +32,8 @@ using namespace svox;
 thread_local char g_error[512] = "";
 // Debug flags of the calling thread (svox_set_debug_flags): bit 0: always take the generic kernels; bit 1: small
 // batches run like large ones; bit 2: forward launches never take the two-wavefront kernel; bit 3: they always
-// do (where it applies).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
+// do (where it applies); bit 4: the bounded waits of that kernel give up at once; bit 5: forward launches cut their rays, as bits 8 and
+// up say (pick_cut).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
 thread_local int g_debug_flags = 0;
 
 // Launch-shape overrides for experiments, read from the environment once, when the first launch of the process
@@ -46,9 +47,12 @@ thread_local int g_debug_flags = 0;
 //   SVOX_SPLIT_FORWARD 0 / 1: forward launches never / always on two wavefronts per tile
 //   SVOX_SPLIT_BLOCKS  largest forward launch (in tiles) that takes two wavefronts per tile
 //   SVOX_REPLAY_SHIFT  4, 5 or 6: log2 of the rays a block of the replay kernels takes
+//   SVOX_CUT           0: forward passes never cut their rays into pieces, 1 to 8: always, so many rays to a wavefront, + 10 x:
+//                      into 2^x pieces at most (62: two rays, 32 pieces of each)
 struct Tuning {
     int per_wave = 0, refill = 0, xcd_group = 0, tile_order = -1, image_run = -1, split_forward = -1, replay_shift = -1;
     long split_blocks = -1;
+    int cut = -1;
 };
 const Tuning& tuning() {
     static const Tuning t = [] {
@@ -65,6 +69,7 @@ const Tuning& tuning() {
         v.split_forward = (int)num("SVOX_SPLIT_FORWARD", -1);
         v.split_blocks = num("SVOX_SPLIT_BLOCKS", -1);
         v.replay_shift = (int)num("SVOX_REPLAY_SHIFT", -1);
+        v.cut = (int)num("SVOX_CUT", -1);
         return v;
     }();
     return t;
@@ -615,6 +620,57 @@ constexpr bool is_image_source(const ImageSource<T>&) { return true; }
 template <typename T>
 constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 
+// How a forward pass cuts its rays into pieces (cut_kernel.h): rays dealt to a wavefront (0: it does not), log2 of a ray's pieces at most.
+struct Cut {
+    int per_wave = 0, most = 6;
+};
+// The pieces pay as long as they find the GPU idle: what each of them walks in vain -- the leaves until two walks agree -- is
+// as much as a fair part of it, and the more of them the shorter.  A tree is small (up to 32^3 leaves: rays of few leaves), large (from
+// 128^3, or the surface of 256^3, on) or between.  The launcher cannot know how many rays meet the cube, so the rule is drawn where a
+// launch of rays that all do gains nothing more.  us, forward pass with notes and without, from 4 096 rays on for both choices,
+// uncut / cut, SH4 to SH16 trees, rays that all meet the cube where it is dense, 18 % of them where it is a shell:
+//   16^3      1 000 rays 43, 40 / 28, 22    4 000 42, 39 / 31, 25    8 000 42, 40 / 34, 26    16 000 43, 40 / 63, 44
+//   32^3      1 000 rays 84, 81 / 36, 29    4 000 81, 79 / 41, 32    8 000 83, 78 / 48, 42    16 000 88, 80 / 94, 69
+//   64^3      1 000 rays 165, 160 / 52, 56  4 000 204, 199 / 68, 67  12 000 202, 197 / 165, 123  16 000 202, 197 / 205, 144
+//   128^3     1 000 rays 418, 412 / 72, 63  4 000 413, 410 / 145, 135  8 000 416, 412 / 255, 184  12 000 424, 418 / 303, 247
+//   64^3 shell   1 000 rays 75, 73 / 38, 31    4 000 83, 80 / 41, 34    16 000 90, 87 / 81, 57
+//   256^3 shell  1 000 rays 149, 145 / 50, 43  4 000 169, 166 / 109, 108  8 000 169, 165 / 89, 72  16 000 196, 189 / 158, 120
+//   512^3 shell  1 000 rays 170, 170 / 67, 72  4 000 224, 225 / 163, 165  8 000 224, 223 / 110, 110  16 000 257, 252 / 225, 186
+// and square pictures of 64 / 90 / 128 pixels a side (4 096, 8 100, 16 384):
+//   16^3   27, 23 / 22, 18      28, 23 / 25, 21       27, 23 / 40, 31
+//   64^3   89, 83 / 37, 30      127, 113 / 44, 31     124, 111 / 75, 52
+//   128^3  206, 192 / 59, 52    242, 237 / 96, 49     237, 231 / 146, 93
+//   512^3 shell  177, 115 / 59, 44  259, 188 / 61, 49  288, 186 / 114, 78
+//   NDC, every ray in the tree, 256^3 and 512^3  133, 86 / 108, 49  151, 114 / 172, 79  146, 117 / 239, 118;
+//                                                227, 129 / 225, 83  245, 158 / 335, 116  243, 156 / 447, 185
+Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRenderOptions* opt, bool noted) {
+    const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : g_debug_flags == 0 ? tuning().cut : 0;
+    Cut c;
+    if (forced >= 0) {
+        c.per_wave = std::min(forced % 10, kCutMostRays);
+        c.most = std::min(forced / 10, 6);
+        return c;
+    }
+    const double cells = (double)tree->capacity * tree->N * tree->N * tree->N;
+    const bool small = cells < 65536.0, large = cells >= 1048576.0;
+    if (image && opt->ndc_width > 0) {
+        if (items <= (noted ? 4096 : 8192)) c.per_wave = small ? 8 : 4;
+    } else if (items <= (small ? 8192 : 12288)) {
+        if (image) {
+            // (most pixels of a picture miss: a wavefront finds one ray or two among four, or eight)
+            c.per_wave = large ? 4 : 8;
+            c.most = large ? 6 : 4;
+        } else if (small) {
+            c.per_wave = items <= 4096 ? 4 : 8;
+        } else if (large) {
+            c.per_wave = items <= 1536 ? 1 : items <= 8192 || !noted ? 2 : 4;
+        } else {
+            c.per_wave = 4;
+        }
+    }
+    return c;
+}
+
 template <class Source, typename T>
 void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, int out_dim,
                     void* out, hipStream_t stream) {
@@ -622,10 +678,16 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
     if constexpr (sizeof(T) == 4) {
         const int D = fast_basis(tree, opt);
         if (D >= 0) {
-            const unsigned blocks = blocks_for(items, src.per_wave);
-            const Source dealt = dealt_out(src, blocks);
             const TreeDev<float> tr = march_tree(tree, opt, opt->sigma_thresh);
             const ReplaySpace none = no_notes();
+            const Cut cut = tree->weight_accum ? Cut() : pick_cut(tree, items, is_image_source(src), opt, false);
+            if (cut.per_wave > 0) {
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(dim3(blocks_for(items, cut.per_wave)), stream, tr, src, *opt, (float*)out,
+                                                                    none, false, nullptr, nullptr, cut.per_wave, cut.most));
+                return;
+            }
+            const unsigned blocks = blocks_for(items, src.per_wave);
+            const Source dealt = dealt_out(src, blocks);
             // Marks made with this launch's own threshold: every leaf they let through is shaded, and the kernel with
             // one wavefront per tile or chunk then reads a leaf's density with its coefficients (one round trip per
             // round instead of two that wait for one another: 4 NDC poses 3.10 -> 2.93 ms).  The two-wavefront kernel
@@ -759,6 +821,13 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
     ws.give_ups = give_up_counter();
+    const Cut cut = pick_cut(tree, total_items_of(src), is_image_source(src), opt, true);
+    if (cut.per_wave > 0) {
+        SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(dim3(blocks_for(total_items_of(src), cut.per_wave)), stream,
+                                                            march_tree(tree, opt), src, *opt, (float*)out, ws, true,
+                                                            (const float*)grad_out, (const float*)color_ref, cut.per_wave, cut.most));
+        return SVOX_OK;
+    }
     const bool refill = src.per_wave > kMarchThreads;
     unsigned at_once = 0;
     SVOX_DISPATCH_OCTREE(D, at_once = MarchLaunch<P, Source>::split_tiles_at_once(true, grad_out != nullptr));

@@ -1,0 +1,128 @@
+"""Rays walked in pieces, several lanes to a ray: every split of a wavefront (one to eight rays, one to 64 pieces), lists that run over,
+rays that miss, end early, or whose notes find no room.
+
+Bar: pictures and noted colours bit-identical to those of the kernel that walks a ray from end to end, as many notes of every
+ray, gradients within 1e-4 of that kernel's -- the terms are the same, added in another order -- beyond the order slack where the
+oracle has one.
+"""
+import pytest
+import torch
+
+import svox_amd as svox
+from svox_amd import csrc as C
+from svox_amd import synth
+from util import cam_spec, grad_close, on_gpu, options, rays_spec
+
+pytestmark = pytest.mark.gpu
+
+END_TO_END = 4
+
+
+def cut(per_wave, most):
+    return 32 | (per_wave + 10 * most) << 8
+
+
+def run(flags, f):
+    C.set_debug_flags(flags)
+    try:
+        return f()
+    finally:
+        C.set_debug_flags(0)
+
+
+def scene(kind, fmt, gen):
+    if kind == "shell":
+        return synth.shell_tree(depth=7, data_format=fmt, n_spheres=6, seed=4)
+    if kind == "deep":
+        return synth.deep_tree(12, data_format=fmt, seed=5)[0]
+    extra = torch.randn(4, 4, generator=gen) if fmt.startswith("SG") else None
+    tree = svox.N3Tree(N=3 if kind == "thirds" else 2, data_format=fmt, init_refine={"thirds": 2, "leaf": 0, "dense": 5}[kind], extra_data=extra)
+    tree.data.data.normal_(generator=gen)
+    keep = torch.rand(tree.child.shape, generator=gen) < 0.6
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 3 * keep
+    return tree
+
+
+@pytest.mark.parametrize("per_wave,most", [(8, 0), (8, 6), (5, 2), (3, 6), (2, 5), (1, 6)])
+@pytest.mark.parametrize("kind,fmt,softplus,fast", [("dense", "SH9", False, False), ("dense", "RGBA", True, False), ("thirds", "SG4", False, False),
+                                                    ("shell", "SH16", False, True), ("deep", "SH4", False, False), ("leaf", "SH25", False, True)])
+def test_rays_in_pieces_are_the_rays_from_end_to_end(gpu, oracle_mod, kind, fmt, softplus, fast, per_wave, most):
+    n = 301
+    gen = torch.Generator().manual_seed(7)
+    tree = scene(kind, fmt, gen)
+    rays = synth.sphere_rays(n, seed=8)
+    rays.dirs[::7] *= -1.0                              # (some look away)
+    rays.dirs[5] = torch.tensor([0.0, 0.0, 1.0])        # (and one along an axis)
+    opt = options(tree, step_size=1e-3, density_softplus=softplus, fast=fast)
+    dev, rs = on_gpu(tree, gpu), rays_spec(rays, gpu)
+    go, target = (torch.randn(n, 3, generator=gen) * 1e-2).to(gpu), torch.rand(n, 3, generator=gen).to(gpu)
+    plain, marked = dev._spec(), dev._spec()
+    marked.child_marks = C.mark_empty_leaves(plain, density_softplus=softplus)
+    marked.child_marks_softplus = softplus
+    slack = None
+    if not softplus:
+        ot = oracle_mod.Tree.from_n3tree(tree)
+        slack = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go.cpu(), want_slack=True)[1]
+
+    def passes(spec):
+        out, notes = C.volume_render_noted(spec, rs, opt, records_per_ray=256)
+        count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+        return (C.volume_render(spec, rs, opt), out, count, C.se_grad(spec, rs, target, opt)[0],
+                C.volume_render_backward_noted(spec, rs, opt, go, notes), C.volume_render_backward(spec, rs, opt, go))
+
+    for spec in (plain, marked):
+        want, got = run(END_TO_END, lambda: passes(spec)), run(cut(per_wave, most), lambda: passes(spec))
+        for what, a, b in zip(("picture", "noted picture", "notes", "colours"), got, want):
+            assert torch.equal(a, b), what
+        for what, a, b in zip(("from notes", "alone"), got[4:], want[4:]):
+            err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
+            assert ok, (what, err)
+    # room for the first chunk of a ray and little more: the others' notes are lost, and the gradient marches
+    want = run(END_TO_END, lambda: C.volume_render_backward(plain, rs, opt, go, workspace=False))
+
+    def short():
+        out, notes = C.volume_render_noted(plain, rs, opt, records_per_ray=16)
+        return out, C.volume_render_backward_noted(plain, rs, opt, go, notes)
+    out, grad = run(cut(per_wave, most), short)
+    assert torch.equal(out, run(END_TO_END, lambda: C.volume_render(plain, rs, opt)))
+    err, ok = grad_close(grad.cpu().numpy(), want.cpu().numpy(), slack=slack, what="lost notes")
+    assert ok, err
+
+
+@pytest.mark.parametrize("ndc", [False, True])
+def test_pictures_in_pieces_and_the_sizes_that_take_them(gpu, ndc):
+    """The sizes around which the launcher changes over, one picture and several; a captured pass, replayed."""
+    tree = synth.shell_tree(depth=6, data_format="SH4", n_spheres=6, seed=4)
+    if ndc:
+        tree.invradius.fill_(0.5)
+        tree.offset.fill_(0.5)
+    dev = on_gpu(tree, gpu)
+    spec = dev._spec()
+    poses = torch.stack(synth.orbit_poses(3, seed=2, radius=3.0))
+    if ndc:
+        poses = torch.cat([torch.eye(3).expand(3, 3, 3), torch.tensor([[0.1, 0.0, 0.2]]).expand(3, 3)[:, :, None]], dim=2)
+    for w, h, k in ((1, 1, 1), (64, 64, 1), (65, 63, 1), (91, 90, 1), (64, 64, 3), (128, 96, 1), (128, 97, 1)):
+        opt = options(tree, step_size=1e-3, ndc=svox.NDCConfig(w, h, 0.8 * w) if ndc else None)
+        cam = cam_spec(poses[:k].contiguous() if k > 1 else poses[0].contiguous(), w, h, 1.4 * w if not ndc else 0.8 * w, device=gpu)
+        f = C.volume_render_images if k > 1 else C.volume_render_image
+        want = run(END_TO_END, lambda: f(spec, cam, opt))
+        assert torch.equal(f(spec, cam, opt), want)
+        out, notes = C.volume_render_images_noted(spec, cam, opt)
+        assert torch.equal(out.reshape(want.shape), want)
+    rs = rays_spec(synth.sphere_rays(2000, seed=1), gpu)
+    opt = options(tree, step_size=1e-3)
+    want = run(END_TO_END, lambda: C.volume_render(spec, rs, opt))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        C.volume_render(spec, rs, opt)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = C.volume_render(spec, rs, opt)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(C.volume_render(spec, rs, opt), want)
