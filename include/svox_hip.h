@@ -134,7 +134,8 @@ const char* svox_status_string(int status);
  * of that kernel give up at the first look that finds nothing (so that a test can see what a give-up leaves
  * behind; every kernel still ends normally).  Bit 5: forward renders take the kernel that walks a ray in several pieces at
  * once, whatever their size (not with a weight accumulator), with as many rays to a wavefront as the last decimal digit of
- * flags >> 8 says (1 to 8; 0: they never take it), in 2^(the digits before it) pieces at most.  With any flag set they
+ * flags >> 8 says (1 to 8; 0: they never take it), in 2^(the digits before it) pieces at most (double precision, gradients
+ * too: two digits, 1 to 16 rays, and 2^2 pieces at least).  With any flag set they
  * do not take it otherwise.  The flags belong to the calling thread. */
 void svox_set_debug_flags(int flags);
 

@@ -419,10 +419,10 @@ int fast_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt) {
 // (group_kernels.h; 0 for RGBA), or -1: three colour channels of a basis size they are built for, cells that 32-bit
 // indices reach, no weight accumulator, and not more rays than kGroupMaxRays.
 //
-// kGroupMaxRays: with more rays than fill the chip the four lanes that walk one ray are work done four times over.
-// Dense 64^3 SH4 tree, gradient: 100 000 rays 1954 -> 1505 us, 600 000 rays 6958 -> 7900 us; a forward pass that only
-// walks (nothing shaded): 469 -> 478 and 1302 -> 1973 us.
-constexpr int64_t kGroupMaxRays = 1 << 17;
+// kGroupMaxRays: with more rays than fill the chip it only costs that the pieces of a ray overlap.  Dense 64^3 SH4 tree, gradient,
+// one ray per lane / pieces: 100 000 rays 1954 / 1214 us, 130 000 rays 2500 / 1550 us.  kGroupMaxPictureRays: beyond, a forward pass gives
+// a ray's four lanes one walk (four walks / one, us: 40 000 rays 322 / 334, 65 000 rays 474 / 380, 130 000 rays 785 / 660).
+constexpr int64_t kGroupMaxRays = 1 << 17, kGroupMaxPictureRays = 40960;
 
 int group_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays) {
     if ((g_debug_flags & 1) || tree->dtype != SVOX_F64 || tree->N != 2 || tree->weight_accum || n_rays > kGroupMaxRays ||
@@ -432,6 +432,41 @@ int group_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t 
     const int D = opt->basis_dim;
     if (D != 1 && D != 4 && D != 9 && D != 16 && D != 25) return -1;
     return tree->data_dim == 3 * D + 1 ? D : -1;
+}
+
+// Rays that a wavefront of those kernels is dealt, and log2 of the pieces a ray is walked in at most (at least 2).
+struct Cut {
+    int per_wave = 0, most = 6;
+};
+Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays) {
+    Cut c;
+    const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : tuning().cut;
+    if (forced > 0) {
+        c.per_wave = std::min(std::max(forced % 100, 1), kGroupRays);
+        c.most = std::min(std::max(forced / 100, 2), 6);
+        return c;
+    }
+    // As many pieces as still are some leaves long -- in a 16^3 grid (up to 16 384 cells) eight, to 64^3 twice as many for twice the
+    // resolution -- while the wavefronts have room on the GPU, fewer with more rays; what was measured beside it, us, forward pass and
+    // gradient of a dense tree, by the rays of a wavefront and the pieces (rays x pieces):
+    //   16^3   1 000 rays 8 x 8 39, 47   4 x 16 95, 100   16 x 4 42, 63     20 000 rays 16 x 4 53, 77   8 x 8 81, 101
+    //   32^3   5 000 rays 4 x 16 58, 93  8 x 8 59, 127    2 x 32 134, 182   20 000 rays 8 x 8 107, 229  4 x 16 182, 259
+    //   64^3   1 000 rays 2 x 32 46, 78  1 x 64 68, 79    4 x 16 55, 102    20 000 rays 4 x 16 175, 286 8 x 8 189, 405  2 x 32 291, 427
+    //   128^3  1 000 rays 1 x 64 65, 133 2 x 32 72, 144   4 x 16 99, 198    5 000 rays 4 x 16 112, 243  2 x 32 133, 252
+    const double cells = (double)tree->capacity * 8.0;
+    if (cells < 16384.0) {
+        c.per_wave = n_rays <= 8192 ? 8 : 16;
+        c.most = n_rays <= 8192 ? 3 : 2;
+    } else if (cells < 131072.0) {
+        c.per_wave = n_rays <= 8192 ? 4 : 8;
+        c.most = n_rays <= 8192 ? 4 : 3;
+    } else if (cells < 1048576.0) {
+        c.per_wave = n_rays <= 2560 ? 2 : 4;
+        c.most = 5;
+    } else {
+        c.per_wave = n_rays <= 1280 ? 1 : n_rays <= 2560 ? 2 : 4;
+    }
+    return c;
 }
 
 Lobes lobes_of(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt) {
@@ -620,10 +655,7 @@ constexpr bool is_image_source(const ImageSource<T>&) { return true; }
 template <typename T>
 constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 
-// How a forward pass cuts its rays into pieces (cut_kernel.h): rays dealt to a wavefront (0: it does not), log2 of a ray's pieces at most.
-struct Cut {
-    int per_wave = 0, most = 6;
-};
+// How a forward pass cuts its rays into pieces (cut_kernel.h); no rays dealt to a wavefront: it does not.
 // The pieces pay as long as they find the GPU idle: what each of them walks in vain -- the leaves until two walks agree -- is
 // as much as a fair part of it, and the more of them the shorter.  A tree is small (up to 32^3 leaves: rays of few leaves), large (from
 // 128^3, or the surface of 256^3, on) or between.  The launcher cannot know how many rays meet the cube, so the rule is drawn where a
@@ -709,7 +741,13 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            launch_group_forward(D, dim3(blocks_for(items, kGroupRays)), stream, make_tree<double>(tree), src, *opt, (double*)out);
+            if (items > kGroupMaxPictureRays && !(g_debug_flags & 32)) {
+                launch_shared_forward(D, dim3(blocks_for(items, kSharedRays)), stream, make_tree<double>(tree), src, *opt, (double*)out);
+                return;
+            }
+            const Cut cut = group_cut(tree, items);
+            launch_group_forward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt, (double*)out,
+                                 cut.per_wave, cut.most);
             return;
         }
     }
@@ -780,8 +818,9 @@ void launch_backward(const SvoxTreeSpec* tree, const Source& src, const SvoxRend
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            launch_group_backward(D, dim3(blocks_for(items, kGroupRays)), stream, make_tree<double>(tree), src, *opt,
-                                  (const double*)grad_out, (double*)grad_data);
+            const Cut cut = group_cut(tree, items);
+            launch_group_backward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt,
+                                  (const double*)grad_out, (double*)grad_data, cut.per_wave, cut.most);
             return;
         }
     }

@@ -126,3 +126,43 @@ def test_pictures_in_pieces_and_the_sizes_that_take_them(gpu, ndc):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         assert torch.equal(C.volume_render(spec, rs, opt), want)
+
+
+@pytest.mark.parametrize("per_wave,most", [(16, 2), (8, 3), (5, 6), (2, 5), (1, 6)])
+@pytest.mark.parametrize("kind,fmt,kw", [("dense", "SH9", {}), ("full", "SH4", {"density_softplus": True}), ("full", "SH1", {}), ("deep", "SH4", {}),
+                                         ("leaf", "RGBA", {}), ("dense", "SH4", {"fast": True, "min_comp": 1, "max_comp": 2})])
+def test_double_precision_rays_in_pieces(gpu, kind, fmt, kw, per_wave, most):
+    """Room for the lists of some rays from end to end, of none (every leaf of 64^3 has density), and of trees deeper than the integer
+    coordinates: the kernels with one ray per lane are the reference, bit for bit where the sums have one order."""
+    n = 333
+    gen = torch.Generator().manual_seed(9)
+    if kind == "full":
+        tree = svox.N3Tree(N=2, data_format=fmt, init_refine=5)
+        tree.data.data.normal_(generator=gen)
+        tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.2 + 0.01
+    elif kind == "deep":
+        tree = synth.deep_tree(27, data_format=fmt, seed=5)[0]
+    else:
+        tree = scene(kind, fmt, gen)
+    tree = tree.double()
+    rays = synth.sphere_rays(n, seed=8, dtype=torch.float64)
+    rays.dirs[::7] *= -1.0
+    opt = options(tree, step_size=1e-3, **kw)
+    spec, rs = on_gpu(tree, gpu)._spec(), rays_spec(rays, gpu)
+    go = torch.randn(n, 3, generator=gen, dtype=torch.float64).to(gpu)
+
+    def passes():
+        return C.volume_render(spec, rs, opt), C.volume_render_backward(spec, rs, opt, go)
+
+    want, got = run(1, passes), run(32 | (per_wave + 100 * most) << 8, passes)
+    assert torch.equal(got[0], want[0])
+    # (sums of at most 333 terms in another order: 333 * 2^-53 of their absolute sum each)
+    assert (got[1] - want[1]).abs().max() <= 1e-11 * want[1].abs().max()
+
+
+@pytest.mark.parametrize("n", [40960, 40961])
+def test_double_precision_batches_on_either_side_of_the_rule(gpu, n):
+    tree = synth.shell_tree(depth=5, n_spheres=5, data_format="SH4", seed=7).double()
+    rs = rays_spec(synth.sphere_rays(n, seed=3, dtype=torch.float64), gpu)
+    spec, opt = on_gpu(tree, gpu)._spec(), options(tree, step_size=1e-3)
+    assert torch.equal(C.volume_render(spec, rs, opt), run(1, lambda: C.volume_render(spec, rs, opt)))
