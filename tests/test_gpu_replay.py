@@ -30,16 +30,12 @@ def test_notes_of_every_number(gpu, oracle_mod, levels, keep, n, fmt):
     out, notes = C.volume_render_noted(dev._spec(), rs, opt, records_per_ray=256)
     assert notes is not None
     got = C.volume_render_backward_noted(dev._spec(), rs, opt, go.to(gpu), notes)
-    if n <= 1000:
-        ot = oracle_mod.Tree.from_n3tree(tree)
-        want = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go)
-    else:
-        C.set_debug_flags(1)
-        try:
-            want = C.volume_render_backward(dev._spec(), rs, opt, go.to(gpu)).cpu().numpy()
-        finally:
-            C.set_debug_flags(0)
-    err, ok = grad_close(got.cpu().numpy(), want)
+    # (70 001 rays add into the leaves of a 64^3 grid in the order the GPU happens to take them: the bare difference of two such sums
+    # is 5e-5 to 1.08e-4 from run to run, so large batches are held against the exact sum beyond the slack that any order has,
+    # sqrt(terms) * 2^-24 * sum |term| of every element)
+    ot = oracle_mod.Tree.from_n3tree(tree)
+    want, slack = oracle_mod.volume_render_backward(ot, rays.origins, rays.dirs, rays.viewdirs, opt, go, n_threads=8, want_slack=True)
+    err, ok = grad_close(got.cpu().numpy(), want, slack=slack if n > 1000 else None)
     assert ok, err
     target = torch.rand(n, 3, generator=gen).to(gpu)
     replayed, marched = C.se_grad(dev._spec(), rs, target, opt), C.se_grad(dev._spec(), rs, target, opt, workspace=False)
