@@ -176,6 +176,23 @@ struct BatchSource {
     }
 };
 
+// Rays of a batch that meet the cube, for noting passes (list_hits_kernel): item i is ray list[i]; without a list, those of the batch.
+// A pass of which only the device knows how many rays it has is launched in several shapes; each has items only if there are as many
+// as it is made for.
+struct ListedSource : BatchSource<float> {
+    const int32_t* list;
+    const unsigned long long* n_listed;
+    int64_t least, most;     // rays listed, for this launch to have any
+    __device__ __forceinline__ int64_t total() const {
+        const int64_t n = (int64_t)*n_listed;
+        return n < least || n > most ? 0 : list ? n : BatchSource<float>::total();
+    }
+    __device__ __forceinline__ int64_t fetch_item(int64_t i, const SvoxRenderOptions& opt, const float* offset,
+                                                  const float* scaling, float* origin, float* dir, float* vdir) const {
+        return BatchSource<float>::fetch_item(list ? (int64_t)list[i] : i, opt, offset, scaling, origin, dir, vdir);
+    }
+};
+
 __host__ __device__ inline int blocks16_of(int extent) { return (extent + 15) / 16; }
 
 // Which chunk of items the wavefront of block `b` (of gridDim.x) works on.  Workgroups are handed
@@ -866,6 +883,7 @@ struct ReplaySpace {
     uint32_t n_stocks;
     // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
     unsigned int* give_ups;
+    int32_t* list;         // room for a number per ray, behind the chunks (ListedSource), or nullptr
 };
 
 // whether the workspace carries the stamp this launch expects

@@ -10,4 +10,7 @@
 namespace svox {
 template struct MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, BatchSource<float>>;
 template struct MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, ImageSource<float>>;
+template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, ListedSource>::noting(
+    dim3, hipStream_t, const TreeDev<float>&, const ListedSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
+    const float*, bool, bool);
 }  // namespace svox

@@ -33,7 +33,7 @@ thread_local char g_error[512] = "";
 // Debug flags of the calling thread (svox_set_debug_flags): bit 0: always take the generic kernels; bit 1: small
 // batches run like large ones; bit 2: forward launches never take the two-wavefront kernel; bit 3: they always
 // do (where it applies); bit 4: the bounded waits of that kernel give up at once; bit 5: forward launches cut their rays, as bits 8 and
-// up say (pick_cut).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
+// up say (pick_cut); bit 6: noting passes list their rays (list_shapes).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
 thread_local int g_debug_flags = 0;
 
 // Launch-shape overrides for experiments, read from the environment once, when the first launch of the process
@@ -504,10 +504,11 @@ ReplaySpace no_notes() {
 // that the launch spreads over as many SIMDs as possible; with many, several chunks, which lets lanes
 // whose rays end early pick up new ones (measured on 1M random rays: forward best at 256 rays per
 // wavefront, backward -- two marches per ray, longer-lived lanes -- at 512).
+constexpr int64_t kRefillRays = 64 * 1024 * 8;
 int pick_per_wave(int64_t total_items, bool backward) {
     const int forced = tuning().per_wave;
     if (forced == 64 || forced == 128 || forced == 256 || forced == 512 || forced == 1024) return forced;
-    if (total_items < (int64_t)64 * 1024 * 8 && !(g_debug_flags & 2)) return 64;
+    if (total_items < kRefillRays && !(g_debug_flags & 2)) return 64;
     return backward ? 512 : 256;
 }
 
@@ -783,16 +784,23 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
 constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
+// (and, from kListRays rays on, where the rays' shared chunks are many beside it, in the place of the last of them: a number per ray.)
+constexpr int64_t kListRays = 1 << 17;
 bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, ReplaySpace* ws) {
     *ws = ReplaySpace{};
-    const int64_t chunks = workspace && n_slots > 0
-                               ? (workspace_bytes - kTailBytes - bitmap_bytes(n_slots)) / kChunkBytes : 0;
+    int64_t chunks = workspace && n_slots > 0
+                         ? (workspace_bytes - kTailBytes - bitmap_bytes(n_slots)) / kChunkBytes : 0;
     if (n_slots <= 0 || chunks < n_slots || chunks >= 0x7fffffffll || ((uintptr_t)workspace & 15u) != 0) return false;
     ws->base = (float2*)workspace;
+    ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
+    const int64_t list_chunks = (n_slots * 4 + kChunkBytes - 1) / kChunkBytes;
+    if ((n_slots >= kListRays || (g_debug_flags & 64)) && chunks - n_slots >= 16 * list_chunks) {
+        chunks -= list_chunks;
+        ws->list = (int32_t*)((char*)workspace + chunks * kChunkBytes);
+    }
     ws->first_shared = n_slots;
     ws->n_chunks = chunks;
     ws->n_stocks = (uint32_t)((chunks - n_slots + kChunkStock - 1) / kChunkStock);
-    ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
     ws->stamp_at = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStampOffset);
     ws->stocks_taken = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStockCounterOffset);
     return true;
@@ -845,6 +853,73 @@ ImageSource<T> noting_shape(const ImageSource<T>& s) { return s; }
 // beforehand.  A launch that does not fill the GPU runs on two wavefronts per 64 rays.  out may be
 // nullptr (notes only); grad_out, if given, is the gradient of the picture the backward pass will be
 // called with: the notes' heads then also carry the sum of that pass's first march.
+// The rays of a batch that meet the cube, in the order they come in block by block (the blocks as they get there); the others are
+// answered as a noting pass answers them.  Reads 24 bytes a ray: 200 000 rays 4 us, 1 Mi rays 9.
+constexpr int kListThreads = 1024;
+__global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> tr, BatchSource<float> src, SvoxRenderOptions opt,
+                                                                        float* __restrict__ out, ReplaySpace ws,
+                                                                        unsigned long long* __restrict__ n_listed) {
+    __shared__ int32_t hits[kListThreads / kMarchThreads];
+    __shared__ unsigned long long first;
+    float offset[3], scaling[3], origin[3], dir[3], vdir[3];
+    load_transform(tr, offset, scaling);
+    const int wave = threadIdx.x / kMarchThreads, lane = threadIdx.x & (kMarchThreads - 1);
+    src.n_waves = 0;
+    const int64_t slot = src.fetch_item(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
+    RayState<float> r;
+    const bool hit = slot >= 0 && setup_ray(r, origin, dir, scaling);
+    if (slot >= 0 && !hit) {
+        if (out) {
+            out[slot * 3] = opt.background_brightness;
+            out[slot * 3 + 1] = opt.background_brightness;
+            out[slot * 3 + 2] = opt.background_brightness;
+        }
+        NoteTaker::missed(ws, slot);
+    }
+    const unsigned long long m = __ballot(hit);
+    if (lane == 0) hits[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < kListThreads / kMarchThreads; ++i) {
+        before += i < wave ? hits[i] : 0;
+        all += hits[i];
+    }
+    if (threadIdx.x == 0) first = all > 0 ? atomicAdd(n_listed, (unsigned long long)all) : 0ull;
+    __syncthreads();
+    if (hit) ws.list[first + before + rank_in(m)] = (int32_t)slot;
+}
+
+// The shapes of a noting pass whose rays are listed first (ListedSource): up to `two` rays that meet the cube two wavefronts per tile,
+// up to `one` one; beyond -- most of the batch does -- the batch as it is.  Only where the batch, if all of it met the cube, would not
+// take two wavefronts anyway (the same rays listed or not: 256^3 shell, 100 000 rays 254 / 255 us, 200 000 rays 283 / 292), and not on
+// trees to 32^3, whose marches are short beside the listing (16^3 RGBA, 300 000 rays that all hit 181 / 192).  us, batch as it is / listed,
+// the noting march, the gradient by itself, the squared error; 18 % of the rays of a shell hit:
+//   256^3 shell SH9   200 003 rays 339, 483, 577 / 290, 413, 524   300 000 rays 405, 573, 665 / 317, 450, 568   500 000 rays 566, 794, 921 / 332, 518, 680
+//   512^3 shell SH16  170 000 rays 452, 820 / 383, 723   500 000 rays 775, 1208 / 457, 870   1 048 576 rays 749, 1332 / 708, 1313
+//   512^3 shell SH25  400 000 rays 727, 1389 / 453, 1025    256^3 shell SH4 700 000 rays 458, 632, 741 / 344, 505, 632
+// Where all of them hit, the listing and the launches without rays are lost: 256^3 shell SH9 200 003 rays 563, 1072, 1469 / 577, 1084, 1492,
+// 500 000 rays 1102, 2183, 3108 / 1127, 2205, 3121, 64^3 SH9 200 000 rays 648, 1832, 2840 / 667, 1835, 2846.
+struct ListShapes {
+    bool any = false;
+    int64_t two = 0, one = 0;
+};
+ListShapes list_shapes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, unsigned at_once) {
+    ListShapes s;
+    if (g_debug_flags & 64) {
+        s.any = true;
+        s.two = (g_debug_flags >> 8 & 255) * kMarchThreads;
+        s.one = (g_debug_flags >> 16) * kMarchThreads;
+        return s;
+    }
+    const Tuning& t = tuning();
+    if (g_debug_flags != 0 || t.per_wave > 0 || t.split_forward >= 0 || t.split_blocks >= 0) return s;
+    s.two = (int64_t)(use_split_forward(tree, at_once, false, opt, false, at_once) ? at_once : std::min(at_once, 2048u)) * kMarchThreads;
+    s.one = std::max(std::min(kRefillRays - 1, n_rays - n_rays / 4), s.two);
+    s.any = n_rays > s.two && (double)tree->capacity * tree->N * tree->N * tree->N >= 131072.0;
+    return s;
+}
+
 template <class Source>
 int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, void* out,
                  void* workspace, int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp,
@@ -855,7 +930,7 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     ReplaySpace ws;
     if (D < 0 || !carve_workspace(workspace, workspace_bytes, n_slots, &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "notes asked for where they cannot be taken");
-    const int rc = zero_fill(ws.stocks_taken, 16, stream);
+    const int rc = zero_fill(ws.stocks_taken, 32, stream);
     if (rc) return rc;
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
@@ -870,6 +945,34 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     const bool refill = src.per_wave > kMarchThreads;
     unsigned at_once = 0;
     SVOX_DISPATCH_OCTREE(D, at_once = MarchLaunch<P, Source>::split_tiles_at_once(true, grad_out != nullptr));
+    if constexpr (!is_image_source(Source())) {
+        // (most of a batch often misses the cube, and the lanes of the rays that do idle; which shape suits those that meet it, the
+        // device decides: every launch but one has no rays)
+        const ListShapes shapes = list_shapes(tree, opt, src.rays.n_rays, at_once);
+        if (ws.list && shapes.any) {
+            unsigned long long* const n_listed = ws.stocks_taken + 2;
+            hipLaunchKernelGGL(list_hits_kernel, dim3(blocks_for(src.rays.n_rays, kListThreads)), dim3(kListThreads), 0, stream,
+                               march_tree(tree, opt), src, *opt, (float*)out, ws, n_listed);
+            auto launch = [&](const Source& s, const int32_t* list, int64_t least, int64_t most, bool two, bool refilled) {
+                ListedSource listed;
+                (Source&)listed = s;
+                listed.list = list;
+                listed.n_listed = n_listed;
+                listed.least = least;
+                listed.most = most;
+                const int64_t items = list ? std::min(most, s.rays.n_rays) : s.rays.n_rays;
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, ListedSource>::noting(
+                                            dim3(blocks_for(items, s.per_wave)), stream, march_tree(tree, opt), listed, *opt, (float*)out,
+                                            ws, (const float*)grad_out, (const float*)color_ref, two, refilled));
+            };
+            Source tiles = src;
+            tiles.per_wave = kMarchThreads;
+            if (shapes.two > 0) launch(tiles, ws.list, 0, shapes.two, true, false);
+            launch(tiles, ws.list, shapes.two + 1, shapes.one, false, false);
+            if (src.rays.n_rays > shapes.one) launch(dealt, nullptr, shapes.one + 1, INT64_MAX, false, refill);
+            return SVOX_OK;
+        }
+    }
     const bool split = !refill && use_split_forward(tree, blocks, is_image_source(src), opt, false, at_once);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
                                                            (float*)out, ws, (const float*)grad_out,

@@ -1,0 +1,87 @@
+"""Noting passes that list the rays of a batch which meet the tree: two wavefronts per tile, one, or the batch as it is, whichever the
+number of them asks for on the device.
+
+Bar: pictures, noted colours and the number of notes of every ray equal to those of the pass that takes the batch as it is, bit for bit;
+gradients the same terms in another order.
+"""
+import pytest
+import torch
+
+from svox_amd import csrc as C
+from svox_amd import synth
+from util import grad_close, on_gpu, options, rays_spec
+
+pytestmark = pytest.mark.gpu
+
+
+def listed(two, one):
+    """flags: up to `two` * 64 listed rays on two wavefronts per tile, up to `one` * 64 on one"""
+    return 64 | two << 8 | one << 16
+
+
+def run(flags, f):
+    C.set_debug_flags(flags)
+    try:
+        return f()
+    finally:
+        C.set_debug_flags(0)
+
+
+# how many rays meet the tree, of 2 500: none, one, a tile and one more, all
+@pytest.mark.parametrize("hits", [0, 1, 64, 65, 1025, 2500])
+@pytest.mark.parametrize("two,one,more", [(255, 256, 0), (16, 32, 0), (1, 16, 2), (0, 40, 0), (1, 1, 2)])
+def test_listed_rays(gpu, oracle_mod, hits, two, one, more):
+    n = 2500
+    tree = synth.shell_tree(depth=6, data_format="SH9", n_spheres=6, seed=4)
+    gen = torch.Generator().manual_seed(hits)
+    rays = synth.sphere_rays(n, seed=8)
+    away = torch.randperm(n, generator=gen)[hits:]
+    rays.dirs[away] = rays.origins[away] - 0.5          # (outwards)
+    opt = options(tree, step_size=1e-3)
+    dev, rs = on_gpu(tree, gpu), rays_spec(rays, gpu)
+    spec = dev._spec()
+    go, target = (torch.randn(n, 3, generator=gen) * 1e-2).to(gpu), torch.rand(n, 3, generator=gen).to(gpu)
+    slack = oracle_mod.volume_render_backward(oracle_mod.Tree.from_n3tree(tree), rays.origins, rays.dirs, rays.viewdirs, opt, go.cpu(),
+                                              want_slack=True)[1]
+
+    def passes():
+        out, notes = C.volume_render_noted(spec, rs, opt, records_per_ray=64)
+        count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+        return (out, count, C.se_grad(spec, rs, target, opt)[0], C.volume_render_backward_noted(spec, rs, opt, go, notes),
+                C.volume_render_backward(spec, rs, opt, go))
+
+    want, got = run(4, passes), run(listed(two, one) | more, passes)
+    for what, a, b in zip(("picture", "notes", "colours"), got, want):
+        assert torch.equal(a, b), what
+    for what, a, b in zip(("from notes", "alone"), got[3:], want[3:]):
+        err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
+        assert ok, (what, err)
+    # no room for the list beside the notes: the batch as it is
+    out = run(listed(two, one) | more, lambda: C.volume_render_noted(spec, rs, opt, records_per_ray=16))[0]
+    assert torch.equal(out, want[0])
+
+
+def test_a_captured_pass_lists_anew_in_every_replay(gpu):
+    n = 200001
+    tree = synth.shell_tree(depth=7, data_format="SH1", n_spheres=6, seed=4)
+    dev, rs = on_gpu(tree, gpu), rays_spec(synth.sphere_rays(n, seed=8), gpu)
+    spec, opt = dev._spec(), options(tree, step_size=1e-3)
+    turned = rs.dirs.clone()
+    turned[::3] *= -1.0
+    kept = rs.dirs.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        C.volume_render_noted(spec, rs, opt)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, notes = C.volume_render_noted(spec, rs, opt)
+    for dirs in (kept, turned, turned, kept):
+        rs.dirs.copy_(dirs)
+        want = run(4, lambda: C.volume_render_noted(spec, rs, opt)[0])
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(C.volume_render_noted(spec, rs, opt)[0], want)
