@@ -660,22 +660,22 @@ constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 // The pieces pay as long as they find the GPU idle: what each of them walks in vain -- the leaves until two walks agree -- is
 // as much as a fair part of it, and the more of them the shorter.  A tree is small (up to 32^3 leaves: rays of few leaves), large (from
 // 128^3, or the surface of 256^3, on) or between.  The launcher cannot know how many rays meet the cube, so the rule is drawn where a
-// launch of rays that all do gains nothing more.  us, forward pass with notes and without, from 4 096 rays on for both choices,
-// uncut / cut, SH4 to SH16 trees, rays that all meet the cube where it is dense, 18 % of them where it is a shell:
-//   16^3      1 000 rays 43, 40 / 28, 22    4 000 42, 39 / 31, 25    8 000 42, 40 / 34, 26    16 000 43, 40 / 63, 44
-//   32^3      1 000 rays 84, 81 / 36, 29    4 000 81, 79 / 41, 32    8 000 83, 78 / 48, 42    16 000 88, 80 / 94, 69
-//   64^3      1 000 rays 165, 160 / 52, 56  4 000 204, 199 / 68, 67  12 000 202, 197 / 165, 123  16 000 202, 197 / 205, 144
-//   128^3     1 000 rays 418, 412 / 72, 63  4 000 413, 410 / 145, 135  8 000 416, 412 / 255, 184  12 000 424, 418 / 303, 247
-//   64^3 shell   1 000 rays 75, 73 / 38, 31    4 000 83, 80 / 41, 34    16 000 90, 87 / 81, 57
-//   256^3 shell  1 000 rays 149, 145 / 50, 43  4 000 169, 166 / 109, 108  8 000 169, 165 / 89, 72  16 000 196, 189 / 158, 120
-//   512^3 shell  1 000 rays 170, 170 / 67, 72  4 000 224, 225 / 163, 165  8 000 224, 223 / 110, 110  16 000 257, 252 / 225, 186
-// and square pictures of 64 / 90 / 128 pixels a side (4 096, 8 100, 16 384):
-//   16^3   27, 23 / 22, 18      28, 23 / 25, 21       27, 23 / 40, 31
-//   64^3   89, 83 / 37, 30      127, 113 / 44, 31     124, 111 / 75, 52
-//   128^3  206, 192 / 59, 52    242, 237 / 96, 49     237, 231 / 146, 93
-//   512^3 shell  177, 115 / 59, 44  259, 188 / 61, 49  288, 186 / 114, 78
-//   NDC, every ray in the tree, 256^3 and 512^3  133, 86 / 108, 49  151, 114 / 172, 79  146, 117 / 239, 118;
-//                                                227, 129 / 225, 83  245, 158 / 335, 116  243, 156 / 447, 185
+// launch of rays that all do gains nothing more.  us, march with notes and without, from end to end / in pieces, rays that all hit:
+//   16^3 SH4     1 000 rays 43, 40 / 28, 22    4 000 42, 39 / 31, 25    8 000 42, 40 / 34, 26    16 000 43, 40 / 63, 44
+//   32^3 SH9     1 000 rays 84, 81 / 36, 29    4 000 81, 79 / 41, 32    8 000 83, 78 / 48, 42    16 000 88, 80 / 94, 69
+//   64^3 SH9     1 000 rays 165, 160 / 47, 39  4 000 204, 199 / 68, 67  12 000 202, 197 / 165, 123  16 000 202, 197 / 205, 144
+//   128^3 SH9    1 000 rays 418, 412 / 72, 63  4 000 413, 410 / 145, 135  8 000 416, 412 / 255, 184  12 000 424, 418 / 303, 247
+//   shells  128^3 SH4   1 000 rays 153, 154 / 50, 58   4 000 154, 153 / 101, 86   8 000 192, 192 / 177, 152  12 000 193, 194 / 227, 180
+//           256^3 SH9   1 000 rays 196, 193 / 60, 55   4 000 261, 256 / 169, 121  8 000 311, 308 / 270, 199  12 000 271, 270 / 334, 255
+//           512^3 SH16  1 000 rays 235, 235 / 99, 108  4 000 332, 333 / 209, 180  8 000 349, 350 / 351, 270  12 000 332, 332 / 436, 365
+// 18 % of the rays hit: 64^3 shell 4 000 rays 83, 80 / 42, 35; 256^3 4 000 169, 166 / 63, 57, 8 000 169, 165 / 89, 72; 512^3 4 000 224, 225 / 97, 108,
+// 8 000 224, 223 / 110, 110.  With the shifted softplus, where every leaf is listed and rays end behind what they met (kOpaqueLight):
+// 32^3 4 000 rays 101, 85 / 59, 54, 12 000 122, 91 / 146, 102; 128^3 4 000 473, 442 / 315, 277, 12 000 499, 463 / 994, 495; 256^3 shell 4 000 75, 70 /
+// 63, 49, 8 000 78, 73 / 92, 53, 12 000 78, 74 / 119, 75; 512^3 shell 4 000 78, 76 / 76, 62.
+// Square pictures of 64 and 90 pixels a side (4 096, 8 100):
+//   16^3   27, 23 / 22, 18      28, 23 / 25, 21       64^3   89, 83 / 37, 30      127, 113 / 44, 31
+//   128^3  206, 192 / 59, 52    242, 237 / 96, 49     512^3 shell  177, 115 / 59, 44  259, 188 / 61, 49
+//   NDC, every ray in the tree, 256^3 and 512^3  133, 86 / 108, 49  151, 114 / 172, 79;  227, 129 / 225, 83  245, 158 / 335, 116
 Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRenderOptions* opt, bool noted) {
     const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : g_debug_flags == 0 ? tuning().cut : 0;
     Cut c;
@@ -685,10 +685,12 @@ Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRend
         return c;
     }
     const double cells = (double)tree->capacity * tree->N * tree->N * tree->N;
-    const bool small = cells < 65536.0, large = cells >= 1048576.0;
+    const bool small = cells < 65536.0, large = cells >= 1048576.0, grid = like_complete_octree(tree);
+    int64_t limit = small ? 8192 : grid ? 12288 : image ? 9216 : noted ? 7168 : 8192;   // (of a picture: in blocks of 16 x 16)
+    if (opt->density_softplus) limit = noted || small ? 4096 : 8192;
     if (image && opt->ndc_width > 0) {
         if (items <= (noted ? 4096 : 8192)) c.per_wave = small ? 8 : 4;
-    } else if (items <= (small ? 8192 : 12288)) {
+    } else if (items <= limit) {
         if (image) {
             // (most pixels of a picture miss: a wavefront finds one ray or two among four, or eight)
             c.per_wave = large ? 4 : 8;
@@ -696,9 +698,9 @@ Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRend
         } else if (small) {
             c.per_wave = items <= 4096 ? 4 : 8;
         } else if (large) {
-            c.per_wave = items <= 1536 ? 1 : items <= 8192 || !noted ? 2 : 4;
+            c.per_wave = items <= (grid ? 1536 : 4096) ? 1 : items <= 8192 || !noted ? 2 : 4;
         } else {
-            c.per_wave = 4;
+            c.per_wave = items <= (grid ? 2048 : 4096) ? 2 : 4;
         }
     }
     return c;
