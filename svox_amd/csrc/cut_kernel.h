@@ -26,7 +26,6 @@ constexpr int cut_listed(bool noted) { return noted ? 16 : 12; }
 constexpr int kCutTurns = kQueue; // of the walk, between looks at the densities of the leaves found
 constexpr int kCutHeads = 8;      // samples of a piece that the piece before can go on from
 constexpr int kCutMostRays = 8;   // of a wavefront
-constexpr int kCutStock = 8;      // chunks a wavefront takes at a time, at least
 
 // n chunks from those that all rays share, one after the other: the number of the first.  The counter of the stocks handed out is
 // kept in step with the one of chunks, beside it, that they are taken from here.
@@ -167,7 +166,6 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     bool painted = kNoted && out == nullptr;
     NoteTaker notes;
     March1Sum sum1;
-    int64_t shared_next = 0, shared_end = 0;
     if constexpr (kNoted) notes.begin(ws, active ? slot : 0);
     int64_t chunk = active ? slot : 0;  // the one its last note is in
     if constexpr (kNoted && kGrad) sum1.begin(grad_out, active ? slot : 0);
@@ -383,18 +381,15 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
             }
             const int all = __builtin_amdgcn_readlane(sum, kMarchThreads - 1);
             if (all > 0) {
-                // (from the wavefront's stock: waves of few rays take small ones)
-                if (shared_next + all > shared_end) {
-                    const int want = all > kCutStock ? all : kCutStock;
-                    unsigned long long t = 0;
-                    if (lane == 0) t = take_chunks(ws, want);
-                    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)t);
-                    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(t >> 32));
-                    shared_next = ws.first_shared + (int64_t)(((unsigned long long)hi << 32) | lo);
-                    shared_end = shared_next + want;
-                }
+                // (as many as there are notes for, no stock: a wavefront of one ray would leave most of it unused, and the notes of
+                // others that find no room cost far more: 1 000 rays, 128^3 SH9, gradient from notes 143 us, with stocks of 8 1240)
+                unsigned long long t = 0;
+                if (lane == 0) t = take_chunks(ws, all);
+                const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)t);
+                const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(t >> 32));
+                const int64_t first_new = ws.first_shared + (int64_t)(((unsigned long long)hi << 32) | lo);
                 if (more > 0) {
-                    const int64_t mine = shared_next + sum - more;
+                    const int64_t mine = first_new + sum - more;
                     if (mine + more > ws.n_chunks) {
                         notes.lost = true;
                     } else {
@@ -404,7 +399,6 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                         ray_more[ray] = (int32_t)mine;
                     }
                 }
-                shared_next += all;
             }
             if (hit && piece == 0) {
                 ray_noted[ray] = before;

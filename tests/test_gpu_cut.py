@@ -77,6 +77,10 @@ def test_rays_in_pieces_are_the_rays_from_end_to_end(gpu, oracle_mod, kind, fmt,
         for what, a, b in zip(("from notes", "alone"), got[4:], want[4:]):
             err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
             assert ok, (what, err)
+    # room for as many chunks of 15 notes as the rays need, beside the first of each: none are lost
+    chunks = -(-int(((want[2] - 1).clamp(min=0) // 15).sum()) // n) + 1
+    notes = run(cut(per_wave, most), lambda: C.volume_render_noted(plain, rs, opt, records_per_ray=15 * chunks))[1]
+    assert torch.equal(notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91], want[2])
     # room for the first chunk of a ray and little more: the others' notes are lost, and the gradient marches
     want = run(END_TO_END, lambda: C.volume_render_backward(plain, rs, opt, go, workspace=False))
 
