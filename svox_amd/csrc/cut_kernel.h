@@ -76,6 +76,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     constexpr float kUnknown = -1.0f;
     const float kNone = __int_as_float(0x7f800000);
     if constexpr (kNoted) {
+        if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
         if (blockIdx.x == 0 && threadIdx.x < kStampWords) ws.stamp_at[threadIdx.x] = ws.stamp[threadIdx.x];
     }
     const int lane = threadIdx.x;
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     bool hit = false;
     {
         float origin[3], dir[3], vdir[3];
-        const int64_t item = (int64_t)lane * gridDim.x + blockIdx.x;
+        const int64_t item = (int64_t)lane * (kNoted ? ws.march_blocks : gridDim.x) + blockIdx.x;
         if (lane < per_wave && item < src.total()) slot = src.fetch_item(item, opt, offset, scaling, origin, dir, vdir);
         if (slot >= 0) hit = setup_ray(r, origin, dir, scaling);
         if (slot >= 0 && !hit) {

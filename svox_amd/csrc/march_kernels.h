@@ -884,7 +884,28 @@ struct ReplaySpace {
     // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
     unsigned int* give_ups;
     int32_t* list;         // room for a number per ray, behind the chunks (ListedSource), or nullptr
+    // a noting launch: the blocks that march; those beyond clear these arrays of clear_words words each
+    uint32_t march_blocks;
+    uint32_t* clear_at[2];
+    int64_t clear_words;
 };
+
+// The arrays a gradient is going to be added to are cleared by further blocks of the launch that takes the notes for it: that one waits
+// for the chains of its longest rays, with the way to memory all but idle, and the blocks behind its last tile fill the places of those
+// that have ended.  (Two arrays of 172 MB, 200 003 rays: the squared error 524 us, 471 with them cleared on the way.)  Written past L2, which holds what the rays read.
+constexpr int64_t kClearWords = 16384;   // a block's share of an array
+static __device__ __forceinline__ void clear_share(const ReplaySpace& ws) {
+    typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+    const int64_t from = (int64_t)(blockIdx.x - ws.march_blocks) * kClearWords;
+    const int64_t n = ws.clear_words - from < kClearWords ? ws.clear_words - from : kClearWords;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (!ws.clear_at[k]) continue;
+        uint32_t* const at = ws.clear_at[k] + from;
+        for (int64_t i = threadIdx.x; i < n / 4; i += blockDim.x) __builtin_nontemporal_store(Words4{0, 0, 0, 0}, (Words4*)at + i);
+        for (int64_t i = n / 4 * 4 + threadIdx.x; i < n; i += blockDim.x) at[i] = 0;
+    }
+}
 
 // whether the workspace carries the stamp this launch expects
 __device__ __forceinline__ bool stamp_matches(const ReplaySpace& ws) {
@@ -1107,6 +1128,9 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
+    if constexpr (kNoted) {
+        if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
+    }
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
     load_transform(tr, offset, scaling);
@@ -1115,7 +1139,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
     const float step = opt.step_size, sigma_thresh = opt.sigma_thresh, stop_thresh = opt.stop_thresh;
 
-    int64_t next = chunk_of_block(blockIdx.x, gridDim.x, src.xcd_group) * (int64_t)src.per_wave;
+    int64_t next = chunk_of_block(blockIdx.x, kNoted ? ws.march_blocks : gridDim.x, src.xcd_group) * (int64_t)src.per_wave;
     const int64_t total = src.total();
     const int64_t end = next + src.per_wave < total ? next + src.per_wave : total;
 
@@ -1864,6 +1888,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ SplitBox box;
     if constexpr (kNoted) {
+        if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
         if (blockIdx.x == 0 && threadIdx.x < kStampWords) ws.stamp_at[threadIdx.x] = ws.stamp[threadIdx.x];
     }
     const int lane = threadIdx.x & (kMarchThreads - 1);
@@ -1876,7 +1901,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     const float step = opt.step_size, sigma_thresh = opt.sigma_thresh, stop_thresh = opt.stop_thresh;
     const int spin_limit = ws.spin_limit > 0 ? ws.spin_limit : kSpinLimit;
 
-    const int64_t item = chunk_of_block(blockIdx.x, gridDim.x, src.xcd_group) * (int64_t)kMarchThreads + lane;
+    const int64_t item = chunk_of_block(blockIdx.x, kNoted ? ws.march_blocks : gridDim.x, src.xcd_group) * (int64_t)kMarchThreads + lane;
     RayState<float> r;
     int64_t slot = -1;
     bool active = false;

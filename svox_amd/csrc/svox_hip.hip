@@ -922,10 +922,18 @@ ListShapes list_shapes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, i
     return s;
 }
 
+// What a noting launch clears on the way (clear_share): up to two arrays of so many bytes.
+struct ClearWork {
+    void* at[2] = {nullptr, nullptr};
+    int64_t bytes = 0;
+};
+constexpr int64_t kMostCleared = kClearWords * 4 * (1 << 24);   // (a launch has fewer than 2^32 threads)
+
 template <class Source>
 int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, void* out,
                  void* workspace, int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp,
-                 hipStream_t stream, const void* grad_out = nullptr, const void* color_ref = nullptr) {
+                 hipStream_t stream, const void* grad_out = nullptr, const void* color_ref = nullptr,
+                 const ClearWork& clear = ClearWork()) {
     const int D = fast_basis(tree, opt);
     const unsigned blocks = blocks_for(total_items_of(src), src.per_wave);
     const Source dealt = dealt_out(src, blocks);
@@ -937,9 +945,18 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
     ws.give_ups = give_up_counter();
+    // (the first launch clears what is to be cleared)
+    ws.clear_at[0] = (uint32_t*)clear.at[0];
+    ws.clear_at[1] = (uint32_t*)clear.at[1];
+    ws.clear_words = clear.bytes / 4;
+    auto with_clearing = [&](unsigned march) {
+        ws.march_blocks = march;
+        return dim3(march + (unsigned)((ws.clear_words + kClearWords - 1) / kClearWords));
+    };
     const Cut cut = pick_cut(tree, total_items_of(src), is_image_source(src), opt, true);
     if (cut.per_wave > 0) {
-        SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(dim3(blocks_for(total_items_of(src), cut.per_wave)), stream,
+        const dim3 grid = with_clearing(blocks_for(total_items_of(src), cut.per_wave));
+        SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(grid, stream,
                                                             march_tree(tree, opt), src, *opt, (float*)out, ws, true,
                                                             (const float*)grad_out, (const float*)color_ref, cut.per_wave, cut.most));
         return SVOX_OK;
@@ -963,20 +980,24 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
                 listed.least = least;
                 listed.most = most;
                 const int64_t items = list ? std::min(most, s.rays.n_rays) : s.rays.n_rays;
+                const dim3 grid = with_clearing(blocks_for(items, s.per_wave));
                 SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, ListedSource>::noting(
-                                            dim3(blocks_for(items, s.per_wave)), stream, march_tree(tree, opt), listed, *opt, (float*)out,
+                                            grid, stream, march_tree(tree, opt), listed, *opt, (float*)out,
                                             ws, (const float*)grad_out, (const float*)color_ref, two, refilled));
+                ws.clear_words = 0;
             };
             Source tiles = src;
             tiles.per_wave = kMarchThreads;
             if (shapes.two > 0) launch(tiles, ws.list, 0, shapes.two, true, false);
-            launch(tiles, ws.list, shapes.two + 1, shapes.one, false, false);
-            if (src.rays.n_rays > shapes.one) launch(dealt, nullptr, shapes.one + 1, INT64_MAX, false, refill);
+            if (shapes.one > shapes.two) launch(tiles, ws.list, shapes.two + 1, shapes.one, false, false);
+            const int64_t listed = std::max(shapes.one, shapes.two);
+            if (src.rays.n_rays > listed) launch(dealt, nullptr, listed + 1, INT64_MAX, false, refill);
             return SVOX_OK;
         }
     }
     const bool split = !refill && use_split_forward(tree, blocks, is_image_source(src), opt, false, at_once);
-    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
+    const dim3 grid = with_clearing(blocks);
+    SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(grid, stream, march_tree(tree, opt), dealt, *opt,
                                                            (float*)out, ws, (const float*)grad_out,
                                                            (const float*)color_ref, split, refill));
     return SVOX_OK;
@@ -1013,11 +1034,12 @@ void launch_se_grad(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
 
 // shared argument checks and zero-fills of the two squared-error entry points
 int se_grad_prepare(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, void* grad, void* hess, int* od,
-                    hipStream_t stream) {
+                    hipStream_t stream, bool fill = true) {
     int rc = check_render(tree, opt, od);
     if (rc) return rc;
     if (*od > 4) return fail(SVOX_ERR_BAD_SHAPE, "Tree's output dim cannot be > 4 for se_grad");
     if (!grad || !hess) return fail(SVOX_ERR_NULL_POINTER, "grad_out / hessdiag_out is NULL");
+    if (!fill) return SVOX_OK;
     rc = zero_fill(grad, data_bytes(tree), stream);
     if (rc) return rc;
     return zero_fill(hess, data_bytes(tree), stream);
@@ -1096,6 +1118,17 @@ SvoxRenderOptions without_thresholds(const SvoxRenderOptions* opt) {
     return o;
 }
 
+// Whether the arrays of a gradient are cleared by the launch that takes its notes: aligned as clear_share stores, not more than a
+// launch has blocks for, and beside a march that leaves the memory room: a gigabyte and more beside one of half a million rays is
+// cleared no faster than before it, and slows it.  us, apart / on the way, the squared error of a 256^3 SH9 shell (345 MB): 20 000 rays 343 / 294, 100 000
+// rays 409 / 360, 200 003 rays 524 / 471, 300 000 rays 568 / 526, 500 000 rays 680 / 655; the gradient by itself of a 512^3 SH16 shell (1.2 GB): 170 000 rays
+// 723 / 631, 300 000 rays 778 / 750, 500 000 rays 870 / 877, 700 000 rays 1129 / 1145; SH25 (1.9 GB) 400 000 rays 1024 / 1049.
+constexpr int64_t kClearBeside = 512ll << 20, kClearRays = 1 << 18;
+bool clears_on_the_way(const SvoxTreeSpec* tree, int64_t n_rays, const void* a, const void* b = nullptr) {
+    return ((uintptr_t)a & 15u) == 0 && ((uintptr_t)b & 15u) == 0 && data_bytes(tree) <= kMostCleared &&
+           (n_rays <= kClearRays || data_bytes(tree) * (b ? 2 : 1) <= kClearBeside);
+}
+
 // The backward pass of a call that brings a workspace but no notes: one noting march without a picture
 // (thresholds play no part in the backward pass, rt_kernel.cu:377, 441), then backward_from_notes.  The
 // reference's two marches per ray become one walk of the tree and one pass over 24 bytes per leaf with
@@ -1104,15 +1137,26 @@ SvoxRenderOptions without_thresholds(const SvoxRenderOptions* opt) {
 template <class Source>
 int backward_by_noting(const SvoxTreeSpec* tree, const Source& all, const Source& rest, const SvoxRenderOptions* opt,
                        const void* grad_output, void* grad_data_out, void* workspace, int64_t workspace_bytes,
-                       int64_t n_slots, NoteStamp stamp, hipStream_t stream) {
+                       int64_t n_slots, NoteStamp stamp, bool accumulate, hipStream_t stream) {
     SvoxTreeSpec quiet = *tree;
     quiet.weight_accum = nullptr;   // (the backward pass accumulates no weights)
     const SvoxRenderOptions plain = without_thresholds(opt);
     if (!noted_ok(&quiet, &plain, n_slots, workspace, workspace_bytes)) return 1;
     // (the notes belong to this call alone: the stamp carries its gradient buffer too)
     stamp.word[0] ^= (unsigned long long)(uintptr_t)grad_output;
-    int rc = launch_noted(&quiet, noting_shape(all), &plain, nullptr, workspace, workspace_bytes, n_slots, stamp, stream,
-                          grad_output);
+    ClearWork clear;
+    int rc = SVOX_OK;
+    if (!accumulate) {
+        if (clears_on_the_way(tree, n_slots, grad_data_out)) {
+            clear.at[0] = grad_data_out;
+            clear.bytes = data_bytes(tree);
+        } else {
+            rc = zero_fill(grad_data_out, data_bytes(tree), stream);
+        }
+    }
+    if (rc) return rc;
+    rc = launch_noted(&quiet, noting_shape(all), &plain, nullptr, workspace, workspace_bytes, n_slots, stamp, stream,
+                      grad_output, nullptr, clear);
     if (rc) return rc;
     rc = check_launch("volume_render_backward");
     if (rc) return rc;
@@ -1129,8 +1173,14 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
                        const void* color_ref, void* color_out, void* grad, void* hess, void* workspace,
                        int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp, hipStream_t stream) {
     const int D = fast_basis(tree, opt);
+    ClearWork clear;
+    if (clears_on_the_way(tree, n_slots, grad, hess)) {
+        clear.at[0] = grad;
+        clear.at[1] = hess;
+        clear.bytes = data_bytes(tree);
+    }
     int rc = launch_noted(tree, noting_shape(all), opt, color_out, workspace, workspace_bytes, n_slots, stamp, stream, nullptr,
-                          color_ref);
+                          color_ref, clear);
     if (rc) return rc;
     rc = check_launch("se_grad");
     if (rc) return rc;
@@ -1480,6 +1530,12 @@ int svox_volume_render_backward_ws(const SvoxTreeSpec* tree, const SvoxRaysSpec*
     rc = check_rays(rays);
     if (rc) return rc;
     if (!grad_data_out) return fail(SVOX_ERR_NULL_POINTER, "grad_data_out is NULL");
+    if (tree->dtype == SVOX_F32 && workspace && workspace_bytes >= 0 && rays->n_rays > 0 && grad_output) {
+        const BatchSource<float> all = batch_source<float>(rays, true);
+        rc = backward_by_noting(tree, all, all, opt, grad_output, grad_data_out, workspace, workspace_bytes,
+                                rays->n_rays, stamp_of(tree, rays, opt), accumulate != 0, (hipStream_t)stream);
+        if (rc <= 0) return rc;
+    }
     if (!accumulate) {
         rc = zero_fill(grad_data_out, data_bytes(tree), (hipStream_t)stream);
         if (rc) return rc;
@@ -1487,12 +1543,6 @@ int svox_volume_render_backward_ws(const SvoxTreeSpec* tree, const SvoxRaysSpec*
     if (rays->n_rays == 0) return SVOX_OK;
     if (!grad_output) return fail(SVOX_ERR_NULL_POINTER, "grad_output is NULL");
     if (workspace_bytes < 0) return fail(SVOX_ERR_BAD_SHAPE, "negative workspace size");
-    if (tree->dtype == SVOX_F32 && workspace) {
-        const BatchSource<float> all = batch_source<float>(rays, true);
-        rc = backward_by_noting(tree, all, all, opt, grad_output, grad_data_out, workspace, workspace_bytes,
-                                rays->n_rays, stamp_of(tree, rays, opt), (hipStream_t)stream);
-        if (rc <= 0) return rc;
-    }
     if (tree->dtype == SVOX_F32)
         launch_backward<BatchSource<float>, float>(tree, batch_source<float>(rays, true), opt, od, grad_output,
                                                    grad_data_out, (hipStream_t)stream);
@@ -1541,6 +1591,13 @@ int svox_volume_render_images_backward_ws(const SvoxTreeSpec* tree, const SvoxCa
     rc = check_camera(cam, n_images, pose_stride);
     if (rc) return rc;
     if (!grad_data_out) return fail(SVOX_ERR_NULL_POINTER, "grad_data_out is NULL");
+    const int64_t n_slots = (int64_t)n_images * cam->width * cam->height;
+    if (tree->dtype == SVOX_F32 && workspace && workspace_bytes >= 0 && n_slots > 0 && grad_output) {
+        const auto src = image_source<float>(cam, n_images, pose_stride, opt);
+        rc = backward_by_noting(tree, src, src, opt, grad_output, grad_data_out, workspace, workspace_bytes, n_slots,
+                                stamp_of_image(tree, cam, n_images, opt), accumulate != 0, (hipStream_t)stream);
+        if (rc <= 0) return rc;
+    }
     if (!accumulate) {
         rc = zero_fill(grad_data_out, data_bytes(tree), (hipStream_t)stream);
         if (rc) return rc;
@@ -1550,12 +1607,6 @@ int svox_volume_render_images_backward_ws(const SvoxTreeSpec* tree, const SvoxCa
     if (workspace_bytes < 0) return fail(SVOX_ERR_BAD_SHAPE, "negative workspace size");
     if (tree->dtype == SVOX_F32) {
         const auto src = image_source<float>(cam, n_images, pose_stride, opt);
-        if (workspace) {
-            rc = backward_by_noting(tree, src, src, opt, grad_output, grad_data_out, workspace, workspace_bytes,
-                                    (int64_t)n_images * cam->width * cam->height,
-                                    stamp_of_image(tree, cam, n_images, opt), (hipStream_t)stream);
-            if (rc <= 0) return rc;
-        }
         launch_backward<ImageSource<float>, float>(tree, src, opt, od, grad_output, grad_data_out, (hipStream_t)stream);
     } else {
         const auto src = image_source<double>(cam, n_images, pose_stride, opt);
@@ -1622,7 +1673,8 @@ int svox_se_grad_ws(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Sv
     if (od != 3 || rays->n_rays == 0 || !color_ref || !color_out ||
         !noted_ok(tree, &plain, rays->n_rays, workspace, workspace_bytes))
         return svox_se_grad(tree, rays, opt, color_ref, color_out, grad_out, hessdiag_out, stream);
-    rc = se_grad_prepare(tree, opt, grad_out, hessdiag_out, &od, (hipStream_t)stream);
+    const bool apart = !clears_on_the_way(tree, rays->n_rays, grad_out, hessdiag_out);
+    rc = se_grad_prepare(tree, opt, grad_out, hessdiag_out, &od, (hipStream_t)stream, apart);
     if (rc) return rc;
     const BatchSource<float> all = batch_source<float>(rays, true);
     return se_grad_from_notes(tree, all, all, &plain, color_ref, color_out, grad_out, hessdiag_out, workspace,
@@ -1643,7 +1695,8 @@ int svox_se_grad_image_ws(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam, c
     if (od != 3 || n_slots == 0 || !color_ref || !color_out ||
         !noted_ok(tree, &plain, n_slots, workspace, workspace_bytes))
         return svox_se_grad_image(tree, cam, opt, color_ref, color_out, grad_out, hessdiag_out, stream);
-    rc = se_grad_prepare(tree, opt, grad_out, hessdiag_out, &od, (hipStream_t)stream);
+    const bool apart = !clears_on_the_way(tree, n_slots, grad_out, hessdiag_out);
+    rc = se_grad_prepare(tree, opt, grad_out, hessdiag_out, &od, (hipStream_t)stream, apart);
     if (rc) return rc;
     const ImageSource<float> all = image_source<float>(cam, 1, 12, opt);
     return se_grad_from_notes(tree, all, all, &plain, color_ref, color_out, grad_out, hessdiag_out, workspace,
