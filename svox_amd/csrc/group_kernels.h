@@ -9,9 +9,9 @@
 // a ray.  The values are those of the generic kernels bit for bit: the same expressions in the same order; multiplying by 2^-levels
 // is dividing by 2^levels.
 // Bound by the chain of a turn (two child reads, the density, some 150 double-precision instructions: 1 to 1.3 us) up to 20 000 rays, by
-// how many wavefronts LDS has room for beyond: 592 entries leave seven to a compute unit (d. = dense 64^3 SH4, 20 000 rays, forward
-// pass and gradient: 592 176, 285 us; 640 181, 332; 768 205, 333; 896 226, 362; 512 172, 285, but where no leaf is empty 405, 933
-// instead of 270, 645; lists of a fixed length for every lane 222, 361).
+// how many wavefronts LDS has room for beyond: with 592 entries seven to a compute unit (dense 64^3 SH4, 20 000 rays, forward pass and
+// gradient, us: 512 entries 172, 285, but 405, 933 instead of 270, 645 where no leaf is empty; 592 176, 285; 640 181, 332; 768 205, 333;
+// 896 226, 362; lists of 20 entries for every lane, none shared, 222, 361).
 // Measured, four lanes that walk a ray together, from end to end, before / pieces, forward pass and gradient, us:
 //   64^3 SH4   200 rays 220, 370 / 46, 71    1 000 232, 391 / 46, 78    5 000 263, 390 / 70, 115    20 000 302, 446 / 176, 286
 //              40 000 334, 766 / 322, 522    100 000 578, 1464 / (757), 1214

@@ -856,7 +856,8 @@ ImageSource<T> noting_shape(const ImageSource<T>& s) { return s; }
 // nullptr (notes only); grad_out, if given, is the gradient of the picture the backward pass will be
 // called with: the notes' heads then also carry the sum of that pass's first march.
 // The rays of a batch that meet the cube, in the order they come in block by block (the blocks as they get there); the others are
-// answered as a noting pass answers them.  Reads 24 bytes a ray: 200 000 rays 4 us, 1 Mi rays 9.
+// answered as a noting pass answers them.  200 003 rays 9 us, 1 Mi rays 30: 24 bytes
+// read of each, and a line written for every one that misses, the head of its notes.
 constexpr int kListThreads = 1024;
 __global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> tr, BatchSource<float> src, SvoxRenderOptions opt,
                                                                         float* __restrict__ out, ReplaySpace ws,
@@ -1120,9 +1121,11 @@ SvoxRenderOptions without_thresholds(const SvoxRenderOptions* opt) {
 
 // Whether the arrays of a gradient are cleared by the launch that takes its notes: aligned as clear_share stores, not more than a
 // launch has blocks for, and beside a march that leaves the memory room: a gigabyte and more beside one of half a million rays is
-// cleared no faster than before it, and slows it.  us, apart / on the way, the squared error of a 256^3 SH9 shell (345 MB): 20 000 rays 343 / 294, 100 000
-// rays 409 / 360, 200 003 rays 524 / 471, 300 000 rays 568 / 526, 500 000 rays 680 / 655; the gradient by itself of a 512^3 SH16 shell (1.2 GB): 170 000 rays
-// 723 / 631, 300 000 rays 778 / 750, 500 000 rays 870 / 877, 700 000 rays 1129 / 1145; SH25 (1.9 GB) 400 000 rays 1024 / 1049.
+// cleared no faster than before it, and slows it.  us, apart / on the way:
+//   squared error, 256^3 SH9 shell (345 MB)          5 000 rays 190 / 147  20 000 350 / 299  100 000 422 / 363  200 003 524 / 471
+//                                                    300 000 rays 568 / 526  500 000 680 / 655
+//   gradient by itself, 512^3 SH16 shell (1.2 GB)    5 000 rays 347 / 274  50 000 584 / 497  170 000 723 / 631  300 000 778 / 750
+//                                                    500 000 rays 870 / 877  700 000 1129 / 1145;  SH25 (1.9 GB) 400 000 1024 / 1049
 constexpr int64_t kClearBeside = 512ll << 20, kClearRays = 1 << 18;
 bool clears_on_the_way(const SvoxTreeSpec* tree, int64_t n_rays, const void* a, const void* b = nullptr) {
     return ((uintptr_t)a & 15u) == 0 && ((uintptr_t)b & 15u) == 0 && data_bytes(tree) <= kMostCleared &&
