@@ -1051,7 +1051,8 @@ struct NoteTaker {
 // the picture, of the sum of the first march and of a gradient.  (What the reference adds to the density gradients of such leaves
 // is the rounding that is left of `accum`, where the exact term is below 2^-126.)  The chain of a batch's longest rays is what such
 // a pass waits for, and those that graze a surface are long because of what they pass through: 50 001 rays of a 256^3 SH9 shell with
-// softplus, march 240 -> 80 us, training step 391 -> 203 us.  Scenes without such densities: within 0.2 %.
+// softplus, march 240 -> 80 us, training step 391 -> 203 us.  Scenes without such densities pay for the look at the light: up to 1 % of the march on
+// two wavefronts (20 000 rays of a 256^3 SH9 shell 198.6 -> 201.6 us; with a flag kept beside the light 206), none on one.
 constexpr float kOpaqueLight = 1.17549435e-38f;
 
 // What a noting pass that has the gradient of the picture at hand accumulates per ray beside its notes:
@@ -1996,7 +1997,6 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     // kNoted: the picture of a ray may be finished (early stop) while its notes go on; without `out`
     // there is no picture to compose
     bool painted = kNoted && out == nullptr;
-    bool opaque = false;   // kNoted: nothing behind the leaves seen so far counts any more
     NoteTaker notes;
     March1Sum sum1;
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
@@ -2008,6 +2008,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) place[q] = ring_read(&box.place[((taken + q) & (kRing - 1)) * kMarchThreads + lane]);
         int n_take = 0;
+        const bool opaque = kNoted && light < kOpaqueLight;   // nothing behind the leaves seen so far counts any more
         bool run = active && !opaque;
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) {
@@ -2017,8 +2018,9 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         }
         const uint32_t next = (uint32_t)place[0];
         const bool over = (next & kOverBit) && (next & kRoundBit) == ring_round(taken);
-        if (active && (over || (kNoted && opaque))) {
+        if (active && (over || opaque)) {
             // the ray left the tree: the background shows through what is left of the light
+            if (kNoted && !over) taken_write(&box.taken[lane], taken | kEndedBit);   // (or the walk may stop)
             const bool broken = over && (next & 1u) != 0;
             if (kNoted && !kGrad && grad_out) {
                 notes.finish_residual(broken, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
@@ -2111,12 +2113,6 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                 painted = true;   // the picture is done; the notes go on to the end of the ray
             } else {
                 active = false;
-                taken_write(&box.taken[lane], taken | kEndedBit);
-            }
-        }
-        if constexpr (kNoted) {
-            if (active && !opaque && light < kOpaqueLight) {
-                opaque = true;
                 taken_write(&box.taken[lane], taken | kEndedBit);
             }
         }
