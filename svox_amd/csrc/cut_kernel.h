@@ -86,6 +86,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     const float pad = opt.rgb_padding;
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
     const float step = opt.step_size, sigma_thresh = opt.sigma_thresh, stop_thresh = opt.stop_thresh;
+    const float opaque = opaque_light(opt, out);
     const float list_thresh = kNoted ? 0.0f : sigma_thresh;
 
     // ---- the wavefront's rays: lane k of the first per_wave looks at the k-th of them
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                     painted = true;
                     if (!kNoted) ended = true;
                 }
-                if (kNoted && there && light < kOpaqueLight) {   // (nothing behind this leaf counts)
+                if (kNoted && there && light <= opaque) {   // (nothing behind this leaf counts)
                     ended = true;
                     limit = k + q + 1;
                 }

@@ -952,7 +952,8 @@ constexpr int kHeadFloat2 = kChunkRecords * 3;          // float2 index of {link
 constexpr int kChunkStock = 64;   // further chunks a wavefront takes at a time (at most 64 lanes ask at once)
 
 // The notes of one lane's ray while they are taken (by the forward kernels, for replay_backward_kernel
-// and replay_se_grad_kernel): every leaf with sigma > 0, in the order the ray meets them.
+// and replay_se_grad_kernel): every leaf with sigma > 0, in the order the ray meets them, up to where nothing shines through
+// any more (opaque_light).
 struct NoteTaker {
     int count, pos;     // notes so far; place in the chunk being written
     bool lost;          // the workspace ran out: the backward pass of this ray will march
@@ -1046,14 +1047,21 @@ struct NoteTaker {
     }
 };
 
-// A noting pass follows a ray beyond the early stop of its picture, but not beyond the leaf behind which the transmittance of what
-// it shades is less than the smallest normal float, 2^-126: every weight further on is less than that, and with it every term of
-// the picture, of the sum of the first march and of a gradient.  (What the reference adds to the density gradients of such leaves
-// is the rounding that is left of `accum`, where the exact term is below 2^-126.)  The chain of a batch's longest rays is what such
-// a pass waits for, and those that graze a surface are long because of what they pass through: 50 001 rays of a 256^3 SH9 shell with
-// softplus, march 240 -> 80 us, training step 391 -> 203 us.  Scenes without such densities pay for the look at the light: up to 1 % of the march on
-// two wavefronts (20 000 rays of a 256^3 SH9 shell 198.6 -> 201.6 us; with a flag kept beside the light 206), none on one.
-constexpr float kOpaqueLight = 1.17549435e-38f;
+// A noting pass follows a ray beyond the early stop of its picture, but not beyond the leaf behind which the transmittance of what it
+// shades is zero: every weight further on is zero there, whatever the gradient of the picture is scaled by, and the picture stops there
+// by itself.  (Not where it never stops, stop_thresh < 0: such a picture is composed to the end of its rays.)  Three things that the
+// reference's gradient has of such leaves are not there, though passes without notes and rays whose notes found no room add them: the
+// rounding that is left of `accum` in their density gradients, where the exact term is zero; a NaN that 0 * NaN makes of a coefficient
+// that is none; and the end of a ray in a malformed tree, where it lies behind.  (Up to kQueue - 1 leaves behind the last that counts
+// are still noted, those of its round: leaving them out, a comparison for every leaf, costs the step below 8 us.)
+// The chain of a batch's longest rays is what such a pass waits for, and those that graze a surface are long because of what they pass
+// through: 50 001 rays of a 256^3 SH9 shell with softplus, training step 342 -> 208 us.  A bound of 2^-126, below which a weight has
+// lost digits, ends them hardly sooner (207 us), and leaves out terms that a large gradient of the picture makes count.
+// Marches on two wavefronts are 1 % longer than before rays ended here (20 000 rays of a 256^3 SH9 shell 302.8 -> 305.8 us, dense 64^3,
+// 30 000 rays 213.7 -> 215.6), though not for the look at the light: without it they measure the same.
+__device__ __forceinline__ float opaque_light(const SvoxRenderOptions& opt, const float* out) {
+    return opt.stop_thresh >= 0.0f || out == nullptr ? 0.0f : -1.0f;   // (light is never below zero)
+}
 
 // What a noting pass that has the gradient of the picture at hand accumulates per ray beside its notes:
 // the sum the backward pass forms in its first march (rt_kernel.cu:358-419; the same expressions, in
@@ -1107,8 +1115,8 @@ struct March1Sum {
 // set up once before the loop, and nothing the set-up needs stays live inside it.
 // kNoted: the forward pass of a training step.  The picture is composed as without it; beside it the
 // launch leaves in the workspace the notes the backward pass works from (NoteTaker): every leaf with
-// sigma > 0 of the whole ray, so a ray is walked to its end also after its picture stopped early, and
-// the colours of the leaves at or below sigma_thresh are evaluated too.  With out == nullptr only the
+// sigma > 0 up to where nothing shines through any more (opaque_light), so a ray is walked on after its
+// picture stopped early, and the colours of the leaves at or below sigma_thresh are evaluated too.  With out == nullptr only the
 // notes are taken (the backward pass without a forward pass before it); kGrad: that backward pass's
 // grad_out is given, and the sum of its first march is formed on the way (March1Sum).  A pass that takes notes for
 // replay_se_grad_kernel (not kGrad, stop_thresh 0) is given the reference colours in grad_out's place
@@ -1139,6 +1147,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     const float pad = opt.rgb_padding;
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
     const float step = opt.step_size, sigma_thresh = opt.sigma_thresh, stop_thresh = opt.stop_thresh;
+    const float opaque = opaque_light(opt, out);
 
     int64_t next = chunk_of_block(blockIdx.x, kNoted ? ws.march_blocks : gridDim.x, src.xcd_group) * (int64_t)src.per_wave;
     const int64_t total = src.total();
@@ -1252,7 +1261,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
             }
 #pragma unroll
             for (int q = 0; q < kQueue; ++q) {
-                // (the light of a ray whose picture is finished goes on: kOpaqueLight)
+                // (the light of a ray whose picture is finished goes on: opaque_light)
                 const bool shade = active && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
                 const bool take = shade && !painted;
                 const float weight = light * (1.0f - q_att[q]);
@@ -1286,11 +1295,11 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
                 out[slot * 3 + 1] = acc[1] * scale;
                 out[slot * 3 + 2] = acc[2] * scale;
                 if constexpr (kNoted)
-                    painted = true;   // the notes go on to the end of the ray
+                    painted = true;   // the notes go on
                 else
                     active = false;
             }
-            if (active && (broken || !(r.t < r.tmax) || (kNoted && light < kOpaqueLight))) {
+            if (active && (broken || !(r.t < r.tmax) || (kNoted && light <= opaque))) {
                 if (kNoted && !kGrad && grad_out) {
                     notes.finish_residual(broken, r.dscale, acc, light, bg, grad_out + slot * 3, out + slot * 3);
                 } else {
@@ -1837,7 +1846,7 @@ static_assert(offsetof(ShadeSharedProbe, who) == sizeof(int32_t) * kQueue * kMar
 // row it gives up, so that a launch ends whatever happens.
 //
 // kNoted: as in render_forward_kernel, the launch also leaves the notes of every ray for the backward
-// pass: every leaf with sigma > 0 of the whole ray, so the walk goes on after the picture's early stop,
+// pass: every leaf with sigma > 0 up to where nothing shines through any more, so the walk goes on after the picture's early stop,
 // and the colours of leaves below sigma_thresh are evaluated too; the picture itself is composed as
 // without notes.
 constexpr int kSplitThreads = 2 * kMarchThreads;
@@ -1900,6 +1909,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     const float pad = opt.rgb_padding;
     const float d_rgb_pad = 1 + 2 * opt.rgb_padding;
     const float step = opt.step_size, sigma_thresh = opt.sigma_thresh, stop_thresh = opt.stop_thresh;
+    const float opaque = opaque_light(opt, out);
     const int spin_limit = ws.spin_limit > 0 ? ws.spin_limit : kSpinLimit;
 
     const int64_t item = chunk_of_block(blockIdx.x, kNoted ? ws.march_blocks : gridDim.x, src.xcd_group) * (int64_t)kMarchThreads + lane;
@@ -2008,8 +2018,8 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) place[q] = ring_read(&box.place[((taken + q) & (kRing - 1)) * kMarchThreads + lane]);
         int n_take = 0;
-        const bool opaque = kNoted && light < kOpaqueLight;   // nothing behind the leaves seen so far counts any more
-        bool run = active && !opaque;
+        const bool ended = kNoted && light <= opaque;   // nothing behind the leaves seen so far counts any more
+        bool run = active && !ended;
 #pragma unroll
         for (int q = 0; q < kQueue; ++q) {
             const uint32_t code = (uint32_t)place[q];
@@ -2018,7 +2028,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         }
         const uint32_t next = (uint32_t)place[0];
         const bool over = (next & kOverBit) && (next & kRoundBit) == ring_round(taken);
-        if (active && (over || opaque)) {
+        if (active && (over || ended)) {
             // the ray left the tree: the background shows through what is left of the light
             if (kNoted && !over) taken_write(&box.taken[lane], taken | kEndedBit);   // (or the walk may stop)
             const bool broken = over && (next & 1u) != 0;
@@ -2085,7 +2095,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             }
 #pragma unroll
             for (int q = 0; q < kQueue; ++q) {
-                // (the light of a ray whose picture is finished goes on: kOpaqueLight)
+                // (the light of a ray whose picture is finished goes on: opaque_light)
                 const bool shade = active && q_leaf[q] >= 0 && !stopped && q_sigma[q] > sigma_thresh;
                 const bool take = shade && !painted;
                 const float weight = light * (1.0f - q_att[q]);
@@ -2110,7 +2120,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
             out[slot * 3 + 1] = acc[1] * scale;
             out[slot * 3 + 2] = acc[2] * scale;
             if constexpr (kNoted) {
-                painted = true;   // the picture is done; the notes go on to the end of the ray
+                painted = true;   // the picture is done; the notes go on
             } else {
                 active = false;
                 taken_write(&box.taken[lane], taken | kEndedBit);

@@ -669,7 +669,7 @@ constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 //           256^3 SH9   1 000 rays 196, 193 / 60, 55   4 000 261, 256 / 169, 121  8 000 311, 308 / 270, 199  12 000 271, 270 / 334, 255
 //           512^3 SH16  1 000 rays 235, 235 / 99, 108  4 000 332, 333 / 209, 180  8 000 349, 350 / 351, 270  12 000 332, 332 / 436, 365
 // 18 % of the rays hit: 64^3 shell 4 000 rays 83, 80 / 42, 35; 256^3 4 000 169, 166 / 63, 57, 8 000 169, 165 / 89, 72; 512^3 4 000 224, 225 / 97, 108,
-// 8 000 224, 223 / 110, 110.  With the shifted softplus, where every leaf is listed and rays end behind what they met (kOpaqueLight):
+// 8 000 224, 223 / 110, 110.  With the shifted softplus, where every leaf is listed and rays end behind what they met (opaque_light):
 // 32^3 4 000 rays 101, 85 / 59, 54, 12 000 122, 91 / 146, 102; 128^3 4 000 473, 442 / 315, 277, 12 000 499, 463 / 994, 495; 256^3 shell 4 000 75, 70 /
 // 63, 49, 8 000 78, 73 / 92, 53, 12 000 78, 74 / 119, 75; 512^3 shell 4 000 78, 76 / 76, 62.
 // Square pictures of 64 and 90 pixels a side (4 096, 8 100):

@@ -33,7 +33,7 @@ def _make_camera_spec(c2w, width, height, fx, fy):
 
 
 # Whether a forward pass that will be differentiated keeps notes for its backward pass (faster
-# training steps; the forward pass itself takes longer, as it follows every ray to its end).
+# training steps; the forward pass itself takes longer, as it follows a ray beyond its early stop).
 KEEP_NOTES = True
 
 
@@ -237,8 +237,10 @@ class VolumeRenderer(nn.Module):
       `csrc.BACKWARD_WORKSPACE_LIMIT` (4 GiB) and at most a quarter of the device memory that is free
       at the time.  Where that leaves no room, or
       the allocation fails, the pass runs without notes and the backward pass marches through the tree
-      twice, as the reference does: same results, slower.  The noted forward pass follows every ray to
-      its end (no early stop), so it is slower than a forward pass under `torch.no_grad()`.  The notes
+      twice, as the reference does: same results, slower.  The noted forward pass follows a ray
+      beyond the early stop of its picture, until nothing at all shines through, so it is slower than a
+      forward pass under `torch.no_grad()`; the picture is the same.  Leaves behind get a gradient of zero,
+      where a march adds the rounding left of its sums (and a NaN, if a coefficient there is one).  The notes
       are used once: a second `backward()` through a retained graph marches.  `renderer.KEEP_NOTES =
       False` switches the notes off.  If `tree.data`, the tree's structure, the rays or the camera are
       written to between the two passes -- through torch (version counters), a method of the tree or a
