@@ -27,6 +27,21 @@ constexpr int kCutTurns = kQueue; // of the walk, between looks at the densities
 constexpr int kCutHeads = 8;      // samples of a piece that the piece before can go on from
 constexpr int kCutMostRays = 8;   // of a wavefront
 
+// Where the first samples of every piece are.  The lanes write and look at them in the same loop, with nothing between that would make the
+// compiler read again or write at once, so both are atomics of the workgroup (ring_read), and nothing else can reach them.
+template <class T, int kHeads>
+class PieceHeads {
+    T at[kHeads * kMarchThreads];
+
+public:
+    __device__ __forceinline__ T read(int head, int lane) const {
+        return __hip_atomic_load(&at[head * kMarchThreads + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ void write(int head, int lane, T t) {
+        __hip_atomic_store(&at[head * kMarchThreads + lane], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+};
+
 // n chunks from those that all rays share, one after the other: the number of the first.  The counter of the stocks handed out is
 // kept in step with the one of chunks, beside it, that they are taken from here.
 __device__ __forceinline__ unsigned long long take_chunks(const ReplaySpace& ws, int n) {
@@ -61,7 +76,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     constexpr int kListed = cut_listed(kNoted);
     constexpr int kMostRays = kCutMostRays;
     __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
-    __shared__ float heads[kCutHeads * kMarchThreads];      // where a piece's first samples are (-1: not known yet)
+    __shared__ PieceHeads<float, kCutHeads> heads;           // (-1: not known yet)
     __shared__ CutLists<kListed> lists;
     __shared__ float atts[kNoted ? kListed * kMarchThreads : 1];      // attenuations (without notes: in lists.dt)
     float* const att_of = kNoted ? atts : lists.dt;
@@ -153,7 +168,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     int sample = 0, count = 0, shaded = 0;
     uint32_t end = 0;
 #pragma unroll
-    for (int i = 0; i < kCutHeads; ++i) heads[i * kMarchThreads + lane] = walking ? (i == 0 ? r.t : kUnknown) : kNone;
+    for (int i = 0; i < kCutHeads; ++i) heads.write(i, lane, walking ? (i == 0 ? r.t : kUnknown) : kNone);
     if (!walking) end = kCutOver;
     OctreeCursor cur;
     cur.reset(path + lane);
@@ -190,7 +205,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
 #pragma unroll
                         for (int k = 0; k < 3; ++k) {
                             if (k > 0 && there != kUnknown && there < r.t && head < kCutHeads - 1) head += 1;
-                            there = heads[head * kMarchThreads + leader + next];
+                            there = heads.read(head, leader + next);
                         }
                         if (there == r.t) {
                             end |= kCutLinked | (uint32_t)head << 8 | (uint32_t)(leader + next) << 11;
@@ -216,7 +231,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                         walking = false;
                         end |= kCutOver | (broken ? kCutBroken : 0u);
                     } else if (q_leaf[q] >= 0 && sample < kCutHeads) {
-                        heads[sample * kMarchThreads + lane] = r.t;
+                        heads.write(sample, lane, r.t);
                     }
                 }
             }
@@ -225,7 +240,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                 const int from = (end & (kCutLinked | kCutBroken)) != 0 ? sample + 1 : sample;
 #pragma unroll
                 for (int i = 0; i < kCutHeads; ++i)
-                    if (i >= from) heads[i * kMarchThreads + lane] = kNone;
+                    if (i >= from) heads.write(i, lane, kNone);
             }
             float q_raw[kCutTurns];
             fetch_sigma<K>(tr.data, q_leaf, q_raw);

@@ -21,7 +21,7 @@
 //   shells, SH9, every ray hits  128^3 2 000 rays 246, 404 / 88, 125, 20 000 321, 537 / 226, 351; 256^3 329, 613 / 93, 178 and 459, 863 / 297, 479
 #pragma once
 
-#include "march_kernels.h"
+#include "cut_kernel.h"
 
 namespace svox {
 
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
     constexpr int DD = D > 0 ? D : 1;
     constexpr int K = D > 0 ? 3 * D + 1 : 4;
     __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
-    __shared__ double heads[kGroupHeads * kMarchThreads];      // where a piece's first samples are (-1: not known yet)
+    __shared__ PieceHeads<double, kGroupHeads> heads;          // (-1: not known yet)
     // the leaves found, and the one after each in its lane's list; the entries that are free
     __shared__ double list_dt[kGroupEntries];
     __shared__ int32_t list_leaf[kGroupEntries];
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
         int sample = 0, count = 0;
         uint32_t end = walking ? 0u : kGroupOver;
 #pragma unroll
-        for (int i = 0; i < kGroupHeads; ++i) heads[i * kMarchThreads + lane] = walking ? (i == 0 ? walk.t : kUnknown) : kNone;
+        for (int i = 0; i < kGroupHeads; ++i) heads.write(i, lane, walking ? (i == 0 ? walk.t : kUnknown) : kNone);
         wave_lds_sync();
         int at_lane = leader, at = 0;      // where the ray's composition stands
         int first = 0, last = 0;           // of this lane's list
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
 #pragma unroll
                         for (int k = 0; k < 3; ++k) {
                             if (k > 0 && there != kUnknown && there < walk.t && head < kGroupHeads - 1) head += 1;
-                            there = heads[head * kMarchThreads + leader + next];
+                            there = heads.read(head, leader + next);
                         }
                         if (there == walk.t) {
                             end |= kGroupLinked | (uint32_t)head << 8 | (uint32_t)(leader + next) << 11;
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
                             walking = false;
                             end |= kGroupOver;
                         } else if (sample < kGroupHeads) {
-                            heads[sample * kMarchThreads + lane] = walk.t;
+                            heads.write(sample, lane, walk.t);
                         }
                     }
                 }
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
                     const int from = (end & (kGroupLinked | kGroupBroken)) != 0 ? sample + 1 : sample;
 #pragma unroll
                     for (int i = 0; i < kGroupHeads; ++i)
-                        if (i >= from) heads[i * kMarchThreads + lane] = kNone;
+                        if (i >= from) heads.write(i, lane, kNone);
                 }
             }
             list_count[lane] = (uint16_t)count;
