@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     bool walking = hit && r.t < r.tmax;
     int next = piece + 1, head = 0;    // the piece ahead, and its next sample to compare with
     float next_at = begin_of(next);
-    int patience = 256;                // turns the lane may yet spend on comparing instead of walking
+    int patience = 256;                // turns the lane may yet spend on waiting for the piece ahead
     int sample = 0, count = 0, shaded = 0;
     uint32_t end = 0;
 #pragma unroll
@@ -210,14 +210,15 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                         if (there == r.t) {
                             end |= kCutLinked | (uint32_t)head << 8 | (uint32_t)(leader + next) << 11;
                             walking = go = false;
-                        } else if (there == kNone || (there != kUnknown && there < r.t && head == kCutHeads - 1) || --patience < 0) {
-                            // it has none after the one here, or tells of none: the one after it
-                            next += 1;
-                            next_at = begin_of(next);
-                            head = 0;
+                        } else if (there == kNone || there < r.t) {
+                            // it has none after the one here, or tells of none: the one after it; otherwise its next sample is not
+                            // known yet, or not looked at (one that lies ahead is walked to)
+                            if (there == kNone || (there != kUnknown && head == kCutHeads - 1) || --patience < 0) {
+                                next += 1;
+                                next_at = begin_of(next);
+                                head = 0;
+                            }
                             go = false;
-                        } else if (there < r.t) {
-                            go = false;   // (its next sample is not known yet, or not looked at)
                         }
                     }
                 }

@@ -329,7 +329,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
         bool fresh = true;             // the sample at walk.t has not been looked at
         int next = piece + 1, head = 0;    // the piece ahead, and its next sample to compare with
         double next_at = begin_of(next);
-        int patience = 32;                 // turns the lane may yet spend on comparing instead of walking (256: 128^3 shell, 2 000 rays 88 -> 247 us)
+        int patience = 32;                 // turns the lane may yet spend on waiting for the piece ahead (256: 128^3 shell, 2 000 rays 88 -> 247 us)
         int sample = 0, count = 0;
         uint32_t end = walking ? 0u : kGroupOver;
 #pragma unroll
@@ -368,15 +368,16 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
                         if (there == walk.t) {
                             end |= kGroupLinked | (uint32_t)head << 8 | (uint32_t)(leader + next) << 11;
                             walking = go = false;
-                        } else if (there == kNone || (there != kUnknown && there < walk.t && head == kGroupHeads - 1) ||
-                                   room < kMarchThreads + kGroupReserve || --patience < 0) {
-                            // it has none after the one here, tells of none, or may not walk on: the one after it
-                            next += 1;
-                            next_at = begin_of(next);
-                            head = 0;
+                        } else if (there == kNone || there < walk.t) {
+                            // it has none after the one here, tells of none, or may not walk on: the one after it; otherwise its next
+                            // sample is not known yet, or not looked at (one that lies ahead is walked to)
+                            if (there == kNone || (there != kUnknown && head == kGroupHeads - 1) || room < kMarchThreads + kGroupReserve ||
+                                --patience < 0) {
+                                next += 1;
+                                next_at = begin_of(next);
+                                head = 0;
+                            }
                             go = false;
-                        } else if (there < walk.t) {
-                            go = false;   // (its next sample is not known yet, or not looked at)
                         }
                     }
                 }

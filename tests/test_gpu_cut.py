@@ -170,3 +170,30 @@ def test_double_precision_batches_on_either_side_of_the_rule(gpu, n):
     rs = rays_spec(synth.sphere_rays(n, seed=3, dtype=torch.float64), gpu)
     spec, opt = on_gpu(tree, gpu)._spec(), options(tree, step_size=1e-3)
     assert torch.equal(C.volume_render(spec, rs, opt), run(1, lambda: C.volume_render(spec, rs, opt)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_many_pieces_are_not_walked_in_vain(gpu, dtype):
+    """64 pieces to a ray and 32 of each of two rays take times of one kind: a lane that walks to the next piece's samples links up
+    with them.  (1 000 rays of a 256^3 SH9 shell in double precision: 95 and 80 us; 323 us where such lanes passed over the pieces ahead of them.)"""
+    tree = synth.shell_tree(depth=8, data_format="SH9", n_spheres=24, seed=0)
+    rs = rays_spec(synth.sphere_rays(1000, seed=5, dtype=dtype), gpu)
+    opt = options(tree, step_size=5e-4)
+    spec = on_gpu(tree.to(dtype), gpu)._spec()
+    flags = {64: cut(1, 6), 32: cut(2, 5)} if dtype == torch.float32 else {64: 32 | 601 << 8, 32: 32 | 502 << 8}
+    times = {64: [], 32: []}
+    for _ in range(7):
+        for pieces, f in flags.items():
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+            def passes():
+                begin.record()
+                for _ in range(5):
+                    C.volume_render(spec, rs, opt)
+                end.record()
+            run(f, passes)
+            end.synchronize()
+            times[pieces].append(begin.elapsed_time(end))
+    many, fewer = (sorted(times[k])[3] for k in (64, 32))
+    print(f"[pieces] {dtype}: 64 to a ray {many * 200:.0f} us, 32 {fewer * 200:.0f} us", flush=True)
+    assert many <= 2 * fewer
