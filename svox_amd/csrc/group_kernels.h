@@ -12,13 +12,11 @@
 // how many wavefronts LDS has room for beyond: with 592 entries seven to a compute unit (dense 64^3 SH4, 20 000 rays, forward pass and
 // gradient, us: 512 entries 172, 285, but 405, 933 instead of 270, 645 where no leaf is empty; 592 176, 285; 640 181, 332; 768 205, 333;
 // 896 226, 362; lists of 20 entries for every lane, none shared, 222, 361).
-// Measured, four lanes that walk a ray together, from end to end, before / pieces, forward pass and gradient, us:
-//   64^3 SH4   200 rays 220, 370 / 46, 71    1 000 232, 391 / 46, 78    5 000 263, 390 / 70, 115    20 000 302, 446 / 176, 286
-//              40 000 334, 766 / 322, 522    100 000 578, 1464 / (757), 1214
-//   no leaf empty  1 000 242, 559 / 64, 153  20 000 312, 678 / 271, 648
-//   16^3 RGBA  1 000 rays 49, 73 / 39, 47    20 000 60, 88 / 53, 77     32^3 SH9  1 000 133, 227 / 51, 74   20 000 163, 290 / 107, 228
-//   128^3 SH4  1 000 rays 520, 950 / 66, 132 5 000 538, 960 / 139, 361  20 000 597, 1109 / 339, 787   60 000 731, 2457 / (862), 1892
-//   shells, SH9, every ray hits  128^3 2 000 rays 246, 404 / 88, 125, 20 000 321, 537 / 226, 351; 256^3 329, 613 / 93, 178 and 459, 863 / 297, 479
+// Measured, four lanes that walk a ray together, from end to end / pieces, forward pass and gradient, us (more: group_cut):
+//   64^3 SH4, half of the leaves empty  1 000 rays 226, 383 / 57, 78    5 000 262, 394 / 78, 121    20 000 295, 442 / 172, 292
+//   no leaf empty                       1 000 rays 232, 541 / 65, 140   5 000 269, 570 / 110, 263   20 000 305, 644 / 280, 658
+//   256^3 shell SH16, every ray hits    1 000 rays 370, 809 / 96, 214   5 000 439, 900 / 131, 364   20 000 509, 1023 / 271, 631
+// The lanes of a ray that walk it together are the kernels for more rays than find room in pieces (below).
 #pragma once
 
 #include "cut_kernel.h"
@@ -329,7 +327,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
         bool fresh = true;             // the sample at walk.t has not been looked at
         int next = piece + 1, head = 0;    // the piece ahead, and its next sample to compare with
         double next_at = begin_of(next);
-        int patience = 32;                 // turns the lane may yet spend on waiting for the piece ahead (256: 128^3 shell, 2 000 rays 88 -> 247 us)
+        int patience = 32;                 // turns the lane may yet spend on waiting for the piece ahead (256: 128^3 shell, 2 000 rays 84 -> 227 us)
         int sample = 0, count = 0;
         uint32_t end = walking ? 0u : kGroupOver;
 #pragma unroll
@@ -515,9 +513,10 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
     }
 }
 
-// ---- pictures of more rays than the pieces of find room on the GPU: four lanes walk a ray together (the same addresses, one
+// ---- more rays than the pieces of find room on the GPU, or in their lists (group_cut): four lanes walk a ray together (the same addresses, one
 // request), each doing one axis' arithmetic, lane c evaluates channel c, and the record of a leaf is asked for before the next step
-// of the walk and used after it.
+// of the walk and used after it.  (128^3 SH4 without empty leaves, four lanes to a ray / pieces: gradient of 20 000 rays
+// 1485 / 1336, of 131 072 6 338 / 7 670 us.)
 constexpr int kSharedLanes = 4;
 constexpr int kSharedRays = kMarchThreads / kSharedLanes;
 
@@ -725,6 +724,187 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_shared_kernel(Tr
     if (channel < 3) out[slot * 3 + channel] = acc;
 }
 
+// trace_ray_backward, rt_kernel.cu:323-477.  The first march sums <render, grad_out> and keeps the leaves with density
+// it met, as far as they fit (kSharedKept to a ray); the second forms the records of the gradient from that list, and
+// walks on only where the list was full.  The wavefront adds the records of a step together: scalar f from lane
+// f mod 64, so that the scalars of a record go out in requests of 64 bytes (the memory system takes a fixed number of
+// those per microsecond).
+constexpr int kSharedKept = 96;
+
+template <int D, class Source>
+__global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(TreeDev<double> tr, Source src,
+                                                                              SvoxRenderOptions opt,
+                                                                              const double* __restrict__ grad_out,
+                                                                              double* __restrict__ grad_data) {
+    constexpr int K = SharedRecord<D>::K;
+    constexpr int DD = D > 0 ? D : 1;
+    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ double basis_rows[kSharedRays * DD];
+    __shared__ double kept_dt[kSharedKept * kSharedRays];     // [place][ray]
+    __shared__ int32_t kept_leaf[kSharedKept * kSharedRays];
+    __shared__ double factors[kSharedRays * 4];       // of the ray's record: the three colour factors, the density term
+    __shared__ int32_t leaves[kSharedRays];           // where the record goes
+    __shared__ uint8_t listed[kSharedRays];           // rays with a record in this step
+    const int lane = threadIdx.x, channel = lane & (kSharedLanes - 1), ray = lane / kSharedLanes;
+    SharedWalk walk;
+    bool live;
+    const int64_t slot = shared_ray<D>(tr, src, opt, lane, path, basis_rows, walk, live);
+    if (!__any(live)) return;
+    const double* const basis = basis_rows + ray * DD;
+    const double pad = (double)opt.rgb_padding, d_rgb_pad = (double)(1 + 2 * opt.rgb_padding);
+    double go[3] = {0.0, 0.0, 0.0};
+    if (live) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) go[j] = grad_out[slot * 3 + j];
+    }
+    const double my_go = channel == 0 ? go[0] : channel == 1 ? go[1] : go[2];
+    double accum = 0.0, light = 1.0;
+    double resume_t = 0.0;     // where the second march walks on
+    int n_kept = 0;
+    bool full = false;
+    // one leaf with density: attenuation, weight and <colour, grad_out>
+    auto shade = [&](const SharedRecord<D>& rec, double sigma, double dt, double& weight, double& sg) {
+        const double att = exp_sp<double>(-dt * sigma * walk.dscale);
+        weight = light * (1.0 - att);
+        sg = rec.colour(opt, basis);
+        const double col = fma_(sg, d_rgb_pad, -pad);
+        double total_color = fma_(from_group<0>(col), go[0], 0.0);
+        total_color = fma_(from_group<1>(col), go[1], total_color);
+        total_color = fma_(from_group<2>(col), go[2], total_color);
+        light *= att;
+        return total_color;
+    };
+    // ---- first march
+    bool whole = live;         // false also for a ray that leaves a malformed tree: no second march (the reference's return)
+    if (live) {
+        bool waiting = false, walking = !walk.ended();
+        double dt = 0.0, at_t = 0.0;       // (at_t: the parameter of the leaf whose record is on its way)
+        int32_t waiting_leaf = 0;
+        SharedRecord<D> rec;
+        if (walking) walk.aim();
+        while (walking || waiting) {
+            int64_t leaf = -1;
+            double next_dt = 0.0;
+            const double next_t = walk.t;
+            if (walking && !walk.turn(tr, (double)opt.step_size, leaf, next_dt)) continue;
+            const bool more = walking && leaf >= 0;
+            if (walking && !more) whole = false;
+            walking = more && !walk.ended();
+            if (walking) walk.aim();
+            if (waiting) {
+                const double sigma = opt.density_softplus ? softplus_m1(rec.raw) : rec.raw;
+                if (sigma > 0.0) {
+                    double weight, sg;
+                    const double total_color = shade(rec, sigma, dt, weight, sg);
+                    accum = fma_(weight, total_color, accum);
+                    if (n_kept < kSharedKept) {
+                        if (channel == 0) {
+                            kept_dt[n_kept * kSharedRays + ray] = dt;
+                            kept_leaf[n_kept * kSharedRays + ray] = waiting_leaf;
+                        }
+                        n_kept += 1;
+                    } else if (!full) {
+                        full = true;
+                        resume_t = at_t;
+                    }
+                }
+            }
+            waiting = more;
+            waiting_leaf = (int32_t)leaf;
+            dt = next_dt;
+            at_t = next_t;
+            if (more) rec.ask(tr.data, leaf, channel);
+        }
+    }
+    wave_lds_sync();
+    if (whole) accum = fma_(light * (double)opt.background_brightness, (go[0] + go[1]) + go[2], accum);
+    // ---- second march
+    light = 1.0;
+    int at = 0;
+    bool waiting = false, walking = false;
+    double dt = 0.0;
+    int32_t waiting_leaf = 0;
+    SharedRecord<D> rec;
+    auto ask_kept = [&]() {
+        waiting = whole && at < n_kept;
+        if (waiting) {
+            waiting_leaf = kept_leaf[at * kSharedRays + ray];
+            dt = kept_dt[at * kSharedRays + ray];
+            rec.ask(tr.data, waiting_leaf, channel);
+            at += 1;
+        } else if (whole && full) {
+            full = false;                   // the list is used up: the rest of the ray is walked again
+            walk.t = resume_t;
+            walking = true;
+            walk.aim();
+        }
+    };
+    ask_kept();
+    while (__any(waiting || walking)) {
+        bool emit = false;
+        bool turned = true;                 // this ray takes part in the step (its search for a leaf is not under way)
+        int64_t leaf = -1;
+        double next_dt = 0.0;
+        if (walking) {
+            turned = walk.turn(tr, (double)opt.step_size, leaf, next_dt);
+            if (turned) {
+                walking = leaf >= 0 && !walk.ended();
+                if (walking) walk.aim();
+            }
+        }
+        if (turned && waiting) {
+            const double raw = rec.raw;
+            const double sigma = opt.density_softplus ? softplus_m1(raw) : raw;
+            if (sigma > 0.0) {
+                double weight, sg;
+                const double total_color = shade(rec, sigma, dt, weight, sg);
+                accum = fma_(-weight, total_color, accum);
+                double f = D == 0 ? weight * sg * (1.0 - sg) * my_go * d_rgb_pad
+                                  : (weight * sg) * (1.0 - sg) * my_go * d_rgb_pad;
+                if (channel == 3) {
+                    const double chain = opt.density_softplus ? sigmoid_(raw - 1.0) : 1.0;
+                    f = dt * walk.dscale * fma_(total_color, light, -accum) * chain;
+                }
+                factors[ray * 4 + channel] = f;
+                if (channel == 0) leaves[ray] = waiting_leaf;
+                emit = true;
+            }
+        }
+        if (turned) {
+            waiting = leaf >= 0;
+            if (waiting) {
+                waiting_leaf = (int32_t)leaf;
+                dt = next_dt;
+                rec.ask(tr.data, leaf, channel);
+            } else if (!walking) {
+                ask_kept();
+            }
+        }
+        // the records of this step, added by the whole wavefront
+        const unsigned long long m = __ballot(emit && channel == 0);
+        if (m != 0) {
+            if (emit && channel == 0) listed[rank_in(m)] = (uint8_t)ray;
+            wave_lds_sync();
+            const int n_scalars = __popcll(m) * K;
+            for (int f = lane; f < n_scalars; f += kMarchThreads) {
+                const int rec_at = f / K, e = f - rec_at * K;
+                const int owner = listed[rec_at];
+                const int c = e / DD < 3 ? e / DD : 3;
+                double v = factors[owner * 4 + c];
+                if constexpr (D > 0) {
+                    const int i = e - c * DD;
+                    if (c < 3) {
+                        if (i < opt.min_comp || i > opt.max_comp) continue;
+                        v = basis_rows[owner * DD + i] * v;
+                    }
+                }
+                atomicAdd(grad_data + (int64_t)leaves[owner] * K + e, v);
+            }
+            wave_lds_sync();
+        }
+    }
+}
+
 // ---- launches (march_double.hip).  D: 0 for RGBA, else the basis size (1, 4, 9, 16 or 25)
 template <class Source>
 void launch_group_forward(int D, dim3 blocks, hipStream_t stream, const TreeDev<double>& tr, const Source& src,
@@ -735,5 +915,8 @@ void launch_shared_forward(int D, dim3 blocks, hipStream_t stream, const TreeDev
 template <class Source>
 void launch_group_backward(int D, dim3 blocks, hipStream_t stream, const TreeDev<double>& tr, const Source& src,
                            const SvoxRenderOptions& opt, const double* grad_out, double* grad_data, int per_wave, int most_cut);
+template <class Source>
+void launch_shared_backward(int D, dim3 blocks, hipStream_t stream, const TreeDev<double>& tr, const Source& src,
+                            const SvoxRenderOptions& opt, const double* grad_out, double* grad_data);
 
 }  // namespace svox

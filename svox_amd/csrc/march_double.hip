@@ -35,13 +35,22 @@ void launch_group_backward(int D, dim3 blocks, hipStream_t stream, const TreeDev
                                            opt, grad_out, grad_data, per_wave, most_cut));
 }
 
+template <class Source>
+void launch_shared_backward(int D, dim3 blocks, hipStream_t stream, const TreeDev<double>& tr, const Source& src,
+                            const SvoxRenderOptions& opt, const double* grad_out, double* grad_data) {
+    SVOX_GROUP_BASIS(D, hipLaunchKernelGGL((render_backward_shared_kernel<kD, Source>), blocks, dim3(kMarchThreads), 0, stream, tr,
+                                           src, opt, grad_out, grad_data));
+}
+
 #define SVOX_GROUP_SOURCE(S)                                                                                               \
     template void launch_group_forward<S>(int, dim3, hipStream_t, const TreeDev<double>&, const S&, const SvoxRenderOptions&, \
                                           double*, int, int);                                                                        \
     template void launch_shared_forward<S>(int, dim3, hipStream_t, const TreeDev<double>&, const S&, const SvoxRenderOptions&, \
                                            double*);                                                                       \
     template void launch_group_backward<S>(int, dim3, hipStream_t, const TreeDev<double>&, const S&,                        \
-                                           const SvoxRenderOptions&, const double*, double*, int, int);
+                                           const SvoxRenderOptions&, const double*, double*, int, int);                    \
+    template void launch_shared_backward<S>(int, dim3, hipStream_t, const TreeDev<double>&, const S&,                       \
+                                            const SvoxRenderOptions&, const double*, double*);
 SVOX_GROUP_SOURCE(BatchSource<double>)
 SVOX_GROUP_SOURCE(ImageSource<double>)
 

@@ -419,10 +419,8 @@ int fast_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt) {
 // (group_kernels.h; 0 for RGBA), or -1: three colour channels of a basis size they are built for, cells that 32-bit
 // indices reach, no weight accumulator, and not more rays than kGroupMaxRays.
 //
-// kGroupMaxRays: with more rays than fill the chip it only costs that the pieces of a ray overlap.  Dense 64^3 SH4 tree, gradient,
-// one ray per lane / pieces: 100 000 rays 1954 / 1214 us, 130 000 rays 2500 / 1550 us.  kGroupMaxPictureRays: beyond, a forward pass gives
-// a ray's four lanes one walk (four walks / one, us: 40 000 rays 322 / 334, 65 000 rays 474 / 380, 130 000 rays 785 / 660).
-constexpr int64_t kGroupMaxRays = 1 << 17, kGroupMaxPictureRays = 40960;
+// kGroupMaxRays: with more rays than fill the chip four lanes to a ray, or pieces of it, are work done several times over.
+constexpr int64_t kGroupMaxRays = 1 << 17;
 
 int group_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays) {
     if ((g_debug_flags & 1) || tree->dtype != SVOX_F64 || tree->N != 2 || tree->weight_accum || n_rays > kGroupMaxRays ||
@@ -434,11 +432,12 @@ int group_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t 
     return tree->data_dim == 3 * D + 1 ? D : -1;
 }
 
-// Rays that a wavefront of those kernels is dealt, and log2 of the pieces a ray is walked in at most (at least 2).
+// Rays that a wavefront of those kernels is dealt, and log2 of the pieces a ray is walked in at most (at least 2); none dealt: four
+// lanes walk a ray together.
 struct Cut {
     int per_wave = 0, most = 6;
 };
-Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays) {
+Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     Cut c;
     const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : tuning().cut;
     if (forced > 0) {
@@ -446,25 +445,50 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays) {
         c.most = std::min(std::max(forced / 100, 2), 6);
         return c;
     }
-    // As many pieces as still are some leaves long -- in a 16^3 grid (up to 16 384 cells) eight, to 64^3 twice as many for twice the
-    // resolution -- while the wavefronts have room on the GPU, fewer with more rays; what was measured beside it, us, forward pass and
-    // gradient of a dense tree, by the rays of a wavefront and the pieces (rays x pieces):
-    //   16^3   1 000 rays 8 x 8 39, 47   4 x 16 95, 100   16 x 4 42, 63     20 000 rays 16 x 4 53, 77   8 x 8 81, 101
-    //   32^3   5 000 rays 4 x 16 58, 93  8 x 8 59, 127    2 x 32 134, 182   20 000 rays 8 x 8 107, 229  4 x 16 182, 259
-    //   64^3   1 000 rays 2 x 32 46, 78  1 x 64 68, 79    4 x 16 55, 102    20 000 rays 4 x 16 175, 286 8 x 8 189, 405  2 x 32 291, 427
-    //   128^3  1 000 rays 1 x 64 65, 133 2 x 32 72, 144   4 x 16 99, 198    5 000 rays 4 x 16 112, 243  2 x 32 133, 252
+    // As many pieces as still are some leaves long, while the wavefronts have room on the GPU, fewer with more rays, and as few rays to a
+    // wavefront as leaves the lists room for all they find: the launcher cannot know how many leaves have density, so the lines are
+    // drawn where trees all of whose leaves do lose nothing or little.  What was measured (us; lanes that walk a ray together / pieces, in
+    // parentheses where they are not taken; half of the leaves with density, all of them):
+    //   forward           1 000 rays                5 000                  20 000                  24 000
+    //   8^3 SH1           -, 25 / (-, 32)           -, 27 / (-, 43)        -, 30 / (-, 35)
+    //   16^3 SH4          57, 58 / 31, 36           58, 60 / 39, 45        67, 70 / 49, 60         68, 70 / (51, 73)
+    //   32^3 SH9          133, 139 / 50, 55         138, 145 / 59, 70      159, 167 / 104, 164     158, 164 / (107, 168)
+    //   64^3 SH4          225, 231 / 56, 65         260, 268 / 77, 109     296, 305 / 172, 277     296, 305 / (205, 320)
+    //   128^3 SH4         512, 521 / 61, 88         528, 543 / 130, 241    595, 619 / 370, 565     594, 611 / (416, 637)
+    //   shell 128^3 SH9   215, 239 / 79, 89         276, 305 / 91, 120     311, 337 / 201, 281     28 672: 313, 340 / (277, 373)
+    //   shell 256^3 SH9   295, 316 / 95, 101        375, 426 / 122, 175    429, 475 / 258, 365     28 672: 409, 446 / (349, 480)
+    //   gradient          1 000 rays                20 000                 24 000                  40 960                    65 536
+    //   16^3 SH4          89, 118 / 50, 72          112, 149 / 96, 164     117, 165 / (106, 201)   192, 265 / (174, 277)     266, 367 / (249, 462)
+    //   32^3 SH9          222, 306 / 80, 146        281, 381 / 223, 385    297, 424 / 263, 436     508, 690 / 404, 610       709, 1007 / 624, 951
+    //   64^3 SH4          382, 539 / 79, 139        442, 643 / 292, 655    463, 688 / 427, 653     766, 1131 / 694, 1033     1084, 1589 / (810, 1773)
+    //   128^3 SH4         910, 1211 / 128, 230      1129, 1489 / 683, 1336 1117, 1526 / (713, 1517) 1861, 2603 / 1147, 2452  2565, 3688 / (1769, 3779)
+    //   shell 128^3 SH9   396, 556 / 115, 146       534, 742 / 321, 640    600, 794 / 399, 738     795, 1163 / 576, 1085     1082, 1669 / 881, 1637
+    //   shell 256^3 SH16  809, 1145 / 214, 262      1023, 1519 / 631, 1250 1054, 1732 / 708, 1493  1324, 2241 / 1011, 2147   1866, 3104 / 1485, 3207
+    // Lanes that walk together fill the GPU with 32 768 rays of a gradient, and take a second turn for the next: there pieces gain once more.
+    // Full trees lose on the near side of some lines: 3 % of a 64^3 SH16 gradient, 9 % of a 16^3 one and 10 % of the forward pass of a 64^3 shell
+    // at 20 000 rays, 5 % of a 128^3 RGBA gradient at 40 960.
     const double cells = (double)tree->capacity * 8.0;
-    if (cells < 16384.0) {
-        c.per_wave = n_rays <= 8192 ? 8 : 16;
-        c.most = n_rays <= 8192 ? 3 : 2;
-    } else if (cells < 131072.0) {
-        c.per_wave = n_rays <= 8192 ? 4 : 8;
-        c.most = n_rays <= 8192 ? 4 : 3;
-    } else if (cells < 1048576.0) {
-        c.per_wave = n_rays <= 2560 ? 2 : 4;
-        c.most = 5;
+    const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
+    const bool grid = like_complete_octree(tree);
+    constexpr int64_t kFill = 20480;
+    if (tiny && !(gradient && n_rays <= 2560)) return c;
+    if (n_rays > kFill) {
+        if (!gradient || small || (!grid && n_rays > 65536)) return c;
+        if (grid && !medium && n_rays > (large ? kFill : 24576) && (n_rays <= 32768 || n_rays > 40960)) return c;
+    }
+    if (small) {
+        c.per_wave = n_rays <= 14336 ? 8 : 12;     // (8 rays to each of 1 792 wavefronts, all that run at once)
+        c.most = n_rays <= 14336 ? 3 : 2;
+    } else if (medium) {
+        const bool short_lists = n_rays <= 8192 || (gradient && n_rays > 14336);
+        c.per_wave = short_lists ? 4 : 8;
+        c.most = short_lists ? 4 : 3;
     } else {
-        c.per_wave = n_rays <= 1280 ? 1 : n_rays <= 2560 ? 2 : 4;
+        // (of a 128^3 grid the lists hold the leaves of two rays, four in a pinch: 4 x 16 / 2 x 32, gradient 20 000 rays 787, 1542 / 683, 1336,
+        // forward pass 12 000 rays 229, 417 / 235, 364, 20 000 rays 336, 623 / 370, 565)
+        const bool two = grid && (large ? gradient || n_rays > 16384 : n_rays > kFill);
+        c.per_wave = large && n_rays <= 1280 ? 1 : n_rays <= 2560 || two ? 2 : 4;
+        c.most = large ? 6 : 5;
     }
     return c;
 }
@@ -744,13 +768,12 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            if (items > kGroupMaxPictureRays && !(g_debug_flags & 32)) {
+            const Cut cut = group_cut(tree, items, false);
+            if (cut.per_wave > 0)
+                launch_group_forward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt, (double*)out,
+                                     cut.per_wave, cut.most);
+            else
                 launch_shared_forward(D, dim3(blocks_for(items, kSharedRays)), stream, make_tree<double>(tree), src, *opt, (double*)out);
-                return;
-            }
-            const Cut cut = group_cut(tree, items);
-            launch_group_forward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt, (double*)out,
-                                 cut.per_wave, cut.most);
             return;
         }
     }
@@ -828,9 +851,13 @@ void launch_backward(const SvoxTreeSpec* tree, const Source& src, const SvoxRend
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            const Cut cut = group_cut(tree, items);
-            launch_group_backward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt,
-                                  (const double*)grad_out, (double*)grad_data, cut.per_wave, cut.most);
+            const Cut cut = group_cut(tree, items, true);
+            if (cut.per_wave > 0)
+                launch_group_backward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt,
+                                      (const double*)grad_out, (double*)grad_data, cut.per_wave, cut.most);
+            else
+                launch_shared_backward(D, dim3(blocks_for(items, kSharedRays)), stream, make_tree<double>(tree), src, *opt,
+                                       (const double*)grad_out, (double*)grad_data);
             return;
         }
     }

@@ -197,3 +197,47 @@ def test_many_pieces_are_not_walked_in_vain(gpu, dtype):
     many, fewer = (sorted(times[k])[3] for k in (64, 32))
     print(f"[pieces] {dtype}: 64 to a ray {many * 200:.0f} us, 32 {fewer * 200:.0f} us", flush=True)
     assert many <= 2 * fewer
+
+
+@pytest.mark.parametrize("levels,n", [(2, 2560), (3, 14336), (3, 14337), (3, 20480), (3, 20481), (4, 8193), (4, 14337), (4, 20481), (4, 70001), (5, 20480), (5, 20481),
+                                      (5, 24577), (5, 32769), (5, 40961), (6, 1281), (6, 16385), (6, 20481), (6, 32769), (1, 2560), (1, 2561)])
+def test_double_precision_rules(gpu, levels, n):
+    """On either side of the lines between the splits, and between pieces and lanes that walk a ray together."""
+    gen = torch.Generator(device=gpu).manual_seed(levels)
+    tree = svox.N3Tree(N=2, data_format="SH1", init_refine=levels, device=gpu, dtype=torch.float64)
+    tree.data.data.normal_(generator=gen)
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.2 + 0.01
+    rs, opt, spec = rays_spec(synth.sphere_rays(n, seed=3, dtype=torch.float64), gpu), options(tree, step_size=1e-3), tree._spec()
+    go = torch.randn(n, 3, generator=gen, device=gpu, dtype=torch.float64)
+    want, ref = run(1, lambda: (C.volume_render(spec, rs, opt), C.volume_render_backward(spec, rs, opt, go)))
+    assert torch.equal(C.volume_render(spec, rs, opt), want)
+    # (up to n terms of a leaf in another order: n * 2^-53 of the sum of their sizes at most, which cancels to a hundredth of it)
+    got = C.volume_render_backward(spec, rs, opt, go)
+    assert (got - ref).abs().max() <= n * 1.2e-14 * ref.abs().max()
+
+
+@pytest.mark.parametrize("gradient,n", [(False, 40960), (True, 131072)])
+def test_full_trees_in_double_precision_take_the_faster_kernel(gpu, gradient, n):
+    """Every leaf of a 128^3 grid has density: lists of pieces run over, and lanes that walk a ray together are faster.  (Forward pass of
+    40 960 rays 670 us, in pieces 1 056; gradient of 131 072 rays 6 338, in pieces 7 670 us.)"""
+    tree = svox.N3Tree(N=2, data_format="SH4", init_refine=6, device=gpu, dtype=torch.float64)
+    tree.data.data.normal_(generator=torch.Generator(device=gpu).manual_seed(2))
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.1 + 0.01
+    rs, opt, spec = rays_spec(synth.sphere_rays(n, seed=3, dtype=torch.float64), gpu), options(tree, step_size=1e-3), tree._spec()
+    go = torch.randn(n, 3, device=gpu, dtype=torch.float64)
+    times = {"rule": [], "pieces": []}
+    for _ in range(5):
+        for way, flags in (("rule", 0), ("pieces", 32 | 604 << 8)):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+            def passes():
+                begin.record()
+                for _ in range(2):
+                    C.volume_render_backward(spec, rs, opt, go) if gradient else C.volume_render(spec, rs, opt)
+                end.record()
+            run(flags, passes)
+            end.synchronize()
+            times[way].append(begin.elapsed_time(end))
+    rule, pieces = (sorted(times[k])[2] for k in ("rule", "pieces"))
+    print(f"[double] {n} rays, gradient {gradient}: {rule * 500:.0f} us, in pieces {pieces * 500:.0f} us", flush=True)
+    assert rule <= 0.92 * pieces
