@@ -682,24 +682,29 @@ constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 
 // How a forward pass cuts its rays into pieces (cut_kernel.h); no rays dealt to a wavefront: it does not.
 // The pieces pay as long as they find the GPU idle: what each of them walks in vain -- the leaves until two walks agree -- is
-// as much as a fair part of it, and the more of them the shorter.  A tree is small (up to 32^3 leaves: rays of few leaves), large (from
-// 128^3, or the surface of 256^3, on) or between.  The launcher cannot know how many rays meet the cube, so the rule is drawn where a
-// launch of rays that all do gains nothing more.  us, march with notes and without, from end to end / in pieces, rays that all hit:
-//   16^3 SH4     1 000 rays 43, 40 / 28, 22    4 000 42, 39 / 31, 25    8 000 42, 40 / 34, 26    16 000 43, 40 / 63, 44
-//   32^3 SH9     1 000 rays 84, 81 / 36, 29    4 000 81, 79 / 41, 32    8 000 83, 78 / 48, 42    16 000 88, 80 / 94, 69
-//   64^3 SH9     1 000 rays 165, 160 / 47, 39  4 000 204, 199 / 68, 67  12 000 202, 197 / 165, 123  16 000 202, 197 / 205, 144
-//   128^3 SH9    1 000 rays 418, 412 / 72, 63  4 000 413, 410 / 145, 135  8 000 416, 412 / 255, 184  12 000 424, 418 / 303, 247
-//   shells  128^3 SH4   1 000 rays 153, 154 / 50, 58   4 000 154, 153 / 101, 86   8 000 192, 192 / 177, 152  12 000 193, 194 / 227, 180
-//           256^3 SH9   1 000 rays 196, 193 / 60, 55   4 000 261, 256 / 169, 121  8 000 311, 308 / 270, 199  12 000 271, 270 / 334, 255
-//           512^3 SH16  1 000 rays 235, 235 / 99, 108  4 000 332, 333 / 209, 180  8 000 349, 350 / 351, 270  12 000 332, 332 / 436, 365
-// 18 % of the rays hit: 64^3 shell 4 000 rays 83, 80 / 42, 35; 256^3 4 000 169, 166 / 63, 57, 8 000 169, 165 / 89, 72; 512^3 4 000 224, 225 / 97, 108,
-// 8 000 224, 223 / 110, 110.  With the shifted softplus, where every leaf is listed and rays end behind what they met (opaque_light):
-// 32^3 4 000 rays 101, 85 / 59, 54, 12 000 122, 91 / 146, 102; 128^3 4 000 473, 442 / 315, 277, 12 000 499, 463 / 994, 495; 256^3 shell 4 000 75, 70 /
-// 63, 49, 8 000 78, 73 / 92, 53, 12 000 78, 74 / 119, 75; 512^3 shell 4 000 78, 76 / 76, 62.
-// Square pictures of 64 and 90 pixels a side (4 096, 8 100):
-//   16^3   27, 23 / 22, 18      28, 23 / 25, 21       64^3   89, 83 / 37, 30      127, 113 / 44, 31
-//   128^3  206, 192 / 59, 52    242, 237 / 96, 49     512^3 shell  177, 115 / 59, 44  259, 188 / 61, 49
-//   NDC, every ray in the tree, 256^3 and 512^3  133, 86 / 108, 49  151, 114 / 172, 79;  227, 129 / 225, 83  245, 158 / 335, 116
+// as much as a fair part of it, and the more of them the shorter; and as long as the lists hold what they find, which the more rays of a wavefront and
+// the more leaves with density fills them the sooner.  The launcher knows neither how many rays meet the cube nor how many leaves have
+// density, so the lines are drawn where launches of rays that all do gain nothing more and, within some per cent, trees all of whose
+// leaves do lose nothing.  Trees are grids (like_complete_octree) or sparse ones, small (up to 32^3 leaves), fine (from 64^3, or the
+// surface of 128^3, on) or large (128^3, the surface of 256^3).  us, march without notes and with, from end to end / in pieces, rays that all hit, half of
+// a grid's leaves empty and a shell's all but the surface | no leaf empty:
+//                1 000 rays                              4 096                                   8 192 (with notes, shells: 7 168)
+//   8^3 SH1      not taken                               | 20, 26 / 34, 36 if it were
+//   32^3 SH9     80, 80 / 27, 34    | 83, 92 / 40, 44    77, 77 / 41, 52     | 80, 91 / 53, 61    79, 82 / 53, 54      | 83, 107 / 76, 82
+//   64^3 SH9     153, 153 / 37, 45  | 171, 194 / 65, 62  194, 192 / 72, 62   | 216, 234 / 104, 115   197, 196 / 110, 115 | 218, 237 / 154, 169
+//   128^3 SH4    377, 377 / 62, 74  | 395, 423 / 86, 99  390, 387 / 112, 141 | 406, 432 / 245, 224   403, 400 / 192, 259 | 416, 437 / 361, 372
+//   shell 128^3 SH9   128, 126 / 54, 60   | 131, 135 / 92, 76   170, 169 / 87, 99    | 185, 194 / 110, 127   180, 180 / 116, 149 | 187, 195 / 163, 206
+//   shell 256^3 SH9   178, 173 / 48, 57   | 181, 188 / 83, 86   260, 257 / 114, 167  | 273, 273 / 150, 222   272, 242 / 185, 198 | 276, 254 / 249, 333
+// (10 000 rays: 64^3 SH9 204, 204 / 132, 147 | 227, 247 / 183, 210, 128^3 417, 414 / 204, 304 | 435, 459 / 419, 447.  Of views from afar, 18 % of whose
+// rays hit a shell, 7 000 with notes take 169 / 89 at 256^3: for those the line of a full shell, 6 000 rays, is passed over.)
+// With the shifted softplus every leaf is listed and rays end behind what they met (opaque_light), from end to end as in pieces.  A shell of 256^3,
+// without notes and with: 1 000 rays 74, 80 / 45, 61, 4 096 84, 95 / (116, 186).
+// Square pictures, 64, 90 pixels a side, from close up (every pixel hits) and from afar, half empty | full:
+//   64^3 SH9          121, 145 / 63, 60, 100, 105 / 32, 40 | 165, 210 / 93, 97     121, 140 / 86, 140 | 157, 191 / 136, 198
+//   128^3 SH4         299, 302 / 115, 129, 209, 222 / 43, 57 | 351, 389 / 167, 218 273, 274 / 182, 279 | 321, 353 / 296, 403
+//   shell 128^3 SH9   142, 149 / 69, 80 | 193, 218 / 91, 116                       149, 159 / 117, 150 | 198, 224 / 158, 210
+//   shell 256^3 SH9   225, 225 / 111, 123 | 257, 285 / 143, 175                    223, 222 / 203, 224 | 266, 295 / 267, 316
+//   NDC, every ray in the tree, half empty, 256^3 and 512^3  133, 86 / 108, 49  151, 114 / 172, 79;  227, 129 / 225, 83  245, 158 / 335, 116 (with notes, without)
 Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRenderOptions* opt, bool noted) {
     const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : g_debug_flags == 0 ? tuning().cut : 0;
     Cut c;
@@ -709,23 +714,42 @@ Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRend
         return c;
     }
     const double cells = (double)tree->capacity * tree->N * tree->N * tree->N;
-    const bool small = cells < 65536.0, large = cells >= 1048576.0, grid = like_complete_octree(tree);
-    int64_t limit = small ? 8192 : grid ? 12288 : image ? 9216 : noted ? 7168 : 8192;   // (of a picture: in blocks of 16 x 16)
-    if (opt->density_softplus) limit = noted || small ? 4096 : 8192;
+    const bool tiny = cells < 2048.0, small = cells < 65536.0, large = cells >= 1048576.0;
+    const bool grid = like_complete_octree(tree), sparse = !grid && !small, fine = cells >= 262144.0;
+    const bool softplus = opt->density_softplus;
+    if (tiny) return c;
     if (image && opt->ndc_width > 0) {
         if (items <= (noted ? 4096 : 8192)) c.per_wave = small ? 8 : 4;
-    } else if (items <= limit) {
-        if (image) {
-            // (most pixels of a picture miss: a wavefront finds one ray or two among four, or eight)
-            c.per_wave = large ? 4 : 8;
-            c.most = large ? 6 : 4;
-        } else if (small) {
-            c.per_wave = items <= 4096 ? 4 : 8;
-        } else if (large) {
-            c.per_wave = items <= (grid ? 1536 : 4096) ? 1 : items <= 8192 || !noted ? 2 : 4;
-        } else {
-            c.per_wave = items <= (grid ? 2048 : 4096) ? 2 : 4;
-        }
+        return c;
+    }
+    int64_t limit = 8192;
+    if (image && !small) limit = grid && !noted ? 12288 : 9216;   // (in blocks of 16 x 16)
+    if (!image && !small) limit = grid ? 10240 : noted ? 7168 : 8192;
+    if (softplus) limit = small ? 4096 : grid ? (noted ? 4096 : 8192) : noted ? (image ? 1024 : 2048) : image ? 4096 : 3072;
+    if (items > limit) return c;
+    if (image) {
+        // (most pixels of a picture miss: a wavefront finds one ray or two among its few)
+        if (small || (grid && !large && items > 9216))
+            c.per_wave = 8, c.most = 4;
+        else if (!large && (grid || !fine))
+            c.per_wave = 4, c.most = 4;
+        else if (sparse && large && !noted && !softplus)
+            c.per_wave = 1;
+        else if (sparse && !large && noted && items > 8192)
+            c.per_wave = 4;
+        else
+            c.per_wave = 2, c.most = 5;
+    } else if (small) {
+        c.per_wave = items <= 4096 || (cells >= 16384.0 && !noted) ? 4 : 8;
+    } else if (!large) {
+        if (noted)
+            c.per_wave = items <= 2048 || (sparse && fine) ? 2 : 4;
+        else
+            c.per_wave = items > 4096 && items <= 6144 && (grid || !fine) ? 4 : 2;
+    } else if (grid) {
+        c.per_wave = items <= 1536 ? 1 : 2;
+    } else {
+        c.per_wave = items <= (softplus ? 1024 : noted ? 4096 : 8192) ? 1 : 2;
     }
     return c;
 }

@@ -241,3 +241,35 @@ def test_full_trees_in_double_precision_take_the_faster_kernel(gpu, gradient, n)
     rule, pieces = (sorted(times[k])[2] for k in ("rule", "pieces"))
     print(f"[double] {n} rays, gradient {gradient}: {rule * 500:.0f} us, in pieces {pieces * 500:.0f} us", flush=True)
     assert rule <= 0.92 * pieces
+
+
+@pytest.mark.parametrize("levels,fmt,n,noted", [(2, "SH1", 4096, False), (6, "SH4", 10000, True), (5, "SH9", 0, True)])
+def test_full_trees_are_not_slower_in_pieces(gpu, levels, fmt, n, noted):
+    """Trees without empty leaves, whose lists of pieces run over, and tiny ones.  (End to end, rule before the lines were drawn for them and now, us:
+    8^3, 4 096 rays 20, 34, 20; 128^3, 10 000 rays with notes 459, 727, 447; 64^3, a picture of 96 x 128 pixels with notes from close up 189, 352, 191.)"""
+    tree = svox.N3Tree(N=2, data_format=fmt, init_refine=levels, device=gpu)
+    tree.data.data.normal_(generator=torch.Generator(device=gpu).manual_seed(2))
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.1 + 0.01
+    spec, opt = tree._spec(), options(tree, step_size=1e-3)
+    if n:
+        rs = rays_spec(synth.sphere_rays(n, seed=5), gpu)
+        f = (lambda: C.volume_render_noted(spec, rs, opt)) if noted else (lambda: C.volume_render(spec, rs, opt))
+    else:
+        cam = cam_spec(synth.orbit_poses(1, seed=1, radius=1.2)[0], 96, 128, 1.39 * 128, device=gpu)
+        f = lambda: C.volume_render_images_noted(spec, cam, opt)
+    times = {"rule": [], "end to end": []}
+    for _ in range(7):
+        for way, flags in (("rule", 0), ("end to end", 8)):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+            def passes():
+                begin.record()
+                for _ in range(20):
+                    f()
+                end.record()
+            run(flags, passes)
+            end.synchronize()
+            times[way].append(begin.elapsed_time(end))
+    rule, marched = (sorted(times[k])[3] for k in ("rule", "end to end"))
+    print(f"[pieces] {levels} {n}: {rule * 50:.0f} us, from end to end {marched * 50:.0f} us", flush=True)
+    assert rule <= 1.2 * marched
