@@ -176,20 +176,14 @@ struct BatchSource {
     }
 };
 
-// Rays of a batch that meet the cube, for noting passes (list_hits_kernel): item i is ray list[i]; without a list, those of the batch.
-// A pass of which only the device knows how many rays it has is launched in several shapes; each has items only if there are as many
-// as it is made for.
+// Rays of a batch that meet the cube, for noting passes (list_hits_kernel): item i is ray list[i].
 struct ListedSource : BatchSource<float> {
     const int32_t* list;
     const unsigned long long* n_listed;
-    int64_t least, most;     // rays listed, for this launch to have any
-    __device__ __forceinline__ int64_t total() const {
-        const int64_t n = (int64_t)*n_listed;
-        return n < least || n > most ? 0 : list ? n : BatchSource<float>::total();
-    }
+    __device__ __forceinline__ int64_t total() const { return (int64_t)*n_listed; }
     __device__ __forceinline__ int64_t fetch_item(int64_t i, const SvoxRenderOptions& opt, const float* offset,
                                                   const float* scaling, float* origin, float* dir, float* vdir) const {
-        return BatchSource<float>::fetch_item(list ? (int64_t)list[i] : i, opt, offset, scaling, origin, dir, vdir);
+        return BatchSource<float>::fetch_item(list[i], opt, offset, scaling, origin, dir, vdir);
     }
 };
 
@@ -888,6 +882,13 @@ struct ReplaySpace {
     uint32_t march_blocks;
     uint32_t* clear_at[2];
     int64_t clear_words;
+    // A pass of which only the device knows how many rays it has (list_hits_kernel) is launched in several shapes: this launch does its
+    // work if there are at least, and at most, as many as it is made for.  nullptr: it does.
+    const unsigned long long* n_listed;
+    int64_t least, most;
+    __device__ __forceinline__ bool chosen() const {
+        return n_listed == nullptr || ((int64_t)*n_listed >= least && (int64_t)*n_listed <= most);
+    }
 };
 
 // The arrays a gradient is going to be added to are cleared by further blocks of the launch that takes the notes for it: that one waits
@@ -1138,6 +1139,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
     if constexpr (kNoted) {
+        if (!ws.chosen()) return;
         if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
     }
     const int lane = threadIdx.x;
@@ -1898,6 +1900,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ SplitBox box;
     if constexpr (kNoted) {
+        if (!ws.chosen()) return;
         if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
         if (blockIdx.x == 0 && threadIdx.x < kStampWords) ws.stamp_at[threadIdx.x] = ws.stamp[threadIdx.x];
     }

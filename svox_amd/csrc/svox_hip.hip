@@ -901,26 +901,39 @@ BatchSource<T> noting_shape(BatchSource<T> s) {
 template <typename T>
 ImageSource<T> noting_shape(const ImageSource<T>& s) { return s; }
 
-// The forward pass of a training step: the picture into `out` and, in the workspace, the notes of
-// every ray under `stamp`.  Needs a usable workspace and the octree kernels, which noted_ok() tells
-// beforehand.  A launch that does not fill the GPU runs on two wavefronts per 64 rays.  out may be
-// nullptr (notes only); grad_out, if given, is the gradient of the picture the backward pass will be
-// called with: the notes' heads then also carry the sum of that pass's first march.
 // The rays of a batch that meet the cube, in the order they come in block by block (the blocks as they get there); the others are
 // answered as a noting pass answers them.  200 003 rays 9 us, 1 Mi rays 30: 24 bytes
-// read of each, and a line written for every one that misses, the head of its notes.
+// read of each, and a line written for every one that misses, the head of its notes.  Where a sample of the rays says that more than
+// `most` hit, nothing is listed (4.5 us), and the number stands for the batch as it is.
 constexpr int kListThreads = 1024;
+constexpr int kListSample = 256;
 __global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> tr, BatchSource<float> src, SvoxRenderOptions opt,
                                                                         float* __restrict__ out, ReplaySpace ws,
-                                                                        unsigned long long* __restrict__ n_listed) {
+                                                                        unsigned long long* __restrict__ n_listed, int64_t most) {
     __shared__ int32_t hits[kListThreads / kMarchThreads];
     __shared__ unsigned long long first;
     float offset[3], scaling[3], origin[3], dir[3], vdir[3];
     load_transform(tr, offset, scaling);
     const int wave = threadIdx.x / kMarchThreads, lane = threadIdx.x & (kMarchThreads - 1);
     src.n_waves = 0;
-    const int64_t slot = src.fetch_item(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
     RayState<float> r;
+    // (the same rays for every block, which all come to the same answer)
+    if (threadIdx.x < kListSample) {
+        const int64_t some = (int64_t)threadIdx.x * src.rays.n_rays / kListSample;
+        src.fetch_item(some, opt, offset, scaling, origin, dir, vdir);
+        const unsigned long long m = __ballot(setup_ray(r, origin, dir, scaling));
+        if (lane == 0) hits[wave] = __popcll(m);
+    }
+    __syncthreads();
+    int sampled = 0;
+#pragma unroll
+    for (int i = 0; i < kListSample / kMarchThreads; ++i) sampled += hits[i];
+    if (sampled * src.rays.n_rays > kListSample * most) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *n_listed = (unsigned long long)src.rays.n_rays;
+        return;
+    }
+    __syncthreads();
+    const int64_t slot = src.fetch_item(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
     const bool hit = slot >= 0 && setup_ray(r, origin, dir, scaling);
     if (slot >= 0 && !hit) {
         if (out) {
@@ -952,8 +965,9 @@ __global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> 
 //   256^3 shell SH9   200 003 rays 339, 483, 577 / 290, 413, 524   300 000 rays 405, 573, 665 / 317, 450, 568   500 000 rays 566, 794, 921 / 332, 518, 680
 //   512^3 shell SH16  170 000 rays 452, 820 / 383, 723   500 000 rays 775, 1208 / 457, 870   1 048 576 rays 749, 1332 / 708, 1313
 //   512^3 shell SH25  400 000 rays 727, 1389 / 453, 1025    256^3 shell SH4 700 000 rays 458, 632, 741 / 344, 505, 632
-// Where all of them hit, the listing and the launches without rays are lost: 256^3 shell SH9 200 003 rays 563, 1072, 1469 / 577, 1084, 1492,
-// 500 000 rays 1102, 2183, 3108 / 1127, 2205, 3121, 64^3 SH9 200 000 rays 648, 1832, 2840 / 667, 1835, 2846.
+// Where all of them hit, what the sample, the launches without rays and the look at which launch has them cost (the noting march, the gradient,
+// the squared error; not listed / listed): 256^3 shell SH9 200 003 rays 540, 1044, 1463 / 548, 1039, 1457, 500 000 rays 1096, 2190, 3129 / 1105,
+// 2189, 3124, 1 000 000 rays 1938, 3949, 5804 / 1951, 3967, 5800; 64^3 SH9 200 003 rays 663, 1877, 2854 / 673, 1893, 2863.
 struct ListShapes {
     bool any = false;
     int64_t two = 0, one = 0;
@@ -981,6 +995,11 @@ struct ClearWork {
 };
 constexpr int64_t kMostCleared = kClearWords * 4 * (1 << 24);   // (a launch has fewer than 2^32 threads)
 
+// The forward pass of a training step: the picture into `out` and, in the workspace, the notes of
+// every ray under `stamp`.  Needs a usable workspace and the octree kernels, which noted_ok() tells
+// beforehand.  A launch that does not fill the GPU runs on two wavefronts per 64 rays.  out may be
+// nullptr (notes only); grad_out, if given, is the gradient of the picture the backward pass will be
+// called with: the notes' heads then also carry the sum of that pass's first march.
 template <class Source>
 int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, void* out,
                  void* workspace, int64_t workspace_bytes, int64_t n_slots, const NoteStamp& stamp,
@@ -997,7 +1016,7 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.spin_limit = (g_debug_flags & 16) ? 1 : 0;
     ws.give_ups = give_up_counter();
-    // (the first launch clears what is to be cleared)
+    // (the launch that has the rays clears what is to be cleared)
     ws.clear_at[0] = (uint32_t*)clear.at[0];
     ws.clear_at[1] = (uint32_t*)clear.at[1];
     ws.clear_words = clear.bytes / 4;
@@ -1022,28 +1041,31 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
         const ListShapes shapes = list_shapes(tree, opt, src.rays.n_rays, at_once);
         if (ws.list && shapes.any) {
             unsigned long long* const n_listed = ws.stocks_taken + 2;
-            hipLaunchKernelGGL(list_hits_kernel, dim3(blocks_for(src.rays.n_rays, kListThreads)), dim3(kListThreads), 0, stream,
-                               march_tree(tree, opt), src, *opt, (float*)out, ws, n_listed);
-            auto launch = [&](const Source& s, const int32_t* list, int64_t least, int64_t most, bool two, bool refilled) {
-                ListedSource listed;
-                (Source&)listed = s;
-                listed.list = list;
-                listed.n_listed = n_listed;
-                listed.least = least;
-                listed.most = most;
-                const int64_t items = list ? std::min(most, s.rays.n_rays) : s.rays.n_rays;
-                const dim3 grid = with_clearing(blocks_for(items, s.per_wave));
-                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, ListedSource>::noting(
-                                            grid, stream, march_tree(tree, opt), listed, *opt, (float*)out,
-                                            ws, (const float*)grad_out, (const float*)color_ref, two, refilled));
-                ws.clear_words = 0;
-            };
-            Source tiles = src;
-            tiles.per_wave = kMarchThreads;
-            if (shapes.two > 0) launch(tiles, ws.list, 0, shapes.two, true, false);
-            if (shapes.one > shapes.two) launch(tiles, ws.list, shapes.two + 1, shapes.one, false, false);
             const int64_t listed = std::max(shapes.one, shapes.two);
-            if (src.rays.n_rays > listed) launch(dealt, nullptr, listed + 1, INT64_MAX, false, refill);
+            hipLaunchKernelGGL(list_hits_kernel, dim3(blocks_for(src.rays.n_rays, kListThreads)), dim3(kListThreads), 0, stream,
+                               march_tree(tree, opt), src, *opt, (float*)out, ws, n_listed, listed);
+            ws.n_listed = n_listed;
+            auto launch_listed = [&](int64_t least, int64_t most, bool two) {
+                ListedSource tiles;
+                (Source&)tiles = src;
+                tiles.per_wave = kMarchThreads;
+                tiles.list = ws.list;
+                tiles.n_listed = n_listed;
+                ws.least = least;
+                ws.most = most;
+                const dim3 grid = with_clearing(blocks_for(std::min(most, src.rays.n_rays), kMarchThreads));
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, ListedSource>::noting(grid, stream, march_tree(tree, opt), tiles, *opt, (float*)out,
+                                                                             ws, (const float*)grad_out, (const float*)color_ref, two, false));
+            };
+            if (shapes.two > 0) launch_listed(0, shapes.two, true);
+            if (shapes.one > shapes.two) launch_listed(shapes.two > 0 ? shapes.two + 1 : 0, shapes.one, false);
+            if (src.rays.n_rays > listed) {
+                ws.least = listed > 0 ? listed + 1 : 0;
+                ws.most = INT64_MAX;
+                const dim3 grid = with_clearing(blocks);
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(grid, stream, march_tree(tree, opt), dealt, *opt, (float*)out, ws,
+                                                                       (const float*)grad_out, (const float*)color_ref, false, refill));
+            }
             return SVOX_OK;
         }
     }
