@@ -1193,16 +1193,18 @@ SvoxRenderOptions without_thresholds(const SvoxRenderOptions* opt) {
 }
 
 // Whether the arrays of a gradient are cleared by the launch that takes its notes: aligned as clear_share stores, not more than a
-// launch has blocks for, and beside a march that leaves the memory room: a gigabyte and more beside one of half a million rays is
-// cleared no faster than before it, and slows it.  us, apart / on the way:
-//   squared error, 256^3 SH9 shell (345 MB)          5 000 rays 190 / 147  20 000 350 / 299  100 000 422 / 363  200 003 524 / 471
-//                                                    300 000 rays 568 / 526  500 000 680 / 655
-//   gradient by itself, 512^3 SH16 shell (1.2 GB)    5 000 rays 347 / 274  50 000 584 / 497  170 000 723 / 631  300 000 778 / 750
-//                                                    500 000 rays 870 / 877  700 000 1129 / 1145;  SH25 (1.9 GB) 400 000 1024 / 1049
-constexpr int64_t kClearBeside = 512ll << 20, kClearRays = 1 << 18;
+// launch has blocks for, and beside a march that leaves the memory room: the more there is to clear the fewer rays that all hit do, and the march is
+// slowed.  us, apart / on the way:
+//   squared error, 256^3 SH9 shell (345 MB), 18 % hit  5 000 rays 190 / 147  20 000 350 / 299  100 000 422 / 363  200 003 543 / 425  500 000 680 / 655
+//                                            all hit   9 000 421 / 381  50 000 629 / 597  100 000 882 / 853  160 000 1173 / 1153  200 003 1463 / 1457
+//   256^3 SH16 shell (310 MB a gradient), all hit      gradient 20 000 476 / 429  160 000 1193 / 1177;  squared error 605 / 549  1625 / 1578
+//   512^3 SH16 shell (1.2 GB), all hit                 gradient 9 000 653 / 549  50 000 871 / 877  100 000 1072 / 1079  200 003 1616 / 1664
+//                                                      squared error 858 / 742  980 / 909  1184 / 1231  2331 / 2453
+//                              18 % hit                gradient 50 000 549 / 455  100 000 593 / 472  500 000 870 / 877;  squared error 50 000 744 / 640
 bool clears_on_the_way(const SvoxTreeSpec* tree, int64_t n_rays, const void* a, const void* b = nullptr) {
-    return ((uintptr_t)a & 15u) == 0 && ((uintptr_t)b & 15u) == 0 && data_bytes(tree) <= kMostCleared &&
-           (n_rays <= kClearRays || data_bytes(tree) * (b ? 2 : 1) <= kClearBeside);
+    if (((uintptr_t)a & 15u) != 0 || ((uintptr_t)b & 15u) != 0 || data_bytes(tree) > kMostCleared) return false;
+    const int64_t bytes = data_bytes(tree) * (b ? 2 : 1);
+    return bytes <= 512ll << 20 || n_rays <= (bytes <= 1ll << 30 ? 1 << 18 : bytes <= 2ll << 30 ? 1 << 17 : 1 << 15);
 }
 
 // The backward pass of a call that brings a workspace but no notes: one noting march without a picture

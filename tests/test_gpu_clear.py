@@ -52,3 +52,16 @@ def test_cleared_by_the_noting_launch(gpu, flags, N, levels, fmt):
             err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), what=f"call {k}")
             assert ok, (k, err)
             assert bool((a[b == 0] == 0).all()), k
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_much_to_clear_beside_many_rays(gpu, n):
+    """Arrays of 1.2 GB each, on either side of the number of rays from which on they are cleared before the march."""
+    tree = synth.shell_tree(depth=9, data_format="SH16", n_spheres=24, seed=0, device=gpu)
+    rs, opt, spec = rays_spec(synth.sphere_rays(n, seed=5), gpu), options(tree, step_size=5e-4), tree._spec()
+    target = torch.rand(n, 3, device=gpu)
+    dirty(tree.data.numel(), gpu)
+    got, want = C.se_grad(spec, rs, target, opt), C.se_grad(spec, rs, target, opt, workspace=False)
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        assert bool(torch.isfinite(a).all()) and bool((a[b == 0] == 0).all())
