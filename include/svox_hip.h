@@ -313,7 +313,8 @@ int64_t svox_volume_render_backward_workspace_bytes(int64_t n_rays, int32_t reco
 /* No counterpart in the reference.  How full a workspace of notes ran: after a call that takes notes
  * (svox_volume_render_noted, svox_volume_render_images_noted, the _ws calls) the 64-bit word at byte
  * *counter_offset of the workspace holds the number of 64-chunk stocks its wavefronts asked for
- * beyond the rays' own chunks, and the workspace has *pool_stocks of them (rounded up).  A count at
+ * beyond the rays' own chunks, and the workspace has *pool_stocks of them (rounded up; a batch of 131 072 rays and
+ * more gives up to n_rays / 6 144 of them to a list of its rays, which a picture of as many pixels has beside those).  A count at
  * or above that number says the shared chunks ran out: some rays' notes are incomplete (those rays are
  * marched by the backward pass: correct, slower) and a larger workspace would serve the same rays
  * better.  Returns 0, or SVOX_ERR_BAD_SHAPE for a workspace too small to hold n_rays chunks. */

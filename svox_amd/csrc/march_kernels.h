@@ -852,13 +852,14 @@ __device__ __forceinline__ int build_shade_list_all(Shared& sh, const int32_t* q
 // holds the index of the ray's next chunk.  Ray number i starts in chunk i; further chunks come
 // from the rest of the workspace, of which a wavefront takes a stock of 64 chunks at a time through
 // one atomic counter (a heavy image tile needs hundreds, most tiles none); the lanes that need a
-// chunk in the same step are ranked by ballot.
+// chunk in the same step are ranked by ballot.  (Rays in pieces take as many as they need through a second
+// counter, and keep the first in step: take_chunks.)
 constexpr int kStampWords = 6;   // ray count; tree data, child; ray origins, directions; step size and threshold
 struct ReplaySpace {
     float2* base;          // chunk c starts at base + c * kChunkFloat2
     int64_t first_shared;  // chunks [0, first_shared) are the rays' first chunks
-    int64_t n_chunks;      // chunks [first_shared, n_chunks) are handed out in stocks of kChunkStock
-    unsigned long long* stocks_taken;   // counter of the stocks handed out (zero when the launch starts)
+    int64_t n_chunks;      // chunks [first_shared, n_chunks) are handed out
+    unsigned long long* stocks_taken;   // counters, zero when the launch starts: stocks handed out; chunks handed out one by one; rays listed
     // the noting forward kernels write `stamp` (what the notes belong to) to stamp_at; replay_backward_kernel uses
     // the notes only if it finds its own stamp there
     unsigned long long* stamp_at;

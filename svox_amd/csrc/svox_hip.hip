@@ -828,14 +828,16 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
 }
 
 // The workspace of the replaying kernels: chunks of notes, then one bit per ray (rays left undone by
-// replay_backward_kernel), then 256 bytes that hold the stamp of the notes and, from byte 128 on, the
-// counter of the chunk stocks (cleared before every launch that takes notes).
+// replay_backward_kernel), then 256 bytes that hold the stamp of the notes and, from byte 128 on, three
+// counters (cleared before every launch that takes notes): the chunk stocks handed out, the chunks that rays in
+// pieces took one by one (take_chunks, which keeps the first in step), and the rays listed (list_hits_kernel).
 constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
-// (and, from kListRays rays on, where the rays' shared chunks are many beside it, in the place of the last of them: a number per ray.)
+// (and, of a batch of kListRays rays and more, where the rays' shared chunks are many beside it, in the place of the last of them: a number per
+// ray.  Every pass over the notes of a batch says that it is one, or the room they are in would not be the same.)
 constexpr int64_t kListRays = 1 << 17;
-bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, ReplaySpace* ws) {
+bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, bool batch, ReplaySpace* ws) {
     *ws = ReplaySpace{};
     int64_t chunks = workspace && n_slots > 0
                          ? (workspace_bytes - kTailBytes - bitmap_bytes(n_slots)) / kChunkBytes : 0;
@@ -843,7 +845,7 @@ bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, 
     ws->base = (float2*)workspace;
     ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
     const int64_t list_chunks = (n_slots * 4 + kChunkBytes - 1) / kChunkBytes;
-    if ((n_slots >= kListRays || (g_debug_flags & 64)) && chunks - n_slots >= 16 * list_chunks) {
+    if (batch && (n_slots >= kListRays || (g_debug_flags & 64)) && chunks - n_slots >= 16 * list_chunks) {
         chunks -= list_chunks;
         ws->list = (int32_t*)((char*)workspace + chunks * kChunkBytes);
     }
@@ -1009,7 +1011,7 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     const unsigned blocks = blocks_for(total_items_of(src), src.per_wave);
     const Source dealt = dealt_out(src, blocks);
     ReplaySpace ws;
-    if (D < 0 || !carve_workspace(workspace, workspace_bytes, n_slots, &ws))
+    if (D < 0 || !carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(src), &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "notes asked for where they cannot be taken");
     const int rc = zero_fill(ws.stocks_taken, 32, stream);
     if (rc) return rc;
@@ -1129,7 +1131,7 @@ bool noted_ok(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_
                      int64_t workspace_bytes) {
     if (!notes_possible(tree, opt)) return false;
     ReplaySpace ws;
-    return carve_workspace(workspace, workspace_bytes, n_slots, &ws);
+    return carve_workspace(workspace, workspace_bytes, n_slots, false, &ws);   // (whether there is room for a list does not matter)
 }
 
 NoteStamp stamp_of_image(const SvoxTreeSpec* tree, const SvoxCameraSpec* cam, int32_t n_images,
@@ -1166,7 +1168,7 @@ int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest
     const int ray_shift = replay_shift(n_slots);
     const unsigned replay_blocks = blocks_for(n_slots, 1 << ray_shift);
     ReplaySpace ws;
-    carve_workspace(workspace, workspace_bytes, n_slots, &ws);
+    carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(all), &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.report = (unsigned long long*)report;
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(replay_blocks), stream, all, *opt, (const float*)grad_output,
@@ -1263,7 +1265,7 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
     rc = check_launch("se_grad");
     if (rc) return rc;
     ReplaySpace ws;
-    carve_workspace(workspace, workspace_bytes, n_slots, &ws);
+    carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(all), &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     const int ray_shift = replay_shift(n_slots);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_se_grad(dim3(blocks_for(n_slots, 1 << ray_shift)), stream, all, *opt,
@@ -1586,7 +1588,7 @@ int svox_notes_pool_info(int64_t n_rays, int64_t workspace_bytes, int64_t* count
     ReplaySpace ws;
     // (any 16-byte aligned address does for the arithmetic)
     char* const base = (char*)(uintptr_t)4096;
-    if (!carve_workspace(base, workspace_bytes, n_rays, &ws))
+    if (!carve_workspace(base, workspace_bytes, n_rays, true, &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "svox_notes_pool_info: the workspace does not hold a chunk per ray");
     *counter_offset = (int64_t)((char*)ws.stocks_taken - base);
     *pool_stocks = ws.n_stocks;

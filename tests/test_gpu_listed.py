@@ -9,7 +9,7 @@ import torch
 
 from svox_amd import csrc as C
 from svox_amd import synth
-from util import grad_close, on_gpu, options, rays_spec
+from util import cam_spec, grad_close, on_gpu, options, rays_spec
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +109,25 @@ def test_batches_that_all_hit_are_hardly_slower(gpu):
     rule, plain = (sorted(times[k])[3] for k in (0, 4))
     print(f"[listed] all hit: {rule * 50:.0f} us, as it is {plain * 50:.0f} us", flush=True)
     assert rule <= 1.018 * plain
+
+
+def test_pictures_leave_no_room_for_a_list(gpu):
+    """All chunks of a picture's workspace are for notes; of a batch of as many rays, a number per ray is taken off."""
+    w, h = 512, 300
+    n = w * h
+    tree = synth.shell_tree(depth=5, data_format="SH1", n_spheres=6, seed=4)
+    spec, opt = on_gpu(tree, gpu)._spec(), options(tree, step_size=1e-3)
+    cam = cam_spec(synth.orbit_poses(1, seed=2, radius=3.0)[0], w, h, 1.4 * w, device=gpu)
+    go = torch.ones(n, 3, device=gpu) * 1e-2
+    report = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    chunks = lambda notes: (notes.numel() * 8 - 256 - 16 * ((n + 127) // 128)) // 384
+
+    notes = C.volume_render_images_noted(spec, cam, opt, records_per_ray=30)[1]
+    C.volume_render_images_backward_noted(spec, cam, opt, go.view(h, w, 3), notes, report.data_ptr())
+    torch.cuda.synchronize()
+    assert int(report[0]) & 0xffffffff == (chunks(notes) - n + 63) // 64
+    rs = rays_spec(synth.sphere_rays(n, seed=8), gpu)
+    notes = C.volume_render_noted(spec, rs, opt, records_per_ray=30)[1]
+    C.volume_render_backward_noted(spec, rs, opt, go, notes, report.data_ptr())
+    torch.cuda.synchronize()
+    assert int(report[0]) & 0xffffffff == (chunks(notes) - -(-n * 4 // 384) - n + 63) // 64 == C.notes_pool_use(notes, n)[1]
