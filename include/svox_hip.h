@@ -134,11 +134,11 @@ const char* svox_status_string(int status);
  * of that kernel give up at the first look that finds nothing (so that a test can see what a give-up leaves
  * behind; every kernel still ends normally).  Bit 5: forward renders take the kernel that walks a ray in several pieces at
  * once, whatever their size (not with a weight accumulator), with as many rays to a wavefront as the last decimal digit of
- * flags >> 8 says (1 to 8; 0: they never take it), in 2^(the digits before it) pieces at most (double precision, gradients
- * too: two digits, 1 to 16 rays, and 2^2 pieces at least).  With any flag set they
- * do not take it otherwise.  Bit 6: noting passes over ray batches list the rays that meet the tree first, where
+ * flags >> 8 says (1 to 8; 0: they never take it), in 2^(the digits before it) pieces at most; in double precision gradients
+ * too, with the last two digits for the rays (1 to 16), and 2^2 pieces at least.  With any other flag set no pass takes it.
+ * Bit 6: noting passes over ray batches list the rays that meet the tree first, where
  * the workspace has room, whatever their size: up to 64 times bits 8 to 15 of them take two wavefronts per tile, up to 64 times
- * bits 16 and up one, more the batch as it is.  The flags belong to the calling thread. */
+ * bits 16 and up one, more the batch as it is (so does one most of whose rays hit by a sample).  The flags belong to the calling thread. */
 void svox_set_debug_flags(int flags);
 
 /* No counterpart in the reference.  The forward kernel that walks and shades on two wavefronts hands leaves over

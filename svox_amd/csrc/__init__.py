@@ -535,7 +535,8 @@ def set_debug_flags(flags):
     """Of the calling thread.  bit 0: route every call to the generic kernels; bit 1: small ray batches run like
     large ones; bit 2 / bit 3: forward renders never / always take the two-wavefront kernel; bit 4: the bounded
     waits of that kernel give up at the first look that finds nothing (tests of what a give-up leaves behind); bit 5: forward
-    renders walk their rays in pieces, (flags >> 8) % 10 rays to a wavefront and 2**((flags >> 8) // 10) pieces of a ray at most;
+    renders walk their rays in pieces, (flags >> 8) % 10 rays to a wavefront (0: never) and 2**((flags >> 8) // 10) pieces of a ray at most
+    (double precision: gradients too, (flags >> 8) % 100 and // 100);
     bit 6: noting passes list the rays of a batch that meet the tree (64 * (flags >> 8 & 255) of them: two wavefronts per tile at most,
     64 * (flags >> 16): one)"""
     _abi.load_library().svox_set_debug_flags(int(flags))

@@ -33,7 +33,7 @@ thread_local char g_error[512] = "";
 // Debug flags of the calling thread (svox_set_debug_flags): bit 0: always take the generic kernels; bit 1: small
 // batches run like large ones; bit 2: forward launches never take the two-wavefront kernel; bit 3: they always
 // do (where it applies); bit 4: the bounded waits of that kernel give up at once; bit 5: forward launches cut their rays, as bits 8 and
-// up say (pick_cut); bit 6: noting passes list their rays (list_shapes).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
+// up say (pick_cut, group_cut); bit 6: noting passes list their rays (list_shapes).  Per thread, so that one thread's tests cannot change the kernels of another's calls.
 thread_local int g_debug_flags = 0;
 
 // Launch-shape overrides for experiments, read from the environment once, when the first launch of the process
@@ -47,8 +47,8 @@ thread_local int g_debug_flags = 0;
 //   SVOX_SPLIT_FORWARD 0 / 1: forward launches never / always on two wavefronts per tile
 //   SVOX_SPLIT_BLOCKS  largest forward launch (in tiles) that takes two wavefronts per tile
 //   SVOX_REPLAY_SHIFT  4, 5 or 6: log2 of the rays a block of the replay kernels takes
-//   SVOX_CUT           0: forward passes never cut their rays into pieces, 1 to 8: always, so many rays to a wavefront, + 10 x:
-//                      into 2^x pieces at most (62: two rays, 32 pieces of each)
+//   SVOX_CUT           single precision, 0: forward passes never cut their rays into pieces, 1 to 8: always, so many rays to a
+//                      wavefront, + 10 x: into 2^x pieces at most (62: two rays, 32 pieces of each, or 64 of one if the other misses)
 struct Tuning {
     int per_wave = 0, refill = 0, xcd_group = 0, tile_order = -1, image_run = -1, split_forward = -1, replay_shift = -1;
     long split_blocks = -1;
@@ -439,9 +439,9 @@ struct Cut {
 };
 Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     Cut c;
-    const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : tuning().cut;
-    if (forced > 0) {
-        c.per_wave = std::min(std::max(forced % 100, 1), kGroupRays);
+    if (g_debug_flags != 0) {
+        const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : 0;
+        c.per_wave = std::min(forced % 100, kGroupRays);
         c.most = std::min(std::max(forced / 100, 2), 6);
         return c;
     }

@@ -78,3 +78,31 @@ def test_pictures_and_trees_deeper_than_the_integer_coordinates(gpu, oracle_mod)
         go = torch.randn(29, 37, 3, generator=gen, dtype=torch.float64).to(gpu)
         grad, generic = both_kernels(lambda: C.volume_render_image_backward(dev._spec(), cam, opt, go))
         assert (grad - generic).abs().max() <= 1e-9 * generic.abs().max()
+
+
+@pytest.mark.parametrize("flags", [2, 4, 32])
+@pytest.mark.parametrize("fmt,kw", [("RGBA", {}), ("SH9", {"fast": True}), ("SH4", {"density_softplus": True, "min_comp": 1, "max_comp": 2})])
+def test_rays_walked_by_four_lanes_together(gpu, flags, fmt, kw):
+    """Any debug flag but those for pieces takes the kernels whose four lanes share a walk, for few rays too: lists of leaves that run over
+    (every leaf of 64^3 has density) and a number of rays that is no multiple of a wavefront's."""
+    n = 333
+    gen = torch.Generator().manual_seed(3)
+    tree = svox.N3Tree(N=2, data_format=fmt, init_refine=5, dtype=torch.float64)
+    tree.data.data.normal_(generator=gen)
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.3 + 0.01
+    rays = synth.sphere_rays(n, seed=4, dtype=torch.float64)
+    rays.dirs[::5] *= -1.0
+    opt = options(tree, step_size=1e-3, **kw)
+    spec, rs = on_gpu(tree, gpu)._spec(), rays_spec(rays, gpu)
+    go = torch.randn(n, 3, generator=gen, dtype=torch.float64).to(gpu)
+
+    def passes(f):
+        C.set_debug_flags(f)
+        try:
+            return C.volume_render(spec, rs, opt), C.volume_render_backward(spec, rs, opt, go)
+        finally:
+            C.set_debug_flags(0)
+
+    (out, grad), (want, ref) = passes(flags), passes(1)
+    assert torch.equal(out, want)
+    assert (grad - ref).abs().max() <= 1e-11 * ref.abs().max()
