@@ -46,7 +46,7 @@ def scene(kind, fmt, gen):
 @pytest.mark.parametrize("per_wave,most", [(8, 0), (8, 6), (5, 2), (3, 6), (2, 5), (1, 6)])
 @pytest.mark.parametrize("kind,fmt,softplus,fast", [("dense", "SH9", False, False), ("dense", "RGBA", True, False), ("thirds", "SG4", False, False),
                                                     ("shell", "SH16", False, True), ("deep", "SH4", False, False), ("leaf", "SH25", False, True)])
-def test_rays_in_pieces_are_the_rays_from_end_to_end(gpu, oracle_mod, kind, fmt, softplus, fast, per_wave, most):
+def test_rays_in_pieces_are_the_rays_from_end_to_end(gpu, oracle_mod, monkeypatch, kind, fmt, softplus, fast, per_wave, most):
     n = 301
     gen = torch.Generator().manual_seed(7)
     tree = scene(kind, fmt, gen)
@@ -78,19 +78,28 @@ def test_rays_in_pieces_are_the_rays_from_end_to_end(gpu, oracle_mod, kind, fmt,
             err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
             assert ok, (what, err)
     # room for as many chunks of 15 notes as the rays need, beside the first of each: none are lost
+    monkeypatch.setattr(C, "SMALL_BATCH_ROOM", 1)
     chunks = -(-int(((want[2] - 1).clamp(min=0) // 15).sum()) // n) + 1
     notes = run(cut(per_wave, most), lambda: C.volume_render_noted(plain, rs, opt, records_per_ray=15 * chunks))[1]
     assert torch.equal(notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91], want[2])
-    # room for the first chunk of a ray and little more: the others' notes are lost, and the gradient marches
-    want = run(END_TO_END, lambda: C.volume_render_backward(plain, rs, opt, go, workspace=False))
+    # room for the first chunk of a ray, and for half of the others: the rest of the notes is lost, and the gradient marches
+    marched = run(END_TO_END, lambda: C.volume_render_backward(plain, rs, opt, go, workspace=False))
+    picture = run(END_TO_END, lambda: C.volume_render(plain, rs, opt))
+    for records in (15, 15 * (chunks // 2 + 1)):
 
-    def short():
-        out, notes = C.volume_render_noted(plain, rs, opt, records_per_ray=16)
-        return out, C.volume_render_backward_noted(plain, rs, opt, go, notes)
-    out, grad = run(cut(per_wave, most), short)
-    assert torch.equal(out, run(END_TO_END, lambda: C.volume_render(plain, rs, opt)))
-    err, ok = grad_close(grad.cpu().numpy(), want.cpu().numpy(), slack=slack, what="lost notes")
-    assert ok, err
+        def short():
+            out, notes = C.volume_render_noted(plain, rs, opt, records_per_ray=records)
+            count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+            return out, count, C.volume_render_backward_noted(plain, rs, opt, go, notes)
+        out, count, grad = run(cut(per_wave, most), short)
+        assert torch.equal(out, picture)
+        lost = count == -1
+        assert torch.equal(count[~lost], want[2][~lost])
+        if records == 15:
+            assert torch.equal(lost, want[2] > 15)
+            assert bool(lost.any()) == (kind != "leaf")
+        err, ok = grad_close(grad.cpu().numpy(), marched.cpu().numpy(), slack=slack, what="lost notes")
+        assert ok, (records, err)
 
 
 @pytest.mark.parametrize("ndc", [False, True])

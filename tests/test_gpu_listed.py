@@ -30,7 +30,7 @@ def run(flags, f):
 # how many rays meet the tree, of 2 500: none, one, a tile and one more, all
 @pytest.mark.parametrize("hits", [0, 1, 64, 65, 1025, 2500])
 @pytest.mark.parametrize("two,one,more", [(255, 256, 0), (16, 32, 0), (1, 16, 2), (0, 40, 0), (1, 1, 2)])
-def test_listed_rays(gpu, oracle_mod, hits, two, one, more):
+def test_listed_rays(gpu, oracle_mod, monkeypatch, hits, two, one, more):
     n = 2500
     tree = synth.shell_tree(depth=6, data_format="SH9", n_spheres=6, seed=4)
     gen = torch.Generator().manual_seed(hits)
@@ -56,9 +56,21 @@ def test_listed_rays(gpu, oracle_mod, hits, two, one, more):
     for what, a, b in zip(("from notes", "alone"), got[3:], want[3:]):
         err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
         assert ok, (what, err)
-    # no room for the list beside the notes: the batch as it is
-    out = run(listed(two, one) | more, lambda: C.volume_render_noted(spec, rs, opt, records_per_ray=16))[0]
+    # no room for the list beside the notes, and for those of a ray beyond the first 15: the batch as it is
+    monkeypatch.setattr(C, "SMALL_BATCH_ROOM", 1)
+
+    def short():
+        out, notes = C.volume_render_noted(spec, rs, opt, records_per_ray=15)
+        assert notes.numel() * 8 // 384 - n < 16 * (n * 4 // 384)
+        count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+        return out, count, C.volume_render_backward_noted(spec, rs, opt, go, notes)
+
+    out, count, grad = run(listed(two, one) | more, short)
     assert torch.equal(out, want[0])
+    assert torch.equal(count, torch.where(want[1] > 15, -1, want[1]))
+    assert bool((count == -1).any()) == (hits >= 64)
+    err, ok = grad_close(grad.cpu().numpy(), want[3].cpu().numpy(), slack=slack, what="no room")
+    assert ok, err
 
 
 def test_a_captured_pass_lists_anew_in_every_replay(gpu):
