@@ -6,6 +6,8 @@
 // (SVOX_DISPATCH_OCTREE) and calls these functions.
 #pragma once
 
+#include <type_traits>
+
 #include "cut_kernel.h"
 #include "march_kernels.h"
 
@@ -99,11 +101,14 @@ void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeD
         SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, true>);
     else if (split)
         SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, false>);
-    else if (refill && grad_out)
-        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
-    else if (refill)
-        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, false>);
-    else if (grad_out)
+    else if (refill) {
+        if constexpr (!std::is_same<Source, ListedSource>::value) {   // (listed rays are marched tile by tile)
+            if (grad_out)
+                SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
+            else
+                SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, false>);
+        }
+    } else if (grad_out)
         SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, true>);
     else
         SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, false>);

@@ -691,7 +691,7 @@ constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 //                1 000 rays                              4 096                                   8 192 (with notes, shells: 7 168)
 //   8^3 SH1      not taken                               | 20, 26 / 34, 36 if it were
 //   32^3 SH9     80, 80 / 27, 34    | 83, 92 / 40, 44    77, 77 / 41, 52     | 80, 91 / 53, 61    79, 82 / 53, 54      | 83, 107 / 76, 82
-//   64^3 SH9     153, 153 / 37, 45  | 171, 194 / 65, 62  194, 192 / 72, 62   | 216, 234 / 104, 115   197, 196 / 110, 115 | 218, 237 / 154, 169
+//   64^3 SH9     153, 153 / 37, 45  | 171, 194 / 65, 62  194, 192 / 62, 62   | 216, 234 / 143, 115   197, 196 / 110, 115 | 218, 237 / 154, 169
 //   128^3 SH4    377, 377 / 62, 74  | 395, 423 / 86, 99  390, 387 / 112, 141 | 406, 432 / 245, 224   403, 400 / 192, 259 | 416, 437 / 361, 372
 //   shell 128^3 SH9   128, 126 / 54, 60   | 131, 135 / 92, 76   170, 169 / 87, 99    | 185, 194 / 110, 127   180, 180 / 116, 149 | 187, 195 / 163, 206
 //   shell 256^3 SH9   178, 173 / 48, 57   | 181, 188 / 83, 86   260, 257 / 114, 167  | 273, 273 / 150, 222   272, 242 / 185, 198 | 276, 254 / 249, 333
@@ -743,9 +743,9 @@ Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRend
         c.per_wave = items <= 4096 || (cells >= 16384.0 && !noted) ? 4 : 8;
     } else if (!large) {
         if (noted)
-            c.per_wave = items <= 2048 || (sparse && fine) ? 2 : 4;
+            c.per_wave = items <= 2048 || (sparse && fine && (tree->N == 2 || items <= 4096)) ? 2 : 4;
         else
-            c.per_wave = items > 4096 && items <= 6144 && (grid || !fine) ? 4 : 2;
+            c.per_wave = items > (grid ? 3072 : 4096) && items <= 6144 && (grid || !fine) ? 4 : 2;
     } else if (grid) {
         c.per_wave = items <= 1536 ? 1 : 2;
     } else {
