@@ -695,7 +695,8 @@ constexpr bool is_image_source(const BatchSource<T>&) { return false; }
 //   128^3 SH4    377, 377 / 62, 74  | 395, 423 / 86, 99  390, 387 / 112, 141 | 406, 432 / 245, 224   403, 400 / 192, 259 | 416, 437 / 361, 372
 //   shell 128^3 SH9   128, 126 / 54, 60   | 131, 135 / 92, 76   170, 169 / 87, 99    | 185, 194 / 110, 127   180, 180 / 116, 149 | 187, 195 / 163, 206
 //   shell 256^3 SH9   178, 173 / 48, 57   | 181, 188 / 83, 86   260, 257 / 114, 167  | 273, 273 / 150, 222   272, 242 / 185, 198 | 276, 254 / 249, 333
-// (10 000 rays: 64^3 SH9 204, 204 / 132, 147 | 227, 247 / 183, 210, 128^3 417, 414 / 204, 304 | 435, 459 / 419, 447.  Of views from afar, 18 % of whose
+// (10 000 rays: 64^3 SH9 204, 204 / 132, 147 | 227, 247 / 183, 210, 128^3 417, 414 / 204, 304 | 435, 459 / 419, 447; 12 288 rays: 64^3 SH9 198, 200 /
+// 158, 165 | 220, 243 / 222, 248, SH4 188, 195 / 161, 158 | 205, 228 / 214, 242, RGBA, not taken, 165, 176 / 144, 147 | 166, 187 / 200, 226.  Of views from afar, 18 % of whose
 // rays hit a shell, 7 000 with notes take 169 / 89 at 256^3: for those the line of a full shell, 6 000 rays, is passed over.)
 // With the shifted softplus every leaf is listed and rays end behind what they met (opaque_light), from end to end as in pieces.  A shell of 256^3,
 // without notes and with: 1 000 rays 74, 80 / 45, 61, 4 096 84, 95 / (116, 186).
@@ -724,7 +725,7 @@ Cut pick_cut(const SvoxTreeSpec* tree, int64_t items, bool image, const SvoxRend
     }
     int64_t limit = 8192;
     if (image && !small) limit = grid && !noted ? 12288 : 9216;   // (in blocks of 16 x 16)
-    if (!image && !small) limit = grid ? 10240 : noted ? 7168 : 8192;
+    if (!image && !small) limit = grid ? (large || tree->data_dim < 13 ? 10240 : 12288) : noted ? 7168 : 8192;
     if (softplus) limit = small ? 4096 : grid ? (noted ? 4096 : 8192) : noted ? (image ? 1024 : 2048) : image ? 4096 : 3072;
     if (items > limit) return c;
     if (image) {
