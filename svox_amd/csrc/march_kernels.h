@@ -137,6 +137,7 @@ __device__ __forceinline__ void maybe_world2ndc(const SvoxRenderOptions& opt, T*
 // tree coordinates.
 template <typename T>
 struct BatchSource {
+    static constexpr bool kGated = false;
     RayBatch<T> rays;
     int per_wave;
     int refill_at;   // idle lanes that trigger taking new rays
@@ -176,8 +177,11 @@ struct BatchSource {
     }
 };
 
-// Rays of a batch that meet the cube, for noting passes (list_hits_kernel): item i is ray list[i].
+// Rays of a batch that meet the cube, for noting passes (list_hits_kernel): item i is ray list[i].  And the batch as it is, where that is
+// one of the shapes such a pass is launched in (kGated, ReplaySpace::chosen; a kernel of their own, as the look at the gate costs others 1 to
+// 2 %: dense 128^3 SH1, 28 456 rays with notes 435.3 -> 443.7 us).
 struct ListedSource : BatchSource<float> {
+    static constexpr bool kGated = true;
     const int32_t* list;
     const unsigned long long* n_listed;
     __device__ __forceinline__ int64_t total() const { return (int64_t)*n_listed; }
@@ -185,6 +189,9 @@ struct ListedSource : BatchSource<float> {
                                                   const float* scaling, float* origin, float* dir, float* vdir) const {
         return BatchSource<float>::fetch_item(list[i], opt, offset, scaling, origin, dir, vdir);
     }
+};
+struct WholeSource : BatchSource<float> {
+    static constexpr bool kGated = true;
 };
 
 __host__ __device__ inline int blocks16_of(int extent) { return (extent + 15) / 16; }
@@ -229,6 +236,7 @@ __device__ __forceinline__ void block_inside_out(int rank, int nbx, int nby, int
 
 template <typename T>
 struct ImageSource {
+    static constexpr bool kGated = false;
     Camera<T> cam;          // cam.c2w: pose of image 0
     int n_images;
     int64_t pose_stride;    // scalars between consecutive poses
@@ -884,12 +892,10 @@ struct ReplaySpace {
     uint32_t* clear_at[2];
     int64_t clear_words;
     // A pass of which only the device knows how many rays it has (list_hits_kernel) is launched in several shapes: this launch does its
-    // work if there are at least, and at most, as many as it is made for.  nullptr: it does.
+    // work if there are at least, and at most, as many as it is made for (sources that are kGated).
     const unsigned long long* n_listed;
     int64_t least, most;
-    __device__ __forceinline__ bool chosen() const {
-        return n_listed == nullptr || ((int64_t)*n_listed >= least && (int64_t)*n_listed <= most);
-    }
+    __device__ __forceinline__ bool chosen() const { return (int64_t)*n_listed >= least && (int64_t)*n_listed <= most; }
 };
 
 // The arrays a gradient is going to be added to are cleared by further blocks of the launch that takes the notes for it: that one waits
@@ -1059,8 +1065,9 @@ struct NoteTaker {
 // The chain of a batch's longest rays is what such a pass waits for, and those that graze a surface are long because of what they pass
 // through: 50 001 rays of a 256^3 SH9 shell with softplus, training step 342 -> 208 us.  A bound of 2^-126, below which a weight has
 // lost digits, ends them hardly sooner (207 us), and leaves out terms that a large gradient of the picture makes count.
-// Marches on two wavefronts are 1 % longer than before rays ended here (20 000 rays of a 256^3 SH9 shell 302.8 -> 305.8 us, dense 64^3,
-// 30 000 rays 213.7 -> 215.6), though not for the look at the light: without it they measure the same.
+// Marches on two wavefronts are 1 % longer with SH9 and RGBA than before rays ended here (50 000 rays of a 256^3 SH9 shell 314.4 -> 317.9 us,
+// dense 64^3 RGBA, 30 000 rays 187.3 -> 189.4), as long with SH1 and SH4, and 0.6 % shorter with SH16 -- though not for the look at the light:
+// without it they measure the same.
 __device__ __forceinline__ float opaque_light(const SvoxRenderOptions& opt, const float* out) {
     return opt.stop_thresh >= 0.0f || out == nullptr ? 0.0f : -1.0f;   // (light is never below zero)
 }
@@ -1140,7 +1147,9 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
     if constexpr (kNoted) {
-        if (!ws.chosen()) return;
+        if constexpr (Source::kGated) {
+            if (!ws.chosen()) return;
+        }
         if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
     }
     const int lane = threadIdx.x;
@@ -1901,7 +1910,9 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ SplitBox box;
     if constexpr (kNoted) {
-        if (!ws.chosen()) return;
+        if constexpr (Source::kGated) {
+            if (!ws.chosen()) return;
+        }
         if (blockIdx.x >= ws.march_blocks) return clear_share(ws);
         if (blockIdx.x == 0 && threadIdx.x < kStampWords) ws.stamp_at[threadIdx.x] = ws.stamp[threadIdx.x];
     }

@@ -97,12 +97,17 @@ void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeD
     // (the colours take the gradient's place in the variants without it)
 #define SVOX_NOTING(THREADS, ...)                                                                                        \
     hipLaunchKernelGGL((__VA_ARGS__), blocks, dim3(THREADS), 0, stream, tr, src, opt, out, ws, grad_out ? grad_out : color_ref)
-    if (split && grad_out)
-        SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, true>);
-    else if (split)
-        SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, false>);
-    else if (refill) {
-        if constexpr (!std::is_same<Source, ListedSource>::value) {   // (listed rays are marched tile by tile)
+    constexpr bool kListed = std::is_same<Source, ListedSource>::value;   // (marched tile by tile)
+    constexpr bool kWhole = std::is_same<Source, WholeSource>::value;     // (on one wavefront per tile or chunk)
+    if (split) {
+        if constexpr (!kWhole) {
+            if (grad_out)
+                SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, true>);
+            else
+                SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, false>);
+        }
+    } else if (refill) {
+        if constexpr (!kListed) {
             if (grad_out)
                 SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
             else

@@ -13,4 +13,7 @@ template struct MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>,
 template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, ListedSource>::noting(
     dim3, hipStream_t, const TreeDev<float>&, const ListedSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
     const float*, bool, bool);
+template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, WholeSource>::noting(
+    dim3, hipStream_t, const TreeDev<float>&, const WholeSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
+    const float*, bool, bool);
 }  // namespace svox

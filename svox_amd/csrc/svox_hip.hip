@@ -1065,9 +1065,11 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
             if (src.rays.n_rays > listed) {
                 ws.least = listed > 0 ? listed + 1 : 0;
                 ws.most = INT64_MAX;
+                WholeSource whole;
+                (Source&)whole = dealt;
                 const dim3 grid = with_clearing(blocks);
-                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(grid, stream, march_tree(tree, opt), dealt, *opt, (float*)out, ws,
-                                                                       (const float*)grad_out, (const float*)color_ref, false, refill));
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, WholeSource>::noting(grid, stream, march_tree(tree, opt), whole, *opt, (float*)out, ws,
+                                                                            (const float*)grad_out, (const float*)color_ref, false, refill));
             }
             return SVOX_OK;
         }
