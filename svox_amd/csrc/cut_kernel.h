@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     constexpr int K = P::kRecord;
     constexpr int kListed = cut_listed(kNoted);
     constexpr int kMostRays = kCutMostRays;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ PieceHeads<float, kCutHeads> heads;           // (-1: not known yet)
     __shared__ CutLists<kListed> lists;
     __shared__ float atts[kNoted ? kListed * kMarchThreads : 1];      // attenuations (without notes: in lists.dt)
@@ -172,6 +172,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     if (!walking) end = kCutOver;
     OctreeCursor cur;
     cur.reset(path + lane);
+    const ChildTable child(tr);
     if (walking) cur.begin(r);
     wave_lds_sync();
 
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                 bool broken = false;
                 q_leaf[q] = -1;
                 q_dt[q] = 0.0f;
-                if (any_lane(go)) walk_turn_flat(tr, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
+                if (any_lane(go)) walk_turn_flat(tr, child, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
                 if (go) {
                     if (q_leaf[q] >= 0) sample += 1;
                     if (broken || !(r.t < r.tmax)) {

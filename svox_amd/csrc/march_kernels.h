@@ -365,38 +365,59 @@ __device__ __forceinline__ Visit step_generic(const TreeDev<T>& tr, const RaySta
     return v;
 }
 
+// The child table of an octree as the march reads it: through a buffer descriptor, so that a read which a lane has no need for, or which a
+// malformed tree leads out of the table, costs neither a branch nor a request -- beyond the last byte it gives 0.  (The table is smaller than
+// 4 GiB, checked on the host.)
+struct ChildTable {
+    __amdgpu_buffer_rsrc_t entries;
+    uint32_t last_cell;
+    bool octree;
+    static constexpr uint32_t kNowhere = 0xffffffe0u;   // a row beyond the largest table
+    __device__ __forceinline__ explicit ChildTable(const TreeDev<float>& tr) {
+        const uint32_t cells = (uint32_t)tr.capacity << 3;
+        octree = tr.N == 2;
+        last_cell = cells - 1u;
+        entries = __builtin_amdgcn_make_buffer_rsrc((void*)tr.child, 0, octree ? cells << 2 : 0u, 0x00020000);
+    }
+    __device__ __forceinline__ int32_t read(uint32_t at) const { return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(entries, (int)at, 0, 0); }
+    __device__ __forceinline__ uint32_t cell(uint32_t at) const { return min(at >> 2, last_cell); }
+};
+
 // The walk of one lane's ray through the tree, sample after sample.  A sample's integer coordinates (24 bits an axis)
 // say which cell it lies in at every level, and those it shares with the sample before say how far up the next search
-// has to start: the node ids of the previous path are kept in LDS, one column per lane (`path`, laid out
-// [kPathLevels + 1][64]: path[64 * l], l < kPathLevels, is the node whose child row is indexed at level l + 1, path[0]
-// the root, node 0; the last row is a dump for the levels below, which no search resumes from).
+// has to start: where the child rows of the previous path begin is kept in LDS, one column per lane (`path`, laid out
+// [kPathLevels + 2][64], the root's row last; the first two rows are a dump for the levels below, which no search resumes from).
 //
 // The march waits for this chain -- position, coordinates, path, child reads, step -- once per leaf, and where no other
-// wavefront fills the gaps its instructions count as much as its reads.  So the ray's origin and direction are kept
+// wavefront fills the gaps what counts are its instructions: a lone wavefront issues one every 7 to 9 cycles, takes 30 to 40 for a
+// branch, 160 for a read that hits L1.  So the ray's origin and direction are kept
 // times 2^24 (exact: the coordinates need no further product), the sample is looked up in the path as soon as it is
-// known (aim) rather than when its turn comes, and there is no state but (level, node): an interrupted descent is one
-// that has not found its leaf yet.  (Before, as selects over pending
-// and finished searches, a turn was 145 vector instructions instead of 110.  Forward kernels: 800x800 picture of a
-// 512^3 SH16 shell 369 -> 343 us, 8 such pictures 688 -> 660 us, an NDC picture 616 -> 583 us; noting: 50 001 rays
-// 266 -> 240 us, 1 Mi rays 710 -> 661 us.  Keeping whole child rows of the last four levels in LDS as well, so that a
+// known (aim) rather than when its turn comes, the levels are counted from below, so that the level to resume from is the highest
+// bit of what the samples differ in, and a lane that has no read to make is turned away by the bounds of the buffer (ChildTable) and not by
+// a branch.  A turn is 75 vector instructions and one branch (110 and five where the reads, the level found and the malformed were each
+// a branch; 145 with selects over pending and finished searches).  A wavefront alone, child table in L2, ns a leaf: 625 to 830 -> 530 to 690 on one
+// wavefront per tile, 705 to 890 -> 460 to 590 on two (by how far the rays are apart).  800x800 picture of a 512^3 SH16 shell 314 -> 270 us, 8 such pictures
+// 762 -> 743, an NDC picture 563 -> 541; squared error of 200 003 rays 481 -> 433, training step of 1 Mi rays 1242 -> 1209.
+// (Keeping whole child rows of the last four levels in LDS as well, so that a
 // step costs one read instead of two, made the two-wavefront kernel 3 to 8 % faster where it runs alone on a CU, and
 // everything else up to 45 % slower.)
 struct OctreeCursor {
-    int32_t* rows;         // the lane's column of the path, counted from level 1: rows[64 * level]
+    int32_t* rows;         // the lane's column of the path: rows[64 * (1 + max(up, kPathUp))]
     float p[3];            // the sample, clamped, times 2^24
     uint32_t ix, iy, iz;   // its integer coordinates
-    int level;             // where the search for its leaf stands: the child row to look into at this level ...
-    int32_t node;          // ... is that of this node
-    int levels;            // of the previous leaf (1: none, or one the path says nothing of)
+    int up;                // where the search for its leaf stands, in levels above the finest the coordinates hold (kCoordBits
+                           // minus the level; negative: the sample lies deeper): the child row to look into ...
+    uint32_t row;          // ... begins at this byte of the table
+    static constexpr int kPathUp = kCoordBits - kPathLevels - 1;   // of the path's upper dump row; the other lies below it
 
     // `lane_path`: this lane's column
     __device__ __forceinline__ void reset(int32_t* lane_path) {
-        rows = lane_path - kMarchThreads;
-        lane_path[0] = 0;
+        rows = lane_path - kPathUp * kMarchThreads;
+        rows[kCoordBits * kMarchThreads] = 0;
         p[0] = p[1] = p[2] = 0.0f;
         ix = iy = iz = 0;
-        level = levels = 1;
-        node = 0;
+        up = kCoordBits - 1;
+        row = 0;
     }
     // the first sample of a ray fresh from setup_ray
     __device__ __forceinline__ void begin(RayState<float>& r) {
@@ -404,104 +425,121 @@ struct OctreeCursor {
         for (int i = 0; i < 3; ++i) {
             r.o[i] *= 16777216.0f;
             r.d[i] *= 16777216.0f;
+            // (a coordinate that is not a number counts as the upper bound, clamp01: so does an infinite one, and fmed3 below has no
+            // say in the matter)
+            if (!(r.o[i] == r.o[i]) || !(r.d[i] == r.d[i])) {
+                r.o[i] = __builtin_inff();
+                r.d[i] = 0.0f;
+            }
         }
-        levels = 1;
-        aim(r);
+        aim(r, kCoordBits - 1);
     }
-    // the sample at r.t
-    __device__ __forceinline__ void aim(const RayState<float>& r) {
+    // the sample at r.t; leaf_up: where the leaf of the sample before it lies (kCoordBits - 1: the path says nothing of it)
+    __device__ __forceinline__ void aim(const RayState<float>& r, int leaf_up) {
         // (clamp01, times 2^24)
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            p[i] = max_(0.0f, min_(__uint_as_float(0x3F7FFFEFu) * 16777216.0f, fma_(r.t, r.d[i], r.o[i])));
+            p[i] = __builtin_amdgcn_fmed3f(fma_(r.t, r.d[i], r.o[i]), 0.0f, __uint_as_float(0x3F7FFFEFu) * 16777216.0f);
         const uint32_t nx = (uint32_t)p[0], ny = (uint32_t)p[1], nz = (uint32_t)p[2];
-        const uint32_t diff = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
-        // the first level the two samples differ at (a huge number: none)
-        const uint32_t first_diff = (diff ? (uint32_t)__builtin_clz(diff) : 0xffffffffu) - (31 - kCoordBits);
-        level = (int)min(min(first_diff, (uint32_t)levels), (uint32_t)kPathLevels);
-        node = rows[level * kMarchThreads];
+        // the first level the two samples differ at is that of the highest bit they differ in; not below the leaf, nor the path
+        const uint32_t diff = (ix ^ nx) | (iy ^ ny) | (iz ^ nz) | 1u << leaf_up | 1u << (kPathUp + 1);
+        up = 31 - __builtin_clz(diff);
+        row = (uint32_t)rows[(up + 1) * kMarchThreads];
         ix = nx;
         iy = ny;
         iz = nz;
     }
+    // (a << n) | b in one instruction: in plain C++ the compiler orders the three of them so that it takes four
+    template <int n>
+    static __device__ __forceinline__ uint32_t shift_or(uint32_t a, uint32_t b) {
+        uint32_t r;
+        asm("v_lshl_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "n"(n), "v"(b));
+        return r;
+    }
+    // the byte of the table that holds the child entry to look at, in the row that begins at `from`
+    __device__ __forceinline__ uint32_t entry(uint32_t from) const {
+        const unsigned bx = __builtin_amdgcn_ubfe(ix, (unsigned)up, 1u), by = __builtin_amdgcn_ubfe(iy, (unsigned)up, 1u),
+                       bz = __builtin_amdgcn_ubfe(iz, (unsigned)up, 1u);
+        return shift_or<2>(shift_or<1>(shift_or<1>(bx, by), bz), from);
+    }
     // One turn of the lanes with `go`: up to kSeekBudget child reads, and if the leaf is found its index (with
     // kEmptyLeafBit if it is marked empty) in slot_leaf, the step of the sample in slot_dt, and the ray moved on; else
-    // slot_leaf is -1.  Returns whether the lane's sample lies deeper than the coordinates resolve.
-    // Node ids read from the table are clamped into [0, last_node]: a malformed tree yields a wrong leaf, never an
-    // access outside the table.  The table is smaller than 4 GiB (checked on the host): a 32-bit byte offset from the
-    // uniform base lets the load use the scalar-base form.
-    __device__ __forceinline__ bool turn(RayState<float>& r, bool go, const int32_t* __restrict__ child, int32_t last_node,
-                                         float step_size, int32_t& slot_leaf, float& slot_dt) {
-        slot_leaf = -1;
-        slot_dt = 0.0f;
-        int32_t cell = 0, skip = 1;   // (a lane that does not search keeps its 1)
-#pragma unroll
-        for (int it = 0; it < kSeekBudget; ++it) {
-            if (go && skip > 0 && level <= kCoordBits) {
-                rows[min(level, kPathLevels + 1) * kMarchThreads] = node;
-                cell = (node << 3) | cell_at(ix, iy, iz, level);
-                skip = *(const int32_t*)((const char*)child + ((uint32_t)cell << 2));
-                // (of a lane that has found its leaf the node is of no more use)
-                node = (int32_t)min((uint32_t)(node + skip), (uint32_t)last_node);
-                level += skip > 0 ? 1 : 0;
-            }
-        }
-        const bool deep = go && level > kCoordBits;
-        if (skip <= 0) {
-            // 2^(levels - 24) and 2^-levels: dividing by the power of two is the multiplication by its reciprocal
-            const uint32_t level_bits = (uint32_t)level << 23;
-            const float to_leaf = __uint_as_float(level_bits + ((uint32_t)(127 - kCoordBits) << 23));
-            const float inv_cube = __uint_as_float((127u << 23) - level_bits);
+    // both are left as they are.  A lane whose sample lies deeper than the coordinates resolve is left with a negative `up`.
+    __device__ __forceinline__ void turn(RayState<float>& r, bool go, const ChildTable& child, float step_size, int32_t& slot_leaf,
+                                         float& slot_dt) {
+        static_assert(kSeekBudget == 2, "two reads, written out");
+        const uint32_t first = entry(go ? row : ChildTable::kNowhere);
+        const int32_t skip1 = child.read(first);
+        const bool below = skip1 > 0;
+        const uint32_t next = row + ((uint32_t)skip1 << 5);
+        // (of a lane that stays where it is the second row means nothing, and is read by nobody)
+        int32_t* const at = rows + max(up, kPathUp) * kMarchThreads;
+        at[kMarchThreads] = (int32_t)row;
+        at[0] = (int32_t)next;
+        up -= below ? 1 : 0;
+        const uint32_t second = entry(below ? next : ChildTable::kNowhere);
+        row = below ? next : row;
+        const int32_t skip2 = child.read(second);
+        const int32_t skip = min(skip1, skip2);   // (the second is 0 where there was no need for it)
+        const int leaf_up = up;
+        row += (uint32_t)max(skip2, 0) << 5;
+        up -= skip2 > 0 ? 1 : 0;
+        if (go & (skip <= 0) & (leaf_up >= 0)) {
+            const uint32_t cell = child.cell(below ? second : first);
+            // 2^-up and 2^(up - 24): dividing by the power of two is the multiplication by its reciprocal
+            const uint32_t up_bits = (uint32_t)leaf_up << 23;
+            const float to_leaf = __uint_as_float((127u << 23) - up_bits);
+            const float inv_cube = __uint_as_float(((uint32_t)(127 - kCoordBits) << 23) + up_bits);
             // leaf-local position frac(pos * 2^levels): s - floor(s), exact for the non-negative s of a clamped
             // coordinate, in one instruction
             float local[3];
 #pragma unroll
             for (int j = 0; j < 3; ++j) local[j] = __builtin_amdgcn_fractf(p[j] * to_leaf);
-            slot_leaf = skip < 0 ? cell | kEmptyLeafBit : cell;
+            slot_leaf = (int32_t)cell | (skip & kEmptyLeafBit);   // (marks are -2)
             slot_dt = leaf_exit(local, r.inv) * inv_cube + step_size;
             const float t_next = r.t + slot_dt;
             r.t = t_next > r.t ? t_next : r.tmax;   // (advance())
-            levels = level;
-            aim(r);
+            aim(r, leaf_up);
         }
-        return deep;
     }
 };
 
+// A sample of the lanes with `go` by the reference's walk from the root: what lies deeper than the integer coordinates hold, and
+// trees with another branching factor, which have no exact integer formulation.  `broken`: the tree is malformed, the ray ends here.
+__device__ __forceinline__ void walk_from_root(const TreeDev<float>& tr, RayState<float>& r, OctreeCursor& cur, float step_size, bool go,
+                                               bool& broken, int32_t& slot_leaf, float& slot_dt) {
+    if (!go) return;
+    float local[3], cells_per_axis;
+    int levels;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) local[j] = cur.p[j] * (1.0f / 16777216.0f);
+    slot_leaf = (int32_t)descend_generic<float>(tr.child, tr.capacity, tr.N, local, &cells_per_axis, &levels, true);
+    if (slot_leaf >= 0) {
+        // (rt_kernel.cu:274 divides by the cell count; for a power of two the product with the reciprocal is
+        // the same number)
+        const float segment = leaf_exit(local, r.inv);
+        slot_dt = (tr.N == 2 ? segment * (1.0f / cells_per_axis) : segment / cells_per_axis) + step_size;
+        const float t_next = r.t + slot_dt;
+        r.t = t_next > r.t ? t_next : r.tmax;
+        cur.aim(r, kCoordBits - 1);
+    } else {
+        broken = true;
+    }
+}
+
 // One turn of the walk for the whole wavefront: the lanes with `go` take one sample (slot_leaf, slot_dt) and advance,
 // or keep a descent open (slot_leaf -1).  `broken`: the tree is malformed, the ray ends here.
-__device__ __forceinline__ void walk_turn_flat(const TreeDev<float>& tr, RayState<float>& r, OctreeCursor& cur,
+__device__ __forceinline__ void walk_turn_flat(const TreeDev<float>& tr, const ChildTable& child, RayState<float>& r, OctreeCursor& cur,
                                                float step_size, bool go, bool& broken, int32_t& slot_leaf,
                                                float& slot_dt) {
-    // (trees with another branching factor have no exact integer formulation: every lane takes the reference's
-    // floating-point walk below, from the root for every sample, and shares everything else with the octrees)
-    const bool octree = tr.N == 2;
     bool deep = go;
     slot_leaf = -1;
     slot_dt = 0.0f;
-    if (octree) deep = cur.turn(r, go, tr.child, (int32_t)(tr.capacity - 1), step_size, slot_leaf, slot_dt);
-    if (__builtin_expect(any_lane(deep), 0)) {
-        if (deep) {
-            // more levels than the integer coordinates hold, another branching factor, or a broken tree
-            float local[3], cells_per_axis;
-            int levels_f;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) local[j] = cur.p[j] * (1.0f / 16777216.0f);
-            slot_leaf = (int32_t)descend_generic<float>(tr.child, tr.capacity, tr.N, local, &cells_per_axis, &levels_f, true);
-            cur.levels = 1;
-            if (slot_leaf >= 0) {
-                // (rt_kernel.cu:274 divides by the cell count; for a power of two the product with the reciprocal is
-                // the same number)
-                const float segment = leaf_exit(local, r.inv);
-                slot_dt = (octree ? segment * (1.0f / cells_per_axis) : segment / cells_per_axis) + step_size;
-                const float t_next = r.t + slot_dt;
-                r.t = t_next > r.t ? t_next : r.tmax;
-                cur.aim(r);
-            } else {
-                broken = true;
-            }
-        }
+    if (child.octree) {
+        cur.turn(r, go, child, step_size, slot_leaf, slot_dt);
+        deep = go && cur.up < 0;
     }
+    if (__builtin_expect(any_lane(deep), 0)) walk_from_root(tr, r, cur, step_size, deep, broken, slot_leaf, slot_dt);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -780,16 +818,27 @@ __device__ __forceinline__ RoundState refill_lanes(bool active, int64_t& next, i
 
 // Walk: kQueue turns; slot q receives the leaf found in turn q and its step length, or -1 (no live
 // ray, or a descent still under way).  `broken` reports a malformed tree: the ray ends there.
-__device__ __forceinline__ void walk_turns(const TreeDev<float>& tr, RayState<float>& r, OctreeCursor& cur,
+__device__ __forceinline__ void walk_turns(const TreeDev<float>& tr, const ChildTable& child, RayState<float>& r, OctreeCursor& cur,
                                            float step, bool active, bool& broken, int32_t* q_leaf, float* q_dt) {
     broken = false;
+    if (__builtin_expect(!child.octree, 0)) {
+#pragma unroll
+        for (int q = 0; q < kQueue; ++q) {
+            q_leaf[q] = -1;
+            q_dt[q] = 0.0f;
+            walk_from_root(tr, r, cur, step, active && !broken && r.t < r.tmax, broken, q_leaf[q], q_dt[q]);
+        }
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < kQueue; ++q) {
-        const bool go = active && !broken && r.t < r.tmax;
         q_leaf[q] = -1;
         q_dt[q] = 0.0f;
-        if (any_lane(go)) walk_turn_flat(tr, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
+        cur.turn(r, active & (r.t < r.tmax), child, step, q_leaf[q], q_dt[q]);
     }
+    // (a descent that has come below the last level the coordinates hold waits for the end of the round)
+    const bool deep = active && cur.up < 0 && r.t < r.tmax;
+    if (__builtin_expect(any_lane(deep), 0)) walk_from_root(tr, r, cur, step, deep, broken, q_leaf[kQueue - 1], q_dt[kQueue - 1]);
 }
 
 // Sigma: the densities of the queued leaves, fetched together (the last scalar of each record).
@@ -1143,7 +1192,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     static_assert(!kAllShaded || (!kNoted && !kAccum), "notes and weights look at leaves the marks may hide");
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
     if constexpr (kNoted) {
@@ -1180,6 +1229,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
     OctreeCursor cur;
     cur.reset(path + lane);
+    const ChildTable child(tr);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
     auto start = [&](int64_t item) {
@@ -1232,7 +1282,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
         int32_t q_leaf[kQueue];
         float q_dt[kQueue];
         bool broken;
-        walk_turns(tr, r, cur, step, active, broken, q_leaf, q_dt);
+        walk_turns(tr, child, r, cur, step, active, broken, q_leaf, q_dt);
         // ---- sigma
         float q_sigma[kQueue], q_raw[kQueue];   // (q_raw: what the notes keep, the stored density)
         int n_entries;
@@ -1862,6 +1912,7 @@ static_assert(offsetof(ShadeSharedProbe, who) == sizeof(int32_t) * kQueue * kMar
 // and the colours of leaves below sigma_thresh are evaluated too; the picture itself is composed as
 // without notes.
 constexpr int kSplitThreads = 2 * kMarchThreads;
+constexpr int kWalkTurns = 4;          // of the walk, between looks at the rays that have ended
 constexpr int kRing = 8;               // leaves a lane's walk may be ahead of its shading (a power of two)
 constexpr int kSpinLimit = 1 << 22;
 constexpr int32_t kEndedBit = 1 << 30;   // in SplitBox::taken: the ray wants no more leaves
@@ -1874,10 +1925,10 @@ constexpr int32_t kEndedBit = 1 << 30;   // in SplitBox::taken: the ray wants no
 // 50 001 rays with notes 241 instead of 225).
 constexpr uint32_t kRoundBit = 1u << 30, kOverBit = 1u << 31;
 struct SplitBox {
-    unsigned long long place[kRing * kMarchThreads];   // [place in the ring][lane]
+    unsigned long long place[(kRing + 1) * kMarchThreads];   // [place in the ring][lane], and a row for what is no leaf
     int32_t taken[kMarchThreads];                      // set by the shading: places taken so far (| kEndedBit)
 };
-__device__ __forceinline__ uint32_t ring_round(int32_t n) { return ((uint32_t)n / kRing & 1u) ? 0u : kRoundBit; }
+__device__ __forceinline__ uint32_t ring_round(int32_t n) { return ((uint32_t)n / kRing & 1u) ? kRoundBit : 0u; }
 
 // Places and counts are read and written as atomics of the workgroup (unlike a volatile access, which the compiler leaves on
 // the generic address path -- a flat instruction with a wait for every store --, it still knows that they live in LDS and
@@ -1906,7 +1957,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                                                                              const float* __restrict__ grad_out = nullptr) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ SplitBox box;
     if constexpr (kNoted) {
@@ -1963,7 +2014,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     if (!any_lane(active)) return;   // (both wavefronts see the same rays: both leave or both stay)
     if (walks) {
 #pragma unroll
-        for (int i = 0; i < kRing; ++i) box.place[i * kMarchThreads + lane] = 0ull;
+        for (int i = 0; i < kRing; ++i) box.place[i * kMarchThreads + lane] = kRoundBit;   // (not the first round)
     } else {
         box.taken[lane] = active ? 0 : kEndedBit;
     }
@@ -1973,43 +2024,66 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         // ---- the walk: one leaf per live lane and turn, into the ring
         OctreeCursor cur;
         cur.reset(path + lane);
+        const ChildTable child(tr);
         if (active) cur.begin(r);
-        int32_t written = 0, taken = 0;
+        // (counts of places in bytes of the ring)
+        constexpr uint32_t kPlace = kMarchThreads * 8, kPlaces = kRing * kPlace;
+        uint32_t written = 0, taken = 0;
         bool live = active, broken = false;
         int spins = 0;
+        if (!active) r.t = r.tmax = 0.0f;
+        auto room = [&]() { return written - taken < kPlaces; };
+        auto hand_over = [&](bool found, uint32_t code, float dt) {
+            // (a lane without one writes to the row behind the ring)
+            unsigned char* const at = (unsigned char*)box.place + lane * 8 + (found ? written & (kPlaces - 1) : kPlaces);
+            ring_write((unsigned long long*)at, code | (written << 18 & kRoundBit), dt);
+            written += found ? kPlace : 0u;
+        };
+        static_assert(kPlaces << 18 == kRoundBit, "the bit of a count that says which round it is");
         // the walk is the longest chain of a tile: it goes first where wavefronts share a SIMD
         // (measured: -10 % on a dense image, nothing elsewhere)
         __builtin_amdgcn_s_setprio(3);
-        while (any_lane(live)) {
-            const bool room = live && written - taken < kRing;
-            const bool over = broken || !(r.t < r.tmax);
-            const bool go = room && !over;
-            if (room && over) {   // the walk of this ray is over: say so once
-                ring_write(&box.place[(written & (kRing - 1)) * kMarchThreads + lane],
-                           kOverBit | ring_round(written) | (broken ? 1u : 0u), 0.0f);
-                live = false;
-            }
-            if (!any_lane(room)) {   // every ring is full: the shading is behind (and the turn below does nothing)
-                if (++spins > spin_limit) {
-                    if (lane == 0) atomicAdd(ws.give_ups, 1u);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            } else {
-                spins = 0;
-            }
-            // asked for here, looked at after the turn: not waited for.  (Reading the shading's count only every few
-            // turns was measured slower: rays that have stopped are then walked further.)
+        while (true) {
+            // asked for here, looked at after the turns: not waited for.  (Four turns to a look: one wavefront alone 620 ns a leaf, with two turns and
+            // looks at the rays that are over 770, with a look at everything in every turn 870.)
             const int32_t taken_next = taken_read(&box.taken[lane]);
-            int32_t leaf;
-            float dt;
-            walk_turn_flat(tr, r, cur, step, go, broken, leaf, dt);
-            if (go && leaf >= 0 && !(leaf & kEmptyLeafBit)) {
-                ring_write(&box.place[(written & (kRing - 1)) * kMarchThreads + lane], (uint32_t)leaf | ring_round(written), dt);
-                written += 1;
+            if (child.octree) {
+#pragma unroll
+                for (int k = 0; k < kWalkTurns; ++k) {
+                    int32_t leaf = -1;
+                    float dt;
+                    cur.turn(r, (r.t < r.tmax) & room(), child, step, leaf, dt);
+                    hand_over((uint32_t)leaf < (uint32_t)kEmptyLeafBit, (uint32_t)leaf, dt);
+                }
             }
-            live = live && !(taken_next & kEndedBit);
-            taken = taken_next & ~kEndedBit;
+            taken = (uint32_t)(taken_next & ~kEndedBit) * kPlace;
+            if (taken_next & kEndedBit) {
+                live = false;
+                r.tmax = r.t;
+            }
+            const bool go = (r.t < r.tmax) & room(), deep = go & (cur.up < 0 || !child.octree);
+            if (__builtin_expect(any_lane(deep), 0)) {
+                int32_t leaf = -1;
+                float dt = 0.0f;
+                walk_from_root(tr, r, cur, step, deep, broken, leaf, dt);
+                if (broken) r.tmax = r.t;
+                hand_over((uint32_t)leaf < (uint32_t)kEmptyLeafBit, (uint32_t)leaf, dt);
+            }
+            spins += 1;
+            if (any_lane(go)) {
+                spins = 0;
+                continue;
+            }
+            // nobody can go on: the rays that are over say so, once, and where every ring is full the shading is behind
+            const bool over = live & !(r.t < r.tmax) & room();
+            hand_over(over, kOverBit | (broken ? 1u : 0u), 0.0f);
+            live = live & !over;
+            if (!any_lane(live)) break;
+            if (spins > spin_limit) {
+                if (lane == 0) atomicAdd(ws.give_ups, 1u);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
         }
         return;
     }
@@ -2155,7 +2229,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
                                                                         ReplaySpace ws) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, true> sh;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
@@ -2178,6 +2252,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
     MergeState merge;
     OctreeCursor cur;
     cur.reset(path + lane);
+    const ChildTable child(tr);
 
     // takes ray `item` into this lane if it hits the tree
     auto start = [&](int64_t item) {
@@ -2233,7 +2308,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
         float q_dt[kQueue];
         bool broken;
         float q_sigma[kQueue];
-        walk_turns(tr, r, cur, step, active, broken, q_leaf, q_dt);
+        walk_turns(tr, child, r, cur, step, active, broken, q_leaf, q_dt);
         // ---- sigma
         float q_raw[kQueue];
         fetch_sigma<K>(tr.data, q_leaf, q_sigma);
@@ -2299,7 +2374,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
                 light = 1.0f;
                 phase = kMarch2;
                 r.t = tmin;
-                cur.aim(r);
+                cur.aim(r, kCoordBits - 1);
             } else {
                 active = false;
             }
@@ -2986,7 +3061,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
                                                                 const unsigned long long* __restrict__ only) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, true> sh;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
@@ -3009,6 +3084,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
     bool active = false, second = false;
     OctreeCursor cur;
     cur.reset(path + lane);
+    const ChildTable child(tr);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
     // (with a bitmap `only` the launch does the rays whose bit is set and no others; a batch launch
@@ -3061,7 +3137,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
         int32_t q_leaf[kQueue];
         float q_dt[kQueue];
         bool broken;
-        walk_turns(tr, r, cur, step, active, broken, q_leaf, q_dt);
+        walk_turns(tr, child, r, cur, step, active, broken, q_leaf, q_dt);
         // ---- sigma
         float q_sigma[kQueue], q_raw[kQueue];
         fetch_sigma<K>(tr.data, q_leaf, q_sigma);
@@ -3172,7 +3248,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
                 }
                 light = 1.0f;
                 r.t = tmin;
-                cur.aim(r);
+                cur.aim(r, kCoordBits - 1);
                 second = true;
             } else {
 #pragma unroll

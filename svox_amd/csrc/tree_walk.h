@@ -12,7 +12,7 @@
 //                        frac(p * 2^L).  The walk therefore runs on integers, and because a ray's
 //                        next sample is close to the previous one, it restarts from the deepest
 //                        node whose cell still contains the new point instead of from the root:
-//                        the node ids of the previous path are kept in LDS, one column per lane
+//                        the child rows of the previous path are kept in LDS, one column per lane
 //                        (keeping only the deepest four levels in registers was measured slower:
 //                        more restarts from the root and select chains on the critical path).
 #pragma once

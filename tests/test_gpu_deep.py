@@ -71,6 +71,23 @@ def test_deep_tree_render(gpu, oracle_mod, levels, fmt):
             assert ok, (workspace, err)
 
 
+@pytest.mark.parametrize("levels", [10, 11, 12, 13, 23, 24, 25])
+def test_walks_at_the_edges_of_the_path_and_of_the_coordinates(gpu, oracle_mod, levels):
+    tree, point = synth.deep_tree(levels, data_format="SH1", seed=levels)
+    rays = rays_through(point, 1500, seed=levels)
+    opt = options(tree, step_size=1e-4)
+    ref = oracle_mod.volume_render(oracle_mod.Tree.from_n3tree(tree), rays.origins, rays.dirs, rays.viewdirs, opt)
+    dev, rs = on_gpu(tree, gpu), rays_spec(rays, gpu)
+    # one wavefront per tile, two, rays in pieces, wavefronts that take new rays
+    for flags in (4, 8, 32 | 24 << 8, 2):
+        C.set_debug_flags(flags)
+        try:
+            out = C.volume_render(dev._spec(), rs, opt).cpu().numpy()
+        finally:
+            C.set_debug_flags(0)
+        assert np.array_equal(out, ref), flags
+
+
 @pytest.mark.parametrize("levels", [14, 27])
 def test_deep_tree_queries(gpu, oracle_mod, levels):
     tree, point = synth.deep_tree(levels, data_format="SH4", seed=levels)
