@@ -70,7 +70,7 @@ typedef struct SvoxTreeSpec {
     int32_t dtype;               /* SvoxDType of data/extra_data/offset/scaling/weight_accum */
     const int32_t* child_marks;  /* optional (NULL: none): what svox_mark_empty_leaves / svox_mark_leaves_below wrote for this tree */
     float child_marks_thresh;    /* the sigma_thresh those marks were made with (0 for svox_mark_empty_leaves) */
-    int32_t child_marks_softplus;/* nonzero: they were made with density_softplus */
+    int32_t child_marks_softplus;/* bit 0: they were made with density_softplus; SVOX_MARKS_WALK, SVOX_MARKS_NONE: see svox_walk_table */
 } SvoxTreeSpec;
 
 /* RaysSpec, svox/csrc/include/data_spec.hpp:51-63 */
@@ -138,7 +138,8 @@ const char* svox_status_string(int status);
  * too, with the last two digits for the rays (1 to 16), and 2^2 pieces at least.  With any other flag set no pass takes it.
  * Bit 6: noting passes over ray batches list the rays that meet the tree first, where
  * the workspace has room, whatever their size: up to 64 times bits 8 to 15 of them take two wavefronts per tile, up to 64 times
- * bits 16 and up one, more the batch as it is (so does one most of whose rays hit by a sample).  The flags belong to the calling thread. */
+ * bits 16 and up one, more the batch as it is (so does one most of whose rays hit by a sample).  Bit 7: every call for which
+ * svox_walk_table could be made is said to gain by one.  The flags belong to the calling thread. */
 void svox_set_debug_flags(int flags);
 
 /* No counterpart in the reference.  The forward kernel that walks and shades on two wavefronts hands leaves over
@@ -388,6 +389,20 @@ int svox_mark_empty_leaves(const SvoxTreeSpec* tree, int32_t* marks_out, void* s
  * marks aside and read the child table.  Results are bit-identical with and without marks. */
 int svox_mark_leaves_below(const SvoxTreeSpec* tree, float sigma_thresh, int32_t density_softplus,
                            int32_t* marks_out, void* stream);
+
+/* A walk table of an octree (no counterpart in the reference): the child table, or the marks that tree->child_marks holds where they apply to a
+ * call with these options, laid out so that a ray knows the leaf it is in without reading the row of a node that has leaves only, the last
+ * step of nearly every search.  table_out (capacity, 2, 2, 2) int32; *with_table_out receives a copy of *tree that carries
+ * the table in place of marks, for the render calls with the same options.  every_positive_leaf: the call is one that works on every leaf with
+ * sigma > 0 whatever the threshold (backward, se_grad, noting forward); image: its rays are those of cameras.  Like marks, the table describes child (and, with marks,
+ * data) as they are.  _bytes: the size of the table where making it for one call of n_rays pays, 0 where it does not or the
+ * call would make no use of it.  Results are bit-identical. */
+#define SVOX_MARKS_WALK 2   /* child_marks_softplus: child_marks is a walk table */
+#define SVOX_MARKS_NONE 4   /* ... made without marks: it hides no leaf, and serves every render call */
+int64_t svox_walk_table_bytes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, int32_t image,
+                              int32_t every_positive_leaf);
+int svox_walk_table(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int32_t every_positive_leaf, int32_t* table_out,
+                    SvoxTreeSpec* with_table_out, void* stream);
 
 /* grid_weight_render(data, CameraSpec&, RenderOptions&, offset, scaling) -> {grid_weight, grid_hit};
  * svox.cpp:38-40, 120, rt_kernel.cu:1174-1203 (kernel :898-1003).

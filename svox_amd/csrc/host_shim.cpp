@@ -31,7 +31,7 @@ namespace {
     X(svox_volume_render_noted) X(svox_volume_render_images_noted) X(svox_volume_render_backward_ws)                    \
     X(svox_volume_render_images_backward_ws) X(svox_volume_render_backward_noted_with)                                  \
     X(svox_volume_render_images_backward_noted_with) X(svox_se_grad_ws) X(svox_se_grad_image_ws) X(svox_notes_serve)    \
-    X(svox_mark_leaves_below)
+    X(svox_mark_leaves_below) X(svox_walk_table_bytes) X(svox_walk_table)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     SVOX_CALLS(X)
@@ -326,6 +326,17 @@ void check_shaped(const Tensor& x, const char* name, at::ScalarType dt, at::IntA
     }
 }
 
+// The walk table of a call of n rays, where one pays: it goes with what is returned.  (every_positive_leaf: svox_walk_table)
+Tensor attach_walk(Tree& t, const SvoxRenderOptions& c, int64_t n_rays, bool image, bool every_positive_leaf, void* stream) {
+    Tensor table;
+    const int64_t bytes = lib.svox_walk_table_bytes(&t.spec, &c, n_rays, image, every_positive_leaf);
+    if (bytes <= 0) return table;
+    table = at::empty({bytes / 4}, t.child.options());
+    const SvoxTreeSpec plain = t.spec;
+    status(lib.svox_walk_table(&plain, &c, every_positive_leaf, (int32_t*)table.data_ptr(), &t.spec, stream), "walk_table");
+    return table;
+}
+
 // ---- point queries
 py::tuple query_vertical(py::handle tree, const py::object& points) {
     const Tensor& p = tensor(points, "indices");
@@ -392,6 +403,7 @@ Tensor volume_render(py::handle tree, py::handle rays, py::handle opt, const py:
     const Unlocked unlocked;
     Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, r.spec.n_rays, false, false, on.stream);
     status(lib.svox_volume_render(&t.spec, &r.spec, &c, out.data_ptr(), on.stream), "volume_render");
     return out;
 }
@@ -404,6 +416,7 @@ Tensor volume_render_images(py::handle tree, py::handle cam, py::handle opt, boo
     const Unlocked unlocked;
     Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, k.rays(), true, false, on.stream);
     status(lib.svox_volume_render_images(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), on.stream), "volume_render_images");
     return out;
 }
@@ -421,6 +434,7 @@ Tensor volume_render_noted(py::handle tree, py::handle rays, py::handle opt, con
     const Unlocked unlocked;
     Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, r.spec.n_rays, false, ws.at != nullptr, on.stream);
     status(lib.svox_volume_render_noted(&t.spec, &r.spec, &c, out.data_ptr(), ws.at, ws.bytes, on.stream), "volume_render_noted");
     return out;
 }
@@ -435,6 +449,7 @@ Tensor volume_render_images_noted(py::handle tree, py::handle cam, py::handle op
     const Unlocked unlocked;
     Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, k.rays(), true, ws.at != nullptr, on.stream);
     status(lib.svox_volume_render_images_noted(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), ws.at, ws.bytes, on.stream),
            "volume_render_images_noted");
     return out;
@@ -453,6 +468,7 @@ Tensor volume_render_backward(py::handle tree, py::handle rays, py::handle opt, 
     const Unlocked unlocked;
     Tensor grad = like_data(t);
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, noted ? 0 : r.spec.n_rays, false, true, on.stream);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
     if (noted)
@@ -479,6 +495,7 @@ Tensor volume_render_images_backward(py::handle tree, py::handle cam, py::handle
     const Unlocked unlocked;
     Tensor grad = like_data(t);
     const On on(t.data);
+    const Tensor walk = attach_walk(t, c, noted ? 0 : k.rays(), true, true, on.stream);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
     if (noted)
@@ -516,6 +533,7 @@ py::tuple se_grad(py::handle tree, py::handle rays_or_cam, py::handle opt, const
         grad = like_data(t);
         hess = like_data(t);
         const On on(t.data);
+        const Tensor walk = attach_walk(t, c, image ? k.rays() : r.spec.n_rays, image, true, on.stream);
         if (image)
             status(lib.svox_se_grad_image_ws(&t.spec, &k.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(),
                                              hess.data_ptr(), ws.at, ws.bytes, on.stream),

@@ -220,6 +220,32 @@ static __global__ __launch_bounds__(256) void last_nodes_kernel(const int32_t* _
     walk[i] = c;
 }
 
+// The walk table (kWalkNodeBits) of an octree from its child table or a copy with marks.  One thread per cell.
+static __global__ __launch_bounds__(256) void walk_table_kernel(const int32_t* __restrict__ child, int32_t capacity,
+                                                                uint32_t* __restrict__ walk) {
+    const int64_t i = blockIdx.x * 256ll + threadIdx.x;
+    const int32_t c = i < capacity * 8ll ? child[i] : 0;
+    // the rows of nodes that have leaves only are read by nobody (but the root's)
+    const unsigned long long inner = __ballot(c > 0);
+    const bool last = (inner >> (threadIdx.x & 56u) & 0xffull) == 0;
+    if (i >= capacity * 8ll || (last && i >= 8)) return;
+    uint32_t word = c < 0 ? kWalkEmptyLeaf : 0u;
+    if (c > 0) {
+        const int64_t node = (i >> 3) + c;
+        word = kWalkNodes;   // (a malformed tree's: past the end of every table)
+        if (node < capacity) {
+            const int4 lo = ((const int4*)child)[node * 2], hi = ((const int4*)child)[node * 2 + 1];
+            word = (uint32_t)c;
+            if (max(max(max(lo.x, lo.y), max(lo.z, lo.w)), max(max(hi.x, hi.y), max(hi.z, hi.w))) <= 0) {
+                const uint32_t marks = (lo.x < 0 ? 1u : 0u) | (lo.y < 0 ? 2u : 0u) | (lo.z < 0 ? 4u : 0u) | (lo.w < 0 ? 8u : 0u) |
+                                       (hi.x < 0 ? 16u : 0u) | (hi.y < 0 ? 32u : 0u) | (hi.z < 0 ? 64u : 0u) | (hi.w < 0 ? 128u : 0u);
+                word |= (uint32_t)kLastNodeBit | marks << kWalkNodeBits;
+            }
+        }
+    }
+    walk[i] = word;
+}
+
 // calc_corner_kernel, svox_kernel.cu:91-115: climb parent links from the leaf's node to the
 // root; per level result = (result + cell index) / N.
 template <typename T>

@@ -141,6 +141,7 @@ TreeDev<T> make_tree(const SvoxTreeSpec* t) {
     d.offset = (const T*)t->offset;
     d.scaling = (const T*)t->scaling;
     d.weight_accum = (T*)t->weight_accum;
+    d.walk = nullptr;
     d.capacity = t->capacity;
     d.N = t->N;
     d.K = t->data_dim;
@@ -500,20 +501,52 @@ Lobes lobes_of(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt) {
 // Whether a launch that works on every leaf with density > need_thresh (the forward pass: opt->sigma_thresh; the
 // backward passes, se_grad and the noting passes: 0) may read the caller's marks in place of the child table: the
 // marks hide the leaves whose density is not > child_marks_thresh, which must all be leaves the launch skips.
+// (SVOX_MARKS_NONE: they hide none.)
 bool marks_apply(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh) {
+    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_NONE)) return true;
     return tree->child_marks && tree->child_marks_thresh >= 0.0f && need_thresh >= tree->child_marks_thresh &&
-           (tree->child_marks_softplus != 0) == (opt->density_softplus != 0);
+           ((tree->child_marks_softplus & 1) != 0) == (opt->density_softplus != 0);
 }
 // ... and whether the marks hide exactly the leaves the launch skips: every leaf they let through is shaded.
 bool marks_decide(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh) {
-    return marks_apply(tree, opt, need_thresh) && need_thresh == tree->child_marks_thresh;
+    return marks_apply(tree, opt, need_thresh) && !(tree->child_marks_softplus & SVOX_MARKS_NONE) && need_thresh == tree->child_marks_thresh;
 }
 
 // The tree as the octree march kernels see it: with the caller's marks in place of the child table where they apply.
 TreeDev<float> march_tree(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh = 0.0f) {
     TreeDev<float> d = make_tree<float>(tree);
-    if (marks_apply(tree, opt, need_thresh)) d.child = tree->child_marks;
+    if (marks_apply(tree, opt, need_thresh)) (tree->child_marks_softplus & SVOX_MARKS_WALK ? d.walk : d.child) = tree->child_marks;
     return d;
+}
+
+// Whether a call makes a walk table (svox_walk_table) for its march.  Making it costs 4 us and 11 ps a node, and a march that starts on a
+// table no cache holds; a turn of the walk then waits for one read instead of two, or for none, though in three turns of ten it only descends.  So it pays
+// where rays are many and apart.  us, whole calls without and with it, forward and with notes (SH9, SH4 on 128^3 and 512^3):
+//   batches that all hit        13 000 rays                   40 000              100 000             300 000
+//     64^3                      178, 196 / 153, 186           184, 240 / 163, 209 264, 351 / 232, 313 662, 983 / 527, 843
+//     128^3                     351, 377 / 279, 334           363, 410 / 302, 384 568, 743 / 467, 610 2106, 2611 / 1495, 1992
+//     shell 256^3               126, 241 / 107, 206           142, 307 / 120, 240 183, 341 / 162, 334 515, 1052 / 441, 910
+//     shell 512^3               188, 308 / 166, 265           224, 334 / 198, 285 254, 439 / 224, 385 759, 1210 / 648, 1110
+//   ... 18 % of which do: shell 128^3  53, 92 / 58, 96        53, 147 / 55, 136   69, 151 / 67, 141   132, 206 / 131, 169
+//     shell 256^3               68, 130 / 82, 140             86, 205 / 89, 165   110, 224 / 105, 189 172, 265 / 181, 213
+//     shell 512^3               96, 163 / 126, 189            128, 270 / 132, 228 161, 252 / 147, 231 240, 306 / 252, 259
+//   pictures, 128, 200, 400, 800 pixels a side: shell 128^3  78, 71, 73, 79 / 70, 71, 70, 75;  256^3  132, 138, 136, 137 / 109, 119, 121, 122;
+//     512^3  187, 193, 204, 205 / 166, 167, 175, 188, eight poses 764 / 687;  64^3  166, 157, 148, 158 / 166, 155, 150, 179;  128^3  332, 317, 290, 294 / 304, 300,
+//     271, 319;  NDC 512^3, 128x96, 256x192, 504x378, 1008x756  123, 136, 171, 350 / 120, 120, 187, 366 (rays that share their nodes find them in L1)
+//   ... with notes, 128, 200, 400, 800, which wait for the colours as much as for the walk: shell 128^3  172, 203, 218, 259 / 157, 203, 219, 256;  256^3  258, 287,
+//     299, 347 / 212, 259, 295, 350;  512^3 SH16  341, 377, 400, 543 / 289, 329, 383, 530;  128^3 SH4  317, 317, 306, 429 / 320, 326, 311, 440
+//   32^3 and smaller (batches of 13 000 and 300 000, picture of 800): 68, 253, 81 / 63, 232, 99
+bool walk_table_pays(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, bool image, bool every_positive_leaf) {
+    if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes || fast_basis(tree, opt) < 0) return false;
+    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_WALK)) return false;
+    if (g_debug_flags & 128) return true;
+    if (tree->capacity < 32768 || n_rays <= 12288) return false;
+    if (opt->density_softplus && every_positive_leaf) return false;   // (rays end behind the first leaves they meet)
+    const bool grid = like_complete_octree(tree);
+    if (image && opt->ndc_width > 0) return !grid && n_rays <= 65536;
+    if (image && every_positive_leaf) return !grid && tree->capacity >= 131072;
+    if (image) return !grid || (tree->capacity >= 262144 && n_rays <= 262144);
+    return grid || n_rays >= (every_positive_leaf ? 40000 : 65536);
 }
 
 // the workspace argument of a forward launch that takes no notes
@@ -1804,6 +1837,30 @@ int svox_mark_leaves_below(const SvoxTreeSpec* tree, float sigma_thresh, int32_t
                            (const double*)tree->data, tree->child, cells, tree->data_dim, (double)sigma_thresh,
                            density_softplus != 0, marks_out);
     return check_launch("mark_leaves_below");
+}
+
+int64_t svox_walk_table_bytes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, int32_t image,
+                              int32_t every_positive_leaf) {
+    int od;
+    if (n_rays <= 0 || check_render(tree, opt, &od) || !walk_table_pays(tree, opt, n_rays, image != 0, every_positive_leaf != 0)) return 0;
+    return tree->capacity * 32;
+}
+
+int svox_walk_table(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int32_t every_positive_leaf, int32_t* table_out,
+                    SvoxTreeSpec* with_table_out, void* stream) {
+    int od;
+    int rc = check_render(tree, opt, &od);
+    if (rc) return rc;
+    if (!table_out || !with_table_out) return fail(SVOX_ERR_NULL_POINTER, "table_out / with_table_out is NULL");
+    if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes) return fail(SVOX_ERR_BAD_SHAPE, "walk tables are for octrees of fewer than 2^22 nodes");
+    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_WALK)) return fail(SVOX_ERR_BAD_SHAPE, "child_marks is a walk table already");
+    const bool marked = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh);
+    hipLaunchKernelGGL(walk_table_kernel, dim3((unsigned)((tree->capacity * 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                       marked ? tree->child_marks : tree->child, (int32_t)tree->capacity, (uint32_t*)table_out);
+    *with_table_out = *tree;
+    with_table_out->child_marks = table_out;
+    with_table_out->child_marks_softplus = marked ? (tree->child_marks_softplus & 1) | SVOX_MARKS_WALK : SVOX_MARKS_WALK | SVOX_MARKS_NONE;
+    return check_launch("walk_table");
 }
 
 int svox_mark_empty_leaves(const SvoxTreeSpec* tree, int32_t* marks_out, void* stream) {

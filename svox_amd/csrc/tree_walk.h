@@ -34,6 +34,7 @@ struct TreeDev {
     const T* offset;   // may be null: zero
     const T* scaling;  // may be null: one
     T* weight_accum;
+    const int32_t* walk;   // a walk table of the octree (kWalkNodeBits), or null
     int64_t capacity;
     int32_t N;
     int32_t K;
@@ -50,6 +51,15 @@ constexpr int32_t kEmptyLeafBit = 1 << 30;
 // The point queries may be given a copy of an octree's child table in which an entry whose node has leaves only carries this
 // bit: the row of such a node, where most searches end, need not be read.  (Entries of a well-formed table stay below 2^28.)
 constexpr int32_t kLastNodeBit = 1 << 30;
+
+// A walk table: the child table of an octree of fewer than 2^kWalkNodeBits nodes, or its copy with marks, made over for the march
+// (walk_table_kernel).  The entry of a cell whose node has leaves only says so (kLastNodeBit), and in the bits from kWalkNodeBits on which of
+// the eight are marked empty: the row of such a node, the one in eight of the table's that a ray finds in no cache, need not be read, and is
+// not written.  A marked leaf is the sign bit and the same eight bits, all set.  So the sum of a node's number and an entry of its
+// row is the child's number, kLastNodeBit and its marks: a word of the walk.
+constexpr int kWalkNodeBits = 22;
+constexpr uint32_t kWalkNodes = (1u << kWalkNodeBits) - 1u;
+constexpr uint32_t kWalkEmptyLeaf = 0x80000000u | 0xffu << kWalkNodeBits;
 
 template <typename T>
 __device__ __forceinline__ void load_transform(const TreeDev<T>& tr, T* offset, T* scaling) {

@@ -1,0 +1,167 @@
+"""Walk tables: the child table made over for the march (a node that has leaves only is known by the entry that leads to it)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import svox_amd as svox
+from svox_amd import csrc as C
+from svox_amd import synth
+from svox_amd.csrc import _abi
+from util import grad_close, on_gpu, options, rays_spec
+
+ALWAYS = 128      # debug flag: every call that could makes one
+
+
+def test_which_calls_make_a_walk_table():
+    lib = _abi.load_library()
+    spec, opt = _abi.TreeSpecC(), _abi.RenderOptionsC()
+    spec.data = spec.child = spec.parent_depth = 16
+    spec.N, spec.data_dim, spec.dtype = 2, 13, 0
+    opt.format, opt.basis_dim, opt.max_comp, opt.ndc_width = 1, 4, 3, -1
+
+    def first(nodes, image, positive, low=1, high=1 << 30):
+        spec.capacity = nodes
+        ask = lambda n: lib.svox_walk_table_bytes(ctypes.byref(spec), ctypes.byref(opt), n, image, positive)
+        assert all(ask(n) in (0, nodes * 32) for n in (1, 20000, 1 << 20, 1 << 24))
+        while low < high:
+            middle = (low + high) // 2
+            low, high = (low, middle) if ask(middle) > 0 else (middle + 1, high)
+        return low
+
+    grid64, grid128, shell = 37449, 299593, 192314
+    assert first(grid64, 0, 0) == first(grid64, 0, 1) == first(grid128, 0, 0) == 12289
+    assert first(shell, 0, 1) == 40000 and first(shell, 0, 0) == 65536 and first(shell, 1, 0) == 12289
+    assert first(4681, 0, 1) == first(grid64, 1, 0) == 1 << 30 and first(grid128, 1, 0, high=262144) == 12289
+    assert first((1 << 22) - 1, 1, 0) == 12289 and first(1 << 22, 1, 0) == 1 << 30      # (a node's number has 22 bits)
+    assert first(shell, 1, 1) == 12289 and first(47433, 1, 1) == first(grid128, 1, 1) == 1 << 30
+    opt.ndc_width = 100
+    assert first(shell, 1, 0, high=65536) == 12289
+    opt.ndc_width, opt.density_softplus = -1, 1
+    assert first(shell, 1, 0) == 12289 and first(grid128, 0, 1) == 1 << 30
+    opt.density_softplus = 0
+    opt.ndc_width, spec.N = -1, 3
+    assert first(shell, 0, 1) == 1 << 30
+
+
+def grown(seed, steps=6):
+    """A tree refined a few leaves at a time, so that its nodes lie in no order, with empty leaves and full ones."""
+    g = torch.Generator().manual_seed(seed)
+    tree = svox.N3Tree(N=2, data_format="SH1", init_refine=1)
+    for _ in range(steps):
+        leaves = tree._all_leaves()
+        pick = leaves[torch.randperm(len(leaves), generator=g)[:24]]
+        tree.refine(sel=tuple(pick.T))
+    tree.data.data.copy_(torch.randn(tree.data.shape, generator=g))
+    tree.data.data[..., -1] = 20 * torch.rand(tree.child.shape, generator=g) * (torch.rand(tree.child.shape, generator=g) < 0.4)
+    return tree
+
+
+def trees():
+    yield "one node", svox.N3Tree(N=2, data_format="SH1", init_refine=0)
+    yield "grown", grown(1)
+    yield "shell", synth.shell_tree(depth=6, n_spheres=4, data_format="SH4", seed=1)
+    for levels in (12, 27):
+        yield f"deep {levels}", synth.deep_tree(levels, data_format="SH1", seed=levels)[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("marks", [False, True])
+def test_what_a_walk_table_holds(gpu, marks):
+    for name, tree in trees():
+        dev = on_gpu(tree, gpu)
+        opt = options(dev, step_size=1e-3, sigma_thresh=0.0)
+        spec = dev._spec()
+        if marks:
+            spec.child_marks = C.mark_empty_leaves(spec, 0.0, False)
+        table = torch.full((dev.child.numel(),), 7, dtype=torch.int32, device=gpu)
+        made = _abi.TreeSpecC()
+        packed = C._pack_tree(spec)
+        C._call("svox_walk_table", ctypes.byref(packed), ctypes.byref(opt._pack()), 0, table.data_ptr(), ctypes.byref(made),
+                torch.cuda.current_stream().cuda_stream)
+        got = table.cpu().numpy().astype(np.int64) & 0xffffffff
+        rows = (spec.child_marks if marks else dev.child).cpu().numpy().reshape(-1, 8).astype(np.int64)
+        bits = ((rows < 0) << np.arange(8)).sum(1)
+        last = (rows <= 0).all(1)
+        for node, row in enumerate(rows):
+            for cell, c in enumerate(row):
+                want = 0 if c == 0 else 0x80000000 | 255 << 22
+                if c > 0:
+                    want = c | (1 << 30 | int(bits[node + c]) << 22 if last[node + c] else 0)
+                if last[node] and node > 0:
+                    want = 7      # (read by nobody)
+                assert got[node * 8 + cell] == want, (name, node, cell)
+        assert made.child_marks == table.data_ptr() and made.child_marks_softplus == (2 if marks else 6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", [4, 8, 2, 32 | 24 << 8, 64 | 1 << 8 | 2 << 16])
+def test_walks_on_a_walk_table_are_those_on_the_child_table(gpu, oracle_mod, kernel):
+    """One wavefront per tile, two, wavefronts that take new rays, rays in pieces, listed rays; with marks and without."""
+    for name, tree in trees():
+        if name == "one node":
+            tree.data.data.copy_(torch.rand(tree.data.shape, generator=torch.Generator().manual_seed(3)) * 2)
+        ot = oracle_mod.Tree.from_n3tree(tree)
+        dev = on_gpu(tree, gpu)
+        rays = synth.sphere_rays(1500, seed=4)
+        rs = rays_spec(rays, gpu)
+        go = torch.randn(1500, 3, generator=torch.Generator().manual_seed(5))
+        for thresh, softplus, marked in ((1e-2, False, False), (1e-2, False, True), (0.0, False, True), (0.0, True, False)):
+            opt = options(tree, step_size=1e-3, sigma_thresh=thresh, density_softplus=softplus)
+            spec = dev._spec()
+            if marked:
+                spec.child_marks, spec.child_marks_thresh = C.mark_empty_leaves(spec, thresh, False), thresh
+            ref = oracle_mod.volume_render(ot, rays.origins, rays.dirs, rays.viewdirs, opt)
+            C.set_debug_flags(kernel | ALWAYS)
+            try:
+                out = C.volume_render(spec, rs, opt).cpu().numpy()
+                noted, notes = C.volume_render_noted(spec, rs, opt)
+                grad = C.volume_render_backward_noted(spec, rs, opt, go.to(gpu), notes).cpu().numpy()
+                marched = C.volume_render_backward(spec, rs, opt, go.to(gpu), workspace=False).cpu().numpy()
+                alone = C.volume_render_backward(spec, rs, opt, go.to(gpu)).cpu().numpy()
+                squared = C.se_grad(spec, rs, ref_colour(gpu), opt)
+            finally:
+                C.set_debug_flags(0)
+            if softplus:      # (logf is the platform's)
+                assert np.abs(out - ref).max() <= 1e-5
+            else:
+                assert np.array_equal(out, ref), (name, thresh, marked)
+            assert np.array_equal(noted.cpu().numpy(), out)
+            plain = dev._spec()
+            want = C.volume_render_backward(plain, rs, opt, go.to(gpu), workspace=False).cpu().numpy()
+            # (the same terms in other orders)
+            scale = np.abs(want).max() + 1e-30
+            for got in (grad, marched, alone):
+                assert np.abs(got - want).max() <= 2e-4 * scale, (name, thresh, softplus, marked)
+            again = C.se_grad(plain, rs, ref_colour(gpu), opt)
+            assert torch.equal(squared[0], again[0])
+            for a, b in zip(squared[1:], again[1:]):
+                assert (a - b).abs().max() <= 2e-4 * b.abs().max() + 1e-30
+
+
+def ref_colour(gpu):
+    return torch.rand(1500, 3, generator=torch.Generator().manual_seed(6)).to(gpu)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", [4, 8, 32 | 24 << 8])
+@pytest.mark.parametrize("thresh,marked", [(1e-2, False), (1e-2, True), (0.0, True)])
+def test_pictures_on_a_walk_table(gpu, oracle_mod, kernel, thresh, marked):
+    tree = synth.shell_tree(depth=7, n_spheres=6, data_format="SH9", seed=2)
+    dev = on_gpu(tree, gpu)
+    poses = torch.stack(synth.orbit_poses(2, seed=1, radius=2.5)).contiguous().to(gpu)
+    opt = options(tree, step_size=1e-3, sigma_thresh=thresh)
+    spec = dev._spec()
+    cam = C.CameraSpec()
+    cam.c2w, cam.fx, cam.fy, cam.width, cam.height = poses, 90.0, 90.0, 61, 45
+    want = C.volume_render_images(spec, cam, opt)
+    if marked:
+        spec.child_marks, spec.child_marks_thresh = C.mark_empty_leaves(spec, thresh, False), thresh
+    C.set_debug_flags(kernel | ALWAYS)
+    try:
+        got = C.volume_render_images(spec, cam, opt)
+        noted, notes = C.volume_render_images_noted(spec, cam, opt)
+    finally:
+        C.set_debug_flags(0)
+    assert torch.equal(got, want) and torch.equal(noted, want)
