@@ -270,19 +270,19 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
         }
         shaded = count;
         wave_lds_sync();
-        for (int p = lane; p < n_fresh * 3; p += kMarchThreads) {
-            const int e = p / 3, c = p - 3 * e;
+        // (a lane to an entry, all of whose record it asks for at once: a lane to a channel waited for memory three times as often.  FIGS)
+        for (int e = lane; e < n_fresh; e += kMarchThreads) {
             const int of = order[e];
             const int at_ray = (of & 63) >> cut;
             const float* rec = tr.data + (int64_t)lists.leaf[of] * K;
-            float s;
+            float s[3];
             if constexpr (P::kFormat == SVOX_FORMAT_RGBA) {
-                s = sigmoid_(rec[c]);
-            } else {
-                const float* co = rec + c * D;
-                float cv[D];
 #pragma unroll
-                for (int i = 0; i < D; ++i) cv[i] = co[i];
+                for (int c = 0; c < 3; ++c) s[c] = rec[c];
+            } else {
+                float co[3 * D];
+#pragma unroll
+                for (int i = 0; i < 3 * D; ++i) co[i] = rec[i];
                 float b[D];
                 if constexpr (P::kForwardRows) {
 #pragma unroll
@@ -291,16 +291,18 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                     const float vd[3] = {ray_basis[at_ray * 3], ray_basis[at_ray * 3 + 1], ray_basis[at_ray * 3 + 2]};
                     sh_basis<float>(P::kBasis, vd, b);
                 }
-                float tmp = 0.0f;
 #pragma unroll
-                for (int i = 0; i < D; ++i) tmp = fma_(b[i], cv[i], tmp);
-                s = sigmoid_(tmp);
+                for (int c = 0; c < 3; ++c) s[c] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < D; ++i) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) s[c] = fma_(b[i], co[c * D + i], s[c]);
+                }
             }
-            lists.colour[of * 3 + c] = s;
-            if (c == 2) {
-                const float raw = lists.raw[of];
-                att_of[of] = expf_fixed(-lists.dt[of] * ray_dscale[at_ray] * (opt.density_softplus ? softplus_m1(raw) : raw));
-            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) lists.colour[of * 3 + c] = sigmoid_(s[c]);
+            const float raw = lists.raw[of];
+            att_of[of] = expf_fixed(-lists.dt[of] * ray_dscale[at_ray] * (opt.density_softplus ? softplus_m1(raw) : raw));
         }
         wave_lds_sync();
         // ---- the rays' order, as far as it is listed
