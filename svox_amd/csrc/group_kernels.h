@@ -13,9 +13,8 @@
 // gradient, us: 512 entries 172, 285, but 405, 933 instead of 270, 645 where no leaf is empty; 592 176, 285; 640 181, 332; 768 205, 333;
 // 896 226, 362; lists of 20 entries for every lane, none shared, 222, 361).
 // Measured, four lanes that walk a ray together, from end to end / pieces, forward pass and gradient, us (more: group_cut):
-//   64^3 SH4, half of the leaves empty  1 000 rays 226, 383 / 57, 78    5 000 262, 394 / 78, 121    20 000 295, 442 / 172, 292
-//   no leaf empty                       1 000 rays 232, 541 / 65, 140   5 000 269, 570 / 110, 263   20 000 305, 644 / 280, 658
-//   256^3 shell SH16, every ray hits    1 000 rays 370, 809 / 96, 214   5 000 439, 900 / 131, 364   20 000 509, 1023 / 271, 631
+//   64^3 SH4, half of the leaves empty  1 000 rays 226, 383 / 51, 72    20 000 279, 561 / 161, 250
+//   no leaf empty                       1 000 rays 232, 541 / 54, 124   20 000 287, 686 / 235, 565
 // The lanes of a ray that walk it together are the kernels for more rays than find room in pieces (below).
 #pragma once
 
@@ -522,7 +521,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
 // ---- more rays than the pieces of find room on the GPU, or in their lists (group_cut): four lanes walk a ray together (the same addresses, one
 // request), each doing one axis' arithmetic, lane c evaluates channel c, and the record of a leaf is asked for before the next step
 // of the walk and used after it.  (128^3 SH4 without empty leaves, four lanes to a ray / pieces: gradient of 20 000 rays
-// 1485 / 1336, of 131 072 6 338 / 7 670 us.)
+// 1511 / 1185, of 131 072 4 683 / 6 633 us.)
 constexpr int kSharedLanes = 4;
 constexpr int kSharedRays = kMarchThreads / kSharedLanes;
 
@@ -543,39 +542,38 @@ __device__ __forceinline__ double from_group(double v) {
 // kGroupSeekBudget child reads; a longer descent goes on in the next turn, so that the other rays of the wavefront do not
 // wait for it.
 struct SharedWalk {
-    double o, d, inv, up;      // this lane's axis, o and d times 2^24; up = max(inv, 0), see leaf_exit
+    double o, d, inv, far;     // this lane's axis, o and d times 2^24; far = max(inv, 0), see leaf_exit
     double t, tmax, dscale;
     double p;                  // the sample's clamped coordinate on this lane's axis, times 2^24
-    int32_t* rows;             // this lane's column of the path, counted from level 1 (OctreeCursor)
+    int32_t* rows;             // this lane's column of the path (OctreeCursor)
     uint32_t nx, ny, nz;       // integer cell coordinates of the sample
-    int levels;                // of the previous leaf (1: none)
-    int level;                 // where the search for the sample's leaf stands
-    int32_t node;
+    int up;                    // where the search for its leaf stands
+    uint32_t row;
+    int leaf_up;               // of the previous leaf (kCoordBits - 1: the path says nothing of it)
 
     __device__ __forceinline__ void begin(const RayState<double>& r, int axis, int32_t* lane_path) {
         o = (axis == 1 ? r.o[1] : axis == 2 ? r.o[2] : r.o[0]) * 16777216.0;
         d = (axis == 1 ? r.d[1] : axis == 2 ? r.d[2] : r.d[0]) * 16777216.0;
         inv = axis == 1 ? r.inv[1] : axis == 2 ? r.inv[2] : r.inv[0];
-        up = max_(inv, 0.0);
+        far = max_(inv, 0.0);
         t = r.t;
         tmax = r.tmax;
         dscale = r.dscale;
-        rows = lane_path - kMarchThreads;
-        rows[kMarchThreads] = 0;
+        rows = lane_path - OctreeCursor::kPathUp * kMarchThreads;
+        rows[kCoordBits * kMarchThreads] = 0;
         nx = ny = nz = 0;
-        levels = 1;
+        leaf_up = kCoordBits - 1;
     }
     __device__ __forceinline__ bool ended() const { return !(t < tmax); }
 
-    // the sample at t: its position, and the deepest node of the previous path it still lies in
+    // the sample at t: its position, and the deepest row of the previous path it still lies in
     __device__ __forceinline__ void aim() {
         p = max_(0.0, min_((1.0 - 1e-6) * 16777216.0, fma_(t, d, o)));   // (clamp01, times 2^24)
         const int n = (int)(uint32_t)p;
         const uint32_t mx = (uint32_t)from_group<0>(n), my = (uint32_t)from_group<1>(n), mz = (uint32_t)from_group<2>(n);
-        const uint32_t diff = (nx ^ mx) | (ny ^ my) | (nz ^ mz);
-        const uint32_t first_diff = (diff ? (uint32_t)__builtin_clz(diff) : 0xffffffffu) - (31 - kCoordBits);
-        level = (int)min(min(first_diff, (uint32_t)levels), (uint32_t)kPathLevels);
-        node = rows[level * kMarchThreads];
+        const uint32_t diff = (nx ^ mx) | (ny ^ my) | (nz ^ mz) | 1u << leaf_up | 1u << (OctreeCursor::kPathUp + 1);
+        up = 31 - __builtin_clz(diff);
+        row = (uint32_t)rows[(up + 1) * kMarchThreads];
         nx = mx;
         ny = my;
         nz = mz;
@@ -583,33 +581,39 @@ struct SharedWalk {
 
     // One turn of the search.  True: the leaf is found (its cell index, -1 in a malformed tree), delta_t is the step of
     // the sample and the ray stands at the next one (aim() is still to be called).  rt_kernel.cu:262-275, 315.
-    __device__ __forceinline__ bool turn(const TreeDev<double>& tr, double step_size, int64_t& leaf, double& delta_t) {
-        int32_t cell = 0, skip = 1;
-#pragma unroll
-        for (int it = 0; it < kGroupSeekBudget; ++it) {
-            if (skip > 0 && level <= kCoordBits) {
-                rows[min(level, kPathLevels + 1) * kMarchThreads] = node;
-                cell = (node << 3) | cell_at(nx, ny, nz, level);
-                skip = tr.child[cell];
-                // (negative: no entry of a well-formed tree; the walk from the root says what comes of it)
-                const bool down = skip != 0;
-                node += skip;
-                level = down ? ((uint32_t)node >= (uint32_t)tr.capacity ? kCoordBits + 1 : level + 1) : level;
-                skip = down ? 1 : 0;
-            }
-        }
-        if (skip > 0 && level <= kCoordBits) return false;
+    __device__ __forceinline__ bool turn(const TreeDev<double>& tr, const ChildTable& child, double step_size, int64_t& leaf, double& delta_t) {
+        static_assert(kGroupSeekBudget == 2, "two reads, written out");
+        const uint32_t first = shift_or<2>(octant_of(nx, ny, nz, up), row);
+        const int32_t skip1 = child.read(first);
+        const bool below = skip1 > 0;
+        const uint32_t next = row + ((uint32_t)skip1 << 5);
+        int32_t* const at = rows + max(up, OctreeCursor::kPathUp) * kMarchThreads;
+        at[kMarchThreads] = (int32_t)row;
+        at[0] = (int32_t)next;
+        up -= below ? 1 : 0;
+        const uint32_t second = shift_or<2>(octant_of(nx, ny, nz, up), below ? next : ChildTable::kNowhere);
+        row = below ? next : row;
+        const int32_t skip2 = child.read(second);
+        const int32_t skip = min(skip1, skip2);
+        const uint32_t cell = (below ? second : first) >> 2;
+        const bool found = skip <= 0;
+        // (a negative entry, of which a well-formed tree has none, and a cell beyond the table: the walk from the root says what comes of it)
+        const bool deep = up < 0 || (found & (skip < 0 || cell > child.last_cell));
+        const int here = up;
+        row += (uint32_t)max(skip2, 0) << 5;
+        up -= skip2 > 0 ? 1 : 0;
+        if (!found && !deep) return false;
         double segment;
         leaf = cell;
-        if (skip == 0) {
-            levels = level;
+        if (!deep) {
+            leaf_up = here;
             // (dda_unit for a point inside the cube: the entry distance is 0, see leaf_exit)
-            const double e = -__builtin_amdgcn_fract(p * __longlong_as_double((long long)(1023 - kCoordBits + level) << 52)) * inv + up;
+            const double e = -__builtin_amdgcn_fract(p * __longlong_as_double((long long)(1023 - here) << 52)) * inv + far;
             const double hi = min_(min_(min_((double)1e9f, from_group<0>(e)), from_group<1>(e)), from_group<2>(e));
-            segment = hi * __longlong_as_double((long long)(1023 - level) << 52);
+            segment = hi * __longlong_as_double((long long)(1023 - kCoordBits + here) << 52);
         } else {
             // more levels than the integer coordinates hold, or a malformed tree
-            levels = 1;
+            leaf_up = kCoordBits - 1;
             const double q = p * (1.0 / 16777216.0);
             double local[3] = {from_group<0>(q), from_group<1>(q), from_group<2>(q)};
             const double all_inv[3] = {from_group<0>(inv), from_group<1>(inv), from_group<2>(inv)};
@@ -680,10 +684,11 @@ __device__ __forceinline__ int64_t shared_ray(const TreeDev<double>& tr, const S
 template <int D, class Source>
 __global__ __launch_bounds__(kMarchThreads) void render_forward_shared_kernel(TreeDev<double> tr, Source src,
                                                                              SvoxRenderOptions opt, double* __restrict__ out) {
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ double basis_rows[kSharedRays * (D > 0 ? D : 1)];
     const int lane = threadIdx.x, channel = lane & (kSharedLanes - 1);
     SharedWalk walk;
+    const ChildTable child(tr);
     bool live;
     const int64_t slot = shared_ray<D>(tr, src, opt, lane, path, basis_rows, walk, live);
     if (slot < 0) return;
@@ -704,7 +709,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_shared_kernel(Tr
         // the next leaf is looked up while the record of the one before it is on its way
         int64_t leaf = -1;
         double next_dt = 0.0;
-        if (walking && !walk.turn(tr, (double)opt.step_size, leaf, next_dt)) continue;
+        if (walking && !walk.turn(tr, child, (double)opt.step_size, leaf, next_dt)) continue;
         const bool more = walking && leaf >= 0;
         walking = more && !walk.ended();
         if (walking) walk.aim();
@@ -735,7 +740,9 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_shared_kernel(Tr
 // walks on only where the list was full.  The wavefront adds the records of a step together: scalar f from lane
 // f mod 64, so that the scalars of a record go out in requests of 64 bytes (the memory system takes a fixed number of
 // those per microsecond).
-constexpr int kSharedKept = 96;
+// (Few, as LDS has room for the more wavefronts: 96 / 64 / 48 / 32, gradient of 131 072 rays, no leaf empty, 128^3 SH4 6 304 / 5 515 / 4 796 / 4 686 us,
+// half of them 4 372 / 4 180 / 3 762 / 3 669, 256^3 shell SH16 6 278 / 5 557 / 5 175 / 5 033.)
+constexpr int kSharedKept = 32;
 
 template <int D, class Source>
 __global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(TreeDev<double> tr, Source src,
@@ -744,7 +751,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(T
                                                                               double* __restrict__ grad_data) {
     constexpr int K = SharedRecord<D>::K;
     constexpr int DD = D > 0 ? D : 1;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ double basis_rows[kSharedRays * DD];
     __shared__ double kept_dt[kSharedKept * kSharedRays];     // [place][ray]
     __shared__ int32_t kept_leaf[kSharedKept * kSharedRays];
@@ -753,6 +760,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(T
     __shared__ uint8_t listed[kSharedRays];           // rays with a record in this step
     const int lane = threadIdx.x, channel = lane & (kSharedLanes - 1), ray = lane / kSharedLanes;
     SharedWalk walk;
+    const ChildTable child(tr);
     bool live;
     const int64_t slot = shared_ray<D>(tr, src, opt, lane, path, basis_rows, walk, live);
     if (!__any(live)) return;
@@ -792,7 +800,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(T
             int64_t leaf = -1;
             double next_dt = 0.0;
             const double next_t = walk.t;
-            if (walking && !walk.turn(tr, (double)opt.step_size, leaf, next_dt)) continue;
+            if (walking && !walk.turn(tr, child, (double)opt.step_size, leaf, next_dt)) continue;
             const bool more = walking && leaf >= 0;
             if (walking && !more) whole = false;
             walking = more && !walk.ended();
@@ -852,7 +860,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_shared_kernel(T
         int64_t leaf = -1;
         double next_dt = 0.0;
         if (walking) {
-            turned = walk.turn(tr, (double)opt.step_size, leaf, next_dt);
+            turned = walk.turn(tr, child, (double)opt.step_size, leaf, next_dt);
             if (turned) {
                 walking = leaf >= 0 && !walk.ended();
                 if (walking) walk.aim();

@@ -373,7 +373,8 @@ struct ChildTable {
     uint32_t last_cell;
     bool octree, words;   // words: it is a walk table
     static constexpr uint32_t kNowhere = 0xffffffe0u;   // a row beyond the largest table
-    __device__ __forceinline__ explicit ChildTable(const TreeDev<float>& tr) {
+    template <typename T>
+    __device__ __forceinline__ explicit ChildTable(const TreeDev<T>& tr) {
         const uint32_t cells = (uint32_t)tr.capacity << 3;
         octree = tr.N == 2;
         last_cell = cells - 1u;
@@ -383,6 +384,20 @@ struct ChildTable {
     __device__ __forceinline__ int32_t read(uint32_t at) const { return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(entries, (int)at, 0, 0); }
     __device__ __forceinline__ uint32_t cell(uint32_t number) const { return min(number, last_cell); }
 };
+
+// (a << n) | b in one instruction: in plain C++ the compiler orders the three below so that it takes four
+template <int n>
+__device__ __forceinline__ uint32_t shift_or(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_lshl_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "n"(n), "v"(b));
+    return r;
+}
+// which cell of its node a sample lies in, `up` levels above the finest that its integer coordinates hold
+__device__ __forceinline__ uint32_t octant_of(uint32_t ix, uint32_t iy, uint32_t iz, int up) {
+    const unsigned bx = __builtin_amdgcn_ubfe(ix, (unsigned)up, 1u), by = __builtin_amdgcn_ubfe(iy, (unsigned)up, 1u),
+                   bz = __builtin_amdgcn_ubfe(iz, (unsigned)up, 1u);
+    return shift_or<1>(shift_or<1>(bx, by), bz);
+}
 
 // The walk of one lane's ray through the tree, sample after sample.  A sample's integer coordinates (24 bits an axis)
 // say which cell it lies in at every level, and those it shares with the sample before say how far up the next search
@@ -450,19 +465,8 @@ struct OctreeCursor {
         iy = ny;
         iz = nz;
     }
-    // (a << n) | b in one instruction: in plain C++ the compiler orders the three of them so that it takes four
-    template <int n>
-    static __device__ __forceinline__ uint32_t shift_or(uint32_t a, uint32_t b) {
-        uint32_t r;
-        asm("v_lshl_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "n"(n), "v"(b));
-        return r;
-    }
     // which cell of its node the sample lies in
-    __device__ __forceinline__ uint32_t octant() const {
-        const unsigned bx = __builtin_amdgcn_ubfe(ix, (unsigned)up, 1u), by = __builtin_amdgcn_ubfe(iy, (unsigned)up, 1u),
-                       bz = __builtin_amdgcn_ubfe(iz, (unsigned)up, 1u);
-        return shift_or<1>(shift_or<1>(bx, by), bz);
-    }
+    __device__ __forceinline__ uint32_t octant() const { return octant_of(ix, iy, iz, up); }
     // the byte of the table that holds the child entry to look at, in the row that begins at `from`
     __device__ __forceinline__ uint32_t entry(uint32_t from) const { return shift_or<2>(octant(), from); }
     // One turn of the lanes with `go`: up to kSeekBudget child reads, and if the leaf is found its index (with

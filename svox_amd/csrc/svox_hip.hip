@@ -450,36 +450,35 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     // wavefront as leaves the lists room for all they find: the launcher cannot know how many leaves have density, so the lines are
     // drawn where trees all of whose leaves do lose nothing or little.  What was measured (us; lanes that walk a ray together / pieces, in
     // parentheses where they are not taken; half of the leaves with density, all of them):
-    //   forward           1 000 rays                5 000                  20 000                  24 000
-    //   8^3 SH1           -, 25 / (-, 32)           -, 27 / (-, 43)        -, 30 / (-, 35)
-    //   16^3 SH4          57, 58 / 31, 36           58, 60 / 39, 45        67, 70 / 49, 60         68, 70 / (51, 73)
-    //   32^3 SH9          133, 139 / 50, 55         138, 145 / 59, 70      159, 167 / 104, 164     158, 164 / (107, 168)
-    //   64^3 SH4          225, 231 / 56, 65         260, 268 / 77, 109     296, 305 / 172, 277     296, 305 / (205, 320)
-    //   128^3 SH4         512, 521 / 61, 88         528, 543 / 130, 241    595, 619 / 370, 565     594, 611 / (416, 637)
-    //   shell 128^3 SH9   215, 239 / 79, 89         276, 305 / 91, 120     311, 337 / 201, 281     28 672: 313, 340 / (277, 373)
-    //   shell 256^3 SH9   295, 316 / 95, 101        375, 426 / 122, 175    429, 475 / 258, 365     28 672: 409, 446 / (349, 480)
-    //   gradient          1 000 rays                20 000                 24 000                  40 960                    65 536
-    //   16^3 SH4          89, 118 / 50, 72          112, 149 / 96, 164     117, 165 / (106, 201)   192, 265 / (174, 277)     266, 367 / (249, 462)
-    //   32^3 SH9          222, 306 / 80, 146        281, 381 / 223, 385    297, 424 / 263, 436     508, 690 / 404, 610       709, 1007 / 624, 951
-    //   64^3 SH4          382, 539 / 79, 139        442, 643 / 292, 655    463, 688 / 427, 653     766, 1131 / 694, 1033     1084, 1589 / (810, 1773)
-    //   128^3 SH4         910, 1211 / 128, 230      1129, 1489 / 683, 1336 1117, 1526 / (713, 1517) 1861, 2603 / 1147, 2452  2565, 3688 / (1769, 3779)
-    //   shell 128^3 SH9   396, 556 / 115, 146       534, 742 / 321, 640    600, 794 / 399, 738     795, 1163 / 576, 1085     1082, 1669 / 881, 1637
-    //   shell 256^3 SH16  809, 1145 / 214, 262      1023, 1519 / 631, 1250 1054, 1732 / 708, 1493  1324, 2241 / 1011, 2147   1866, 3104 / 1485, 3207
-    // Lanes that walk together fill the GPU with 32 768 rays of a gradient, and take a second turn for the next: there pieces gain once more.
-    // Full trees lose on the near side of some lines: 3 % of a 64^3 SH16 gradient, 9 % of a 16^3 one and 10 % of the forward pass of a 64^3 shell
-    // at 20 000 rays, 5 % of a 128^3 RGBA gradient at 40 960.
+    //   forward           20 000 rays               26 000                 40 960
+    //   16^3 SH4          65, 67 / 43, 51           66, 69 / (73, 79)      76, 79 / (94, 106)
+    //   32^3 SH9          155, 162 / 96, 139        160, 167 / 102, 146    182, 183 / (141, 212)
+    //   64^3 SH4          279, 287 / 153, 234       286, 294 / 194, 288    333, 335 / (283, 426)
+    //   64^3 SH16         407, 428 / 178, 282       436, 458 / 223, 349    492, 514 / (335, 515)
+    //   128^3 SH4         548, 568 / 338, 491       577, 591 / 423, 614    628, 647 / (634, 934)
+    //   shell 128^3 SH9   303, 346 / 199, 281       305, 334 / 246, 333    345, 389 / (369, 493)
+    //   shell 256^3 SH16  506, 594 / 290, 416       532, 659 / 344, 525    585, 701 / (513, 756)
+    //   gradient          20 000 rays               26 000                 40 960                    65 536                    131 072
+    //   16^3 SH4          115, 154 / 88, 154        121, 173 / 111, 144    153, 220 / (156, 208)     226, 328 / (223, 303)     335, 497 / (412, 558)
+    //   32^3 SH9          307, 426 / 209, 331       337, 478 / 256, 410    427, 594 / 371, 571       602, 957 / 562, 834       913, 1500 / (1088, 1599)
+    //   64^3 SH4          561, 686 / 250, 565       602, 744 / 309, 703    699, 903 / 628, 910       1030, 1401 / 986, 1413    1576, 2184 / (1909, 2709)
+    //   64^3 SH16         932, 1271 / 515, 1090     1050, 1404 / 627, 1316 1248, 1801 / 1079, 1723   1939, 2885 / 1679, 2675   3125, 4880 / (3283, 5134)
+    //   128^3 SH4         1304, 1511 / 559, 1185    1375, 1604 / 692, 1464 1562, 1858 / 1025, 2211   2361, 2987 / (1574, 3416) 3695, 4683 / (3038, 6633)
+    //   shell 128^3 SH9   601, 899 / 325, 689       658, 887 / 398, 809    677, 1165 / 581, 1168     979, 1681 / 862, 1761     1477, 2587 / (1659, 3300)
+    //   shell 256^3 SH16  1094, 1668 / 639, 1400    1174, 1819 / 732, 1674 1286, 2329 / 1019, 2367   1898, 3235 / 1527, 3604   2903, 5093 / (2827, 6745)
+    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full 128^3 grids lose a fifth of a gradient beyond
+    // 32 768 rays, full shells a tenth at 65 536, for the sake of trees with empty leaves, which gain a third.
     const double cells = (double)tree->capacity * 8.0;
     const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
     const bool grid = like_complete_octree(tree);
     constexpr int64_t kFill = 20480;
     if (tiny && !(gradient && n_rays <= 2560)) return c;
-    if (n_rays > kFill) {
-        if (!gradient || small || (!grid && n_rays > 65536)) return c;
-        if (grid && !medium && n_rays > (large ? kFill : 24576) && (n_rays <= 32768 || n_rays > 40960)) return c;
-    }
+    const int64_t most_rays = gradient ? (small ? 32768 : grid && large ? 40960 : 65536) : small ? kFill : 26624;
+    if (n_rays > most_rays) return c;
     if (small) {
-        c.per_wave = n_rays <= 14336 ? 8 : 12;     // (8 rays to each of 1 792 wavefronts, all that run at once)
-        c.most = n_rays <= 14336 ? 3 : 2;
+        const bool eight = n_rays <= 14336 || n_rays > kFill;
+        c.per_wave = eight ? 8 : 12;     // (8 rays to each of 1 792 wavefronts, all that run at once)
+        c.most = eight ? 3 : 2;
     } else if (medium) {
         const bool short_lists = n_rays <= 8192 || (gradient && n_rays > 14336);
         c.per_wave = short_lists ? 4 : 8;
@@ -487,7 +486,7 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     } else {
         // (of a 128^3 grid the lists hold the leaves of two rays, four in a pinch: 4 x 16 / 2 x 32, gradient 20 000 rays 787, 1542 / 683, 1336,
         // forward pass 12 000 rays 229, 417 / 235, 364, 20 000 rays 336, 623 / 370, 565)
-        const bool two = grid && (large ? gradient || n_rays > 16384 : n_rays > kFill);
+        const bool two = grid && (large ? gradient || n_rays > 16384 : n_rays > 28672);
         c.per_wave = large && n_rays <= 1280 ? 1 : n_rays <= 2560 || two ? 2 : 4;
         c.most = large ? 6 : 5;
     }
