@@ -60,7 +60,8 @@ struct CutLists {
     float colour[kListed * kMarchThreads * 3];
     int32_t count[kMarchThreads];
     // what is composed in this round: from which entry on, how many, and from which place in the ray's order on
-    int32_t from[kMarchThreads], taken[kMarchThreads], place[kMarchThreads];
+    // (16 bits: with 26 880 bytes of LDS six wavefronts run on a compute unit, with more five; 8 000 rays of a 128^3 SH4 grid 174 / 193 us)
+    int16_t from[kMarchThreads], taken[kMarchThreads], place[kMarchThreads];
     // which of the piece's first samples are listed (bits 0 to 7); the sample (8 to 10) of the lane (11 to 16) the ray goes on
     // with, if it does (kLinked), or whether it ends here (kOver), in a malformed tree (kBroken)
     uint32_t end[kMarchThreads];
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
     constexpr int kListed = cut_listed(kNoted);
     constexpr int kMostRays = kCutMostRays;
     __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
-    __shared__ PieceHeads<float, kCutHeads> heads;           // (-1: not known yet)
+    __shared__ PieceHeads<float, kCutHeads + 1> heads;       // (-1: not known yet; the last row is for what is to be kept from nobody)
     __shared__ CutLists<kListed> lists;
     __shared__ float atts[kNoted ? kListed * kMarchThreads : 1];      // attenuations (without notes: in lists.dt)
     float* const att_of = kNoted ? atts : lists.dt;
@@ -195,10 +196,18 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
             int32_t q_leaf[kCutTurns];
             float q_dt[kCutTurns];
             int number = sample;       // of the sample the next leaf found belongs to
+            // the sample of a lane with `found` is looked at, the next one stands at r.t
+            auto arrive = [&](bool found) {
+                sample += found ? 1 : 0;
+                const bool over = found & !(r.t < r.tmax);
+                walking = walking & !over;
+                end |= over ? kCutOver : 0u;
+                heads.write(found & !over ? min(sample, kCutHeads) : kCutHeads, lane, r.t);
+            };
 #pragma unroll
             for (int q = 0; q < kCutTurns; ++q) {
-                bool go = walking && room;
-                const bool ahead = go && r.t >= next_at;
+                bool go = walking & room;
+                const bool ahead = go & (r.t >= next_at);
                 if (any_lane(ahead)) {
                     if (ahead) {
                         // on the ground of the piece ahead: is this one of its samples?
@@ -223,17 +232,23 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                         }
                     }
                 }
-                bool broken = false;
                 q_leaf[q] = -1;
                 q_dt[q] = 0.0f;
-                if (any_lane(go)) walk_turn_flat(tr, child, r, cur, step, go, broken, q_leaf[q], q_dt[q]);
-                if (go) {
-                    if (q_leaf[q] >= 0) sample += 1;
-                    if (broken || !(r.t < r.tmax)) {
-                        walking = false;
-                        end |= kCutOver | (broken ? kCutBroken : 0u);
-                    } else if (q_leaf[q] >= 0 && sample < kCutHeads) {
-                        heads.write(sample, lane, r.t);
+                if (child.octree) {
+                    cur.turn(r, go, child, step, q_leaf[q], q_dt[q]);
+                    arrive(q_leaf[q] >= 0);
+                }
+                // (lanes whose sample lies deeper than the coordinates wait for the last turn)
+                if (q == kCutTurns - 1 || !child.octree) {
+                    const bool deep = go & (cur.up < 0 || !child.octree);
+                    if (__builtin_expect(any_lane(deep), 0)) {
+                        bool broken = false;
+                        walk_from_root(tr, r, cur, step, deep, broken, q_leaf[q], q_dt[q]);
+                        if (broken) {
+                            walking = false;
+                            end |= kCutOver | kCutBroken;
+                        }
+                        arrive(deep & !broken);
                     }
                 }
             }
@@ -270,7 +285,8 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
         }
         shaded = count;
         wave_lds_sync();
-        // (a lane to an entry, all of whose record it asks for at once: a lane to a channel waited for memory three times as often.  FIGS)
+        // (a lane to an entry, all of whose record it asks for at once: a lane to a channel waited for memory three times as often.  8 000 rays, without notes and with:
+        // 64^3 SH9 112, 117 -> 106, 109 us, no leaf empty 149, 190 -> 138, 176; 128^3 SH4 184, 264 -> 174, 251; 256^3 shell SH9 215, 242 -> 214, 243.)
         for (int e = lane; e < n_fresh; e += kMarchThreads) {
             const int of = order[e];
             const int at_ray = (of & 63) >> cut;
@@ -318,9 +334,9 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_cut_kernel(TreeD
                 if (going) {
                     const int have = lists.count[at_lane];
                     const uint32_t e = lists.end[at_lane];
-                    lists.from[at_lane] = at;
-                    lists.taken[at_lane] = have - at;
-                    lists.place[at_lane] = n_order;
+                    lists.from[at_lane] = (int16_t)at;
+                    lists.taken[at_lane] = (int16_t)(have - at);
+                    lists.place[at_lane] = (int16_t)n_order;
                     n_order += have - at;
                     if (e & kCutLinked) {
                         at_lane = (int)(e >> 11 & 63u);

@@ -579,24 +579,6 @@ __device__ __forceinline__ void walk_from_root(const TreeDev<float>& tr, RayStat
     }
 }
 
-// One turn of the walk for the whole wavefront: the lanes with `go` take one sample (slot_leaf, slot_dt) and advance,
-// or keep a descent open (slot_leaf -1).  `broken`: the tree is malformed, the ray ends here.
-__device__ __forceinline__ void walk_turn_flat(const TreeDev<float>& tr, const ChildTable& child, RayState<float>& r, OctreeCursor& cur,
-                                               float step_size, bool go, bool& broken, int32_t& slot_leaf,
-                                               float& slot_dt) {
-    bool deep = go;
-    slot_leaf = -1;
-    slot_dt = 0.0f;
-    if (child.octree) {
-        if (child.words)
-            cur.turn_words(r, go, child, step_size, slot_leaf, slot_dt);
-        else
-            cur.turn(r, go, child, step_size, slot_leaf, slot_dt);
-        deep = go && cur.up < 0;
-    }
-    if (__builtin_expect(any_lane(deep), 0)) walk_from_root(tr, r, cur, step_size, deep, broken, slot_leaf, slot_dt);
-}
-
 // ------------------------------------------------------------------------------------------------
 // policies
 // ------------------------------------------------------------------------------------------------

@@ -518,6 +518,12 @@ TreeDev<float> march_tree(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt
     return d;
 }
 
+// ... and of rays in pieces, who walk on the child table alone (calls of so few rays make no walk table)
+TreeDev<float> on_child_table(TreeDev<float> tr) {
+    tr.walk = nullptr;
+    return tr;
+}
+
 // Whether a call makes a walk table (svox_walk_table) for its march.  Making it costs 4 us and 11 ps a node, and a march that starts on a
 // table no cache holds; a turn of the walk then waits for one read instead of two, or for none, though in three turns of ten it only descends.  So it pays
 // where rays are many and apart.  us, whole calls without and with it, forward and with notes (SH9, SH4 on 128^3 and 512^3):
@@ -798,7 +804,7 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
             const ReplaySpace none = no_notes();
             const Cut cut = tree->weight_accum ? Cut() : pick_cut(tree, items, is_image_source(src), opt, false);
             if (cut.per_wave > 0) {
-                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(dim3(blocks_for(items, cut.per_wave)), stream, tr, src, *opt, (float*)out,
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(dim3(blocks_for(items, cut.per_wave)), stream, on_child_table(tr), src, *opt, (float*)out,
                                                                     none, false, nullptr, nullptr, cut.per_wave, cut.most));
                 return;
             }
@@ -1063,7 +1069,7 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     if (cut.per_wave > 0) {
         const dim3 grid = with_clearing(blocks_for(total_items_of(src), cut.per_wave));
         SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::cut(grid, stream,
-                                                            march_tree(tree, opt), src, *opt, (float*)out, ws, true,
+                                                            on_child_table(march_tree(tree, opt)), src, *opt, (float*)out, ws, true,
                                                             (const float*)grad_out, (const float*)color_ref, cut.per_wave, cut.most));
         return SVOX_OK;
     }
