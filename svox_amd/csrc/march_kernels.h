@@ -969,6 +969,8 @@ struct ReplaySpace {
     // bitmap as `only` does those rays and no others
     unsigned long long* undone;
     const unsigned long long* only;
+    // not zero if any bit is set: the launch for those rays, which most passes have none of, then need not look for them (training step of an 800x800 picture 899 -> 887 us)
+    unsigned long long* any_undone;
     // > 0: the looks in a row after which a waiting wavefront of render_forward_split_kernel gives up, in place of
     // kSpinLimit (set by a debug flag, so that a test can see what a give-up leaves behind)
     int32_t spin_limit;
@@ -2282,6 +2284,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
     constexpr int K = P::kRecord;
     __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, true> sh;
+    if (ws.only && *ws.any_undone == 0) return;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
     load_transform(tr, offset, scaling);
@@ -2530,6 +2533,7 @@ struct ReplayRays {
             }
             const unsigned long long undone = __ballot(count < 0), m = __ballot(count > 0);
             if ((lane & 15) == 0 && seated) ((uint16_t*)ws.undone)[ray >> 4] = (uint16_t)(undone >> lane);
+            if (lane == 0 && undone) *ws.any_undone = 1;
             if (lane == 0) n = __popcll(m);
             wave_lds_sync();
             bool known = false;
@@ -3109,11 +3113,13 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
                                                                 float* __restrict__ color_out,
                                                                 float* __restrict__ grad_data,
                                                                 float* __restrict__ hess_data,
-                                                                const unsigned long long* __restrict__ only) {
+                                                                const unsigned long long* __restrict__ only,
+                                                               const unsigned long long* __restrict__ any_undone) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
     __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, true> sh;
+    if (only && *any_undone == 0) return;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
     load_transform(tr, offset, scaling);

@@ -35,7 +35,7 @@ struct MarchLaunch {
                                 const Lobes& lobes);
     static void se_grad(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                         const SvoxRenderOptions& opt, const float* color_ref, float* color_out, float* grad, float* hess,
-                        const unsigned long long* only, bool refill);
+                        const unsigned long long* only, const unsigned long long* any_undone, bool refill);
     static void replay_se_grad(dim3 blocks, hipStream_t stream, const Source& src, const SvoxRenderOptions& opt,
                                float* grad, float* hess, const ReplaySpace& ws, int ray_shift, const Lobes& lobes);
 };
@@ -165,13 +165,13 @@ void MarchLaunch<P, Source>::replay_backward(dim3 blocks, hipStream_t stream, co
 template <class P, class Source>
 void MarchLaunch<P, Source>::se_grad(dim3 blocks, hipStream_t stream, const TreeDev<float>& tr, const Source& src,
                                      const SvoxRenderOptions& opt, const float* color_ref, float* color_out, float* grad,
-                                     float* hess, const unsigned long long* only, bool refill) {
+                                     float* hess, const unsigned long long* only, const unsigned long long* any_undone, bool refill) {
     if (refill)
         hipLaunchKernelGGL((se_grad_kernel<P, Source, true>), blocks, dim3(kMarchThreads), 0, stream, tr, src, opt,
-                           color_ref, color_out, grad, hess, only);
+                           color_ref, color_out, grad, hess, only, any_undone);
     else
         hipLaunchKernelGGL((se_grad_kernel<P, Source, false>), blocks, dim3(kMarchThreads), 0, stream, tr, src, opt,
-                           color_ref, color_out, grad, hess, only);
+                           color_ref, color_out, grad, hess, only, any_undone);
 }
 
 template <class P, class Source>

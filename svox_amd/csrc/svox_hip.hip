@@ -867,9 +867,9 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
 }
 
 // The workspace of the replaying kernels: chunks of notes, then one bit per ray (rays left undone by
-// replay_backward_kernel), then 256 bytes that hold the stamp of the notes and, from byte 128 on, three
-// counters (cleared before every launch that takes notes): the chunk stocks handed out, the chunks that rays in
-// pieces took one by one (take_chunks, which keeps the first in step), and the rays listed (list_hits_kernel).
+// replay_backward_kernel), then 256 bytes that hold the stamp of the notes and, from byte 128 on, four
+// words (cleared before every launch that takes notes): the chunk stocks handed out, the chunks that rays in
+// pieces took one by one (take_chunks, which keeps the first in step), and the rays listed (list_hits_kernel); and whether any ray was left undone.
 constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
@@ -893,6 +893,7 @@ bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, 
     ws->n_stocks = (uint32_t)((chunks - n_slots + kChunkStock - 1) / kChunkStock);
     ws->stamp_at = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStampOffset);
     ws->stocks_taken = (unsigned long long*)((char*)ws->undone + bitmap_bytes(n_slots) + kStockCounterOffset);
+    ws->any_undone = ws->stocks_taken + 3;
     return true;
 }
 
@@ -1129,7 +1130,7 @@ int64_t data_bytes(const SvoxTreeSpec* t) {
 template <class Source, typename T>
 void launch_se_grad(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOptions* opt, int out_dim,
                     const void* color_ref, void* color_out, void* grad, void* hess, hipStream_t stream,
-                    const unsigned long long* only = nullptr) {
+                    const unsigned long long* only = nullptr, const unsigned long long* any_undone = nullptr) {
     const int64_t items = total_items_of(src);
     if constexpr (sizeof(T) == 4) {
         const int D = fast_basis(tree, opt);
@@ -1138,7 +1139,7 @@ void launch_se_grad(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
             const Source dealt = only ? src : dealt_out(src, blocks);
             SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::se_grad(dim3(blocks), stream, march_tree(tree, opt), dealt, *opt,
                                                                     (const float*)color_ref, (float*)color_out,
-                                                                    (float*)grad, (float*)hess, only,
+                                                                    (float*)grad, (float*)hess, only, any_undone,
                                                                     src.per_wave > kMarchThreads));
             return;
         }
@@ -1220,6 +1221,7 @@ int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest
     ReplaySpace only{};
     only.base = ws.base;
     only.only = ws.undone;
+    only.any_undone = ws.any_undone;
     const unsigned blocks = blocks_for(total_items_of(rest), rest.per_wave);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::backward(dim3(blocks), stream, march_tree(tree, opt), rest, *opt,
                                                              (const float*)grad_output, (float*)grad_data_out, only,
@@ -1314,7 +1316,7 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
                                                                    lobes_of(tree, opt)));
     rc = check_launch("se_grad");
     if (rc) return rc;
-    launch_se_grad<Source, float>(tree, rest, opt, 3, color_ref, color_out, grad, hess, stream, ws.undone);
+    launch_se_grad<Source, float>(tree, rest, opt, 3, color_ref, color_out, grad, hess, stream, ws.undone, ws.any_undone);
     return check_launch("se_grad");
 }
 
