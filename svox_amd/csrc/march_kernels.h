@@ -287,6 +287,10 @@ struct ImageSource {
         const int ix = bx * 16 + (sub & 1) * 8 + (pos & 7);
         const int iy = by * 16 + (sub >> 1) * 8 + (pos >> 3);
         if (ix >= cam.width || iy >= cam.height) return -1;
+        return fetch_pixel(image, ix, iy, opt, offset, scaling, origin, dir, vdir);
+    }
+    __device__ __forceinline__ int64_t fetch_pixel(int image, int ix, int iy, const SvoxRenderOptions& opt, const T* offset,
+                                                   const T* scaling, T* origin, T* dir, T* vdir) const {
         Camera<T> c = cam;
         c.c2w = cam.c2w + (int64_t)image * pose_stride;
         cam2world_ray(ix, iy, c, dir, origin);
@@ -296,6 +300,31 @@ struct ImageSource {
         transform_coord(origin, offset, scaling);
         return ((int64_t)image * cam.height + iy) * cam.width + ix;
     }
+    // the pixel of a number as the pixels are numbered, of which there are n_slots()
+    __device__ __forceinline__ int64_t fetch_slot(int64_t slot, const SvoxRenderOptions& opt, const T* offset, const T* scaling,
+                                                  T* origin, T* dir, T* vdir) const {
+        const int64_t per_image = (int64_t)cam.height * cam.width;
+        const int image = (int)(slot / per_image);
+        const int pixel = (int)(slot - image * per_image);
+        const int iy = pixel / cam.width;
+        return fetch_pixel(image, pixel - iy * cam.width, iy, opt, offset, scaling, origin, dir, vdir);
+    }
+};
+
+// Pixels of pictures that meet the cube, for noting passes, as ListedSource has the rays of a batch; and the pictures as they are, where that
+// is the shape such a pass is launched in.  (One kernel for both, which looks at the number, took 1.15 to 2 times as long where most pixels do.)
+struct ListedImageSource : ImageSource<float> {
+    static constexpr bool kGated = true;
+    const int32_t* list;
+    const unsigned long long* n_listed;
+    __device__ __forceinline__ int64_t total() const { return (int64_t)*n_listed; }
+    __device__ __forceinline__ int64_t fetch_item(int64_t i, const SvoxRenderOptions& opt, const float* offset,
+                                                  const float* scaling, float* origin, float* dir, float* vdir) const {
+        return fetch_slot(list[i], opt, offset, scaling, origin, dir, vdir);
+    }
+};
+struct WholeImageSource : ImageSource<float> {
+    static constexpr bool kGated = true;
 };
 
 // ------------------------------------------------------------------------------------------------
@@ -980,7 +1009,7 @@ struct ReplaySpace {
     uint32_t n_stocks;
     // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
     unsigned int* give_ups;
-    int32_t* list;         // room for a number per ray, behind the chunks (ListedSource), or nullptr
+    int32_t* list;         // room for a number per ray, behind the chunks (ListedSource, ListedImageSource), or nullptr
     // a noting launch: the blocks that march; those beyond clear these arrays of clear_words words each
     uint32_t march_blocks;
     uint32_t* clear_at[2];

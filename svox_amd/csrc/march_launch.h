@@ -99,6 +99,7 @@ void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeD
     hipLaunchKernelGGL((__VA_ARGS__), blocks, dim3(THREADS), 0, stream, tr, src, opt, out, ws, grad_out ? grad_out : color_ref)
     constexpr bool kListed = std::is_same<Source, ListedSource>::value;   // (marched tile by tile)
     constexpr bool kWhole = std::is_same<Source, WholeSource>::value;     // (on one wavefront per tile or chunk)
+    constexpr bool kPixels = Source::kGated && !Source::kItemsAreSlots;   // (on two wavefronts per tile)
     if (split) {
         if constexpr (!kWhole) {
             if (grad_out)
@@ -106,17 +107,19 @@ void MarchLaunch<P, Source>::noting(dim3 blocks, hipStream_t stream, const TreeD
             else
                 SVOX_NOTING(kSplitThreads, render_forward_split_kernel<P, Source, true, false>);
         }
-    } else if (refill) {
-        if constexpr (!kListed) {
-            if (grad_out)
-                SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
-            else
-                SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, false>);
-        }
-    } else if (grad_out)
-        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, true>);
-    else
-        SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, false>);
+    } else if constexpr (!kPixels) {
+        if (refill) {
+            if constexpr (!kListed) {
+                if (grad_out)
+                    SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, true>);
+                else
+                    SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, true, true, false>);
+            }
+        } else if (grad_out)
+            SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, true>);
+        else
+            SVOX_NOTING(kMarchThreads, render_forward_kernel<P, Source, false, false, true, false>);
+    }
 #undef SVOX_NOTING
 }
 

@@ -16,4 +16,10 @@ template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, L
 template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, WholeSource>::noting(
     dim3, hipStream_t, const TreeDev<float>&, const WholeSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
     const float*, bool, bool);
+template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, ListedImageSource>::noting(
+    dim3, hipStream_t, const TreeDev<float>&, const ListedImageSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
+    const float*, bool, bool);
+template void MarchLaunch<OctreePolicy<SVOX_POLICY_FORMAT, SVOX_POLICY_BASIS>, WholeImageSource>::noting(
+    dim3, hipStream_t, const TreeDev<float>&, const WholeImageSource&, const SvoxRenderOptions&, float*, const ReplaySpace&, const float*,
+    const float*, bool, bool);
 }  // namespace svox

@@ -15,6 +15,7 @@
 #include "partition_kernels.h"
 
 #include <mutex>
+#include <numeric>
 
 // Workspace of svox_volume_render_backward_static: one array per GPU, inside the library's code object.
 // In host code the name `scratch` is only a handle for hipGetSymbolAddress (static_workspace below); it
@@ -866,6 +867,34 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
     return st;
 }
 
+// Whether a noting pass over pictures lists the pixels that meet the cube first, and deals them out so that every tile has some from all over the
+// picture (PicturesSpread).  A tile of 8 x 8 pixels has long rays or short ones, and leaves to shade in the same rounds or none, and the pass takes as long as
+// the worst of them; dealt out they are alike: 800x800 picture of a 512^3 SH16 shell 538 -> 417 us, of a 256^3 SH16 shell 453 -> 332, of 400x400 322 -> 251.
+// Not for grids that are as fine everywhere, whose rays are alike and read the same lines (64^3 SH9 400x400 175 / 178, 800x800 218 / 239; 128^3 SH4 435 / 507), trees
+// of fewer than 65 536 cells (16^3 RGBA 132 / 245), pictures in normalised device coordinates, all of whose rays meet the cube, and where what is to be gone through
+// is small beside the launches or large beside the hits: under 16 384 pixels, over 2 Mi (1700x1700, 16 000 hits: 412 / 428).
+bool lists_pixels(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_pixels) {
+    if (g_debug_flags & 64) return true;
+    const Tuning& t = tuning();
+    return g_debug_flags == 0 && t.per_wave <= 0 && t.split_forward < 0 && t.split_blocks < 0 && opt->ndc_width <= 0 && n_pixels >= 1 << 14 &&
+           n_pixels <= 1 << 21 && (double)tree->capacity * tree->N * tree->N * tree->N >= 65536.0 && !like_complete_octree(tree);
+}
+// Up to how many: tiles that are alike must all find a place at once, or the last of them take as long again when the first have ended (800x800, 256^3 SH9 shell:
+// 2 530 tiles 262 -> 225 us, 2 712 tiles 256 -> 402, of 2 816 places, as LDS has them; SH16, of 2 560: 2 290 tiles 439 -> 343, 2 446 445 -> 490).  Few functions leave little to
+// level, while rays from all over read more lines: half as many then (512^3 SH1 shell 125 000 hits 318 / 332; 74 000 hits, 512^3 SH4 392 -> 334, 256^3 SH1 252 -> 241).
+// Pictures with more hits pay for the sample and a launch without tiles: 5 to 10 us (800x800 close up, 512^3 SH16 868 / 876, 128^3 SH4 328 / 334).
+int64_t most_listed_pixels(const SvoxRenderOptions* opt, int64_t n_pixels, unsigned at_once) {
+    if (g_debug_flags & 64) return std::min((int64_t)(g_debug_flags >> 8 & 255) * kMarchThreads, n_pixels);
+    const bool light = opt->format == SVOX_FORMAT_RGBA || opt->basis_dim < 9;
+    const int64_t tiles = (int64_t)std::min(at_once, 2816u) * 9 / 10;
+    return std::min((light ? tiles / 2 : tiles) * kMarchThreads, n_pixels);
+}
+constexpr int64_t kListRays = 1 << 17;
+template <class Source>
+bool keeps_list(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, const Source& src, int64_t n_slots) {
+    return is_image_source(src) ? lists_pixels(tree, opt, n_slots) : n_slots >= kListRays || (g_debug_flags & 64);
+}
+
 // The workspace of the replaying kernels: chunks of notes, then one bit per ray (rays left undone by
 // replay_backward_kernel), then 256 bytes that hold the stamp of the notes and, from byte 128 on, four
 // words (cleared before every launch that takes notes): the chunk stocks handed out, the chunks that rays in
@@ -873,10 +902,9 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
 constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
-// (and, of a batch of kListRays rays and more, where the rays' shared chunks are many beside it, in the place of the last of them: a number per
-// ray.  Every pass over the notes of a batch says that it is one, or the room they are in would not be the same.)
-constexpr int64_t kListRays = 1 << 17;
-bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, bool batch, ReplaySpace* ws) {
+// (and, of a batch or pictures whose rays may be listed, where the rays' shared chunks are many beside it, in the place of the last of them: a number per
+// ray.  Every pass over the notes says so alike (keeps_list), or the room they are in would not be the same.)
+bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, bool list, ReplaySpace* ws) {
     *ws = ReplaySpace{};
     int64_t chunks = workspace && n_slots > 0
                          ? (workspace_bytes - kTailBytes - bitmap_bytes(n_slots)) / kChunkBytes : 0;
@@ -884,7 +912,7 @@ bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, 
     ws->base = (float2*)workspace;
     ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
     const int64_t list_chunks = (n_slots * 4 + kChunkBytes - 1) / kChunkBytes;
-    if (batch && (n_slots >= kListRays || (g_debug_flags & 64)) && chunks - n_slots >= 16 * list_chunks) {
+    if (list && chunks - n_slots >= 16 * list_chunks) {
         chunks -= list_chunks;
         ws->list = (int32_t*)((char*)workspace + chunks * kChunkBytes);
     }
@@ -943,39 +971,70 @@ BatchSource<T> noting_shape(BatchSource<T> s) {
 template <typename T>
 ImageSource<T> noting_shape(const ImageSource<T>& s) { return s; }
 
-// The rays of a batch that meet the cube, in the order they come in block by block (the blocks as they get there); the others are
+// The rays of a batch or of pictures that meet the cube, in the order they come in block by block (the blocks as they get there); the others are
 // answered as a noting pass answers them.  200 003 rays 9 us, 1 Mi rays 30: 24 bytes
 // read of each, and a line written for every one that misses, the head of its notes.  Where a sample of the rays says that more than
-// `most` hit, nothing is listed (4.5 us), and the number stands for the batch as it is.
+// `most` hit, nothing is listed (4.5 us), and the number stands for the batch as it is.  Pixels of an 800x800 picture 20 us.
 constexpr int kListThreads = 1024;
-constexpr int kListSample = 256;
-__global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> tr, BatchSource<float> src, SvoxRenderOptions opt,
-                                                                        float* __restrict__ out, ReplaySpace ws,
-                                                                        unsigned long long* __restrict__ n_listed, int64_t most) {
+// The rays as a listing launch goes through them, place by place.
+struct BatchInOrder {
+    static constexpr int kSample = 256;
+    BatchSource<float> rays;
+    __device__ __forceinline__ int64_t n_rays() const { return rays.rays.n_rays; }
+    __device__ __forceinline__ int64_t sample(int i) const { return (int64_t)i * n_rays() / kSample; }
+    __device__ __forceinline__ int64_t fetch(int64_t place, const SvoxRenderOptions& opt, const float* offset, const float* scaling,
+                                             float* origin, float* dir, float* vdir) const {
+        return rays.fetch_item(place, opt, offset, scaling, origin, dir, vdir);
+    }
+};
+// Pieces of a row of 16 pixels, from all over the pictures in turn: the next piece lies `step` pieces on, about 0.618 of all there are and without a common
+// factor with their number, so that any run of places is spread evenly.
+constexpr int kListPiece = 16;
+struct PicturesSpread {
+    static constexpr int kSample = 256;
+    ImageSource<float> pictures;
+    int64_t n_pieces, step;
+    __device__ __forceinline__ int64_t n_rays() const { return pictures.n_slots(); }
+    __device__ __forceinline__ int64_t sample(int i) const { return (int64_t)i * kListPiece + i % kListPiece; }
+    __device__ __forceinline__ int64_t fetch(int64_t place, const SvoxRenderOptions& opt, const float* offset, const float* scaling,
+                                             float* origin, float* dir, float* vdir) const {
+        const int64_t piece = place / kListPiece;
+        const int64_t slot = piece * step % n_pieces * kListPiece + place % kListPiece;
+        if (piece >= n_pieces || slot >= n_rays()) return -1;
+        return pictures.fetch_slot(slot, opt, offset, scaling, origin, dir, vdir);
+    }
+};
+int64_t spread_step(int64_t n_pieces) {
+    int64_t step = std::max((int64_t)((double)n_pieces * 0.6180339887), (int64_t)1);
+    while (std::gcd(step, n_pieces) != 1) ++step;
+    return step;
+}
+template <class Places>
+__global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> tr, Places src, SvoxRenderOptions opt,
+                                                                 float* __restrict__ out, ReplaySpace ws,
+                                                                 unsigned long long* __restrict__ n_listed, int64_t most) {
     __shared__ int32_t hits[kListThreads / kMarchThreads];
     __shared__ unsigned long long first;
     float offset[3], scaling[3], origin[3], dir[3], vdir[3];
     load_transform(tr, offset, scaling);
     const int wave = threadIdx.x / kMarchThreads, lane = threadIdx.x & (kMarchThreads - 1);
-    src.n_waves = 0;
     RayState<float> r;
     // (the same rays for every block, which all come to the same answer)
-    if (threadIdx.x < kListSample) {
-        const int64_t some = (int64_t)threadIdx.x * src.rays.n_rays / kListSample;
-        src.fetch_item(some, opt, offset, scaling, origin, dir, vdir);
-        const unsigned long long m = __ballot(setup_ray(r, origin, dir, scaling));
+    if (threadIdx.x < Places::kSample) {
+        const int64_t some = src.fetch(src.sample(threadIdx.x), opt, offset, scaling, origin, dir, vdir);
+        const unsigned long long m = __ballot(some >= 0 && setup_ray(r, origin, dir, scaling));
         if (lane == 0) hits[wave] = __popcll(m);
     }
     __syncthreads();
     int sampled = 0;
 #pragma unroll
-    for (int i = 0; i < kListSample / kMarchThreads; ++i) sampled += hits[i];
-    if (sampled * src.rays.n_rays > kListSample * most) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *n_listed = (unsigned long long)src.rays.n_rays;
+    for (int i = 0; i < Places::kSample / kMarchThreads; ++i) sampled += hits[i];
+    if (sampled * src.n_rays() > Places::kSample * most) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *n_listed = (unsigned long long)src.n_rays();
         return;
     }
     __syncthreads();
-    const int64_t slot = src.fetch_item(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
+    const int64_t slot = src.fetch(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
     const bool hit = slot >= 0 && setup_ray(r, origin, dir, scaling);
     if (slot >= 0 && !hit) {
         if (out) {
@@ -1051,7 +1110,7 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
     const unsigned blocks = blocks_for(total_items_of(src), src.per_wave);
     const Source dealt = dealt_out(src, blocks);
     ReplaySpace ws;
-    if (D < 0 || !carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(src), &ws))
+    if (D < 0 || !carve_workspace(workspace, workspace_bytes, n_slots, keeps_list(tree, opt, src, n_slots), &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "notes asked for where they cannot be taken");
     const int rc = zero_fill(ws.stocks_taken, 32, stream);
     if (rc) return rc;
@@ -1084,8 +1143,10 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
         if (ws.list && shapes.any) {
             unsigned long long* const n_listed = ws.stocks_taken + 2;
             const int64_t listed = std::max(shapes.one, shapes.two);
-            hipLaunchKernelGGL(list_hits_kernel, dim3(blocks_for(src.rays.n_rays, kListThreads)), dim3(kListThreads), 0, stream,
-                               march_tree(tree, opt), src, *opt, (float*)out, ws, n_listed, listed);
+            BatchInOrder places{src};
+            places.rays.n_waves = 0;
+            hipLaunchKernelGGL(list_hits_kernel<BatchInOrder>, dim3(blocks_for(src.rays.n_rays, kListThreads)), dim3(kListThreads), 0, stream,
+                               march_tree(tree, opt), places, *opt, (float*)out, ws, n_listed, listed);
             ws.n_listed = n_listed;
             auto launch_listed = [&](int64_t least, int64_t most, bool two) {
                 ListedSource tiles;
@@ -1114,6 +1175,39 @@ int launch_noted(const SvoxTreeSpec* tree, const Source& src, const SvoxRenderOp
         }
     }
     const bool split = !refill && use_split_forward(tree, blocks, is_image_source(src), opt, false, at_once);
+    if constexpr (is_image_source(Source())) {
+        const int64_t most = split && ws.list ? most_listed_pixels(opt, n_slots, at_once) : 0;
+        if (most > 0) {
+            unsigned long long* const n_listed = ws.stocks_taken + 2;
+            const int64_t n_pieces = (n_slots + kListPiece - 1) / kListPiece;
+            const PicturesSpread places{src, n_pieces, spread_step(n_pieces)};
+            // (nothing is listed only where the number that then stands for all of them, n_slots, is more than the listed shape takes; a sample is
+            // some per cent off)
+            const int64_t sampled_most = n_slots > most ? most - most / 32 : n_slots;
+            hipLaunchKernelGGL(list_hits_kernel<PicturesSpread>, dim3(blocks_for(n_pieces * kListPiece, kListThreads)), dim3(kListThreads), 0,
+                               stream, march_tree(tree, opt), places, *opt, (float*)out, ws, n_listed, sampled_most);
+            ws.n_listed = n_listed;
+            auto launch_pixels = [&](auto pixels, int64_t tiles, int64_t least, int64_t most_here) {
+                ws.least = least;
+                ws.most = most_here;
+                const dim3 grid = with_clearing((unsigned)tiles);
+                SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, decltype(pixels)>::noting(grid, stream, march_tree(tree, opt), pixels, *opt, (float*)out,
+                                                                                 ws, (const float*)grad_out, (const float*)color_ref, true, false));
+            };
+            ListedImageSource listed;
+            (Source&)listed = src;
+            listed.xcd_group = 1;
+            listed.list = ws.list;
+            listed.n_listed = n_listed;
+            launch_pixels(listed, blocks_for(most, kMarchThreads), 0, most);
+            if (n_slots > most) {
+                WholeImageSource whole;
+                (Source&)whole = src;
+                launch_pixels(whole, blocks, most + 1, INT64_MAX);
+            }
+            return SVOX_OK;
+        }
+    }
     const dim3 grid = with_clearing(blocks);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::noting(grid, stream, march_tree(tree, opt), dealt, *opt,
                                                            (float*)out, ws, (const float*)grad_out,
@@ -1210,7 +1304,7 @@ int backward_from_notes(const SvoxTreeSpec* tree, const Source& all, Source rest
     const int ray_shift = replay_shift(n_slots);
     const unsigned replay_blocks = blocks_for(n_slots, 1 << ray_shift);
     ReplaySpace ws;
-    carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(all), &ws);
+    carve_workspace(workspace, workspace_bytes, n_slots, keeps_list(tree, opt, all, n_slots), &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     ws.report = (unsigned long long*)report;
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_backward(dim3(replay_blocks), stream, all, *opt, (const float*)grad_output,
@@ -1308,7 +1402,7 @@ int se_grad_from_notes(const SvoxTreeSpec* tree, const Source& all, const Source
     rc = check_launch("se_grad");
     if (rc) return rc;
     ReplaySpace ws;
-    carve_workspace(workspace, workspace_bytes, n_slots, !is_image_source(all), &ws);
+    carve_workspace(workspace, workspace_bytes, n_slots, keeps_list(tree, opt, all, n_slots), &ws);
     memcpy(ws.stamp, stamp.word, sizeof(ws.stamp));
     const int ray_shift = replay_shift(n_slots);
     SVOX_DISPATCH_OCTREE(D, MarchLaunch<P, Source>::replay_se_grad(dim3(blocks_for(n_slots, 1 << ray_shift)), stream, all, *opt,
@@ -1631,7 +1725,7 @@ int svox_notes_pool_info(int64_t n_rays, int64_t workspace_bytes, int64_t* count
     ReplaySpace ws;
     // (any 16-byte aligned address does for the arithmetic)
     char* const base = (char*)(uintptr_t)4096;
-    if (!carve_workspace(base, workspace_bytes, n_rays, true, &ws))
+    if (!carve_workspace(base, workspace_bytes, n_rays, n_rays >= kListRays || (g_debug_flags & 64), &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "svox_notes_pool_info: the workspace does not hold a chunk per ray");
     *counter_offset = (int64_t)((char*)ws.stocks_taken - base);
     *pool_stocks = ws.n_stocks;

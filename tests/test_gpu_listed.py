@@ -1,4 +1,4 @@
-"""Noting passes that list the rays of a batch which meet the tree: two wavefronts per tile, one, or the batch as it is, whichever the
+"""Noting passes that list the rays of a batch, or the pixels of pictures, which meet the tree: two wavefronts per tile, one, or all as they are, whichever the
 number of them asks for on the device.
 
 Bar: pictures, noted colours and the number of notes of every ray equal to those of the pass that takes the batch as it is, bit for bit;
@@ -143,3 +143,72 @@ def test_pictures_leave_no_room_for_a_list(gpu):
     C.volume_render_backward_noted(spec, rs, opt, go, notes, report.data_ptr())
     torch.cuda.synchronize()
     assert int(report[0]) & 0xffffffff == (chunks(notes) - -(-n * 4 // 384) - n + 63) // 64 == C.notes_pool_use(notes, n)[1]
+
+
+# pictures: of which no pixel meets the tree, some, all; pieces of 16 pixels with a rest and without; one and several; listed, or more than are
+@pytest.mark.parametrize("w,h,n_images", [(16, 1, 1), (33, 31, 1), (48, 40, 2), (100, 67, 3), (128, 96, 1)])
+@pytest.mark.parametrize("view", ["none", "some", "all"])
+@pytest.mark.parametrize("tiles", [255, 1])
+def test_listed_pixels(gpu, oracle_mod, w, h, n_images, view, tiles):
+    n = w * h * n_images
+    tree = synth.shell_tree(depth=6, data_format="SH9", n_spheres=6, seed=4)
+    gen = torch.Generator().manual_seed(n)
+    poses = torch.stack([p[:3] for p in synth.orbit_poses(n_images, seed=2, radius=3.0)])
+    poses[:, :, 3] += 100.0 if view == "none" else 0.0
+    fx = 1.1 * w if view == "some" else 12.0 * w
+    opt = options(tree, step_size=1e-3)
+    dev = on_gpu(tree, gpu)
+    spec = dev._spec()
+    cam, one = cam_spec(poses, w, h, fx, device=gpu), cam_spec(poses[0], w, h, fx, device=gpu)
+    go, target = (torch.randn(n_images, h, w, 3, generator=gen) * 1e-2).to(gpu), torch.rand(h, w, 3, generator=gen).to(gpu)
+    slack = sum(oracle_mod.volume_render_image_backward(oracle_mod.Tree.from_n3tree(tree), p, fx, fx, w, h, opt, g, want_slack=True)[1]
+                for p, g in zip(poses, go.cpu()))
+
+    def passes():
+        out, notes = C.volume_render_images_noted(spec, cam, opt, records_per_ray=64)
+        count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+        hit = notes.view(torch.float32)[: n * 96].view(n, 96)[:, 93] != 1.0
+        assert {"none": bool(~hit.any()), "some": bool(hit.any()) and not bool(hit.all()) or n == 16, "all": bool(hit.all())}[view]
+        number = C.notes_pool_use(notes, n)[0]
+        said = int(notes.view(torch.int64)[number.storage_offset() + 2])
+        return (out, count, C.se_grad_persp(spec, one, opt, target)[0], said, int(hit.sum()), C.volume_render_images_backward_noted(spec, cam, opt, go, notes),
+                C.volume_render_images_backward(spec, cam, opt, go))
+
+    want, got = run(8, passes), run(64 | tiles << 8, passes)
+    for what, a, b in zip(("pictures", "notes", "colours"), got, want):
+        assert torch.equal(a, b), what
+    assert want[3] == 0 and got[3] in (got[4], n)
+    for what, a, b in zip(("from notes", "alone"), got[5:], want[5:]):
+        err, ok = grad_close(a.cpu().numpy(), b.cpu().numpy(), slack=slack, what=what)
+        assert ok, (what, err)
+
+
+def test_pictures_of_shells_take_less_time_listed(gpu):
+    """(400x400 picture of a 256^3 SH9 shell, noting march 307 us as it is, 252 listed.)  And the rule takes the list where it says so: the last of
+    the chunks are not for notes."""
+    w = 400
+    tree = synth.shell_tree(depth=8, data_format="SH9", n_spheres=24, seed=0, device=gpu)
+    spec, opt = tree._spec(), options(tree, step_size=5e-4)
+    cam = cam_spec(synth.orbit_poses(1, seed=2, radius=4.0)[0], w, w, 1.39 * w, device=gpu)
+    out, notes = C.volume_render_images_noted(spec, cam, opt, records_per_ray=30)
+    report = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    C.volume_render_images_backward_noted(spec, cam, opt, torch.ones_like(out), notes, report.data_ptr())
+    torch.cuda.synchronize()
+    assert int(report[0]) & 0xffffffff == C.notes_pool_use(notes, w * w)[1]
+    assert torch.equal(out, run(8, lambda: C.volume_render_images_noted(spec, cam, opt, records_per_ray=30)[0]))
+    times = {0: [], 8: []}
+    for _ in range(7):
+        for flags in times:
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+            def passes():
+                begin.record()
+                for _ in range(20):
+                    C.volume_render_images_noted(spec, cam, opt)
+                end.record()
+            run(flags, passes)
+            end.synchronize()
+            times[flags].append(begin.elapsed_time(end))
+    rule, plain = (sorted(times[k])[3] for k in (0, 8))
+    print(f"[listed] picture: {rule * 50:.0f} us, as it is {plain * 50:.0f} us", flush=True)
+    assert rule <= 0.95 * plain
