@@ -331,8 +331,7 @@ def _backward_workspace(tree, n_rays, records_per_ray=None):
     if size_of(n_rays, per_ray) > _ASK_DEVICE_ABOVE:
         device = tree.data.device
         free, _ = torch.cuda.mem_get_info(device)
-        cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
-        limit = min(limit, int((free + cached) * BACKWARD_WORKSPACE_FREE_FRACTION))
+        limit = min(limit, int((free + _shim().cached_bytes(device.index)) * BACKWARD_WORKSPACE_FREE_FRACTION))
     while per_ray > 0 and size_of(n_rays, per_ray) > limit:
         per_ray -= 15
     nbytes = int(size_of(n_rays, per_ray)) if per_ray > 0 else 0
