@@ -4,17 +4,16 @@
 // and what a ray waits for is its chain: descent, density, colour, step.  One ray per lane (the generic kernels) leaves
 // that chain to one lane.  Here every ray is walked in 4 to 64 pieces at once, a lane to each, as cut_kernel.h does it: the lanes of a
 // piece walk until their samples are, bit for bit, those of the next one, and list the leaves with density in LDS; the lists are
-// put in the ray's order, and its entries are evaluated by all lanes together (a lane to a channel) and composed one after the
+// put in the ray's order, and its entries are evaluated by all lanes together (a lane to an entry) and composed one after the
 // other.  The gradient forms its records from the same lists, and walks a second time only where one round did not hold all of
 // a ray.  The values are those of the generic kernels bit for bit: the same expressions in the same order; multiplying by 2^-levels
 // is dividing by 2^levels.
 // Bound by the chain of a turn (two child reads, the density, some 150 double-precision instructions: 1 to 1.3 us) up to 20 000 rays, by
-// how many wavefronts LDS has room for beyond: with 592 entries seven to a compute unit (dense 64^3 SH4, 20 000 rays, forward pass and
-// gradient, us: 512 entries 172, 285, but 405, 933 instead of 270, 645 where no leaf is empty; 592 176, 285; 640 181, 332; 768 205, 333;
-// 896 226, 362; lists of 20 entries for every lane, none shared, 222, 361).
+// how many wavefronts LDS has room for beyond: with 592 entries nine to a compute unit up to SH4, eight to SH16 (GroupBlock; seven and six where
+// everything had its own place: dense 64^3 SH4, 65 536 rays, gradient 986 us instead of 596, 256^3 shell SH16 1527 instead of 1161; 20 000 rays 250 instead of 245).
 // Measured, four lanes that walk a ray together, from end to end / pieces, forward pass and gradient, us (more: group_cut):
-//   64^3 SH4, half of the leaves empty  1 000 rays 226, 383 / 51, 72    20 000 279, 561 / 161, 250
-//   no leaf empty                       1 000 rays 232, 541 / 54, 124   20 000 287, 686 / 235, 565
+//   64^3 SH4, half of the leaves empty  1 000 rays 226, 383 / 51, 72    20 000 278, 553 / 144, 245
+//   no leaf empty                       1 000 rays 232, 541 / 54, 124   20 000 285, 686 / 220, 518
 // The lanes of a ray that walk it together are the kernels for more rays than find room in pieces (below).
 #pragma once
 
@@ -42,8 +41,12 @@ struct GroupWalk {
 
     __device__ __forceinline__ void begin(int32_t* lane_path) {
         rows = lane_path - kMarchThreads;
-        rows[kMarchThreads] = 0;
         nx = ny = nz = 0;
+        from_root();
+    }
+    // the path is lost: the next aim() starts at the root
+    __device__ __forceinline__ void from_root() {
+        rows[kMarchThreads] = 0;
         levels = 1;
     }
     __device__ __forceinline__ bool ended() const { return !(t < tmax); }
@@ -115,25 +118,48 @@ constexpr uint32_t kGroupLinked = 1u << 20, kGroupOver = 1u << 21, kGroupBroken 
 // trace_ray, rt_kernel.cu:222-321 (result: the picture), and trace_ray_backward, rt_kernel.cu:323-477 (result: grad_data).  The
 // gradient's first pass sums <render, grad_out>, its second forms the records, whose scalars the wavefront adds together: scalar f
 // from lane f mod 64, so that they go out in requests of 64 bytes (the memory system takes a fixed number of those per microsecond).
+//
+// LDS says how many wavefronts a compute unit holds (granules of 1 280 bytes), so what is not needed at the same time lies in the same place: what a block of
+// entries evaluates and what puts the lists in order lies where the walk keeps its path, which starts at the root again in a round after one that
+// was composed (few rays have one); the rays' order fills the list of free entries from behind.
+template <bool kBackward>
+struct GroupBlock {
+    // of the entries of a block: the colour, then the factors of the coefficients' gradient; the attenuation, then the weight;
+    // <colour, grad_out>, then the density's gradient
+    union {
+        double colour[kMarchThreads * 3];
+        uint32_t end[kMarchThreads];       // (before there is one) of a lane's list: how it ends
+    };
+    double attenuation[kMarchThreads], total[kBackward ? kMarchThreads : 1];
+    // of a lane's list: how many there are, from which on and how many are composed now, and where in the ray's order
+    uint16_t count[kMarchThreads], from[kMarchThreads], taken[kMarchThreads], place[kMarchThreads];
+};
 template <int D, class Source, bool kBackward>
 __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<double> tr, Source src, SvoxRenderOptions opt,
                                                                      const double* __restrict__ grad_out, double* __restrict__ result,
                                                                      int per_wave, int most_cut) {
     constexpr int DD = D > 0 ? D : 1;
     constexpr int K = D > 0 ? 3 * D + 1 : 4;
-    __shared__ int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __shared__ union {
+        int32_t path[(kPathLevels + 1) * kMarchThreads];
+        GroupBlock<kBackward> block;
+    } sh;
     __shared__ PieceHeads<double, kGroupHeads> heads;          // (-1: not known yet)
     // the leaves found, and the one after each in its lane's list; the entries that are free
     __shared__ double list_dt[kGroupEntries];
     __shared__ int32_t list_leaf[kGroupEntries];
-    __shared__ uint16_t list_next[kGroupEntries], spare[kGroupEntries];
-    __shared__ uint16_t order[kGroupEntries];                  // the entries of every ray in its order, ray by ray
-    // of a lane's list: how many there are, from which on and how many are composed now, and where in the ray's order
-    __shared__ uint16_t list_count[kMarchThreads], list_from[kMarchThreads], list_taken[kMarchThreads], list_place[kMarchThreads];
-    __shared__ uint32_t list_end[kMarchThreads];
-    // of the entries of a block: the colour, then the factors of the coefficients' gradient; the attenuation, then the weight;
-    // <colour, grad_out>, then the density's gradient
-    __shared__ double colour[kMarchThreads * 3], attenuation[kMarchThreads], total[kBackward ? kMarchThreads : 1];
+    __shared__ uint16_t list_next[kGroupEntries];
+    // from the front the entries that are free, from behind those of every ray in its order, ray by ray (each once, and none that is free)
+    __shared__ uint16_t spare[kGroupEntries];
+    auto order = [&](int place) -> uint16_t& { return spare[kGroupEntries - 1 - place]; };
+    double* const colour = sh.block.colour;
+    double* const attenuation = sh.block.attenuation;
+    double* const total = sh.block.total;
+    uint16_t* const list_count = sh.block.count;
+    uint16_t* const list_from = sh.block.from;
+    uint16_t* const list_taken = sh.block.taken;
+    uint16_t* const list_place = sh.block.place;
+    uint32_t* const list_end = sh.block.end;
     __shared__ double ray_basis[kGroupRays * DD], ray_go[kBackward ? kGroupRays * 3 : 1], ray_dscale[kGroupRays];
     __shared__ int32_t ray_count[kGroupRays], ray_at[kGroupRays], ray_lane[kGroupRays];
     constexpr double kUnknown = -1.0;
@@ -196,7 +222,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
         walk.tmax = __shfl(r.tmax, from);
         slot = (int64_t)__shfl((long long)slot, from);
     }
-    walk.begin(path + lane);
+    walk.begin(sh.path + lane);
     const double length = walk.tmax - t0, part = 1.0 / (double)pieces;
     auto begin_of = [&](int k) { return k < pieces ? fma_((double)k * part, length, t0) : kNone; };
 
@@ -213,7 +239,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
             auto entry_of = [&](int e, int& of_ray) {      // entry e of the block, -1: there is none
                 of_ray = e >> cut;
                 const int k = base + (e & (pieces - 1));
-                return of_ray < n_rays && k < ray_count[of_ray] ? (int)order[ray_at[of_ray] + k] : -1;
+                return of_ray < n_rays && k < ray_count[of_ray] ? (int)order(ray_at[of_ray] + k) : -1;
             };
             // (a lane to an entry: what it reads of a record is asked for at once; a lane to a channel waited three times, and once more for the density.
             // Forward pass, gradient step of 20 000 rays: 64^3 SH4 177, 467 -> 161, 414 us, no leaf empty 267, 897 -> 235, 797; 128^3 SH4 359, 992 -> 330, 901;
@@ -346,6 +372,8 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
         int rounds = 0, n_order = 0;
         while (true) {
             rounds += 1;
+            walk.from_root();
+            if (!fresh) walk.aim();    // (a search that was under way)
             // ---- walk; the density of a leaf is looked at a turn after the leaf was found
             int32_t leaf_before = -1;
             double dt_before = 0.0, raw_before = 0.0;
@@ -433,6 +461,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
                         if (i >= from) heads.write(i, lane, kNone);
                 }
             }
+            wave_lds_sync();
             list_count[lane] = (uint16_t)count;
             list_end[lane] = end;
             list_taken[lane] = 0;
@@ -472,7 +501,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<dou
                 int id = first;
                 for (int i = 0; any_lane(i < from + taken); ++i) {
                     if (i < from + taken) {
-                        if (i >= from) order[to + i] = (uint16_t)id;
+                        if (i >= from) order(to + i) = (uint16_t)id;
                         id = list_next[id];
                     }
                 }

@@ -451,34 +451,34 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     // wavefront as leaves the lists room for all they find: the launcher cannot know how many leaves have density, so the lines are
     // drawn where trees all of whose leaves do lose nothing or little.  What was measured (us; lanes that walk a ray together / pieces, in
     // parentheses where they are not taken; half of the leaves with density, all of them):
-    //   forward           20 000 rays               26 000                 40 960
-    //   16^3 SH4          65, 67 / 43, 51           66, 69 / (73, 79)      76, 79 / (94, 106)
-    //   32^3 SH9          155, 162 / 96, 139        160, 167 / 102, 146    182, 183 / (141, 212)
-    //   64^3 SH4          279, 287 / 153, 234       286, 294 / 194, 288    333, 335 / (283, 426)
-    //   64^3 SH16         407, 428 / 178, 282       436, 458 / 223, 349    492, 514 / (335, 515)
-    //   128^3 SH4         548, 568 / 338, 491       577, 591 / 423, 614    628, 647 / (634, 934)
-    //   shell 128^3 SH9   303, 346 / 199, 281       305, 334 / 246, 333    345, 389 / (369, 493)
-    //   shell 256^3 SH16  506, 594 / 290, 416       532, 659 / 344, 525    585, 701 / (513, 756)
-    //   gradient          20 000 rays               26 000                 40 960                    65 536                    131 072
-    //   16^3 SH4          115, 154 / 88, 154        121, 173 / 111, 144    153, 220 / (156, 208)     226, 328 / (223, 303)     335, 497 / (412, 558)
-    //   32^3 SH9          307, 426 / 209, 331       337, 478 / 256, 410    427, 594 / 371, 571       602, 957 / 562, 834       913, 1500 / (1088, 1599)
-    //   64^3 SH4          561, 686 / 250, 565       602, 744 / 309, 703    699, 903 / 628, 910       1030, 1401 / 986, 1413    1576, 2184 / (1909, 2709)
-    //   64^3 SH16         932, 1271 / 515, 1090     1050, 1404 / 627, 1316 1248, 1801 / 1079, 1723   1939, 2885 / 1679, 2675   3125, 4880 / (3283, 5134)
-    //   128^3 SH4         1304, 1511 / 559, 1185    1375, 1604 / 692, 1464 1562, 1858 / 1025, 2211   2361, 2987 / (1574, 3416) 3695, 4683 / (3038, 6633)
-    //   shell 128^3 SH9   601, 899 / 325, 689       658, 887 / 398, 809    677, 1165 / 581, 1168     979, 1681 / 862, 1761     1477, 2587 / (1659, 3300)
-    //   shell 256^3 SH16  1094, 1668 / 639, 1400    1174, 1819 / 732, 1674 1286, 2329 / 1019, 2367   1898, 3235 / 1527, 3604   2903, 5093 / (2827, 6745)
-    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full 128^3 grids lose a fifth of a gradient beyond
-    // 32 768 rays, full shells a tenth at 65 536, for the sake of trees with empty leaves, which gain a third.
+    //   forward           20 000 rays               26 000                    40 960
+    //   16^3 SH4          66, 67 / 46, 52           68, 70 / (72, 78)         78, 81 / (88, 100)
+    //   32^3 SH9          158, 163 / 95, 139        160, 167 / 104, 151       177, 182 / (136, 207)
+    //   64^3 SH4          278, 285 / 144, 220       285, 294 / 165, 254       318, 328 / (242, 365)
+    //   64^3 SH16         404, 427 / 174, 280       439, 463 / 219, 338       478, 496 / (312, 487)
+    //   128^3 SH4         550, 565 / 296, 430       576, 590 / 358, 531       622, 646 / (528, 797)
+    //   shell 128^3 SH9   290, 315 / 195, 247       320, 354 / 238, 291       330, 351 / (329, 421)
+    //   shell 256^3 SH16  507, 599 / 253, 349       526, 620 / 303, 432       575, 677 / (434, 618)
+    //   gradient          20 000 rays               26 000                    40 960                    65 536                    131 072
+    //   16^3 SH4          120, 157 / 95, 158        129, 180 / 115, 147       162, 228 / 155, 209       224, 332 / 201, 276       341, 502 / (355, 486)
+    //   32^3 SH9          308, 435 / 204, 327       343, 480 / 242, 398       418, 627 / 350, 542       610, 959 / 521, 771       917, 1502 / (974, 1451)
+    //   64^3 SH4          553, 686 / 245, 518       597, 745 / 279, 601       696, 904 / 402, 867       1036, 1404 / 596, 1308    1574, 2196 / (1106, 2469)
+    //   64^3 SH16         935, 1268 / 473, 965      1041, 1400 / 578, 1149    1271, 1850 / 815, 1625    1926, 2878 / 1201, 2454   3110, 4904 / (2221, 4617)
+    //   128^3 SH4         1312, 1515 / 500, 1020    1355, 1599 / 597, 1261    1534, 1854 / 876, 1877    2385, 2987 / 1329, 2858   3678, 4680 / (2535, 5498)
+    //   shell 128^3 SH9   611, 812 / 292, 563       644, 911 / 360, 654       688, 1071 / 487, 911      869, 1554 / 754, 1396     1362, 2308 / (1359, 2464)
+    //   shell 256^3 SH16  1182, 1617 / 503, 1019    1147, 1732 / 587, 1223    1336, 1993 / 777, 1649    1600, 2816 / 1161, 2553   2532, 4447 / (2011, 4364)
+    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full shells of 256^3 and 128^3 grids lose 2 % of a gradient
+    // at 40 960 rays and nothing beyond; gradients of 131 072 gain in half-empty trees what full 128^3 grids lose, 31 % and 17 %.
     const double cells = (double)tree->capacity * 8.0;
     const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
     const bool grid = like_complete_octree(tree);
     constexpr int64_t kFill = 20480;
     if (tiny && !(gradient && n_rays <= 2560)) return c;
-    const int64_t most_rays = gradient ? (small ? 32768 : grid && large ? 40960 : 65536) : small ? kFill : 26624;
+    const int64_t most_rays = gradient ? 65536 : small ? kFill : 26624;
     if (n_rays > most_rays) return c;
     if (small) {
         const bool eight = n_rays <= 14336 || n_rays > kFill;
-        c.per_wave = eight ? 8 : 12;     // (8 rays to each of 1 792 wavefronts, all that run at once)
+        c.per_wave = eight ? 8 : 12;     // (8 rays to each of as many wavefronts as run at once)
         c.most = eight ? 3 : 2;
     } else if (medium) {
         const bool short_lists = n_rays <= 8192 || (gradient && n_rays > 14336);
@@ -487,7 +487,7 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     } else {
         // (of a 128^3 grid the lists hold the leaves of two rays, four in a pinch: 4 x 16 / 2 x 32, gradient 20 000 rays 787, 1542 / 683, 1336,
         // forward pass 12 000 rays 229, 417 / 235, 364, 20 000 rays 336, 623 / 370, 565)
-        const bool two = grid && (large ? gradient || n_rays > 16384 : n_rays > 28672);
+        const bool two = grid && large && (gradient || n_rays > 16384);
         c.per_wave = large && n_rays <= 1280 ? 1 : n_rays <= 2560 || two ? 2 : 4;
         c.most = large ? 6 : 5;
     }
