@@ -467,8 +467,8 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     //   128^3 SH4         1312, 1515 / 500, 1020    1355, 1599 / 597, 1261    1534, 1854 / 876, 1877    2385, 2987 / 1329, 2858   3678, 4680 / (2535, 5498)
     //   shell 128^3 SH9   611, 812 / 292, 563       644, 911 / 360, 654       688, 1071 / 487, 911      869, 1554 / 754, 1396     1362, 2308 / (1359, 2464)
     //   shell 256^3 SH16  1182, 1617 / 503, 1019    1147, 1732 / 587, 1223    1336, 1993 / 777, 1649    1600, 2816 / 1161, 2553   2532, 4447 / (2011, 4364)
-    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full shells of 256^3 and 128^3 grids lose 2 % of a gradient
-    // at 40 960 rays and nothing beyond; gradients of 131 072 gain in half-empty trees what full 128^3 grids lose, 31 % and 17 %.
+    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full 128^3 grids lose 1 % of a gradient of
+    // 40 960 rays; of 131 072 rays they would lose 17 % (half-empty trees would gain up to a third).
     const double cells = (double)tree->capacity * 8.0;
     const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
     const bool grid = like_complete_octree(tree);
