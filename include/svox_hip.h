@@ -70,7 +70,7 @@ typedef struct SvoxTreeSpec {
     int32_t dtype;               /* SvoxDType of data/extra_data/offset/scaling/weight_accum */
     const int32_t* child_marks;  /* optional (NULL: none): what svox_mark_empty_leaves / svox_mark_leaves_below wrote for this tree */
     float child_marks_thresh;    /* the sigma_thresh those marks were made with (0 for svox_mark_empty_leaves) */
-    int32_t child_marks_softplus;/* bit 0: they were made with density_softplus; SVOX_MARKS_WALK, SVOX_MARKS_NONE: see svox_walk_table */
+    int32_t child_marks_softplus;/* nonzero: they were made with density_softplus */
 } SvoxTreeSpec;
 
 /* RaysSpec, svox/csrc/include/data_spec.hpp:51-63 */
@@ -397,7 +397,7 @@ int svox_mark_leaves_below(const SvoxTreeSpec* tree, float sigma_thresh, int32_t
  * sigma > 0 whatever the threshold (backward, se_grad, noting forward); image: its rays are those of cameras.  Like marks, the table describes child (and, with marks,
  * data) as they are.  _bytes: the size of the table where making it for one call of n_rays pays, 0 where it does not or the
  * call would make no use of it.  Results are bit-identical. */
-#define SVOX_MARKS_WALK 2   /* child_marks_softplus: child_marks is a walk table */
+#define SVOX_MARKS_WALK 2   /* child_marks_softplus, beside a child_marks_thresh below zero, which no marks that apply to a call have: child_marks is a walk table */
 #define SVOX_MARKS_NONE 4   /* ... made without marks: it hides no leaf, and serves every render call */
 int64_t svox_walk_table_bytes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, int32_t image,
                               int32_t every_positive_leaf);

@@ -498,24 +498,55 @@ Lobes lobes_of(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt) {
     return Lobes{(const float*)tree->extra_data, tree->extra_cols, opt->format};
 }
 
+// Whether child_marks is a walk table, as svox_walk_table leaves it: one of its numbers in child_marks_softplus, and a child_marks_thresh below
+// zero (or no number), which marks that apply to any call do not have.  Marks by themselves may say by any number but 0 that they were made with
+// density_softplus.
+bool has_walk_table(const SvoxTreeSpec* tree) {
+    uint32_t bits;
+    memcpy(&bits, &tree->child_marks_thresh, 4);
+    const int32_t is = tree->child_marks_softplus;
+    return tree->child_marks && bits > 0x80000000u &&
+           (is == SVOX_MARKS_WALK || is == (SVOX_MARKS_WALK | 1) || is == (SVOX_MARKS_WALK | SVOX_MARKS_NONE));
+}
+// The threshold of the marks a walk table was made from, as it carries it: the next number of the other sign.
+float walk_thresh(float thresh) {
+    uint32_t bits;
+    thresh += 0.0f;   // (-0 is 0)
+    memcpy(&bits, &thresh, 4);
+    bits = (bits + 1u) | 0x80000000u;
+    memcpy(&thresh, &bits, 4);
+    return thresh;
+}
+float marks_thresh(const SvoxTreeSpec* tree) {
+    float thresh = tree->child_marks_thresh;
+    if (!has_walk_table(tree)) return thresh;
+    uint32_t bits;
+    memcpy(&bits, &thresh, 4);
+    bits = (bits & 0x7fffffffu) - 1u;
+    memcpy(&thresh, &bits, 4);
+    return thresh;
+}
+// Whether they are a walk table made without marks, which hides no leaf.
+bool marks_none(const SvoxTreeSpec* tree) { return has_walk_table(tree) && (tree->child_marks_softplus & SVOX_MARKS_NONE); }
+
 // Whether a launch that works on every leaf with density > need_thresh (the forward pass: opt->sigma_thresh; the
 // backward passes, se_grad and the noting passes: 0) may read the caller's marks in place of the child table: the
-// marks hide the leaves whose density is not > child_marks_thresh, which must all be leaves the launch skips.
-// (SVOX_MARKS_NONE: they hide none.)
+// marks hide the leaves whose density is not > the threshold they were made with, which must all be leaves the launch skips.
 bool marks_apply(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh) {
-    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_NONE)) return true;
-    return tree->child_marks && tree->child_marks_thresh >= 0.0f && need_thresh >= tree->child_marks_thresh &&
-           ((tree->child_marks_softplus & 1) != 0) == (opt->density_softplus != 0);
+    if (marks_none(tree)) return true;
+    const bool softplus = has_walk_table(tree) ? (tree->child_marks_softplus & 1) != 0 : tree->child_marks_softplus != 0;
+    const float thresh = marks_thresh(tree);
+    return tree->child_marks && thresh >= 0.0f && need_thresh >= thresh && softplus == (opt->density_softplus != 0);
 }
 // ... and whether the marks hide exactly the leaves the launch skips: every leaf they let through is shaded.
 bool marks_decide(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh) {
-    return marks_apply(tree, opt, need_thresh) && !(tree->child_marks_softplus & SVOX_MARKS_NONE) && need_thresh == tree->child_marks_thresh;
+    return marks_apply(tree, opt, need_thresh) && !marks_none(tree) && need_thresh == marks_thresh(tree);
 }
 
 // The tree as the octree march kernels see it: with the caller's marks in place of the child table where they apply.
 TreeDev<float> march_tree(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh = 0.0f) {
     TreeDev<float> d = make_tree<float>(tree);
-    if (marks_apply(tree, opt, need_thresh)) (tree->child_marks_softplus & SVOX_MARKS_WALK ? d.walk : d.child) = tree->child_marks;
+    if (marks_apply(tree, opt, need_thresh)) (has_walk_table(tree) ? d.walk : d.child) = tree->child_marks;
     return d;
 }
 
@@ -544,7 +575,7 @@ TreeDev<float> on_child_table(TreeDev<float> tr) {
 //   32^3 and smaller (batches of 13 000 and 300 000, picture of 800): 68, 253, 81 / 63, 232, 99
 bool walk_table_pays(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, bool image, bool every_positive_leaf) {
     if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes || fast_basis(tree, opt) < 0) return false;
-    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_WALK)) return false;
+    if (has_walk_table(tree)) return false;
     if (g_debug_flags & 128) return true;
     if (tree->capacity < 32768 || n_rays <= 12288) return false;
     if (opt->density_softplus && every_positive_leaf) return false;   // (rays end behind the first leaves they meet)
@@ -1954,13 +1985,14 @@ int svox_walk_table(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int3
     if (rc) return rc;
     if (!table_out || !with_table_out) return fail(SVOX_ERR_NULL_POINTER, "table_out / with_table_out is NULL");
     if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes) return fail(SVOX_ERR_BAD_SHAPE, "walk tables are for octrees of fewer than 2^22 nodes");
-    if (tree->child_marks && (tree->child_marks_softplus & SVOX_MARKS_WALK)) return fail(SVOX_ERR_BAD_SHAPE, "child_marks is a walk table already");
+    if (has_walk_table(tree)) return fail(SVOX_ERR_BAD_SHAPE, "child_marks is a walk table already");
     const bool marked = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh);
     hipLaunchKernelGGL(walk_table_kernel, dim3((unsigned)((tree->capacity * 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        marked ? tree->child_marks : tree->child, (int32_t)tree->capacity, (uint32_t*)table_out);
     *with_table_out = *tree;
     with_table_out->child_marks = table_out;
-    with_table_out->child_marks_softplus = marked ? (tree->child_marks_softplus & 1) | SVOX_MARKS_WALK : SVOX_MARKS_WALK | SVOX_MARKS_NONE;
+    with_table_out->child_marks_softplus = !marked ? SVOX_MARKS_WALK | SVOX_MARKS_NONE : tree->child_marks_softplus ? SVOX_MARKS_WALK | 1 : SVOX_MARKS_WALK;
+    with_table_out->child_marks_thresh = walk_thresh(marked ? tree->child_marks_thresh : 0.0f);
     return check_launch("walk_table");
 }
 

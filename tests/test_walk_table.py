@@ -45,6 +45,60 @@ def test_which_calls_make_a_walk_table():
     assert first(shell, 0, 1) == 1 << 30
 
 
+@pytest.mark.parametrize("softplus", [0, 1, 2, 3, 4, 6, 7, -1])
+def test_any_number_but_0_says_that_marks_are_softened(softplus):
+    """... and none that they are a walk table, of which no second one is made."""
+    lib = _abi.load_library()
+    spec, opt = _abi.TreeSpecC(), _abi.RenderOptionsC()
+    spec.data = spec.child = spec.parent_depth = spec.child_marks = 16
+    spec.capacity, spec.N, spec.data_dim, spec.dtype = 192314, 2, 13, 0
+    opt.format, opt.basis_dim, opt.max_comp, opt.ndc_width = 1, 4, 3, -1
+    spec.child_marks_softplus = softplus
+    for thresh in (0.0, -0.0, 1e-2, float("inf")):
+        spec.child_marks_thresh = thresh
+        assert lib.svox_walk_table_bytes(ctypes.byref(spec), ctypes.byref(opt), 1 << 20, 1, 0) == 192314 * 32, thresh
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("softplus", [1, 2, 3, 6, -1])
+@pytest.mark.parametrize("thresh", [0.0, 0.6])
+def test_marks_with_softplus_whatever_number_says_so(gpu, softplus, thresh):
+    """Marks, and walk tables made from them; a call to which they do not apply leaves them aside."""
+    tree = grown(2)
+    # (softened, -200 is 0, and 0.7 less than 0.6)
+    some = torch.rand(tree.child.shape, generator=torch.Generator().manual_seed(7))
+    tree.data.data[..., -1][some < 0.2] = -200.0
+    tree.data.data[..., -1][some > 0.8] = 0.7
+    rs, spec = rays_spec(synth.sphere_rays(1500, seed=4), gpu), on_gpu(tree, gpu)._spec()
+    rays = C._pack_rays(rs, torch.float32)
+    for soft in (True, False):
+        opt = options(tree, step_size=1e-3, sigma_thresh=thresh, density_softplus=soft)
+        want = C.volume_render(spec, rs, opt)
+        grad = C.volume_render_backward(spec, rs, opt, want, workspace=False)
+        packed, marks = C._pack_tree(spec), C.mark_empty_leaves(spec, thresh, True)
+        assert int((marks < 0).sum()) > marks.numel() // 10
+        packed.child_marks, packed.child_marks_thresh, packed.child_marks_softplus = marks.data_ptr(), thresh, softplus
+        table, made = torch.empty_like(marks), _abi.TreeSpecC()
+        stream = torch.cuda.current_stream().cuda_stream
+        for positive in (0, 1):
+            C._call("svox_walk_table", ctypes.byref(packed), ctypes.byref(opt._pack()), positive, table.data_ptr(), ctypes.byref(made), stream)
+            applies = soft and (thresh == 0.0 or not positive)
+            assert made.child_marks_softplus == (3 if applies else 6)
+            for kernel in (4, 8):
+                C.set_debug_flags(kernel)
+                try:
+                    for given in (packed, made):
+                        out, again = torch.empty_like(want), torch.empty_like(grad)
+                        C._call("svox_volume_render", ctypes.byref(given), ctypes.byref(rays), ctypes.byref(opt._pack()), out.data_ptr(), stream)
+                        C._call("svox_volume_render_backward", ctypes.byref(given), ctypes.byref(rays), ctypes.byref(opt._pack()),
+                                want.data_ptr(), again.data_ptr(), 0, stream)
+                        assert torch.equal(out, want), (soft, kernel)
+                        # (the same terms in another order, as above)
+                        assert (again - grad).abs().max() <= 2e-4 * grad.abs().max(), (soft, kernel)
+                finally:
+                    C.set_debug_flags(0)
+
+
 def grown(seed, steps=6):
     """A tree refined a few leaves at a time, so that its nodes lie in no order, with empty leaves and full ones."""
     g = torch.Generator().manual_seed(seed)
