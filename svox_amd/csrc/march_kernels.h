@@ -448,7 +448,7 @@ __device__ __forceinline__ uint32_t octant_of(uint32_t ix, uint32_t iy, uint32_t
 // everything else up to 45 % slower.)
 struct OctreeCursor {
     int32_t* rows;         // the lane's column of the path: rows[64 * (1 + max(up, kPathUp))]
-    float p[3];            // the sample, clamped, times 2^24
+    float m[3];            // the sample, clamped, times -2^24
     uint32_t ix, iy, iz;   // its integer coordinates
     int up;                // where the search for its leaf stands, in levels above the finest the coordinates hold (kCoordBits
                            // minus the level; negative: the sample lies deeper): the child row to look into ...
@@ -459,7 +459,7 @@ struct OctreeCursor {
     __device__ __forceinline__ void reset(int32_t* lane_path) {
         rows = lane_path - kPathUp * kMarchThreads;
         rows[kCoordBits * kMarchThreads] = 0;
-        p[0] = p[1] = p[2] = 0.0f;
+        m[0] = m[1] = m[2] = 0.0f;
         ix = iy = iz = 0;
         up = kCoordBits - 1;
         row = 0;
@@ -470,22 +470,19 @@ struct OctreeCursor {
         for (int i = 0; i < 3; ++i) {
             r.o[i] *= 16777216.0f;
             r.d[i] *= 16777216.0f;
-            // (a coordinate that is not a number counts as the upper bound, clamp01: so does an infinite one, and fmed3 below has no
-            // say in the matter)
-            if (!(r.o[i] == r.o[i]) || !(r.d[i] == r.d[i])) {
-                r.o[i] = __builtin_inff();
-                r.d[i] = 0.0f;
-            }
         }
         aim(r, kCoordBits - 1);
     }
     // the sample at r.t; leaf_up: where the leaf of the sample before it lies (kCoordBits - 1: the path says nothing of it)
     __device__ __forceinline__ void aim(const RayState<float>& r, int leaf_up) {
-        // (clamp01, times 2^24)
+        // (clamp01, times -2^24: of a coordinate that is no number, as 0 times an infinite direction is, clamp01 makes the upper bound, and fmed3 the
+        // least of the other two.  The asm keeps the compiler from taking the signs out again.)
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-            p[i] = __builtin_amdgcn_fmed3f(fma_(r.t, r.d[i], r.o[i]), 0.0f, __uint_as_float(0x3F7FFFEFu) * 16777216.0f);
-        const uint32_t nx = (uint32_t)p[0], ny = (uint32_t)p[1], nz = (uint32_t)p[2];
+        for (int i = 0; i < 3; ++i) {
+            m[i] = __builtin_amdgcn_fmed3f(-fma_(r.t, r.d[i], r.o[i]), 0.0f, -__uint_as_float(0x3F7FFFEFu) * 16777216.0f);
+            asm("" : "+v"(m[i]));
+        }
+        const uint32_t nx = (uint32_t)-m[0], ny = (uint32_t)-m[1], nz = (uint32_t)-m[2];
         // the first level the two samples differ at is that of the highest bit they differ in; not below the leaf, nor the path
         const uint32_t diff = (ix ^ nx) | (iy ^ ny) | (iz ^ nz) | 1u << leaf_up | 1u << (kPathUp + 1);
         up = 31 - __builtin_clz(diff);
@@ -538,12 +535,12 @@ struct OctreeCursor {
         int32_t* const at = rows + max(up, kPathUp) * kMarchThreads;
         at[kMarchThreads] = (int32_t)word;
         const uint32_t up_bits = (uint32_t)up << 23;
-        const float to_leaf = __uint_as_float((127u << 23) - up_bits);
+        const float to_leaf = __uint_as_float((383u << 23) - up_bits);
         const float inv_cube = __uint_as_float(((uint32_t)(127 - kCoordBits) << 23) + up_bits);
         float here[3], below_it[3];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const float s = p[j] * to_leaf;
+            const float s = m[j] * to_leaf;
             here[j] = __builtin_amdgcn_fractf(s);
             below_it[j] = __builtin_amdgcn_fractf(s + s);
         }
@@ -564,15 +561,15 @@ struct OctreeCursor {
     }
     // the step to the far side of the leaf the sample lies in
     __device__ __forceinline__ float step_out(const RayState<float>& r, int leaf_up, float step_size) const {
-        // 2^-up and 2^(up - 24): dividing by the power of two is the multiplication by its reciprocal
+        // -2^-up and 2^(up - 24): dividing by the power of two is the multiplication by its reciprocal
         const uint32_t up_bits = (uint32_t)leaf_up << 23;
-        const float to_leaf = __uint_as_float((127u << 23) - up_bits);
+        const float to_leaf = __uint_as_float((383u << 23) - up_bits);
         const float inv_cube = __uint_as_float(((uint32_t)(127 - kCoordBits) << 23) + up_bits);
         // leaf-local position frac(pos * 2^levels): s - floor(s), exact for the non-negative s of a clamped
         // coordinate, in one instruction
         float local[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) local[j] = __builtin_amdgcn_fractf(p[j] * to_leaf);
+        for (int j = 0; j < 3; ++j) local[j] = __builtin_amdgcn_fractf(m[j] * to_leaf);
         return leaf_exit(local, r.inv) * inv_cube + step_size;
     }
     // the sample's leaf is found, at the level `up` says: on to the next sample
@@ -593,7 +590,7 @@ __device__ __forceinline__ void walk_from_root(const TreeDev<float>& tr, RayStat
     float local[3], cells_per_axis;
     int levels;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) local[j] = cur.p[j] * (1.0f / 16777216.0f);
+    for (int j = 0; j < 3; ++j) local[j] = -cur.m[j] * (1.0f / 16777216.0f);
     slot_leaf = (int32_t)descend_generic<float>(tr.child, tr.capacity, tr.N, local, &cells_per_axis, &levels, true);
     if (slot_leaf >= 0) {
         // (rt_kernel.cu:274 divides by the cell count; for a power of two the product with the reciprocal is

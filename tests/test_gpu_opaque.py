@@ -162,3 +162,24 @@ def test_values_that_are_no_numbers(gpu, dtype, kind):
                     fine = grad.isfinite()
                     err, ok = grad_close(g[fine].cpu().numpy(), grad[fine].cpu().numpy())
                     assert ok, (kw, f, err)
+
+
+@pytest.mark.parametrize("flags", FLAGS)
+@pytest.mark.parametrize("N", [2, 3])
+def test_directions_without_a_length(gpu, oracle_mod, flags, N):
+    """The norm of a tiny direction is zero and its unit vector infinite: from an infinite origin the first sample has no number for a coordinate, and
+    counts as the upper corner.  (Every leaf ends such a ray.)"""
+    inf, tiny = float("inf"), 1e-30
+    signs = torch.tensor([[x, y, z] for x in (1, -1) for y in (1, -1) for z in (1, -1)], dtype=torch.float32)
+    origins = torch.cat([signs * inf] * 3 + [torch.rand(8, 3, generator=torch.Generator().manual_seed(2))])
+    dirs = torch.cat([signs * tiny, -signs * tiny, signs * 0.0, signs * tiny])
+    gen = torch.Generator().manual_seed(1)
+    tree = svox.N3Tree(N=N, data_format="SH1", init_refine=1)
+    tree.data.data.normal_(generator=gen)
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() + 1.0
+    rays = svox.Rays(origins, dirs, synth.unit_vectors(32, gen))
+    spec, rs, opt = on_gpu(tree, gpu)._spec(), rays_spec(rays, gpu), options(tree, step_size=1e-3)
+    want = torch.from_numpy(oracle_mod.volume_render(oracle_mod.Tree.from_n3tree(tree), rays.origins, rays.dirs, rays.viewdirs, opt))
+    assert torch.equal(run(1, lambda: C.volume_render(spec, rs, opt)).cpu(), want)
+    assert torch.equal(run(flags, lambda: C.volume_render(spec, rs, opt)).cpu(), want)
+    assert torch.equal(run(flags, lambda: C.volume_render_noted(spec, rs, opt)[0]).cpu(), want)
