@@ -395,8 +395,9 @@ int svox_mark_leaves_below(const SvoxTreeSpec* tree, float sigma_thresh, int32_t
  * step of nearly every search.  table_out (capacity, 2, 2, 2) int32; *with_table_out receives a copy of *tree that carries
  * the table in place of marks, for the render calls with the same options.  every_positive_leaf: the call is one that works on every leaf with
  * sigma > 0 whatever the threshold (backward, se_grad, noting forward); image: its rays are those of cameras.  Like marks, the table describes child (and, with marks,
- * data) as they are.  _bytes: the size of the table where making it for one call of n_rays pays, 0 where it does not or the
- * call would make no use of it.  Results are bit-identical. */
+ * data) as they are.  _bytes: the size of the table where making it for one call of n_rays pays, 0 where it does not, where the
+ * call would make no use of it, or where the child table (or the marks) does not begin at a multiple of 16 bytes: svox_walk_table refuses that.
+ * Results are bit-identical. */
 #define SVOX_MARKS_WALK 2   /* child_marks_softplus, beside a child_marks_thresh below zero, which no marks that apply to a call have: child_marks is a walk table */
 #define SVOX_MARKS_NONE 4   /* ... made without marks: it hides no leaf, and serves every render call */
 int64_t svox_walk_table_bytes(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, int32_t image,

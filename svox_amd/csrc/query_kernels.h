@@ -220,7 +220,7 @@ static __global__ __launch_bounds__(256) void last_nodes_kernel(const int32_t* _
     walk[i] = c;
 }
 
-// The walk table (kWalkNodeBits) of an octree from its child table or a copy with marks.  One thread per cell.
+// The walk table (kWalkNodeBits) of an octree from its child table or a copy with marks, which begins at a multiple of 16 bytes.  One thread per cell.
 static __global__ __launch_bounds__(256) void walk_table_kernel(const int32_t* __restrict__ child, int32_t capacity,
                                                                 uint32_t* __restrict__ walk) {
     const int64_t i = blockIdx.x * 256ll + threadIdx.x;

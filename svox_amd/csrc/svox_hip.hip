@@ -573,9 +573,15 @@ TreeDev<float> on_child_table(TreeDev<float> tr) {
 //   ... with notes, 128, 200, 400, 800, which wait for the colours as much as for the walk: shell 128^3  172, 203, 218, 259 / 157, 203, 219, 256;  256^3  258, 287,
 //     299, 347 / 212, 259, 295, 350;  512^3 SH16  341, 377, 400, 543 / 289, 329, 383, 530;  128^3 SH4  317, 317, 306, 429 / 320, 326, 311, 440
 //   32^3 and smaller (batches of 13 000 and 300 000, picture of 800): 68, 253, 81 / 63, 232, 99
+// The table a walk table is made from.  Its rows are read 16 bytes at a time (walk_table_kernel): one that begins elsewhere, which the march itself
+// reads entry by entry, serves no walk table.
+const int32_t* walk_source(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, bool every_positive_leaf) {
+    const int32_t* from = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh) ? tree->child_marks : tree->child;
+    return ((uintptr_t)from & 15u) == 0 ? from : nullptr;
+}
 bool walk_table_pays(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, bool image, bool every_positive_leaf) {
     if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes || fast_basis(tree, opt) < 0) return false;
-    if (has_walk_table(tree)) return false;
+    if (has_walk_table(tree) || !walk_source(tree, opt, every_positive_leaf)) return false;
     if (g_debug_flags & 128) return true;
     if (tree->capacity < 32768 || n_rays <= 12288) return false;
     if (opt->density_softplus && every_positive_leaf) return false;   // (rays end behind the first leaves they meet)
@@ -1986,9 +1992,11 @@ int svox_walk_table(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int3
     if (!table_out || !with_table_out) return fail(SVOX_ERR_NULL_POINTER, "table_out / with_table_out is NULL");
     if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes) return fail(SVOX_ERR_BAD_SHAPE, "walk tables are for octrees of fewer than 2^22 nodes");
     if (has_walk_table(tree)) return fail(SVOX_ERR_BAD_SHAPE, "child_marks is a walk table already");
-    const bool marked = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh);
-    hipLaunchKernelGGL(walk_table_kernel, dim3((unsigned)((tree->capacity * 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       marked ? tree->child_marks : tree->child, (int32_t)tree->capacity, (uint32_t*)table_out);
+    const int32_t* const from = walk_source(tree, opt, every_positive_leaf != 0);
+    if (!from) return fail(SVOX_ERR_BAD_SHAPE, "a walk table is made from a table that begins at a multiple of 16 bytes");
+    const bool marked = from != tree->child;
+    hipLaunchKernelGGL(walk_table_kernel, dim3((unsigned)((tree->capacity * 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, from,
+                       (int32_t)tree->capacity, (uint32_t*)table_out);
     *with_table_out = *tree;
     with_table_out->child_marks = table_out;
     with_table_out->child_marks_softplus = !marked ? SVOX_MARKS_WALK | SVOX_MARKS_NONE : tree->child_marks_softplus ? SVOX_MARKS_WALK | 1 : SVOX_MARKS_WALK;

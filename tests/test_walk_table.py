@@ -45,6 +45,38 @@ def test_which_calls_make_a_walk_table():
     assert first(shell, 0, 1) == 1 << 30
 
 
+def test_tables_that_do_not_begin_at_16_bytes_serve_no_walk_table():
+    lib = _abi.load_library()
+    spec, opt = _abi.TreeSpecC(), _abi.RenderOptionsC()
+    spec.data = spec.parent_depth = 16
+    spec.capacity, spec.N, spec.data_dim, spec.dtype = 192314, 2, 13, 0
+    opt.format, opt.basis_dim, opt.max_comp, opt.ndc_width, opt.sigma_thresh = 1, 4, 3, -1, 0.0
+    made = _abi.TreeSpecC()
+    for always in (0, ALWAYS):
+        C.set_debug_flags(always)
+        try:
+            # (marks that do not apply to the call, softened ones here, are not what the table is made from)
+            for child, marks, softened, pays in ((4096, 0, 0, True), (4100, 0, 0, False), (4104, 0, 0, False), (4100, 8192, 0, True), (4096, 8196, 0, False),
+                                                 (4096, 8196, 1, True), (4100, 8192, 1, False)):
+                spec.child, spec.child_marks, spec.child_marks_softplus = child, marks, softened
+                assert lib.svox_walk_table_bytes(ctypes.byref(spec), ctypes.byref(opt), 1 << 20, 1, 0) == (192314 * 32 if pays else 0), (child, marks)
+                if not pays:
+                    assert lib.svox_walk_table(ctypes.byref(spec), ctypes.byref(opt), 0, 4096, ctypes.byref(made), None) == -2
+        finally:
+            C.set_debug_flags(0)
+
+
+@pytest.mark.gpu
+def test_a_child_table_that_does_not_begin_at_16_bytes(gpu):
+    tree = synth.shell_tree(depth=8, data_format="SH1", n_spheres=24, seed=0, device=gpu)
+    rs, opt, spec = rays_spec(synth.sphere_rays(70001, seed=4), gpu), options(tree, step_size=1e-3), tree._spec()
+    want = C.volume_render(spec, rs, opt)
+    room = torch.empty(spec.child.numel() + 1, dtype=torch.int32, device=gpu)
+    room[1:] = spec.child.flatten()
+    spec.child = room[1:].view(spec.child.shape)
+    assert spec.child.data_ptr() % 16 == 4 and torch.equal(C.volume_render(spec, rs, opt), want)
+
+
 @pytest.mark.parametrize("softplus", [0, 1, 2, 3, 4, 6, 7, -1])
 def test_any_number_but_0_says_that_marks_are_softened(softplus):
     """... and none that they are a walk table, of which no second one is made."""
