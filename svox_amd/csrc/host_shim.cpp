@@ -327,12 +327,16 @@ void check_shaped(const Tensor& x, const char* name, at::ScalarType dt, at::IntA
     }
 }
 
-// The walk table of a call of n rays, where one pays: it goes with what is returned.  (every_positive_leaf: svox_walk_table)
+// The walk table of a call of n rays, where one pays and there is memory for it: it goes with what is returned.  (every_positive_leaf: svox_walk_table)
 Tensor attach_walk(Tree& t, const SvoxRenderOptions& c, int64_t n_rays, bool image, bool every_positive_leaf, void* stream) {
     Tensor table;
     const int64_t bytes = lib.svox_walk_table_bytes(&t.spec, &c, n_rays, image, every_positive_leaf);
     if (bytes <= 0) return table;
-    table = at::empty({bytes / 4}, t.child.options());
+    try {
+        table = at::empty({bytes / 4}, t.child.options());
+    } catch (const c10::OutOfMemoryError&) {
+        return table;   // (the march does without)
+    }
     const SvoxTreeSpec plain = t.spec;
     status(lib.svox_walk_table(&plain, &c, every_positive_leaf, (int32_t*)table.data_ptr(), &t.spec, stream), "walk_table");
     return table;

@@ -77,6 +77,27 @@ def test_a_child_table_that_does_not_begin_at_16_bytes(gpu):
     assert spec.child.data_ptr() % 16 == 4 and torch.equal(C.volume_render(spec, rs, opt), want)
 
 
+@pytest.mark.gpu
+def test_calls_without_memory_for_a_walk_table_do_without(gpu):
+    """The table takes 6 MB, for which torch asks for 20; the picture fits 2."""
+    tree = synth.shell_tree(depth=8, data_format="SH1", n_spheres=24, seed=0, device=gpu)
+    rs, opt, spec = rays_spec(synth.sphere_rays(70001, seed=4), gpu), options(tree, step_size=1e-3), tree._spec()
+    want = C.volume_render(spec, rs, opt)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(gpu) + (6 << 20)) / total, gpu)
+    held = []
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(100):      # (what is left of the blocks there are)
+                held.append(torch.empty(tree.child.numel(), dtype=torch.int32, device=gpu))
+        got = C.volume_render(spec, rs, opt)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("softplus", [0, 1, 2, 3, 4, 6, 7, -1])
 def test_any_number_but_0_says_that_marks_are_softened(softplus):
     """... and none that they are a walk table, of which no second one is made."""
