@@ -136,9 +136,9 @@ const char* svox_status_string(int status);
  * once, whatever their size (not with a weight accumulator), with as many rays to a wavefront as the last decimal digit of
  * flags >> 8 says (1 to 8; 0: they never take it), in 2^(the digits before it) pieces at most; in double precision gradients
  * too, with the last two digits for the rays (1 to 16), and 2^2 pieces at least.  With any other flag set no pass takes it.
- * Bit 6: noting passes over ray batches list the rays that meet the tree first, where
+ * Bit 6: noting passes over ray batches and pictures list the rays that meet the tree first, where
  * the workspace has room, whatever their size: up to 64 times bits 8 to 15 of them take two wavefronts per tile, up to 64 times
- * bits 16 and up one, more the batch as it is (so does one most of whose rays hit by a sample).  Bit 7: every call for which
+ * bits 16 and up one (of batches), more the batch or the pictures as they are (so does one most of whose rays hit by a sample).  Bit 7: every call for which
  * svox_walk_table could be made is said to gain by one.  The flags belong to the calling thread. */
 void svox_set_debug_flags(int flags);
 
@@ -314,8 +314,9 @@ int64_t svox_volume_render_backward_workspace_bytes(int64_t n_rays, int32_t reco
 /* No counterpart in the reference.  How full a workspace of notes ran: after a call that takes notes
  * (svox_volume_render_noted, svox_volume_render_images_noted, the _ws calls) the 64-bit word at byte
  * *counter_offset of the workspace holds the number of 64-chunk stocks its wavefronts asked for
- * beyond the rays' own chunks, and the workspace has *pool_stocks of them (rounded up; a batch of 131 072 rays and
- * more gives up to n_rays / 6 144 of them to a list of its rays, which a picture of as many pixels has beside those).  A count at
+ * beyond the rays' own chunks, and the workspace has *pool_stocks of them (rounded up; of 131 072 rays and more up to n_rays / 6 144
+ * are given to a list of them beside those, which pictures whose pixels are not listed have besides; pictures with fewer pixels
+ * that are listed count the stocks of their list among those asked for).  A count at
  * or above that number says the shared chunks ran out: some rays' notes are incomplete (those rays are
  * marched by the backward pass: correct, slower) and a larger workspace would serve the same rays
  * better.  Returns 0, or SVOX_ERR_BAD_SHAPE for a workspace too small to hold n_rays chunks. */

@@ -1006,7 +1006,8 @@ struct ReplaySpace {
     uint32_t n_stocks;
     // counts the wavefronts of render_forward_split_kernel that gave up waiting (svox_give_up_count)
     unsigned int* give_ups;
-    int32_t* list;         // room for a number per ray, behind the chunks (ListedSource, ListedImageSource), or nullptr
+    int32_t* list;         // room for a number per ray, behind the chunks or in the first stocks (ListedSource, ListedImageSource), or nullptr
+    uint32_t list_stocks;  // of the stocks, those that a launch which fills the list takes for it
     // a noting launch: the blocks that march; those beyond clear these arrays of clear_words words each
     uint32_t march_blocks;
     uint32_t* clear_at[2];

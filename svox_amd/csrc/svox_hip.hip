@@ -927,9 +927,10 @@ int64_t most_listed_pixels(const SvoxRenderOptions* opt, int64_t n_pixels, unsig
     return std::min((light ? tiles / 2 : tiles) * kMarchThreads, n_pixels);
 }
 constexpr int64_t kListRays = 1 << 17;
+bool list_at_end(int64_t n_slots) { return n_slots >= kListRays || (g_debug_flags & 64); }
 template <class Source>
 bool keeps_list(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, const Source& src, int64_t n_slots) {
-    return is_image_source(src) ? lists_pixels(tree, opt, n_slots) : n_slots >= kListRays || (g_debug_flags & 64);
+    return is_image_source(src) ? lists_pixels(tree, opt, n_slots) : list_at_end(n_slots);
 }
 
 // The workspace of the replaying kernels: chunks of notes, then one bit per ray (rays left undone by
@@ -940,7 +941,9 @@ constexpr int64_t kStampOffset = 0;
 constexpr int64_t kStockCounterOffset = 128;
 int64_t bitmap_bytes(int64_t n_slots) { return ((n_slots + 63) / 64 * 8 + 15) / 16 * 16; }
 // (and, of a batch or pictures whose rays may be listed, where the rays' shared chunks are many beside it, in the place of the last of them: a number per
-// ray.  Every pass over the notes says so alike (keeps_list), or the room they are in would not be the same.)
+// ray.  Every pass over the notes says so alike (keeps_list), or the room they are in would not be the same.  Of pictures with fewer pixels than
+// kListRays the list lies in the first stocks instead, which a launch that lists takes like any others: svox_notes_pool_info, which knows of
+// a workspace neither the tree nor whether its rays are a batch, has to know how many stocks it had.)
 bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, bool list, ReplaySpace* ws) {
     *ws = ReplaySpace{};
     int64_t chunks = workspace && n_slots > 0
@@ -950,8 +953,11 @@ bool carve_workspace(void* workspace, int64_t workspace_bytes, int64_t n_slots, 
     ws->undone = (unsigned long long*)((char*)workspace + chunks * kChunkBytes);
     const int64_t list_chunks = (n_slots * 4 + kChunkBytes - 1) / kChunkBytes;
     if (list && chunks - n_slots >= 16 * list_chunks) {
-        chunks -= list_chunks;
-        ws->list = (int32_t*)((char*)workspace + chunks * kChunkBytes);
+        if (list_at_end(n_slots))
+            chunks -= list_chunks;
+        else
+            ws->list_stocks = (uint32_t)((list_chunks + kChunkStock - 1) / kChunkStock);
+        ws->list = (int32_t*)((char*)workspace + (ws->list_stocks ? n_slots : chunks) * kChunkBytes);
     }
     ws->first_shared = n_slots;
     ws->n_chunks = chunks;
@@ -1070,6 +1076,7 @@ __global__ __launch_bounds__(kListThreads) void list_hits_kernel(TreeDev<float> 
         if (blockIdx.x == 0 && threadIdx.x == 0) *n_listed = (unsigned long long)src.n_rays();
         return;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && ws.list_stocks) *ws.stocks_taken = ws.list_stocks;
     __syncthreads();
     const int64_t slot = src.fetch(blockIdx.x * (int64_t)kListThreads + threadIdx.x, opt, offset, scaling, origin, dir, vdir);
     const bool hit = slot >= 0 && setup_ray(r, origin, dir, scaling);
@@ -1762,7 +1769,7 @@ int svox_notes_pool_info(int64_t n_rays, int64_t workspace_bytes, int64_t* count
     ReplaySpace ws;
     // (any 16-byte aligned address does for the arithmetic)
     char* const base = (char*)(uintptr_t)4096;
-    if (!carve_workspace(base, workspace_bytes, n_rays, n_rays >= kListRays || (g_debug_flags & 64), &ws))
+    if (!carve_workspace(base, workspace_bytes, n_rays, list_at_end(n_rays), &ws))
         return fail(SVOX_ERR_BAD_SHAPE, "svox_notes_pool_info: the workspace does not hold a chunk per ray");
     *counter_offset = (int64_t)((char*)ws.stocks_taken - base);
     *pool_stocks = ws.n_stocks;

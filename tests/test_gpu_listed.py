@@ -183,6 +183,38 @@ def test_listed_pixels(gpu, oracle_mod, w, h, n_images, view, tiles):
         assert ok, (what, err)
 
 
+@pytest.mark.parametrize("w", [128, 200, 361, 363])
+@pytest.mark.parametrize("fx", [1.39, 4.0])
+@pytest.mark.parametrize("records", [30, 300])
+def test_the_pool_of_a_picture_of_any_size(gpu, monkeypatch, w, fx, records):
+    """svox_notes_pool_info knows the number of rays and no more: of pictures with fewer than 131 072 pixels, which are listed where a batch of as
+    many rays is not, and of larger ones (363 x 363), it says what the pass and its replay go by, and a count below that says that no note was lost."""
+    monkeypatch.setattr(C, "SMALL_BATCH_ROOM", 1)
+    n = w * w
+    tree = synth.shell_tree(depth=7, data_format="SH9", n_spheres=24, seed=0, device=gpu)
+    spec, opt = tree._spec(), options(tree, step_size=5e-4)
+    cam = cam_spec(synth.orbit_poses(1, seed=2, radius=4.0)[0], w, w, fx * w, device=gpu)
+    report = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    got = []
+    for flags in (0, 8):
+        out, notes = run(flags, lambda: C.volume_render_images_noted(spec, cam, opt, records_per_ray=records))
+        counter, pool = C.notes_pool_use(notes, n)
+        asked, listed = (int(v) for v in notes.view(torch.int64)[counter.storage_offset():][[0, 2]])
+        count = notes.view(torch.int32)[: n * 96].view(n, 96)[:, 91].clone()
+        grad = run(flags, lambda: C.volume_render_images_backward_noted(spec, cam, opt, torch.ones_like(out), notes, report.data_ptr()))
+        torch.cuda.synchronize()
+        if flags == 0:
+            assert int(report[0]) == asked << 32 | pool and listed > 0
+            assert asked <= pool or bool((count < 0).any())      # (the last stock may be a part of one)
+        assert asked >= pool or bool((count >= 0).all())
+        got.append((out, count, grad, asked))
+    assert torch.equal(got[0][0], got[1][0])
+    if records == 300:
+        assert torch.equal(got[0][1], got[1][1])
+    err, ok = grad_close(got[0][2].cpu().numpy(), got[1][2].cpu().numpy())
+    assert ok, err
+
+
 def test_pictures_of_shells_take_less_time_listed(gpu):
     """(400x400 picture of a 256^3 SH9 shell, noting march 307 us as it is, 252 listed.)  And the rule takes the list where it says so: the last of
     the chunks are not for notes."""
