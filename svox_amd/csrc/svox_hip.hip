@@ -908,13 +908,14 @@ NoteStamp stamp_of(const SvoxTreeSpec* tree, const SvoxRaysSpec* rays, const Svo
 // picture (PicturesSpread).  A tile of 8 x 8 pixels has long rays or short ones, and leaves to shade in the same rounds or none, and the pass takes as long as
 // the worst of them; dealt out they are alike: 800x800 picture of a 512^3 SH16 shell 538 -> 417 us, of a 256^3 SH16 shell 453 -> 332, of 400x400 322 -> 251.
 // Not for grids that are as fine everywhere, whose rays are alike and read the same lines (64^3 SH9 400x400 175 / 178, 800x800 218 / 239; 128^3 SH4 435 / 507), trees
-// of fewer than 65 536 cells (16^3 RGBA 132 / 245), pictures in normalised device coordinates, all of whose rays meet the cube, and where what is to be gone through
-// is small beside the launches or large beside the hits: under 16 384 pixels, over 2 Mi (1700x1700, 16 000 hits: 412 / 428).
+// of fewer than 65 536 cells (16^3 RGBA 132 / 245), trees of other branching factors, whose rays walk longer and are no longer alike (gradient of an 800x800 picture,
+// us, as it is / listed: 81^3 SH9 full 1047 / 1100, one leaf in twenty 363 / 435, 64^3 (N = 4) SH1 400x400 208 / 221), pictures in normalised device coordinates, all of
+// whose rays meet the cube, and where what is to be gone through is small beside the launches or large beside the hits: under 16 384 pixels, over 2 Mi (1700x1700, 16 000 hits: 412 / 428).
 bool lists_pixels(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_pixels) {
     if (g_debug_flags & 64) return true;
     const Tuning& t = tuning();
     return g_debug_flags == 0 && t.per_wave <= 0 && t.split_forward < 0 && t.split_blocks < 0 && opt->ndc_width <= 0 && n_pixels >= 1 << 14 &&
-           n_pixels <= 1 << 21 && (double)tree->capacity * tree->N * tree->N * tree->N >= 65536.0 && !like_complete_octree(tree);
+           n_pixels <= 1 << 21 && tree->N == 2 && tree->capacity * 8 >= 65536 && !like_complete_octree(tree);
 }
 // Up to how many: tiles that are alike must all find a place at once, or the last of them take as long again when the first have ended (800x800, 256^3 SH9 shell:
 // 2 530 tiles 262 -> 225 us, 2 712 tiles 256 -> 402, of 2 816 places, as LDS has them; SH16, of 2 560: 2 290 tiles 439 -> 343, 2 446 445 -> 490).  Few functions leave little to

@@ -7,6 +7,7 @@ gradients the same terms in another order.
 import pytest
 import torch
 
+import svox_amd as svox
 from svox_amd import csrc as C
 from svox_amd import synth
 from util import cam_spec, grad_close, on_gpu, options, rays_spec
@@ -213,6 +214,19 @@ def test_the_pool_of_a_picture_of_any_size(gpu, monkeypatch, w, fx, records):
         assert torch.equal(got[0][1], got[1][1])
     err, ok = grad_close(got[0][2].cpu().numpy(), got[1][2].cpu().numpy())
     assert ok, err
+
+
+@pytest.mark.parametrize("N,levels", [(3, 3), (4, 2)])
+def test_pictures_of_other_branching_factors_are_not_listed(gpu, N, levels):
+    tree = svox.N3Tree(N=N, data_format="SH1", init_refine=levels, device=gpu)
+    tree.data.data[..., -1] = 1.0
+    w = 150
+    spec, opt = tree._spec(), options(tree, step_size=1e-3)
+    cam = cam_spec(synth.orbit_poses(1, seed=2, radius=4.0)[0], w, w, 1.39 * w, device=gpu)
+    for flags, listed in ((0, False), (64 | 255 << 8, True)):
+        notes = run(flags, lambda: C.volume_render_images_noted(spec, cam, opt)[1])
+        counter = C.notes_pool_use(notes, w * w)[0]
+        assert bool(notes.view(torch.int64)[counter.storage_offset() + 2] > 0) == listed
 
 
 def test_pictures_of_shells_take_less_time_listed(gpu):
