@@ -134,8 +134,11 @@ struct GroupBlock {
     // of a lane's list: how many there are, from which on and how many are composed now, and where in the ray's order
     uint16_t count[kMarchThreads], from[kMarchThreads], taken[kMarchThreads], place[kMarchThreads];
 };
+// (With 25 functions the coefficients of an entry take 150 registers: the compiler is told to leave room for two wavefronts on a SIMD, which costs 20 to 28
+// bytes of scratch.  Forward pass and gradient of 20 000 rays, one / two: 64^3 SH25 289, 912 / 203, 683 us, no leaf empty 483, 1934 / 335, 1432, 256^3 shell
+// 435, 974 / 271, 752.)
 template <int D, class Source, bool kBackward>
-__global__ __launch_bounds__(kMarchThreads) void render_group_kernel(TreeDev<double> tr, Source src, SvoxRenderOptions opt,
+__global__ __launch_bounds__(kMarchThreads, D > 16 ? 2 : 1) void render_group_kernel(TreeDev<double> tr, Source src, SvoxRenderOptions opt,
                                                                      const double* __restrict__ grad_out, double* __restrict__ result,
                                                                      int per_wave, int most_cut) {
     constexpr int DD = D > 0 ? D : 1;
