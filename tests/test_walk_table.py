@@ -39,7 +39,7 @@ def test_which_calls_make_a_walk_table():
     opt.ndc_width = 100
     assert first(shell, 1, 0, high=65536) == 12289
     opt.ndc_width, opt.density_softplus = -1, 1
-    assert first(shell, 1, 0) == 12289 and first(grid128, 0, 1) == 1 << 30
+    assert first(shell, 1, 0) == first(shell, 0, 0) == first(grid128, 1, 0) == first(grid128, 0, 1) == 1 << 30 and first(grid64, 0, 0) == 12289
     opt.density_softplus = 0
     opt.ndc_width, spec.N = -1, 3
     assert first(shell, 0, 1) == 1 << 30
