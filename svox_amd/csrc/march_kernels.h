@@ -792,18 +792,28 @@ template <int D, bool kRows>
 struct ShadeShared;
 template <int D>
 struct ShadeShared<D, true> {
+    float basis[kMarchThreads * D];             // [lane][coefficient]
+    float colour[kQueue * kMarchThreads * 3];   // [slot][lane][channel]: sigmoid(basis . coefficients)
     int32_t leaf[kQueue * kMarchThreads];       // leaf cell index of entry e
     uint8_t who[kQueue * kMarchThreads];        // owner lane | slot << 6
-    float colour[kQueue * kMarchThreads * 3];   // [slot][lane][channel]: sigmoid(basis . coefficients)
-    float basis[kMarchThreads * D];             // [lane][coefficient]
 };
 template <int D>
 struct ShadeShared<D, false> {
+    float vdir[kMarchThreads * 3];              // [lane][xyz]
+    float colour[kQueue * kMarchThreads * 3];
     int32_t leaf[kQueue * kMarchThreads];
     uint8_t who[kQueue * kMarchThreads];
-    float colour[kQueue * kMarchThreads * 3];
-    float vdir[kMarchThreads * 3];              // [lane][xyz]
 };
+// The LDS of a wavefront that walks and shades in turn.  The lowest row of its path, a dump, is `who`, which lives from a shade list to the end of its
+// round: 256 bytes more are a granule more for some, and two wavefronts fewer on a compute unit (march without notes of 200 000 rays, 81^3 SH16, 3 797 us instead of
+// 3 130; forward pass of 200 000 rays of a 128^3 shell with 16 lobes 414 instead of 321, of 285 000 rays of a 512^3 SH16 shell 890 instead of 754).
+template <int D, bool kRows>
+struct MarchShared {
+    ShadeShared<D, kRows> sh;
+    int32_t path[(kPathLevels + 1) * kMarchThreads];
+    __device__ __forceinline__ int32_t* lane_path(int lane) { return (int32_t*)((char*)this + offsetof(MarchShared, path)) - kMarchThreads + lane; }
+};
+static_assert(sizeof(((ShadeShared<1, true>*)nullptr)->who) == sizeof(int32_t) * kMarchThreads, "the row before the path is `who`");
 
 // Colours of all list entries, computed by the whole wavefront: item p = 3 * entry + channel goes to
 // lane p mod 64.  One item is the reference's dot product for one channel, evaluated in the
@@ -1264,8 +1274,8 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     static_assert(!kAllShaded || (!kNoted && !kAccum), "notes and weights look at leaves the marks may hide");
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
-    __shared__ ShadeShared<D, P::kForwardRows> sh;
+    __shared__ MarchShared<D, P::kForwardRows> lds;
+    auto& sh = lds.sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
     if constexpr (kNoted) {
         if constexpr (Source::kGated) {
@@ -1300,7 +1310,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_forward_kernel(TreeDev<f
     March1Sum sum1;
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
     OctreeCursor cur;
-    cur.reset(path + lane);
+    cur.reset(lds.lane_path(lane));
     const ChildTable child(tr);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
@@ -1959,7 +1969,7 @@ static_assert(kEmitCap <= kMarchThreads, "group_by_leaf holds one record per lan
 static_assert(sizeof(GroupScratch) + kEmitCap <= sizeof(float) * kQueue * kMarchThreads * 3,
               "GroupScratch and the owners live in ShadeShared::colour");
 using ShadeSharedProbe = ShadeShared<1, true>;
-static_assert(offsetof(ShadeSharedProbe, who) == sizeof(int32_t) * kQueue * kMarchThreads,
+static_assert(offsetof(ShadeSharedProbe, who) - offsetof(ShadeSharedProbe, leaf) == sizeof(int32_t) * kQueue * kMarchThreads,
               "the record list runs from ShadeShared::leaf into ShadeShared::who");
 
 
@@ -1997,9 +2007,11 @@ constexpr int32_t kEndedBit = 1 << 30;   // in SplitBox::taken: the ray wants no
 // 50 001 rays with notes 241 instead of 225).
 constexpr uint32_t kRoundBit = 1u << 30, kOverBit = 1u << 31;
 struct SplitBox {
-    unsigned long long place[(kRing + 1) * kMarchThreads];   // [place in the ring][lane], and a row for what is no leaf
+    unsigned long long place[kRing * kMarchThreads];   // [place in the ring][lane]
+    int32_t path[(kPathLevels + 2) * kMarchThreads];   // of the walk (OctreeCursor); its two dump rows are also the ring's, for what is no leaf
     int32_t taken[kMarchThreads];                      // set by the shading: places taken so far (| kEndedBit)
 };
+static_assert(offsetof(SplitBox, path) == sizeof(unsigned long long) * kRing * kMarchThreads, "a row of places behind the ring is two of the path");
 __device__ __forceinline__ uint32_t ring_round(int32_t n) { return ((uint32_t)n / kRing & 1u) ? kRoundBit : 0u; }
 
 // Places and counts are read and written as atomics of the workgroup (unlike a volatile access, which the compiler leaves on
@@ -2029,7 +2041,6 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
                                                                              const float* __restrict__ grad_out = nullptr) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
     __shared__ ShadeShared<D, P::kForwardRows> sh;
     __shared__ SplitBox box;
     if constexpr (kNoted) {
@@ -2095,7 +2106,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
     if (walks) {
         // ---- the walk: one leaf per live lane and turn, into the ring
         OctreeCursor cur;
-        cur.reset(path + lane);
+        cur.reset(box.path + lane);
         const ChildTable child(tr);
         if (active) cur.begin(r);
         // (counts of places in bytes of the ring)
@@ -2107,7 +2118,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         auto room = [&]() { return written - taken < kPlaces; };
         auto hand_over = [&](bool found, uint32_t code, float dt) {
             // (a lane without one writes to the row behind the ring)
-            unsigned char* const at = (unsigned char*)box.place + lane * 8 + (found ? written & (kPlaces - 1) : kPlaces);
+            unsigned char* const at = (unsigned char*)&box + lane * 8 + (found ? written & (kPlaces - 1) : kPlaces);
             ring_write((unsigned long long*)at, code | (written << 18 & kRoundBit), dt);
             written += found ? kPlace : 0u;
         };
@@ -2309,8 +2320,8 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
                                                                         ReplaySpace ws) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
-    __shared__ ShadeShared<D, true> sh;
+    __shared__ MarchShared<D, true> lds;
+    auto& sh = lds.sh;
     if (ws.only && *ws.any_undone == 0) return;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
@@ -2332,7 +2343,7 @@ __global__ __launch_bounds__(kMarchThreads) void render_backward_kernel(TreeDev<
     int phase = kMarch1;
     MergeState merge;
     OctreeCursor cur;
-    cur.reset(path + lane);
+    cur.reset(lds.lane_path(lane));
     const ChildTable child(tr);
 
     // takes ray `item` into this lane if it hits the tree
@@ -3144,8 +3155,8 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
                                                                const unsigned long long* __restrict__ any_undone) {
     constexpr int D = P::kBasis > 0 ? P::kBasis : 1;
     constexpr int K = P::kRecord;
-    __shared__ int32_t path[(kPathLevels + 2) * kMarchThreads];
-    __shared__ ShadeShared<D, true> sh;
+    __shared__ MarchShared<D, true> lds;
+    auto& sh = lds.sh;
     if (only && *any_undone == 0) return;
     const int lane = threadIdx.x;
     float offset[3], scaling[3];
@@ -3167,7 +3178,7 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> t
     int64_t slot = -1;
     bool active = false, second = false;
     OctreeCursor cur;
-    cur.reset(path + lane);
+    cur.reset(lds.lane_path(lane));
     const ChildTable child(tr);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray

@@ -922,7 +922,7 @@ bool lists_pixels(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_
            n_pixels <= 1 << 21 && tree->N == 2 && tree->capacity * 8 >= 65536 && !like_complete_octree(tree);
 }
 // Up to how many: tiles that are alike must all find a place at once, or the last of them take as long again when the first have ended (800x800, 256^3 SH9 shell:
-// 2 530 tiles 262 -> 225 us, 2 712 tiles 256 -> 402, of 2 816 places, as LDS has them; SH16, of 2 560: 2 290 tiles 439 -> 343, 2 446 445 -> 490).  Few functions leave little to
+// 2 530 tiles 262 -> 225 us, 2 712 tiles 256 -> 402, of 2 816 places; SH16, of 2 560: 2 290 tiles 439 -> 343, 2 446 445 -> 490).  Few functions leave little to
 // level, while rays from all over read more lines: half as many then (512^3 SH1 shell 125 000 hits 318 / 332; 74 000 hits, 512^3 SH4 392 -> 334, 256^3 SH1 252 -> 241).
 // Pictures with more hits pay for the sample and a launch without tiles: 5 to 10 us (800x800 close up, 512^3 SH16 868 / 876, 128^3 SH4 328 / 334).
 int64_t most_listed_pixels(const SvoxRenderOptions* opt, int64_t n_pixels, unsigned at_once) {

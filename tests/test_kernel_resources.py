@@ -47,3 +47,23 @@ def wavefronts(kernel):
 def test_double_precision_rays_in_pieces(kernels, basis, forward, backward, source):
     assert wavefronts(kernels[f"render_group_kernel<{basis}, {source}, false>"]) >= forward
     assert wavefronts(kernels[f"render_group_kernel<{basis}, {source}, true>"]) >= backward
+
+
+def by_lds(kernel):
+    return LDS // (-(-kernel[0] // GRANULE) * GRANULE) * (kernel[2] // 64)
+
+
+# (a path of 11 levels and its dump rows, beside the shading's lists: MarchShared, SplitBox)
+@pytest.mark.parametrize("policy,walks_and_shades,splits,marches", [("0, 0", 18, 24, 21), ("1, 1", 18, 24, 21), ("1, 4", 18, 24, 18), ("1, 9", 18, 24, 16), ("1, 16", 18, 24, 14),
+                                                                    ("1, 25", 18, 24, 11), ("2, 1", 21, 24, 21), ("2, 4", 18, 22, 18), ("2, 9", 16, 20, 16),
+                                                                    ("2, 16", 14, 16, 14), ("2, 25", 11, 16, 11)])
+@pytest.mark.parametrize("source", ["BatchSource<float>", "ImageSource<float>"])
+def test_wavefronts_lds_has_room_for(kernels, policy, walks_and_shades, splits, marches, source):
+    policy = f"OctreePolicy<{policy}>"
+    for refill in ("false", "true"):
+        for noted in ("false", "true"):
+            assert by_lds(kernels[f"render_forward_kernel<{policy}, {source}, false, {refill}, {noted}, false, false>"]) >= walks_and_shades
+            assert by_lds(kernels[f"render_forward_split_kernel<{policy}, {source}, {noted}, false>"]) >= splits
+        for mode in (0, 1):
+            assert by_lds(kernels[f"render_backward_kernel<{policy}, {source}, {refill}, {mode}>"]) >= marches
+        assert by_lds(kernels[f"se_grad_kernel<{policy}, {source}, {refill}>"]) >= marches
