@@ -67,3 +67,14 @@ def test_wavefronts_lds_has_room_for(kernels, policy, walks_and_shades, splits, 
         for mode in (0, 1):
             assert by_lds(kernels[f"render_backward_kernel<{policy}, {source}, {refill}, {mode}>"]) >= marches
         assert by_lds(kernels[f"se_grad_kernel<{policy}, {source}, {refill}>"]) >= marches
+
+
+@pytest.mark.parametrize("policy,notes,marches", [("0, 0", 16, 20), ("1, 16", 16, 14), ("2, 4", 16, 16), ("2, 9", 16, 16), ("2, 16", 14, 14)])
+@pytest.mark.parametrize("source", ["BatchSource<float>", "ImageSource<float>"])
+def test_wavefronts_that_take_notes_or_march_without(kernels, policy, notes, marches, source):
+    for refill in ("false", "true"):
+        for mode in (0, 1):
+            assert wavefronts(kernels[f"render_backward_kernel<OctreePolicy<{policy}>, {source}, {refill}, {mode}>"]) >= marches
+        if policy.startswith("2"):
+            for grad in ("false", "true"):
+                assert wavefronts(kernels[f"render_forward_kernel<OctreePolicy<{policy}>, {source}, false, {refill}, true, {grad}, false>"]) >= notes
