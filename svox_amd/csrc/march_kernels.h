@@ -410,6 +410,35 @@ struct ChildTable {
         words = octree && tr.walk != nullptr;
         entries = __builtin_amdgcn_make_buffer_rsrc((void*)(words ? tr.walk : tr.child), 0, octree ? cells << 2 : 0u, 0x00020000);
     }
+    // The table for a wavefront whose first rays are these, before any of them begins.  Rays that run close together find the rows they read in L1, and
+    // the turns of a walk on a walk table that only descend then cost more than the reads it saves: it stays with the child table where most
+    // neighbours enter the cube less than 0.7 of the square root of 1/nodes apart -- of a surface 0.4 of its leaves -- unless marks went into the walk table,
+    // which the child table has not.  (Pictures, us, child table / walk table, by that distance over the square root: 128^3 shell RGBA 0.34 175 / 198, 0.38 147 / 173,
+    // 0.48 117 / 131, 0.64 114 / 116, 0.69 118 / 111, SH9 0.38 175 / 197, 0.43 173 / 166; 256^3 RGBA 0.48 345 / 387, 0.68 228 / 247, 0.77 203 / 219, 0.86 189 / 181, SH9 0.6 299 / 318, 0.68
+    // 260 / 272, 0.77 241 / 248, 0.86 229 / 215; 512^3 RGBA 0.6 465 / 514, 0.96 410 / 446, 1.2 323 / 337, 1.5 266 / 254, SH9 0.6 605 / 596, 0.96 629 / 578; 128^3 grid SH4 0.6
+    // 384 / 411, 1.2 281 / 293, 1.6 267 / 244.)
+    template <typename T>
+    __device__ __forceinline__ void settle(const TreeDev<T>& tr, const RayState<T>& r, bool active) {
+        if (!words || tr.walk_marked) return;
+        T apart = T(0);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T at = active ? fma_(r.t, r.d[i], r.o[i]) : T(0);
+            const T by = at - neighbour(at);
+            apart = fma_(by, by, apart);
+        }
+        const unsigned long long rays = __builtin_amdgcn_ballot_w64(active), odd = 0x5555555555555555ull;
+        const unsigned long long pairs = rays & ((rays >> 1 & odd) | (rays & odd) << 1);
+        const unsigned long long close = __builtin_amdgcn_ballot_w64(apart * (T)tr.capacity < T(0.5)) & pairs;
+        if (2 * __popcll(close) > __popcll(pairs)) {
+            words = false;
+            entries = __builtin_amdgcn_make_buffer_rsrc((void*)tr.child, 0, (last_cell + 1u) << 2, 0x00020000);
+        }
+    }
+    // the value of the lane beside, of each pair
+    static __device__ __forceinline__ float neighbour(float v) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+    }
     __device__ __forceinline__ int32_t read(uint32_t at) const { return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(entries, (int)at, 0, 0); }
     __device__ __forceinline__ uint32_t cell(uint32_t number) const { return min(number, last_cell); }
 };
@@ -1312,7 +1341,7 @@ __global__ __launch_bounds__(kMarchThreads, kNoted && P::kForwardRows && P::kBas
     int64_t shared_next = 0, shared_end = 0;   // the wavefront's stock of chunks for notes (uniform)
     OctreeCursor cur;
     cur.reset(lds.lane_path(lane));
-    const ChildTable child(tr);
+    ChildTable child(tr);
 
     // takes ray `item` into this lane: a miss is answered at once, a hit becomes the lane's ray
     auto start = [&](int64_t item) {
@@ -1332,7 +1361,7 @@ __global__ __launch_bounds__(kMarchThreads, kNoted && P::kForwardRows && P::kBas
             }
             acc[0] = acc[1] = acc[2] = 0.0f;
             light = 1.0f;
-            cur.begin(r);
+            if constexpr (kRefill) cur.begin(r);
             active = true;
             if constexpr (kNoted) {
                 painted = out == nullptr;   // no picture asked for: nothing to compose
@@ -1350,6 +1379,8 @@ __global__ __launch_bounds__(kMarchThreads, kNoted && P::kForwardRows && P::kBas
     };
     if constexpr (!kRefill) {
         if (next + lane < end) start(next + lane);
+        child.settle(tr, r, active);
+        if (active) cur.begin(r);
     }
 
     while (true) {
@@ -2109,7 +2140,8 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         // ---- the walk: one leaf per live lane and turn, into the ring
         OctreeCursor cur;
         cur.reset(box.path + lane);
-        const ChildTable child(tr);
+        ChildTable child(tr);
+        child.settle(tr, r, active);
         if (active) cur.begin(r);
         // (counts of places in bytes of the ring)
         constexpr uint32_t kPlace = kMarchThreads * 8, kPlaces = kRing * kPlace;

@@ -143,6 +143,7 @@ TreeDev<T> make_tree(const SvoxTreeSpec* t) {
     d.scaling = (const T*)t->scaling;
     d.weight_accum = (T*)t->weight_accum;
     d.walk = nullptr;
+    d.walk_marked = false;
     d.capacity = t->capacity;
     d.N = t->N;
     d.K = t->data_dim;
@@ -547,6 +548,7 @@ bool marks_decide(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float 
 TreeDev<float> march_tree(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, float need_thresh = 0.0f) {
     TreeDev<float> d = make_tree<float>(tree);
     if (marks_apply(tree, opt, need_thresh)) (has_walk_table(tree) ? d.walk : d.child) = tree->child_marks;
+    d.walk_marked = d.walk && !marks_none(tree);
     return d;
 }
 

@@ -35,6 +35,7 @@ struct TreeDev {
     const T* scaling;  // may be null: one
     T* weight_accum;
     const int32_t* walk;   // a walk table of the octree (kWalkNodeBits), or null
+    bool walk_marked;      // ... made from marks
     int64_t capacity;
     int32_t N;
     int32_t K;

@@ -255,14 +255,16 @@ def ref_colour(gpu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kernel", [4, 8, 32 | 24 << 8])
 @pytest.mark.parametrize("thresh,marked", [(1e-2, False), (1e-2, True), (0.0, True)])
-def test_pictures_on_a_walk_table(gpu, oracle_mod, kernel, thresh, marked):
+@pytest.mark.parametrize("fx", [90.0, 700.0, 4000.0])
+def test_pictures_on_a_walk_table(gpu, oracle_mod, kernel, thresh, marked, fx):
+    """From afar, and from where some tiles' rays, or all, run so close together that they walk on the child table."""
     tree = synth.shell_tree(depth=7, n_spheres=6, data_format="SH9", seed=2)
     dev = on_gpu(tree, gpu)
     poses = torch.stack(synth.orbit_poses(2, seed=1, radius=2.5)).contiguous().to(gpu)
     opt = options(tree, step_size=1e-3, sigma_thresh=thresh)
     spec = dev._spec()
     cam = C.CameraSpec()
-    cam.c2w, cam.fx, cam.fy, cam.width, cam.height = poses, 90.0, 90.0, 61, 45
+    cam.c2w, cam.fx, cam.fy, cam.width, cam.height = poses, fx, fx, 61, 45
     want = C.volume_render_images(spec, cam, opt)
     if marked:
         spec.child_marks, spec.child_marks_thresh = C.mark_empty_leaves(spec, thresh, False), thresh
