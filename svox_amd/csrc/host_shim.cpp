@@ -328,8 +328,13 @@ void check_shaped(const Tensor& x, const char* name, at::ScalarType dt, at::IntA
 }
 
 // The walk table of a call of n rays, where one pays and there is memory for it: it goes with what is returned.  (every_positive_leaf: svox_walk_table)
-Tensor attach_walk(Tree& t, const SvoxRenderOptions& c, int64_t n_rays, bool image, bool every_positive_leaf, void* stream) {
+// Marks leave the march no way back to the child table where the rays of a picture run close together, as one pose's do from close up: on trees of few
+// nodes such a picture is marched on its marks.  (128^3 shell, RGBA and SH9, 800x800, marks / walk table: from afar 118, 182 / 109, 172 us, closer 123, 167 / 127,
+// 164, 264, 323 / 305, 344, 417, 491 / 486, 539; eight poses of 400x400, from afar and closer, 149, 192, 290, 345 / 141, 186, 316, 352.)
+Tensor attach_walk(Tree& t, const SvoxRenderOptions& c, int64_t n_rays, int64_t n_images, bool every_positive_leaf, void* stream) {
     Tensor table;
+    const bool image = n_images > 0;
+    if (n_images == 1 && t.spec.child_marks && t.spec.capacity < 65536) return table;
     const int64_t bytes = lib.svox_walk_table_bytes(&t.spec, &c, n_rays, image, every_positive_leaf);
     if (bytes <= 0) return table;
     try {
@@ -408,7 +413,7 @@ Tensor volume_render(py::handle tree, py::handle rays, py::handle opt, const py:
     const Unlocked unlocked;
     Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, r.spec.n_rays, false, false, on.stream);
+    const Tensor walk = attach_walk(t, c, r.spec.n_rays, 0, false, on.stream);
     status(lib.svox_volume_render(&t.spec, &r.spec, &c, out.data_ptr(), on.stream), "volume_render");
     return out;
 }
@@ -421,7 +426,7 @@ Tensor volume_render_images(py::handle tree, py::handle cam, py::handle opt, boo
     const Unlocked unlocked;
     Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, k.rays(), true, false, on.stream);
+    const Tensor walk = attach_walk(t, c, k.rays(), k.n, false, on.stream);
     status(lib.svox_volume_render_images(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), on.stream), "volume_render_images");
     return out;
 }
@@ -439,7 +444,7 @@ Tensor volume_render_noted(py::handle tree, py::handle rays, py::handle opt, con
     const Unlocked unlocked;
     Tensor out = like(r.origins, {r.spec.n_rays, out_dim(t, c)});
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, r.spec.n_rays, false, ws.at != nullptr, on.stream);
+    const Tensor walk = attach_walk(t, c, r.spec.n_rays, 0, ws.at != nullptr, on.stream);
     status(lib.svox_volume_render_noted(&t.spec, &r.spec, &c, out.data_ptr(), ws.at, ws.bytes, on.stream), "volume_render_noted");
     return out;
 }
@@ -454,7 +459,7 @@ Tensor volume_render_images_noted(py::handle tree, py::handle cam, py::handle op
     const Unlocked unlocked;
     Tensor out = like(t.data, k.shape(out_dim(t, c)));
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, k.rays(), true, ws.at != nullptr, on.stream);
+    const Tensor walk = attach_walk(t, c, k.rays(), k.n, ws.at != nullptr, on.stream);
     status(lib.svox_volume_render_images_noted(&t.spec, &k.spec, k.n, k.stride, &c, out.data_ptr(), ws.at, ws.bytes, on.stream),
            "volume_render_images_noted");
     return out;
@@ -473,7 +478,7 @@ Tensor volume_render_backward(py::handle tree, py::handle rays, py::handle opt, 
     const Unlocked unlocked;
     Tensor grad = like_data(t);
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, noted ? 0 : r.spec.n_rays, false, true, on.stream);
+    const Tensor walk = attach_walk(t, c, noted ? 0 : r.spec.n_rays, 0, true, on.stream);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
     if (noted)
@@ -500,7 +505,7 @@ Tensor volume_render_images_backward(py::handle tree, py::handle cam, py::handle
     const Unlocked unlocked;
     Tensor grad = like_data(t);
     const On on(t.data);
-    const Tensor walk = attach_walk(t, c, noted ? 0 : k.rays(), true, true, on.stream);
+    const Tensor walk = attach_walk(t, c, noted ? 0 : k.rays(), k.n, true, on.stream);
     SvoxNotesExtras extras{};
     extras.report = (int64_t*)report;
     if (noted)
@@ -538,7 +543,7 @@ py::tuple se_grad(py::handle tree, py::handle rays_or_cam, py::handle opt, const
         grad = like_data(t);
         hess = like_data(t);
         const On on(t.data);
-        const Tensor walk = attach_walk(t, c, image ? k.rays() : r.spec.n_rays, image, true, on.stream);
+        const Tensor walk = attach_walk(t, c, image ? k.rays() : r.spec.n_rays, image ? k.n : 0, true, on.stream);
         if (image)
             status(lib.svox_se_grad_image_ws(&t.spec, &k.spec, &c, ref.data_ptr(), result.data_ptr(), grad.data_ptr(),
                                              hess.data_ptr(), ws.at, ws.bytes, on.stream),

@@ -78,6 +78,22 @@ def test_a_child_table_that_does_not_begin_at_16_bytes(gpu):
 
 
 @pytest.mark.gpu
+def test_a_picture_of_a_small_tree_with_marks_is_marched_on_them(gpu):
+    """Allocations of a call: what it returns, and a walk table."""
+    tree = synth.shell_tree(depth=7, data_format="SH1", n_spheres=24, seed=0, device=gpu)
+    opt, spec = options(tree, step_size=1e-3, fast=True), tree._spec()
+    poses = torch.stack(synth.orbit_poses(2, seed=1, radius=4.0)).contiguous().to(gpu)
+    marks = C.mark_empty_leaves(spec, opt.sigma_thresh, False)
+    for n, marked, made in ((1, False, 2), (1, True, 1), (2, False, 2), (2, True, 2)):
+        spec.child_marks, spec.child_marks_thresh = (marks, opt.sigma_thresh) if marked else (None, 0.0)
+        cam = C.CameraSpec()
+        cam.c2w, cam.fx, cam.fy, cam.width, cam.height = poses[:n], 170.0, 170.0, 128, 128
+        before = torch.cuda.memory_stats(gpu)["allocation.all.allocated"]
+        C.volume_render_images(spec, cam, opt)
+        assert torch.cuda.memory_stats(gpu)["allocation.all.allocated"] - before == made, (n, marked)
+
+
+@pytest.mark.gpu
 def test_calls_without_memory_for_a_walk_table_do_without(gpu):
     """The table takes 6 MB, for which torch asks for 20; the picture fits 2."""
     tree = synth.shell_tree(depth=8, data_format="SH1", n_spheres=24, seed=0, device=gpu)
