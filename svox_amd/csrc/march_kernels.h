@@ -2171,7 +2171,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
 #pragma unroll
                 for (int k = 0; k < kWalkTurns; ++k) {
                     int32_t leaf = -1;
-                    float dt;
+                    float dt = 0.0f;
                     cur.turn_words(r, (r.t < r.tmax) & room(), child, step, leaf, dt);
                     hand_over((uint32_t)leaf < (uint32_t)kEmptyLeafBit, (uint32_t)leaf, dt);
                 }
@@ -2179,7 +2179,7 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
 #pragma unroll
                 for (int k = 0; k < kWalkTurns; ++k) {
                     int32_t leaf = -1;
-                    float dt;
+                    float dt = 0.0f;
                     cur.turn(r, (r.t < r.tmax) & room(), child, step, leaf, dt);
                     hand_over((uint32_t)leaf < (uint32_t)kEmptyLeafBit, (uint32_t)leaf, dt);
                 }
