@@ -468,7 +468,8 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     //   128^3 SH4         1312, 1515 / 500, 1020    1355, 1599 / 597, 1261    1534, 1854 / 876, 1877    2385, 2987 / 1329, 2858   3678, 4680 / (2535, 5498)
     //   shell 128^3 SH9   611, 812 / 292, 563       644, 911 / 360, 654       688, 1071 / 487, 911      869, 1554 / 754, 1396     1362, 2308 / (1359, 2464)
     //   shell 256^3 SH16  1182, 1617 / 503, 1019    1147, 1732 / 587, 1223    1336, 1993 / 777, 1649    1600, 2816 / 1161, 2553   2532, 4447 / (2011, 4364)
-    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.)  Full 128^3 grids lose 1 % of a gradient of
+    // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.  25 functions: 64^3, forward pass and gradient of 20 000 rays 203, 335 and 683,
+    // 1432, gradient of 40 960 1136, 2449, shell 256^3 of 65 536 1675.)  Full 128^3 grids lose 1 % of a gradient of
     // 40 960 rays; of 131 072 rays they would lose 17 % (half-empty trees would gain up to a third).
     const double cells = (double)tree->capacity * 8.0;
     const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
@@ -486,8 +487,8 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
         c.per_wave = short_lists ? 4 : 8;
         c.most = short_lists ? 4 : 3;
     } else {
-        // (of a 128^3 grid the lists hold the leaves of two rays, four in a pinch: 4 x 16 / 2 x 32, gradient 20 000 rays 787, 1542 / 683, 1336,
-        // forward pass 12 000 rays 229, 417 / 235, 364, 20 000 rays 336, 623 / 370, 565)
+        // (of a 128^3 grid the lists hold the leaves of two rays, four in a pinch: SH4, 4 x 16 / 2 x 32, gradient 12 000 rays 465, 910 / 342, 705, 20 000 650, 1302 / 503,
+        // 1056, forward pass 12 000 rays 207, 361 / 189, 292, 20 000 286, 523 / 290, 450: from fewer rays on than here)
         const bool two = grid && large && (gradient || n_rays > 16384);
         c.per_wave = large && n_rays <= 1280 ? 1 : n_rays <= 2560 || two ? 2 : 4;
         c.most = large ? 6 : 5;

@@ -222,7 +222,8 @@ def test_what_a_walk_table_holds(gpu, marks):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kernel", [4, 8, 2, 32 | 24 << 8, 64 | 1 << 8 | 2 << 16])
 def test_walks_on_a_walk_table_are_those_on_the_child_table(gpu, oracle_mod, kernel):
-    """One wavefront per tile, two, wavefronts that take new rays, rays in pieces, listed rays; with marks and without."""
+    """One wavefront per tile, two, wavefronts that take new rays, rays in pieces (which are given the table and leave it aside: they walk on the child
+    table alone), listed rays; with marks and without."""
     for name, tree in trees():
         if name == "one node":
             tree.data.data.copy_(torch.rand(tree.data.shape, generator=torch.Generator().manual_seed(3)) * 2)
