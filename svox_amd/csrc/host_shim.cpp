@@ -563,7 +563,8 @@ int notes_serve(py::handle tree, py::handle opt) {
 }
 
 // The bytes torch holds on a device that no tensor has: torch.cuda.memory_reserved - memory_allocated.  (Each of these makes a dictionary of
-// every figure the allocator keeps, 37 us: the training step of 50 001 rays of a 256^3 SH9 shell, whose kernels take 165 us, waited for its host, 213 us; now 162.)
+// every figure the allocator keeps, 37 us: the training step of 50 001 rays of a 256^3 SH9 shell, whose kernels take 165 us, waited for its host.  In turn with the step
+// as it was 206 / 178 and 210 / 189 us, where two runs of one side differ by 11 to 17 %.)
 int64_t cached_bytes(int device) {
     const auto stats = c10::hip::HIPCachingAllocator::getDeviceStats((c10::DeviceIndex)device);
     constexpr size_t all = (size_t)c10::CachingAllocator::StatType::AGGREGATE;

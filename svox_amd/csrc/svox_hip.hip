@@ -576,6 +576,10 @@ TreeDev<float> on_child_table(TreeDev<float> tr) {
 //   ... with notes, 128, 200, 400, 800, which wait for the colours as much as for the walk: shell 128^3  172, 203, 218, 259 / 157, 203, 219, 256;  256^3  258, 287,
 //     299, 347 / 212, 259, 295, 350;  512^3 SH16  341, 377, 400, 543 / 289, 329, 383, 530;  128^3 SH4  317, 317, 306, 429 / 320, 326, 311, 440
 //   32^3 and smaller (batches of 13 000 and 300 000, picture of 800): 68, 253, 81 / 63, 232, 99
+// Forward batches through shells most of whose rays miss lose by it from some 200 000 rays on, where making the table costs more than the few rays that hit
+// gain: 18 % of 200 000, 300 000, 500 000 and 1 Mi rays, with thresholds, without and with it 256^3 SH9 150, 163, 240, 214 / 152, 174, 248, 226, 512^3 SH9 215, 231, 342,
+// 321 / 220, 246, 362, 330, 256^3 RGBA 128, 153, 223, 194 / 142, 161, 234, 213.  They make one all the same, for those that all hit: 239, 373, 490, 881 / 218, 332, 442,
+// 753, 366, 625, 787, 1400 / 355, 578, 717, 1238, 203, 297, 388, 621 / 196, 273, 370, 589.  How many hit the launcher does not know.
 // The table a walk table is made from.  Its rows are read 16 bytes at a time (walk_table_kernel): one that begins elsewhere, which the march itself
 // reads entry by entry, serves no walk table.
 const int32_t* walk_source(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, bool every_positive_leaf) {
