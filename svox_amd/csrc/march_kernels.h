@@ -3185,8 +3185,11 @@ __global__ __launch_bounds__(kMarchThreads) void se_grad_generic_kernel(TreeDev<
 // (the reference's second march) and the density terms (its third).  Every term has the reference's
 // value; records are added cooperatively, one coalesced atomic instruction per record element and
 // output array, after summing the lanes whose rays sit in the same leaf.
+// (Room for five wavefronts on a SIMD with up to four functions, 2 to 6 registers fewer than the compiler takes by itself; lobes on wavefronts that take new rays: for
+// four.  285 000 rays that all hit, four wavefronts / five: 64^3 grid RGBA 3 282 / 2 602, SH4 4 197 / 3 263 us, 128^3 shell 1 440 / 1 176, 1 675 / 1 300, 512^3
+// 1 816 / 1 473, 2 326 / 1 801; 700 000, 128^3 shell, 9 lobes, three / four 2 527 / 2 357.)
 template <class P, class Source, bool kRefill>
-__global__ __launch_bounds__(kMarchThreads) void se_grad_kernel(TreeDev<float> tr, Source src, SvoxRenderOptions opt,
+__global__ __launch_bounds__(kMarchThreads, !kRefill && P::kBasis <= 4 ? 5 : P::kForwardRows && P::kBasis <= 9 ? 4 : 1) void se_grad_kernel(TreeDev<float> tr, Source src, SvoxRenderOptions opt,
                                                                 const float* __restrict__ color_ref,
                                                                 float* __restrict__ color_out,
                                                                 float* __restrict__ grad_data,

@@ -78,3 +78,10 @@ def test_wavefronts_that_take_notes_or_march_without(kernels, policy, notes, mar
         if policy.startswith("2"):
             for grad in ("false", "true"):
                 assert wavefronts(kernels[f"render_forward_kernel<OctreePolicy<{policy}>, {source}, false, {refill}, true, {grad}, false>"]) >= notes
+
+
+@pytest.mark.parametrize("policy,walks,takes_new_rays", [("0, 0", 20, 16), ("1, 1", 20, 16), ("1, 4", 18, 16), ("2, 1", 20, 16), ("2, 4", 18, 16), ("2, 9", 16, 16)])
+@pytest.mark.parametrize("source", ["BatchSource<float>", "ImageSource<float>"])
+def test_wavefronts_of_squared_errors_without_notes(kernels, policy, walks, takes_new_rays, source):
+    for refill, most in (("false", walks), ("true", takes_new_rays)):
+        assert wavefronts(kernels[f"se_grad_kernel<OctreePolicy<{policy}>, {source}, {refill}>"]) >= most
