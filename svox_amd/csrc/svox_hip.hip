@@ -440,7 +440,7 @@ int group_basis(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t 
 struct Cut {
     int per_wave = 0, most = 6;
 };
-Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
+Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient, bool image) {
     Cut c;
     if (g_debug_flags != 0) {
         const int forced = (g_debug_flags & 32) ? g_debug_flags >> 8 : 0;
@@ -471,12 +471,18 @@ Cut group_cut(const SvoxTreeSpec* tree, int64_t n_rays, bool gradient) {
     // (1 000 and 5 000 rays, pieces: 64^3 SH4 51, 54 and 68, 96, gradient step 123, 178 and 166, 329.  25 functions: 64^3, forward pass and gradient of 20 000 rays 203, 335 and 683,
     // 1432, gradient of 40 960 1136, 2449, shell 256^3 of 65 536 1675.)  Full 128^3 grids lose 1 % of a gradient of
     // 40 960 rays; of 131 072 rays they would lose 17 % (half-empty trees would gain up to a third).
+    // The rays that meet the cube lie together in a picture, and fill the lists of a few wavefronts, while a batch deals them out: with more than kFill pixels small trees have
+    // no gradient in pieces, and those of up to 32^3 leaves with fewer than nine functions no picture.  (Gradient of a picture from radius 1.5, 2.5 and 4, 150x150: 16^3 RGBA
+    // 59 / 68, 52 / 72, 46 / 60, SH9 133 / 122, 90 / 94, 79 / 75, 250x250: 94 / 142, 58 / 135, 51 / 105, 261 / 267, 124 / 191, 86 / 137; picture, 150x150: 32^3 RGBA 65 / 69,
+    // 60 / 77, 57 / 55, SH9 98 / 80, 86 / 83, 77 / 62.)  Larger trees lose at some distances and gain at others: 64^3 SH4, gradient, 200x200 459 / 353,
+    // 330 / 267, 307 / 189, 250x250 593 / 518, 349 / 414, 300 / 249, 128^3 1129 / 1139, 876 / 798, 769 / 403.
     const double cells = (double)tree->capacity * 8.0;
     const bool tiny = cells < 2048.0, small = cells < 16384.0, medium = cells < 131072.0, large = cells >= 1048576.0;
     const bool grid = like_complete_octree(tree);
     constexpr int64_t kFill = 20480;
     if (tiny && !(gradient && n_rays <= 2560)) return c;
-    const int64_t most_rays = gradient ? 65536 : small ? kFill : 26624;
+    const bool few = image && (gradient ? small : medium && tree->data_dim < 28);
+    const int64_t most_rays = few ? kFill : gradient ? 65536 : small ? kFill : 26624;
     if (n_rays > most_rays) return c;
     if (small) {
         const bool eight = n_rays <= 14336 || n_rays > kFill;
@@ -880,7 +886,7 @@ void launch_forward(const SvoxTreeSpec* tree, const Source& src, const SvoxRende
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            const Cut cut = group_cut(tree, items, false);
+            const Cut cut = group_cut(tree, items, false, is_image_source(src));
             if (cut.per_wave > 0)
                 launch_group_forward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt, (double*)out,
                                      cut.per_wave, cut.most);
@@ -1000,7 +1006,7 @@ void launch_backward(const SvoxTreeSpec* tree, const Source& src, const SvoxRend
     if constexpr (sizeof(T) == 8) {
         const int D = group_basis(tree, opt, items);
         if (D >= 0) {
-            const Cut cut = group_cut(tree, items, true);
+            const Cut cut = group_cut(tree, items, true, is_image_source(src));
             if (cut.per_wave > 0)
                 launch_group_backward(D, dim3(blocks_for(items, cut.per_wave)), stream, make_tree<double>(tree), src, *opt,
                                       (const double*)grad_out, (double*)grad_data, cut.per_wave, cut.most);

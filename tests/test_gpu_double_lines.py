@@ -38,3 +38,25 @@ def test_lines_and_lists_that_run_over(gpu, levels, n, split):
     assert torch.equal(got[0], want[0])
     # (up to n terms of a leaf in another order: n * 2^-53 of the sum of their sizes at most, which cancels to a hundredth of it)
     assert (got[1] - want[1]).abs().max() <= n * 1.2e-14 * want[1].abs().max()
+
+
+@pytest.mark.parametrize("levels,fmt", [(3, "RGBA"), (3, "SH9"), (4, "SH4"), (4, "SH9")])
+@pytest.mark.parametrize("size", [128, 144, 160, 176])
+def test_pictures_on_either_side(gpu, levels, fmt, size):
+    """Small trees have gradients of pictures in pieces up to 20 480 pixels, those of 32^3 leaves pictures of few functions up to as many and others up to 26 624."""
+    gen = torch.Generator(device=gpu).manual_seed(levels)
+    tree = svox.N3Tree(N=2, data_format=fmt, init_refine=levels, device=gpu, dtype=torch.float64)
+    tree.data.data.normal_(generator=gen)
+    tree.data.data[..., -1] = tree.data.data[..., -1].abs() * 0.1 + 0.01
+    opt, spec, cam = options(tree, step_size=1e-3), tree._spec(), C.CameraSpec()
+    cam.c2w = synth.orbit_poses(1, seed=3, radius=2.5)[0].to(gpu).double().contiguous()
+    cam.fx, cam.fy, cam.width, cam.height = size * 1.4, size * 1.4, size, size
+    go = torch.randn(size, size, 3, generator=gen, device=gpu, dtype=torch.float64)
+
+    def passes():
+        return C.volume_render_image(spec, cam, opt), C.volume_render_image_backward(spec, cam, opt, go)
+
+    want, got = run(1, passes), run(0, passes)
+    assert torch.equal(got[0], want[0])
+    # (as above)
+    assert (got[1] - want[1]).abs().max() <= size * size * 1.2e-14 * want[1].abs().max()
