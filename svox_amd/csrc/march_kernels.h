@@ -2158,12 +2158,13 @@ __global__ __launch_bounds__(kSplitThreads) void render_forward_split_kernel(Tre
         };
         static_assert(kPlaces << 18 == kRoundBit, "the bit of a count that says which round it is");
         // The walk is the longest chain of a tile: it goes first where wavefronts share a SIMD, on trees whose child rows lie beyond L2 for all batches, on others
-        // for batches of up to 147 000 rays without notes, and in normalised device coordinates.  Where many tiles run, rays of a picture or notes to write, it keeps the shading from its
+        // for batches of up to 147 000 rays without notes, in normalised device coordinates, and on trees of other branching factors, whose walk is the reference's.  Where many tiles run, rays of a picture or notes to write, it keeps the shading from its
         // turns, and every ring is full.  (us, walk first / as they come.  Batches, 100 000 rays: 128^3 shell SH9 165 / 174, 18 % hit 118 / 127, 32^3 SH9 94 / 101,
         // 190 000: 128^3 shell RGBA 264 / 215, SH9 266 / 259, 150 000: 512^3 shell SH9 403 / 425, 222 / 245; with notes, the gradient, 100 000: 128^3 shell SH9
         // 201 / 188, 150 000: 512^3 368 / 384.  Pictures of 800x800: 512^3 SH16 354 / 350, 64^3 RGBA from close up 424 / 352, 128^3 shell SH9 432 / 346, eight of 400x400 416 / 351.
-        // Pictures in normalised device coordinates, all of whose tiles are long, 504x378: blobs 128^3 SH16 93 / 98, 256^3 114 / 127, SH4 of 512^3 167 / 179, SH25 290 / 285.)
-        if (opt.ndc_width > 0 || (Source::kItemsAreSlots && (tr.capacity >= kBeyondL2 || (!kNoted && gridDim.x <= 2304u)))) __builtin_amdgcn_s_setprio(3);
+        // Pictures in normalised device coordinates, all of whose tiles are long, 504x378: blobs 128^3 SH16 93 / 98, 256^3 114 / 127, SH4 of 512^3 167 / 179, SH25 290 / 285.  N = 3, 81^3 SH9,
+        // 800x800 193 / 215, four of 400x400 298 / 370, training step of 60 000 rays 894 / 919.)
+        if (opt.ndc_width > 0 || !child.octree || (Source::kItemsAreSlots && (tr.capacity >= kBeyondL2 || (!kNoted && gridDim.x <= 2304u)))) __builtin_amdgcn_s_setprio(3);
         while (true) {
             // asked for here, looked at after the turns: not waited for.  (Four turns to a look: one wavefront alone 620 ns a leaf, with two turns and
             // looks at the rays that are over 770, with a look at everything in every turn 870.)
