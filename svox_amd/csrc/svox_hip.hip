@@ -565,6 +565,13 @@ TreeDev<float> on_child_table(TreeDev<float> tr) {
     return tr;
 }
 
+// The table a walk table is made from.  Its rows are read 16 bytes at a time (walk_table_kernel): one that begins elsewhere, which the march itself
+// reads entry by entry, serves no walk table.
+const int32_t* walk_source(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, bool every_positive_leaf) {
+    const int32_t* from = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh) ? tree->child_marks : tree->child;
+    return ((uintptr_t)from & 15u) == 0 ? from : nullptr;
+}
+
 // Whether a call makes a walk table (svox_walk_table) for its march.  Making it costs 4 us and 11 ps a node, and a march that starts on a
 // table no cache holds; a turn of the walk then waits for one read instead of two, or for none, though in three turns of ten it only descends.  So it pays
 // where rays are many and apart.  us, whole calls without and with it, forward and with notes (SH9, SH4 on 128^3 and 512^3):
@@ -586,12 +593,6 @@ TreeDev<float> on_child_table(TreeDev<float> tr) {
 // gain: 18 % of 200 000, 300 000, 500 000 and 1 Mi rays, with thresholds, without and with it 256^3 SH9 150, 163, 240, 214 / 152, 174, 248, 226, 512^3 SH9 215, 231, 342,
 // 321 / 220, 246, 362, 330, 256^3 RGBA 128, 153, 223, 194 / 142, 161, 234, 213.  They make one all the same, for those that all hit: 239, 373, 490, 881 / 218, 332, 442,
 // 753, 366, 625, 787, 1400 / 355, 578, 717, 1238, 203, 297, 388, 621 / 196, 273, 370, 589.  How many hit the launcher does not know.
-// The table a walk table is made from.  Its rows are read 16 bytes at a time (walk_table_kernel): one that begins elsewhere, which the march itself
-// reads entry by entry, serves no walk table.
-const int32_t* walk_source(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, bool every_positive_leaf) {
-    const int32_t* from = marks_apply(tree, opt, every_positive_leaf ? 0.0f : opt->sigma_thresh) ? tree->child_marks : tree->child;
-    return ((uintptr_t)from & 15u) == 0 ? from : nullptr;
-}
 bool walk_table_pays(const SvoxTreeSpec* tree, const SvoxRenderOptions* opt, int64_t n_rays, bool image, bool every_positive_leaf) {
     if (tree->N != 2 || tree->capacity > (int64_t)kWalkNodes || fast_basis(tree, opt) < 0) return false;
     if (has_walk_table(tree) || !walk_source(tree, opt, every_positive_leaf)) return false;
