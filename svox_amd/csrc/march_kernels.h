@@ -1307,6 +1307,10 @@ __global__ __launch_bounds__(kMarchThreads, kNoted && P::kForwardRows && P::kBas
     __shared__ MarchShared<D, P::kForwardRows> lds;
     auto& sh = lds.sh;
     __shared__ float sh_sigma[kAllShaded ? kQueue * kMarchThreads : 1];
+    // Wavefronts that take new rays, with 16 functions: four to a SIMD, not the five that 94 registers leave room for.  A batch of 1 Mi rays is 4 096 of them, four to
+    // a SIMD, and where five find room some SIMDs have five and others three: 1 Mi rays drawn from pictures of a 512^3 SH16 shell 395 us with room for five, 367 for
+    // four.  (launch_bounds has a say in the least only.)
+    if constexpr (kRefill && !kNoted && P::kFormat == SVOX_FORMAT_SH && P::kBasis == 16) asm volatile("" ::: "v103");
     if constexpr (kNoted) {
         if constexpr (Source::kGated) {
             if (!ws.chosen()) return;

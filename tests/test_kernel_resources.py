@@ -85,3 +85,9 @@ def test_wavefronts_that_take_notes_or_march_without(kernels, policy, notes, mar
 def test_wavefronts_of_squared_errors_without_notes(kernels, policy, walks, takes_new_rays, source):
     for refill, most in (("false", walks), ("true", takes_new_rays)):
         assert wavefronts(kernels[f"se_grad_kernel<OctreePolicy<{policy}>, {source}, {refill}>"]) >= most
+
+
+# (render_forward_kernel: four to a SIMD, as many as a batch of 1 Mi rays has, and not a fifth)
+def test_wavefronts_that_take_new_rays_are_four_to_a_simd(kernels):
+    kernel = kernels["render_forward_kernel<OctreePolicy<1, 16>, BatchSource<float>, false, true, false, false, false>"]
+    assert SIMDS * (REGISTERS // (-(-kernel[1] // 8) * 8)) == 16
